@@ -497,6 +497,63 @@ int spr_energy_exchange(int64_t T, int64_t P, int64_t D, int64_t B,
                         void *workspace, int64_t workspace_bytes,
                         void *stream);
 
+/* An exchange plan of one scene, as the plan builders above fill it, for
+ * spr_exchange_orders and spr_exchange_sum.  kind SPR_PLAN_PAIRS: row_ptr, src, lag, dir, coef
+ * (spr_plan_from_geometry / _from_dense).  SPR_PLAN_GROUPED: row_ptr,
+ * grp_ptr, grp_key, rowid, lag, scal, rtab (spr_plan_grouped_fill).
+ * SPR_PLAN_DS: the same with dscal, rtab not read (spr_plan_ds_fill).  With
+ * M > 0 the last two gather on destination tiles of tile_rows rows
+ * (spr_plan_tile_order / _fill / _span): tptr, gstart [tile_slots], mlag,
+ * mw, and mspan for 16 rows (tile_r 8 or 16 bins per lane) or mrow for 4
+ * and 8; diffuse + specular tiles have 16 rows and gdiff, mdw besides.
+ * Unused pointers are NULL. */
+#define SPR_PLAN_PAIRS 0
+#define SPR_PLAN_GROUPED 1
+#define SPR_PLAN_DS 2
+
+typedef struct spr_exchange_plan {
+  int64_t kind, P, D, B, Vd;
+  int64_t tile_slots, tile_rows, tile_r, M;
+  const int64_t *row_ptr;
+  const int32_t *src, *lag, *dir;
+  const double *coef;
+  const int64_t *grp_ptr;
+  const int32_t *grp_key, *rowid;
+  const double *scal, *dscal, *rtab;
+  const int64_t *tptr, *gstart, *gdiff;
+  const int32_t *mspan, *mrow, *mlag;
+  const double *mw, *mdw;
+} spr_exchange_plan;
+
+/* out[P,D,B,T] (float32) = the sum of orders 0..K (RadiosityFast.py:
+ * 1037-1145; the histogram energy_exchange_etc): every bin of out is
+ * written.  Each order is summed in float64 and rounded to float32; the
+ * total is kept as a compensated pair and rounded once, the bits of
+ * spr_exchange_init, K orders of gather and spread with the total updated
+ * every other order (per-pair plans: every order) and spr_exchange_finalize.
+ * e0dir [P,D,B] and d0 [P] as for spr_exchange_init; lo, prev, cur
+ * [P,D,B,T] and gsum [groups,B,T] (grouped and diffuse + specular plans)
+ * are workspaces, not read, needed for K >= 1; n0 [P] (int32) receives each
+ * patch's source bin.  Bit 0 of *err_flag is set where a source delay lies
+ * outside the histogram (the reference raises IndexError); such a patch
+ * injects nothing.  Enqueues kernels only: no allocation, no
+ * synchronisation, safe to capture. */
+int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T, int64_t K,
+                        const double *e0dir, const double *d0, double c,
+                        double dt, float *out, float *lo, float *prev,
+                        float *cur, float *gsum, int32_t *n0, int *err_flag,
+                        void *stream);
+
+/* The same sum by the recurrence x_{k+1} = x_0 + A x_k, x_0 the injected
+ * energy: two state buffers (out and tmp [P,D,B,T]) and no total.  Each x_k
+ * is summed in float64 and rounded to float32 once, so the error against
+ * float64 is that of spr_exchange_orders, but not every last bit agrees
+ * with it.  Other arguments as there. */
+int spr_exchange_sum(const spr_exchange_plan *plan, int64_t T, int64_t K,
+                     const double *e0dir, const double *d0, double c,
+                     double dt, float *out, float *tmp, float *gsum,
+                     int32_t *n0, int *err_flag, void *stream);
+
 /* hkey[e] (uint64, Vd entries) = hash of entry e's F~ row fft[src[e], j]
  * (destination j of row_ptr's row holding e) with every band divided by its
  * first element of largest magnitude and rounded to multiples of 2^-30:

@@ -151,6 +151,10 @@ SYMBOLS = {
     "spr_energy_exchange": (_int, [_i64, _i64, _i64, _i64, _vp, _vp, _vp,
                                    _vp, _vp, _dbl, _dbl, _i64, _i64, _vp,
                                    _vp, _vp, _i64, _vp]),
+    "spr_exchange_orders": (_int, [_vp, _i64, _i64, _vp, _vp, _dbl, _dbl,
+                                   _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "spr_exchange_sum": (_int, [_vp, _i64, _i64, _vp, _vp, _dbl, _dbl, _vp,
+                                _vp, _vp, _vp, _vp, _vp]),
     "spr_plan_dense_hash": (_int, [_i64, _i64, _i64, _vp, _vp, _vp, _vp,
                                    _vp]),
     "spr_energy_exchange_groups": (_i64, []),
@@ -161,6 +165,19 @@ SYMBOLS = {
     "spr_collect": (_int, [_i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp,
                            _vp, _vp, _dbl, _dbl, _int, _vp, _vp]),
 }
+
+
+class ExchangePlanStruct(ctypes.Structure):
+    """``spr_exchange_plan`` (sparrow_hip.h)."""
+
+    PAIRS, GROUPED, DS = 0, 1, 2
+    SIZES = ("kind", "P", "D", "B", "Vd", "tile_slots", "tile_rows",
+             "tile_r", "M")
+    ARRAYS = ("row_ptr", "src", "lag", "dir", "coef", "grp_ptr", "grp_key",
+              "rowid", "scal", "dscal", "rtab", "tptr", "gstart", "gdiff",
+              "mspan", "mrow", "mlag", "mw", "mdw")
+    _fields_ = [(n, _i64) for n in SIZES] + [(n, _vp) for n in ARRAYS]
+
 
 _lib = None
 _lock = threading.Lock()

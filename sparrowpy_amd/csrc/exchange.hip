@@ -170,10 +170,11 @@ __global__ void init_kernel(int64_t P, int64_t D, int64_t B, int64_t T,
 // the prev histogram row `row(e)` shifted by the entry's delay.  Metadata
 // loads are unconditional (the index is clamped into the row) so they can
 // be issued together; entries past the row end or whose delay reaches
-// beyond the tile are inactive and load nothing.
+// beyond the tile are inactive and load nothing.  Bins of prev from Tp on
+// count as 0.
 template <int R, int BS, int C, typename RowFn>
 __device__ __forceinline__ void gather_chunk(
-    int64_t e, int64_t e_end, int B, int T, int b, int t0, int t_end,
+    int64_t e, int64_t e_end, int B, int T, int Tp, int b, int t0, int t_end,
     RowFn row_of, const int32_t *__restrict__ lag,
     const float *__restrict__ prev, float (&buf)[C][R], int (&n)[C],
     bool (&act)[C]) {
@@ -194,34 +195,71 @@ __device__ __forceinline__ void gather_chunk(
     for (int r = 0; r < R; ++r) {
       const int t = t0 + (int)threadIdx.x + BS * r;
       const int ts = t - nc;
-      buf[c][r] = (act[c] && t < T && ts >= 0) ? s[ts] : 0.f;
+      buf[c][r] = (act[c] && ts >= 0 && ts < Tp) ? s[ts] : 0.f;
     }
   }
 }
 
-// Write one order's tile (cur) and add it to the compensated total
-// (tot_hi + tot_lo, updated in float64 and split back into two floats).
+// Add one value of an order to the compensated total (tot_hi + tot_lo,
+// updated in float64 and split back into two floats); the last order leaves
+// the rounded total only.
+__device__ __forceinline__ void add_to_total(double a, int64_t idx, int t,
+                                             const OrderSpan &sp,
+                                             float *__restrict__ cur,
+                                             float *__restrict__ tot_hi,
+                                             float *__restrict__ tot_lo) {
+  const double old =
+      t < sp.Tv ? (double)tot_hi[idx] + (double)tot_lo[idx] : 0.0;
+  const double sum = old + a;
+  const float h = (float)sum;
+  tot_hi[idx] = h;
+  if (sp.last) return;
+  cur[idx] = (float)a;
+  tot_lo[idx] = (float)(sum - (double)h);
+}
+
+// Write one order's tile (cur) and add it to the total.
 template <int DP, int R, int BS>
 __device__ __forceinline__ void store_tile(const double (&acc)[DP][R], int D,
-                                           int B, int T, int64_t j, int b,
-                                           int t0, float *__restrict__ cur,
+                                           int B, int T, const OrderSpan &sp,
+                                           int64_t j, int b, int t0,
+                                           float *__restrict__ cur,
                                            float *__restrict__ tot_hi,
                                            float *__restrict__ tot_lo) {
   const int64_t dstride = (int64_t)B * T;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int t = t0 + (int)threadIdx.x + BS * r;
-    if (t >= T) continue;
+    if (t >= sp.Tc) continue;
 #pragma unroll
     for (int d = 0; d < DP; ++d) {
       if (d >= D) continue;  // padded direction (compile-time d)
       const int64_t idx = (j * D + d) * dstride + (int64_t)b * T + t;
-      const double a = acc[d][r];
-      cur[idx] = (float)a;
-      const double sum = ((double)tot_hi[idx] + (double)tot_lo[idx]) + a;
-      const float h = (float)sum;
-      tot_hi[idx] = h;
-      tot_lo[idx] = (float)(sum - (double)h);
+      add_to_total(acc[d][r], idx, t, sp, cur, tot_hi, tot_lo);
+    }
+  }
+}
+
+// One tile of an order of the running sum: cur = acc on bins [0, Tc), plus
+// the injected energy in each row's source bin.
+template <int DP, int R, int BS>
+__device__ __forceinline__ void store_sum_tile(const double (&acc)[DP][R],
+                                               int D, int B, int T, int Tc,
+                                               int64_t j, int b, int t0,
+                                               const Injection &inj,
+                                               float *__restrict__ cur) {
+  const int64_t dstride = (int64_t)B * T;
+  const int nj = inj.n0[j];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int t = t0 + (int)threadIdx.x + BS * r;
+    if (t >= Tc) continue;
+#pragma unroll
+    for (int d = 0; d < DP; ++d) {
+      if (d >= D) continue;
+      double a = acc[d][r];
+      if (t == nj) a += inj.e0[(j * D + d) * B + b];
+      cur[(j * D + d) * dstride + (int64_t)b * T + t] = (float)a;
     }
   }
 }
@@ -233,14 +271,15 @@ __device__ __forceinline__ void store_tile(const double (&acc)[DP][R], int D,
 // for L2 every time) come through LDS: the workgroup loads the rows of the
 // next NBE entries with coalesced vector loads while the current NBE are
 // summed, and every wave reads the current rows by broadcast.
-template <int DP, int R, int BS, int C>
+// SUM: an order of the running sum (no total, the injection added).
+template <int DP, int R, int BS, int C, bool SUM>
 __global__ __launch_bounds__(BS) void exchange_step_kernel(
-    int D, int B, int T, int n_tblk, int64_t nblocks,
+    int D, int B, int T, OrderSpan sp, int n_tblk, int64_t nblocks,
     const int64_t *__restrict__ row_ptr, const int32_t *__restrict__ src,
     const int32_t *__restrict__ lag, const int32_t *__restrict__ dir,
     const double *__restrict__ coef, const float *__restrict__ prev,
     float *__restrict__ cur, float *__restrict__ tot_hi,
-    float *__restrict__ tot_lo) {
+    float *__restrict__ tot_lo, Injection inj) {
   constexpr int NBE = 16;                      // entries per row batch
   constexpr int NW = NBE * DP;                 // doubles per batch
   constexpr int NLD = (NW + BS - 1) / BS;      // of them per thread
@@ -252,7 +291,7 @@ __global__ __launch_bounds__(BS) void exchange_step_kernel(
   const int b = (int)(jb % B);
   const int64_t j = jb / B;
   const int t0 = tb * (BS * R);
-  const int t_end = min(T, t0 + BS * R);
+  const int t_end = min(sp.Tc, t0 + BS * R);
 
   double acc[DP][R];
 #pragma unroll
@@ -290,7 +329,7 @@ __global__ __launch_bounds__(BS) void exchange_step_kernel(
     float buf[C][R];
     int n[C];
     bool act[C];
-    gather_chunk<R, BS, C>(e_begin, e_end, B, T, b, t0, t_end, row_of, lag,
+    gather_chunk<R, BS, C>(e_begin, e_end, B, T, sp.Tp, b, t0, t_end, row_of, lag,
                            prev, buf, n, act);
     int cb = 0;
     for (int64_t eb = e_begin; eb < e_end; eb += NBE) {
@@ -303,7 +342,7 @@ __global__ __launch_bounds__(BS) void exchange_step_kernel(
         float nbuf[C][R];
         int nn[C];
         bool nact[C];
-        gather_chunk<R, BS, C>(e + C, e_end, B, T, b, t0, t_end, row_of,
+        gather_chunk<R, BS, C>(e + C, e_end, B, T, sp.Tp, b, t0, t_end, row_of,
                                lag, prev, nbuf, nn, nact);
 #pragma unroll
         for (int c = 0; c < C; ++c) {
@@ -334,7 +373,10 @@ __global__ __launch_bounds__(BS) void exchange_step_kernel(
       cb ^= 1;
     }
   }
-  store_tile<DP, R, BS>(acc, D, B, T, j, b, t0, cur, tot_hi, tot_lo);
+  if constexpr (SUM)
+    store_sum_tile<DP, R, BS>(acc, D, B, T, sp.Tc, j, b, t0, inj, cur);
+  else
+    store_tile<DP, R, BS>(acc, D, B, T, sp, j, b, t0, cur, tot_hi, tot_lo);
 }
 
 // Per-pair plan on the matrix cores (DP >= 16).  For destination j and band
@@ -353,14 +395,15 @@ __global__ __launch_bounds__(BS) void exchange_step_kernel(
 // vector kernel's (float64 rounding).
 typedef double mfma_d4 __attribute__((ext_vector_type(4)));
 
-template <int DP, int NT>
+// SUM: an order of the running sum (no total, the injection added).
+template <int DP, int NT, bool SUM>
 __global__ __launch_bounds__(256) void exchange_mfma_kernel(
-    int D, int B, int T, int n_tblk, int64_t nblocks,
+    int D, int B, int T, OrderSpan sp, int n_tblk, int64_t nblocks,
     const int64_t *__restrict__ row_ptr, const int32_t *__restrict__ src,
     const int32_t *__restrict__ lag, const int32_t *__restrict__ dir,
     const double *__restrict__ coef, const float *__restrict__ prev,
     float *__restrict__ cur, float *__restrict__ tot_hi,
-    float *__restrict__ tot_lo) {
+    float *__restrict__ tot_lo, Injection inj) {
   constexpr int MT = DP / 16;
   constexpr int WBINS = 16 * NT;  // bins per wave
   static_assert(MT * NT == 8, "eight accumulator tiles per wave");
@@ -419,7 +462,7 @@ __global__ __launch_bounds__(256) void exchange_mfma_kernel(
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       const int ts = tw + nt * 16 + cc - m.lag;
-      o.ok[nt] = m.in && (unsigned)ts < (unsigned)T;
+      o.ok[nt] = m.in && (unsigned)ts < (unsigned)sp.Tp;
       o.x[nt] = row[o.ok[nt] ? ts : 0];
     }
     return o;
@@ -455,7 +498,8 @@ __global__ __launch_bounds__(256) void exchange_mfma_kernel(
     }
   }
 
-  // cur and the compensated total (as store_tile)
+  // cur and the compensated total (as store_tile), or the running sum
+  const int nj = SUM ? inj.n0[j] : 0;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -464,14 +508,15 @@ __global__ __launch_bounds__(256) void exchange_mfma_kernel(
       for (int r = 0; r < 4; ++r) {
         const int d = mt * 16 + kk + 4 * r;
         const int t = tw + nt * 16 + cc;
-        if (d >= D || t >= T) continue;
+        if (d >= D || t >= sp.Tc) continue;
         const int64_t idx = (j * D + d) * BT + (int64_t)b * T + t;
-        const double v = acc[mt][nt][r];
-        cur[idx] = (float)v;
-        const double sum = ((double)tot_hi[idx] + (double)tot_lo[idx]) + v;
-        const float h = (float)sum;
-        tot_hi[idx] = h;
-        tot_lo[idx] = (float)(sum - (double)h);
+        double v = acc[mt][nt][r];
+        if (SUM) {
+          if (t == nj) v += inj.e0[(j * D + d) * B + b];
+          cur[idx] = (float)v;
+        } else {
+          add_to_total(v, idx, t, sp, cur, tot_hi, tot_lo);
+        }
       }
 }
 
@@ -514,7 +559,7 @@ __device__ __forceinline__ EntryMeta load_meta(
 
 template <int R, int BS, int C>
 __global__ __launch_bounds__(BS) void group_gather_kernel(
-    int B, int T, int n_tblk, int64_t nblocks, int64_t Vd,
+    int B, int T, int Tp, int n_tblk, int64_t nblocks, int64_t Vd,
     const int64_t *__restrict__ row_ptr, const int64_t *__restrict__ grp_ptr,
     const int32_t *__restrict__ rowid, const int32_t *__restrict__ lag,
     const double *__restrict__ scal, const float *__restrict__ prev,
@@ -530,7 +575,8 @@ __global__ __launch_bounds__(BS) void group_gather_kernel(
   const int64_t e_begin = row_ptr[j], e_end = row_ptr[j + 1];
   if (e_end <= e_begin) return;
   const double *w = scal + (int64_t)b * Vd;
-  const uint32_t row_bytes = (uint32_t)T * 4u;
+  const uint32_t row_bytes = (uint32_t)T * 4u;   // of a group's sums
+  const uint32_t src_bytes = (uint32_t)Tp * 4u;  // of a source row
   const int tl = t0 + (int)threadIdx.x;
   int64_t g = grp_ptr[j];
 
@@ -544,7 +590,7 @@ __global__ __launch_bounds__(BS) void group_gather_kernel(
       const int n = min(lk & kLagMask, T);
       const float *src = prev + ((int64_t)rk * B + b) * T;
       const __amdgpu_buffer_rsrc_t rs =
-          make_rsrc(src, n < t_end ? row_bytes : 0u);
+          make_rsrc(src, n < t_end ? src_bytes : 0u);
 #pragma unroll
       for (int r = 0; r < R; ++r)
         v[c][r] = buffer_load(rs, bin_offset(tl + BS * r - n));
@@ -603,7 +649,7 @@ __global__ __launch_bounds__(BS) void group_gather_kernel(
 // register file.
 template <int R, int BS, int C>
 __global__ __launch_bounds__(BS) void ds_gather_kernel(
-    int B, int T, int n_tblk, int64_t nblocks, int64_t Vd,
+    int B, int T, int Tp, int n_tblk, int64_t nblocks, int64_t Vd,
     const int64_t *__restrict__ row_ptr, const int64_t *__restrict__ grp_ptr,
     const int32_t *__restrict__ rowid, const int32_t *__restrict__ lag,
     const double *__restrict__ scal, const double *__restrict__ dscal,
@@ -619,6 +665,7 @@ __global__ __launch_bounds__(BS) void ds_gather_kernel(
   const double *w = scal + (int64_t)b * Vd;
   const double *w2 = dscal + (int64_t)b * Vd;
   const uint32_t row_bytes = (uint32_t)T * 4u;
+  const uint32_t src_bytes = (uint32_t)Tp * 4u;
   const int tl = t0 + (int)threadIdx.x;
   int64_t g = grp_ptr[j];
 
@@ -630,7 +677,7 @@ __global__ __launch_bounds__(BS) void ds_gather_kernel(
       const int n = min(lag[ee] & kLagMask, T);
       const float *src = prev + ((int64_t)rowid[ee] * B + b) * T;
       const __amdgpu_buffer_rsrc_t rs =
-          make_rsrc(src, in_row && n < t_end ? row_bytes : 0u);
+          make_rsrc(src, in_row && n < t_end ? src_bytes : 0u);
 #pragma unroll
       for (int r = 0; r < R; ++r)
         v[c][r] = buffer_load(rs, bin_offset(tl + BS * r - n));
@@ -701,14 +748,16 @@ struct SpreadShape {
 };
 
 // MODE: 0 writes cur only; 1 adds cur to the total; 2 adds prev + cur (two
-// orders at once, so the total is read and written every other order).
+// orders at once, so the total is read and written every other order);
+// kSumMode writes an order of the running sum (the injection added).
+constexpr int kSumMode = 3;
 template <int DP, int MODE>
 __global__ __launch_bounds__(256) void group_spread_kernel(
-    int D, int B, int T, int n_tblk, int64_t nblocks,
+    int D, int B, int T, OrderSpan sp, int n_tblk, int64_t nblocks,
     const int64_t *__restrict__ grp_ptr, const int32_t *__restrict__ grp_key,
     const double *__restrict__ rtab, const float *__restrict__ gsum,
     const float *__restrict__ prev, float *__restrict__ cur,
-    float *__restrict__ tot_hi, float *__restrict__ tot_lo) {
+    float *__restrict__ tot_hi, float *__restrict__ tot_lo, Injection inj) {
   using Sh = SpreadShape<DP>;
   constexpr int DW = Sh::DW, R = Sh::R, K = 8;
   // time-major tile order: the blocks one XCD runs at a time write long
@@ -727,7 +776,7 @@ __global__ __launch_bounds__(256) void group_spread_kernel(
   const int wd = wave % Sh::NWD, wt = wave / Sh::NWD;
   const int d0 = wd * DW;  // first direction of this wave
   const int tl = tb * Sh::TILE + wt * (64 * R) + lane;  // bin of r = 0
-  const uint32_t row_bytes = (uint32_t)T * 4u;
+  const uint32_t row_bytes = (uint32_t)sp.Tc * 4u;
 
   double acc[DW][R];
 #pragma unroll
@@ -784,14 +833,26 @@ __global__ __launch_bounds__(256) void group_spread_kernel(
   const int64_t dstride = (int64_t)B * T;
   const int64_t base = j * D * dstride + (int64_t)b * T;
   const uint32_t span = (uint32_t)(((int64_t)(D - 1) * dstride + T) * 4);
-  const __amdgpu_buffer_rsrc_t rc = make_rsrc(cur + base, span);
+  // the last order leaves the rounded total only
+  const __amdgpu_buffer_rsrc_t rc = make_rsrc(cur + base, sp.last ? 0u : span);
   constexpr int NP = DW * R;  // (d, r) pairs of this lane
-  if (MODE == 0) {  // order histogram only (no running total)
+  if (MODE == kSumMode) {     // the injected energy, where this tile has it
+    const int nj = inj.n0[j];
+    if (nj >= tb * Sh::TILE && nj < (tb + 1) * Sh::TILE) {  // uniform
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        const int d = d0 + p / R;
+        if (d < D && tl + 64 * (p % R) == nj)
+          acc[p / R][p % R] += inj.e0[(j * D + d) * B + b];
+      }
+    }
+  }
+  if (MODE == 0 || MODE == kSumMode) {  // no running total
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
       const int d = d0 + p / R, r = p % R;
       const int t = tl + 64 * r;
-      const uint32_t off = (d < D && t < T)
+      const uint32_t off = (d < D && t < sp.Tc)
                                ? (uint32_t)((int64_t)d * dstride + t) * 4u
                                : kNoOffset;
       buffer_store((float)acc[p / R][r], rc, off);
@@ -800,6 +861,8 @@ __global__ __launch_bounds__(256) void group_spread_kernel(
   }
   const __amdgpu_buffer_rsrc_t rh = make_rsrc(tot_hi + base, span);
   const __amdgpu_buffer_rsrc_t rl = make_rsrc(tot_lo + base, span);
+  const __amdgpu_buffer_rsrc_t wl =
+      make_rsrc(tot_lo + base, sp.last ? 0u : span);
   const __amdgpu_buffer_rsrc_t rp =
       make_rsrc(MODE == 2 ? prev + base : cur + base, MODE == 2 ? span : 0u);
 #pragma unroll
@@ -812,24 +875,27 @@ __global__ __launch_bounds__(256) void group_spread_kernel(
       if (p >= NP) break;
       const int d = d0 + p / R, r = p % R;
       const int t = tl + 64 * r;
-      off[q] = (d < D && t < T) ? (uint32_t)((int64_t)d * dstride + t) * 4u
-                                : kNoOffset;
-      h[q] = buffer_load(rh, off[q]);
-      l[q] = buffer_load(rl, off[q]);
-      if (MODE == 2) e[q] = buffer_load(rp, off[q]);
+      off[q] = (d < D && t < sp.Tc)
+                   ? (uint32_t)((int64_t)d * dstride + t) * 4u
+                   : kNoOffset;
+      const uint32_t ot = t < sp.Tv ? off[q] : kNoOffset;
+      h[q] = buffer_load(rh, ot);
+      l[q] = buffer_load(rl, ot);
+      if (MODE == 2) e[q] = buffer_load(rp, t < sp.Tp ? off[q] : kNoOffset);
     }
 #pragma unroll
     for (int q = 0; q < K; ++q) {
       const int p = p0 + q;
       if (p >= NP) break;
-      const double a = acc[p / R][p % R];
+      const double a = sp.round ? (double)(float)acc[p / R][p % R]
+                                : acc[p / R][p % R];
       double sum = (double)h[q] + (double)l[q];
       if (MODE == 2) sum += (double)e[q];
       sum += a;
       const float hs = (float)sum;
       buffer_store((float)a, rc, off[q]);
       buffer_store(hs, rh, off[q]);
-      buffer_store((float)(sum - (double)hs), rl, off[q]);
+      buffer_store((float)(sum - (double)hs), wl, off[q]);
     }
   }
 }
@@ -846,11 +912,11 @@ __global__ __launch_bounds__(256) void group_spread_kernel(
 // group_spread_kernel.
 template <int DP, int MODE>
 __global__ __launch_bounds__(256) void ds_spread_kernel(
-    int D, int B, int T, int n_tblk, int64_t nblocks,
+    int D, int B, int T, OrderSpan sp, int n_tblk, int64_t nblocks,
     const int64_t *__restrict__ grp_ptr, const int32_t *__restrict__ grp_key,
     const float *__restrict__ gsum, const float *__restrict__ prev,
     float *__restrict__ cur, float *__restrict__ tot_hi,
-    float *__restrict__ tot_lo) {
+    float *__restrict__ tot_lo, Injection inj) {
   constexpr int K = 8;
   __shared__ int32_t gmap[DP];  // direction -> specular group offset, or -1
   const int64_t tile = xcd_tile(blockIdx.x, nblocks);
@@ -859,7 +925,7 @@ __global__ __launch_bounds__(256) void ds_spread_kernel(
   const int64_t j = (tile / n_tblk) % P;
   const int b = (int)(tile / (n_tblk * P));
   const int t = tb * 256 + (int)threadIdx.x;
-  const uint32_t row_bytes = (uint32_t)T * 4u;
+  const uint32_t row_bytes = (uint32_t)sp.Tc * 4u;
   const int64_t g0 = grp_ptr[j], g1 = grp_ptr[j + 1];
   for (int d = (int)threadIdx.x; d < DP; d += 256) gmap[d] = -1;
   __syncthreads();
@@ -885,19 +951,26 @@ __global__ __launch_bounds__(256) void ds_spread_kernel(
   const int64_t dstride = (int64_t)B * T;
   const int64_t base = j * D * dstride + (int64_t)b * T;
   const uint32_t span = (uint32_t)(((int64_t)(D - 1) * dstride + T) * 4);
-  const __amdgpu_buffer_rsrc_t rc = make_rsrc(cur + base, span);
+  // the last order leaves the rounded total only
+  const __amdgpu_buffer_rsrc_t rc = make_rsrc(cur + base, sp.last ? 0u : span);
   auto offset = [&](int d) {
-    return (d < D && t < T) ? (uint32_t)((int64_t)d * dstride + t) * 4u
-                            : kNoOffset;
+    return (d < D && t < sp.Tc) ? (uint32_t)((int64_t)d * dstride + t) * 4u
+                             : kNoOffset;
   };
-  if (MODE == 0) {
+  if (MODE == 0 || MODE == kSumMode) {
+    const bool here = MODE == kSumMode && t == inj.n0[j];
 #pragma unroll
-    for (int d = 0; d < DP; ++d)
-      buffer_store((float)((double)v[d] + gd), rc, offset(d));
+    for (int d = 0; d < DP; ++d) {
+      double a = (double)v[d] + gd;
+      if (here && d < D) a += inj.e0[(j * D + d) * B + b];
+      buffer_store((float)a, rc, offset(d));
+    }
     return;
   }
   const __amdgpu_buffer_rsrc_t rh = make_rsrc(tot_hi + base, span);
   const __amdgpu_buffer_rsrc_t rl = make_rsrc(tot_lo + base, span);
+  const __amdgpu_buffer_rsrc_t wl =
+      make_rsrc(tot_lo + base, sp.last ? 0u : span);
   const __amdgpu_buffer_rsrc_t rp =
       make_rsrc(MODE == 2 ? prev + base : cur + base, MODE == 2 ? span : 0u);
 #pragma unroll
@@ -908,21 +981,23 @@ __global__ __launch_bounds__(256) void ds_spread_kernel(
     for (int q = 0; q < K; ++q) {
       if (d0 + q >= DP) break;
       off[q] = offset(d0 + q);
-      h[q] = buffer_load(rh, off[q]);
-      l[q] = buffer_load(rl, off[q]);
-      if (MODE == 2) e[q] = buffer_load(rp, off[q]);
+      const uint32_t ot = t < sp.Tv ? off[q] : kNoOffset;
+      h[q] = buffer_load(rh, ot);
+      l[q] = buffer_load(rl, ot);
+      if (MODE == 2) e[q] = buffer_load(rp, t < sp.Tp ? off[q] : kNoOffset);
     }
 #pragma unroll
     for (int q = 0; q < K; ++q) {
       if (d0 + q >= DP) break;
-      const double a = (double)v[d0 + q] + gd;
+      double a = (double)v[d0 + q] + gd;
+      if (sp.round) a = (double)(float)a;
       double sum = (double)h[q] + (double)l[q];
       if (MODE == 2) sum += (double)e[q];
       sum += a;
       const float hs = (float)sum;
       buffer_store((float)a, rc, off[q]);
       buffer_store(hs, rh, off[q]);
-      buffer_store((float)(sum - (double)hs), rl, off[q]);
+      buffer_store((float)(sum - (double)hs), wl, off[q]);
     }
   }
 }
@@ -931,17 +1006,23 @@ template <int DP>
 int launch_ds_spread(int64_t P, int64_t D, int64_t B, int64_t T,
                      const int64_t *grp_ptr, const int32_t *grp_key,
                      const float *gsum, const float *prev, float *cur,
-                     float *tot_hi, float *tot_lo, hipStream_t s) {
-  const int64_t nt = ceil_div(T, (int64_t)256);
+                     float *tot_hi, float *tot_lo, const OrderStep *step,
+                     hipStream_t s) {
+  const OrderSpan sp = span_of(step, T);
+  const Injection inj = step ? step->inj : Injection{};
+  const int64_t nt = ceil_div((int64_t)sp.Tc, (int64_t)256);
   const int64_t nb = P * B * nt;
   SPR_REQUIRE(nb < (int64_t)0x7fffffff, "exchange grid too large");
   SPR_REQUIRE(D * B * T < ((int64_t)1 << 29),
               "histogram too large for one patch (D*B*T >= 2^29)");
 #define SPR_DS_MODE(M)                                                        \
   hipLaunchKernelGGL((ds_spread_kernel<DP, M>), dim3((unsigned)nb),           \
-                     dim3(256), 0, s, (int)D, (int)B, (int)T, (int)nt, nb,    \
-                     grp_ptr, grp_key, gsum, prev, cur, tot_hi, tot_lo)
-  if (!tot_hi)
+                     dim3(256), 0, s, (int)D, (int)B, (int)T, sp,             \
+                     (int)nt, nb, grp_ptr, grp_key, gsum, prev, cur, tot_hi,  \
+                     tot_lo, inj)
+  if (step && !tot_hi && step->inj.n0)
+    SPR_DS_MODE(kSumMode);
+  else if (!tot_hi)
     SPR_DS_MODE(0);
   else if (!prev)
     SPR_DS_MODE(1);
@@ -957,28 +1038,42 @@ int launch_step(int64_t P, int64_t D, int64_t B, int64_t T,
                 const int64_t *row_ptr, const int32_t *src,
                 const int32_t *lag, const int32_t *dir, const double *coef,
                 const float *prev, float *cur, float *tot_hi, float *tot_lo,
-                hipStream_t s) {
+                const OrderStep *step, hipStream_t s) {
+  const OrderSpan sp = span_of(step, T);
+  const Injection inj = step ? step->inj : Injection{};
   if constexpr (DP >= 16) {
     constexpr int NT = 8 / (DP / 16);
-    const int64_t n_tblk = ceil_div(T, (int64_t)4 * 16 * NT);
+    const int64_t n_tblk = ceil_div((int64_t)sp.Tc, (int64_t)4 * 16 * NT);
     const int64_t nblocks = P * B * n_tblk;
     SPR_REQUIRE(nblocks < (int64_t)0x7fffffff, "exchange grid too large");
-    hipLaunchKernelGGL((exchange_mfma_kernel<DP, NT>),
-                       dim3((unsigned)nblocks), dim3(256), 0, s, (int)D,
-                       (int)B, (int)T, (int)n_tblk, nblocks, row_ptr, src,
-                       lag, dir, coef, prev, cur, tot_hi, tot_lo);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)nblocks), dim3(256), 0, s,
+                         (int)D, (int)B, (int)T, sp, (int)n_tblk, nblocks,
+                         row_ptr, src, lag, dir, coef, prev, cur, tot_hi, tot_lo, inj);
+    };
+    if (step && !tot_hi)
+      go(exchange_mfma_kernel<DP, NT, true>);
+    else
+      go(exchange_mfma_kernel<DP, NT, false>);
     SPR_LAUNCH_CHECK();
     return SPR_OK;
   }
-  constexpr int BS = 256;
-  const int64_t n_tblk = ceil_div(T, (int64_t)BS * R);
-  const int64_t nblocks = P * B * n_tblk;
-  SPR_REQUIRE(nblocks < (int64_t)0x7fffffff, "exchange grid too large");
-  hipLaunchKernelGGL((exchange_step_kernel<DP, R, BS, 4>),
-                     dim3((unsigned)nblocks), dim3(BS), 0, s, (int)D, (int)B,
-                     (int)T, (int)n_tblk, nblocks, row_ptr, src, lag, dir,
-                     coef, prev, cur, tot_hi, tot_lo);
-  SPR_LAUNCH_CHECK();
+  else {
+    constexpr int BS = 256;
+    const int64_t n_tblk = ceil_div((int64_t)sp.Tc, (int64_t)BS * R);
+    const int64_t nblocks = P * B * n_tblk;
+    SPR_REQUIRE(nblocks < (int64_t)0x7fffffff, "exchange grid too large");
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)nblocks), dim3(BS), 0, s,
+                         (int)D, (int)B, (int)T, sp, (int)n_tblk, nblocks,
+                         row_ptr, src, lag, dir, coef, prev, cur, tot_hi, tot_lo, inj);
+    };
+    if (step && !tot_hi)
+      go(exchange_step_kernel<DP, R, BS, 4, true>);
+    else
+      go(exchange_step_kernel<DP, R, BS, 4, false>);
+    SPR_LAUNCH_CHECK();
+  }
   return SPR_OK;
 }
 
@@ -1005,23 +1100,24 @@ int launch_gather(int64_t P, int64_t B, int64_t T, int64_t Vd,
                   const int64_t *row_ptr, const int64_t *grp_ptr,
                   const int32_t *rowid, const int32_t *lag,
                   const double *scal, const double *dscal, const float *prev,
-                  float *gsum, hipStream_t s) {
+                  float *gsum, const OrderStep *step, hipStream_t s) {
   constexpr int BS = 256;
+  const OrderSpan sp = span_of(step, T);
   const int64_t nt =
-      ceil_div(T, (int64_t)BS * (dscal ? kDsGatherR : kGatherR));
+      ceil_div((int64_t)sp.Tc, (int64_t)BS * (dscal ? kDsGatherR : kGatherR));
   const int64_t nb = P * B * nt;
   SPR_REQUIRE(nb < (int64_t)0x7fffffff, "exchange grid too large");
   SPR_REQUIRE(T < ((int64_t)1 << 29), "histogram too long (T >= 2^29)");
   if (dscal)
     hipLaunchKernelGGL((ds_gather_kernel<kDsGatherR, BS, kDsGatherC>),
                        dim3((unsigned)nb), dim3(BS), 0, s, (int)B, (int)T,
-                       (int)nt, nb, Vd, row_ptr, grp_ptr, rowid, lag, scal,
-                       dscal, prev, gsum);
+                       sp.Tp, (int)nt, nb, Vd, row_ptr, grp_ptr, rowid, lag,
+                       scal, dscal, prev, gsum);
   else
     hipLaunchKernelGGL((group_gather_kernel<kGatherR, BS, kGatherC>),
                        dim3((unsigned)nb), dim3(BS), 0, s, (int)B, (int)T,
-                       (int)nt, nb, Vd, row_ptr, grp_ptr, rowid, lag, scal,
-                       prev, gsum);
+                       sp.Tp, (int)nt, nb, Vd, row_ptr, grp_ptr, rowid, lag,
+                       scal, prev, gsum);
   SPR_LAUNCH_CHECK();
   return SPR_OK;
 }
@@ -1030,17 +1126,23 @@ template <int DP>
 int launch_spread(int64_t P, int64_t D, int64_t B, int64_t T,
                   const int64_t *grp_ptr, const int32_t *grp_key,
                   const double *rtab, const float *gsum, const float *prev,
-                  float *cur, float *tot_hi, float *tot_lo, hipStream_t s) {
-  const int64_t nt = ceil_div(T, (int64_t)SpreadShape<DP>::TILE);
+                  float *cur, float *tot_hi, float *tot_lo,
+                  const OrderStep *step, hipStream_t s) {
+  const OrderSpan sp = span_of(step, T);
+  const Injection inj = step ? step->inj : Injection{};
+  const int64_t nt = ceil_div((int64_t)sp.Tc, (int64_t)SpreadShape<DP>::TILE);
   const int64_t nb = P * B * nt;
   SPR_REQUIRE(nb < (int64_t)0x7fffffff, "exchange grid too large");
   SPR_REQUIRE(D * B * T < ((int64_t)1 << 29),
               "histogram too large for one patch (D*B*T >= 2^29)");
 #define SPR_SPREAD_MODE(M)                                                    \
   hipLaunchKernelGGL((group_spread_kernel<DP, M>), dim3((unsigned)nb),        \
-                     dim3(256), 0, s, (int)D, (int)B, (int)T, (int)nt, nb,    \
-                     grp_ptr, grp_key, rtab, gsum, prev, cur, tot_hi, tot_lo)
-  if (!tot_hi)
+                     dim3(256), 0, s, (int)D, (int)B, (int)T, sp,             \
+                     (int)nt, nb, grp_ptr, grp_key, rtab, gsum, prev, cur,    \
+                     tot_hi, tot_lo, inj)
+  if (step && !tot_hi && step->inj.n0)
+    SPR_SPREAD_MODE(kSumMode);
+  else if (!tot_hi)
     SPR_SPREAD_MODE(0);
   else if (!prev)
     SPR_SPREAD_MODE(1);
@@ -1658,6 +1760,29 @@ extern "C" int spr_exchange_init(int64_t P, int64_t D, int64_t B, int64_t T,
   return SPR_OK;
 }
 
+int spr::step_pairs(int64_t P, int64_t D, int64_t B, int64_t T,
+                    const int64_t *row_ptr, const int32_t *src,
+                    const int32_t *lag, const int32_t *dir,
+                    const double *coef, const float *prev, float *cur,
+                    float *tot_hi, float *tot_lo, const OrderStep *step,
+                    hipStream_t s) {
+  const int64_t DP = spr_padded_directions(D);
+#define SPR_STEP(DPV, RV)                                                   \
+  return launch_step<DPV, RV>(P, D, B, T, row_ptr, src, lag, dir, coef,     \
+                              prev, cur, tot_hi, tot_lo, step, s)
+  switch (DP) {
+    case 1: SPR_STEP(1, 8);
+    case 2: SPR_STEP(2, 8);
+    case 4: SPR_STEP(4, 8);
+    case 8: SPR_STEP(8, 8);
+    case 16: SPR_STEP(16, 4);
+    case 32: SPR_STEP(32, 2);
+    case 64: SPR_STEP(64, 1);
+  }
+#undef SPR_STEP
+  return fail(SPR_ERR_UNSUPPORTED, "spr_exchange_step: D unsupported");
+}
+
 extern "C" int spr_exchange_step(int64_t P, int64_t D, int64_t B, int64_t T,
                                  const int64_t *row_ptr, const int32_t *src,
                                  const int32_t *lag, const int32_t *dir,
@@ -1673,21 +1798,8 @@ extern "C" int spr_exchange_step(int64_t P, int64_t D, int64_t B, int64_t T,
                   tot_lo,
               "spr_exchange_step: null pointer");
   SPR_REQUIRE(prev != cur, "spr_exchange_step: prev and cur must differ");
-  hipStream_t s = as_stream(stream);
-#define SPR_STEP(DPV, RV)                                                   \
-  return launch_step<DPV, RV>(P, D, B, T, row_ptr, src, lag, dir, coef,     \
-                              prev, cur, tot_hi, tot_lo, s)
-  switch (DP) {
-    case 1: SPR_STEP(1, 8);
-    case 2: SPR_STEP(2, 8);
-    case 4: SPR_STEP(4, 8);
-    case 8: SPR_STEP(8, 8);
-    case 16: SPR_STEP(16, 4);
-    case 32: SPR_STEP(32, 2);
-    case 64: SPR_STEP(64, 1);
-  }
-#undef SPR_STEP
-  return fail(SPR_ERR_UNSUPPORTED, "spr_exchange_step: D unsupported");
+  return step_pairs(P, D, B, T, row_ptr, src, lag, dir, coef, prev, cur,
+                    tot_hi, tot_lo, nullptr, as_stream(stream));
 }
 
 extern "C" int spr_exchange_finalize(int64_t n, const float *tot_hi,
@@ -1889,7 +2001,7 @@ extern "C" int spr_exchange_gather_ds(
                   gsum,
               "spr_exchange_gather_ds: null pointer");
   return launch_gather(P, B, T, Vd, row_ptr, grp_ptr, rowid, lag, scal,
-                       dscal, prev, gsum, as_stream(stream));
+                       dscal, prev, gsum, nullptr, as_stream(stream));
 }
 
 extern "C" int spr_plan_ds_transpose_rows(int64_t P, int64_t D,
@@ -1964,14 +2076,15 @@ extern "C" int spr_exchange_gather_grouped(
   SPR_REQUIRE(row_ptr && grp_ptr && rowid && lag && scal && prev && gsum,
               "spr_exchange_gather_grouped: null pointer");
   return launch_gather(P, B, T, Vd, row_ptr, grp_ptr, rowid, lag, scal,
-                       nullptr, prev, gsum, as_stream(stream));
+                       nullptr, prev, gsum, nullptr, as_stream(stream));
 }
 
 namespace {
 int spread_grouped(const char *name, int64_t P, int64_t D, int64_t B,
                    int64_t T, const int64_t *grp_ptr, const int32_t *grp_key,
                    const double *rtab, const float *gsum, const float *prev,
-                   float *cur, float *tot_hi, float *tot_lo, void *stream) {
+                   float *cur, float *tot_hi, float *tot_lo,
+                   const OrderStep *step, hipStream_t s) {
   const int64_t DP = spr_padded_directions(D);
   SPR_REQUIRE(DP > 0, "%s: D=%lld unsupported", name, (long long)D);
   SPR_REQUIRE(P > 0 && B > 0 && T > 0 && T < 0x3fffffff, "%s: bad sizes",
@@ -1982,10 +2095,9 @@ int spread_grouped(const char *name, int64_t P, int64_t D, int64_t B,
               name);
   SPR_REQUIRE(!prev || (tot_hi && prev != cur),
               "%s: prev needs the total and a separate buffer", name);
-  hipStream_t s = as_stream(stream);
 #define SPR_SPREAD(DPV)                                                       \
   return launch_spread<DPV>(P, D, B, T, grp_ptr, grp_key, rtab, gsum, prev,   \
-                            cur, tot_hi, tot_lo, s)
+                            cur, tot_hi, tot_lo, step, s)
   switch (DP) {
     case 1: SPR_SPREAD(1);
     case 2: SPR_SPREAD(2);
@@ -2006,7 +2118,7 @@ extern "C" int spr_exchange_spread_grouped(
     float *cur, float *tot_hi, float *tot_lo, void *stream) {
   return spread_grouped("spr_exchange_spread_grouped", P, D, B, T, grp_ptr,
                         grp_key, rtab, gsum, nullptr, cur, tot_hi, tot_lo,
-                        stream);
+                        nullptr, as_stream(stream));
 }
 
 extern "C" int spr_exchange_spread_grouped_pair(
@@ -2018,8 +2130,31 @@ extern "C" int spr_exchange_spread_grouped_pair(
               "spr_exchange_spread_grouped_pair: null pointer");
   return spread_grouped("spr_exchange_spread_grouped_pair", P, D, B, T,
                         grp_ptr, grp_key, rtab, gsum, prev, cur, tot_hi,
-                        tot_lo, stream);
+                        tot_lo, nullptr, as_stream(stream));
 }
+
+namespace {
+int spread_ds(int64_t P, int64_t D, int64_t B, int64_t T,
+              const int64_t *grp_ptr, const int32_t *grp_key,
+              const float *gsum, const float *prev, float *cur, float *tot_hi,
+              float *tot_lo, const OrderStep *step, hipStream_t s) {
+  const int64_t DP = spr_padded_directions(D);
+#define SPR_DSS(DPV)                                                          \
+  return launch_ds_spread<DPV>(P, D, B, T, grp_ptr, grp_key, gsum, prev, cur, \
+                               tot_hi, tot_lo, step, s)
+  switch (DP) {
+    case 1: SPR_DSS(1);
+    case 2: SPR_DSS(2);
+    case 4: SPR_DSS(4);
+    case 8: SPR_DSS(8);
+    case 16: SPR_DSS(16);
+    case 32: SPR_DSS(32);
+    case 64: SPR_DSS(64);
+  }
+#undef SPR_DSS
+  return fail(SPR_ERR_UNSUPPORTED, "diffuse + specular spread: bad D");
+}
+}  // namespace
 
 extern "C" int spr_exchange_spread_ds(int64_t P, int64_t D, int64_t B,
                                       int64_t T, const int64_t *grp_ptr,
@@ -2039,21 +2174,26 @@ extern "C" int spr_exchange_spread_ds(int64_t P, int64_t D, int64_t B,
   SPR_REQUIRE(!prev || (tot_hi && prev != cur),
               "spr_exchange_spread_ds: prev needs the total and a separate "
               "buffer");
-  hipStream_t s = as_stream(stream);
-#define SPR_DSS(DPV)                                                          \
-  return launch_ds_spread<DPV>(P, D, B, T, grp_ptr, grp_key, gsum, prev, cur, \
-                               tot_hi, tot_lo, s)
-  switch (DP) {
-    case 1: SPR_DSS(1);
-    case 2: SPR_DSS(2);
-    case 4: SPR_DSS(4);
-    case 8: SPR_DSS(8);
-    case 16: SPR_DSS(16);
-    case 32: SPR_DSS(32);
-    case 64: SPR_DSS(64);
-  }
-#undef SPR_DSS
-  return fail(SPR_ERR_UNSUPPORTED, "spr_exchange_spread_ds: bad D");
+  return spread_ds(P, D, B, T, grp_ptr, grp_key, gsum, prev, cur, tot_hi,
+                   tot_lo, nullptr, as_stream(stream));
+}
+
+int spr::gather_rows(const spr_exchange_plan &p, int64_t T, const float *prev,
+                     float *gsum, const OrderStep &step, hipStream_t s) {
+  return launch_gather(p.P, p.B, T, p.Vd, p.row_ptr, p.grp_ptr, p.rowid,
+                       p.lag, p.scal, p.kind == SPR_PLAN_DS ? p.dscal : nullptr,
+                       prev, gsum, &step, s);
+}
+
+int spr::spread_rows(const spr_exchange_plan &p, int64_t T, const float *gsum,
+                     const float *prev, float *cur, float *tot_hi,
+                     float *tot_lo, const OrderStep &step, hipStream_t s) {
+  if (p.kind == SPR_PLAN_DS)
+    return spread_ds(p.P, p.D, p.B, T, p.grp_ptr, p.grp_key, gsum, prev, cur,
+                     tot_hi, tot_lo, &step, s);
+  return spread_grouped("grouped spread", p.P, p.D, p.B, T, p.grp_ptr,
+                        p.grp_key, p.rtab, gsum, prev, cur, tot_hi, tot_lo,
+                        &step, s);
 }
 
 extern "C" int spr_exchange_total_add(int64_t n, const float *x,
@@ -2086,7 +2226,8 @@ extern "C" int spr_exchange_step_grouped(
 
 namespace {
 // Workspace of spr_energy_exchange.  Besides the per-pair plan and the
-// three state buffers it holds the grouped plan built from the dense F~
+// state buffers (prev, beside the caller's etc, for the running sum; lo
+// holds the source bins) it holds the grouped plan built from the dense F~
 // (hashes alias coef, which is filled after the sort) with group sums for
 // at most gcap = min(ceil(Vd / 4), 2 P D) groups: beyond a quarter of the
 // entries the per-pair plan is used, and the group sums never take more
@@ -2230,15 +2371,15 @@ int energy_exchange_on(const char *name, int64_t T, int64_t P, int64_t D,
   auto *dir = reinterpret_cast<int32_t *>(ws + L.dir);
   auto *coef = reinterpret_cast<double *>(ws + L.coef);
   auto *prev = reinterpret_cast<float *>(ws + L.prev);
-  auto *cur = reinterpret_cast<float *>(ws + L.cur);
-  auto *lo = reinterpret_cast<float *>(ws + L.lo);
+  auto *n0 = reinterpret_cast<int32_t *>(ws + L.lo);
   auto *err = reinterpret_cast<int *>(ws + L.err);
   last_dense_groups = 0;
   int rc;
   if ((rc = fill<int32_t>(err, 1, 0, s))) return rc;
-  if ((rc = spr_exchange_init(P, D, B, T, e0dir, d0, c, dt, prev, etc, lo,
-                              err, stream)))
-    return rc;
+  spr_exchange_plan p{};
+  p.P = P;
+  p.D = D;
+  p.B = B;
   if (K >= 1 && V > 0) {
     const int64_t Vd = 2 * V;
     if ((rc = fill<uint8_t>(vis, P * P, 0, s))) return rc;
@@ -2251,31 +2392,16 @@ int energy_exchange_on(const char *name, int64_t T, int64_t P, int64_t D,
     if ((rc = dense_grouped_plan(T, P, D, B, dist, fft, p2o, c, dt, V, ws, L,
                                  s, &G)))
       return rc;
+    p.Vd = Vd;
+    p.row_ptr = row_ptr;
+    p.lag = lag;
     if (G > 0) {
-      // two passes per order; the total is updated every other order with
-      // two orders at once (spread mode 2), an odd last order on its own
-      auto *grp_ptr = reinterpret_cast<const int64_t *>(ws + L.grp_ptr);
-      auto *grp_key = reinterpret_cast<const int32_t *>(ws + L.grp_key);
-      auto *rowid = reinterpret_cast<const int32_t *>(ws + L.rowid);
-      auto *scal = reinterpret_cast<const double *>(ws + L.scal);
-      auto *gsum = reinterpret_cast<float *>(ws + L.gsum);
-      for (int64_t k = 0; k < K; ++k) {
-        if ((rc = launch_gather(P, B, T, Vd, row_ptr, grp_ptr, rowid, lag,
-                                scal, nullptr, prev, gsum, s)))
-          return rc;
-        const bool pair = k % 2 == 1;
-        if ((rc = spread_grouped(name, P, D, B, T, grp_ptr, grp_key, coef,
-                                 gsum, pair ? prev : nullptr, cur,
-                                 pair ? etc : nullptr, pair ? lo : nullptr,
-                                 stream)))
-          return rc;
-        float *t = prev;
-        prev = cur;
-        cur = t;
-      }
-      if (K % 2 == 1 &&
-          (rc = spr_exchange_total_add(P * D * B * T, prev, etc, lo, stream)))
-        return rc;
+      p.kind = SPR_PLAN_GROUPED;
+      p.grp_ptr = reinterpret_cast<const int64_t *>(ws + L.grp_ptr);
+      p.grp_key = reinterpret_cast<const int32_t *>(ws + L.grp_key);
+      p.rowid = reinterpret_cast<const int32_t *>(ws + L.rowid);
+      p.scal = reinterpret_cast<const double *>(ws + L.scal);
+      p.rtab = coef;
       last_dense_groups = G;
     } else {
       // the sort may have reordered the rows: rebuild them in source order
@@ -2283,17 +2409,15 @@ int energy_exchange_on(const char *name, int64_t T, int64_t P, int64_t D,
       if ((rc = spr_plan_from_dense(P, D, B, c, dt, Vd, row_ptr, src, dist,
                                     p2o, fft, lag, dir, coef, stream)))
         return rc;
-      for (int64_t k = 0; k < K; ++k) {
-        if ((rc = spr_exchange_step(P, D, B, T, row_ptr, src, lag, dir, coef,
-                                    prev, cur, etc, lo, stream)))
-          return rc;
-        float *t = prev;
-        prev = cur;
-        cur = t;
-      }
+      p.kind = SPR_PLAN_PAIRS;
+      p.src = src;
+      p.dir = dir;
+      p.coef = coef;
     }
   }
-  if ((rc = spr_exchange_finalize(P * D * B * T, etc, lo, etc, stream)))
+  if ((rc = spr_exchange_sum(&p, T, K, e0dir, d0, c, dt, etc, prev,
+                             reinterpret_cast<float *>(ws + L.gsum), n0, err,
+                             stream)))
     return rc;
   int h_err = 0;
   SPR_HIP(hipMemcpyAsync(&h_err, err, sizeof(int), hipMemcpyDeviceToHost, s));

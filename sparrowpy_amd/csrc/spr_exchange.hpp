@@ -92,4 +92,43 @@ __device__ __forceinline__ int64_t entry_brdf_row(
   return brdf_index[w] * S + nearest_direction(in_dirs + w * S * 3, S, u);
 }
 
+// The bins of one order that can hold energy: bins of the source histograms
+// from Tp on, of the result from Tc on and of the total so far from Tv on
+// are 0 and are neither read nor written.  Of the last order only the total
+// is kept, rounded; round adds the order to the total as rounded to float32
+// (as when it is read back from its histogram).
+struct OrderSpan {
+  int Tp, Tc, Tv;
+  int last, round;
+};
+// Energy injected into every order of the running sum x_{k+1} = x_0 + A x_k
+// (spr_exchange_sum): one bin n0[i] per patch.
+struct Injection {
+  const double *e0 = nullptr;   // [P, D, B]
+  const int32_t *n0 = nullptr;  // [P]
+};
+struct OrderStep {
+  OrderSpan span;
+  Injection inj;
+};
+inline OrderSpan span_of(const OrderStep *step, int64_t T) {
+  return step ? step->span : OrderSpan{(int)T, (int)T, (int)T, 0, 0};
+}
+
+// The passes of an order (exchange.hip, tiles.hip): the group sums row by
+// row or on destination tiles, the spread over the directions, and the
+// per-pair order.
+int gather_rows(const spr_exchange_plan &p, int64_t T, const float *prev,
+                float *gsum, const OrderStep &step, hipStream_t s);
+int gather_tiles(const spr_exchange_plan &p, int64_t T, const float *prev,
+                 float *gsum, const OrderStep &step, hipStream_t s);
+int spread_rows(const spr_exchange_plan &p, int64_t T, const float *gsum,
+                const float *prev, float *cur, float *tot_hi, float *tot_lo,
+                const OrderStep &step, hipStream_t s);
+int step_pairs(int64_t P, int64_t D, int64_t B, int64_t T,
+               const int64_t *row_ptr, const int32_t *src, const int32_t *lag,
+               const int32_t *dir, const double *coef, const float *prev,
+               float *cur, float *tot_hi, float *tot_lo, const OrderStep *step,
+               hipStream_t s);
+
 }  // namespace spr

@@ -1,0 +1,216 @@
+// All reflection orders of one source: the order loop, and the sum of the
+// orders.
+//
+// Reference: the order loop of _energy_exchange and its running total
+// (sparrowpy/classes/RadiosityFast.py:1073-1145).  With A the exchange of
+// one order and E_0 the injected energy (:1037-1070), E_{k+1} = A E_k and the
+// result is E_0 + ... + E_K.  Two forms:
+//
+// spr_exchange_orders carries the order beside the running total (a
+// compensated pair of float32): what stepping spr_exchange_gather_* /
+// _spread_* does, in one call.  The total starts as the injected energy and
+// the last order writes the rounded total alone, so nothing is cleared
+// before the loop and no pass follows it.
+//
+// spr_exchange_sum carries the sum instead of the order, x_{k+1} = E_0 +
+// A x_k, x_K being the result: no total to read and write, two state
+// buffers instead of four.  x_k is rounded to float32 once per order like
+// E_k, and A averages that rounding over all sources, so the error against
+// float64 is the same; its bits are not those of the order-by-order sum.
+#include <algorithm>
+
+#include "spr_common.hpp"
+#include "spr_exchange.hpp"
+#include "spr_util.hpp"
+
+namespace spr {
+namespace {
+
+// Bins [t0, t1) of every histogram row: E_0 (with e0dir), or 0; with lo, x
+// and lo as a compensated pair and x's rounded value in prev too.  A wave
+// takes kFillBins bins of one row at a time; bound by the writes.
+constexpr int kFillBins = 1024;
+
+__global__ __launch_bounds__(256) void row_fill_kernel(
+    int64_t P, int64_t DB, int64_t T, int64_t t0, int64_t t1, int64_t chunks,
+    const double *__restrict__ e0dir, const double *__restrict__ d0, double c,
+    double dt, float *__restrict__ x, float *__restrict__ lo,
+    float *__restrict__ prev, int32_t *__restrict__ n0,
+    int *__restrict__ err) {
+  const int lane = (int)threadIdx.x & 63;
+  const int64_t waves = (int64_t)gridDim.x * 4;
+  for (int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+       q < P * DB * chunks; q += waves) {
+    const int64_t row = q / chunks, chunk = q % chunks;
+    int64_t n = -1;
+    float v = 0.f, w = 0.f;
+    if (e0dir) {
+      const int64_t i = row / DB;
+      n = delay_floor(d0[i], c, dt);
+      // a delay outside the histogram injects nothing and is reported
+      const bool bad = n < 0 || n >= T;
+      if (bad) n = -1;
+      if (chunk == 0 && lane == 0 && row % DB == 0) {
+        n0[i] = (int32_t)n;
+        if (bad) atomicOr(err, 1);
+      }
+      const double e = e0dir[row];
+      v = (float)e;
+      w = (float)(e - (double)v);
+    }
+    const int64_t a = t0 + chunk * kFillBins;
+    const int64_t b = a + kFillBins < t1 ? a + kFillBins : t1;
+    for (int64_t t = a + lane; t < b; t += 64) {
+      x[row * T + t] = t == n ? v : 0.f;
+      if (lo) {
+        lo[row * T + t] = t == n ? w : 0.f;
+        prev[row * T + t] = t == n ? v : 0.f;
+      }
+    }
+  }
+}
+
+int fill_rows(const spr_exchange_plan &p, int64_t T, int64_t t0, int64_t t1,
+              const double *e0dir, const double *d0, double c, double dt,
+              float *x, float *lo, float *prev, int32_t *n0, int *err,
+              hipStream_t s) {
+  if (t1 <= t0) return SPR_OK;
+  const int64_t chunks = ceil_div(t1 - t0, kFillBins);
+  const int64_t nb = ceil_div(p.P * p.D * p.B * chunks, 4);
+  hipLaunchKernelGGL(row_fill_kernel,
+                     dim3((unsigned)std::min<int64_t>(nb, 1 << 20)),
+                     dim3(256), 0, s, p.P, p.D * p.B, T, t0, t1, chunks,
+                     e0dir, d0, c, dt, x, lo, prev, n0, err);
+  SPR_LAUNCH_CHECK();
+  return SPR_OK;
+}
+
+int check_plan(const char *name, const spr_exchange_plan &p) {
+  SPR_REQUIRE(p.row_ptr && p.lag, "%s: null plan array", name);
+  if (p.kind == SPR_PLAN_PAIRS) {
+    SPR_REQUIRE(p.src && p.dir && p.coef, "%s: null plan array", name);
+    return SPR_OK;
+  }
+  SPR_REQUIRE(p.kind == SPR_PLAN_GROUPED || p.kind == SPR_PLAN_DS,
+              "%s: unknown plan kind %lld", name, (long long)p.kind);
+  SPR_REQUIRE(p.grp_ptr && p.grp_key && p.rowid && p.scal,
+              "%s: null plan array", name);
+  SPR_REQUIRE(p.kind == SPR_PLAN_DS ? p.dscal != nullptr : p.rtab != nullptr,
+              "%s: null plan array", name);
+  if (!p.M) return SPR_OK;
+  SPR_REQUIRE(p.tile_slots > 0 && p.tptr && p.gstart && p.mlag && p.mw,
+              "%s: null tile array", name);
+  if (p.kind == SPR_PLAN_DS)
+    SPR_REQUIRE(p.tile_rows == 16 && p.gdiff && p.mspan && p.mdw,
+                "%s: diffuse + specular tiles have 16 rows", name);
+  else if (p.tile_rows == 16)
+    SPR_REQUIRE(p.mspan && (p.tile_r == 8 || p.tile_r == 16),
+                "%s: 16-row tiles gather 8 or 16 bins per lane", name);
+  else
+    SPR_REQUIRE(p.mrow && (p.tile_rows == 4 || p.tile_rows == 8),
+                "%s: tiles have 4, 8 or 16 rows", name);
+  return SPR_OK;
+}
+
+// The arguments both forms share; *K becomes 0 where there is no order to
+// run (none asked for, or no pair of patches sees another).
+int check_call(const char *name, const spr_exchange_plan &p, int64_t T,
+               int64_t *K, const double *e0dir, const double *d0, double c,
+               double dt, const float *out, const float *gsum,
+               const int32_t *n0, const int *err_flag) {
+  SPR_REQUIRE(p.P > 0 && p.D > 0 && p.B > 0 && p.Vd >= 0 && T > 0 && c > 0 &&
+                  dt > 0,
+              "%s: bad sizes", name);
+  SPR_REQUIRE(e0dir && d0 && out && n0 && err_flag, "%s: null pointer", name);
+  if (*K < 0 || p.Vd == 0) *K = 0;
+  if (!*K) return SPR_OK;
+  SPR_REQUIRE(T < 0x3fffffff, "%s: histogram too long", name);
+  SPR_REQUIRE(spr_padded_directions(p.D) > 0,
+              "%s: D=%lld unsupported (max 64)", name, (long long)p.D);
+  SPR_REQUIRE(p.kind == SPR_PLAN_PAIRS || gsum, "%s: null pointer", name);
+  return check_plan(name, p);
+}
+
+// Pass 1 of an order on a grouped or diffuse + specular plan.
+int gather(const spr_exchange_plan &p, int64_t T, const float *x, float *gsum,
+           const OrderStep &step, hipStream_t s) {
+  return p.M ? gather_tiles(p, T, x, gsum, step, s)
+             : gather_rows(p, T, x, gsum, step, s);
+}
+
+}  // namespace
+}  // namespace spr
+
+using namespace spr;
+
+extern "C" int spr_exchange_sum(const spr_exchange_plan *plan, int64_t T,
+                                int64_t K, const double *e0dir,
+                                const double *d0, double c, double dt,
+                                float *out, float *tmp, float *gsum,
+                                int32_t *n0, int *err_flag, void *stream) {
+  SPR_REQUIRE(plan, "spr_exchange_sum: null plan");
+  const spr_exchange_plan &p = *plan;
+  int rc = check_call("spr_exchange_sum", p, T, &K, e0dir, d0, c, dt, out,
+                      gsum, n0, err_flag);
+  if (rc) return rc;
+  SPR_REQUIRE(!K || (tmp && tmp != out), "spr_exchange_sum: null pointer");
+  hipStream_t s = as_stream(stream);
+  float *x = K % 2 ? tmp : out, *y = K % 2 ? out : tmp;
+  OrderStep step{{(int)T, (int)T, 0, 0, 0}, {e0dir, n0}};
+  if ((rc = fill_rows(p, T, 0, T, e0dir, d0, c, dt, x, nullptr, nullptr, n0,
+                      err_flag, s)))
+    return rc;
+  for (int64_t k = 0; k < K; ++k) {
+    if (p.kind == SPR_PLAN_PAIRS) {
+      rc = step_pairs(p.P, p.D, p.B, T, p.row_ptr, p.src, p.lag, p.dir,
+                      p.coef, x, y, nullptr, nullptr, &step, s);
+    } else {
+      rc = gather(p, T, x, gsum, step, s);
+      if (!rc)
+        rc = spread_rows(p, T, gsum, nullptr, y, nullptr, nullptr, step, s);
+    }
+    if (rc) return rc;
+    std::swap(x, y);
+  }
+  return SPR_OK;
+}
+
+extern "C" int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T,
+                                   int64_t K, const double *e0dir,
+                                   const double *d0, double c, double dt,
+                                   float *out, float *lo, float *prev,
+                                   float *cur, float *gsum, int32_t *n0,
+                                   int *err_flag, void *stream) {
+  SPR_REQUIRE(plan, "spr_exchange_orders: null plan");
+  const spr_exchange_plan &p = *plan;
+  int rc = check_call("spr_exchange_orders", p, T, &K, e0dir, d0, c, dt, out,
+                      gsum, n0, err_flag);
+  if (rc) return rc;
+  SPR_REQUIRE(!K || (lo && prev && cur && prev != cur),
+              "spr_exchange_orders: null pointer");
+  hipStream_t s = as_stream(stream);
+  if ((rc = fill_rows(p, T, 0, T, e0dir, d0, c, dt, out, K ? lo : nullptr,
+                      prev, n0, err_flag, s)))
+    return rc;
+  OrderStep step{{(int)T, (int)T, (int)T, 0, 0}, {}};
+  for (int64_t k = 1; k <= K; ++k) {
+    OrderSpan &sp = step.span;
+    sp.last = k == K;
+    if (p.kind == SPR_PLAN_PAIRS) {
+      rc = step_pairs(p.P, p.D, p.B, T, p.row_ptr, p.src, p.lag, p.dir,
+                      p.coef, prev, cur, out, lo, &step, s);
+    } else {
+      // the total takes two orders at a time (the even ones' spread); an
+      // odd last order is added on its own, as rounded
+      rc = gather(p, T, prev, gsum, step, s);
+      const bool pair = k % 2 == 0, add = pair || sp.last;
+      sp.round = add && !pair;
+      if (!rc)
+        rc = spread_rows(p, T, gsum, pair ? prev : nullptr, cur,
+                         add ? out : nullptr, add ? lo : nullptr, step, s);
+    }
+    if (rc) return rc;
+    std::swap(prev, cur);
+  }
+  return SPR_OK;
+}

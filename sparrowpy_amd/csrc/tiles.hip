@@ -214,9 +214,10 @@ __device__ __forceinline__ TileMeta<JW> load_tile_meta(
 // bins, so the groups' gathers of one source row meet in the CU's cache.
 template <int R, int C, int JT, int JW, int MB>
 __global__ __launch_bounds__(256 * (JT / JW)) void tile_gather_kernel(
-    int64_t P, int B, int T, int n_tblk, int64_t nblocks, int64_t M,
-    const int64_t *__restrict__ tptr, const int64_t *__restrict__ grp_ptr,
-    const int32_t *__restrict__ mrow, const int32_t *__restrict__ mlag,
+    int64_t P, int B, int T, int Tp, int Tc, int n_tblk, int64_t nblocks,
+    int64_t M, const int64_t *__restrict__ tptr,
+    const int64_t *__restrict__ grp_ptr, const int32_t *__restrict__ mrow,
+    const int32_t *__restrict__ mlag,
     const double *__restrict__ mw, const float *__restrict__ prev,
     float *__restrict__ gsum) {
   static_assert(MB <= 64 && MB % (2 * C) == 0, "chunks pair up in a block");
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(256 * (JT / JW)) void tile_gather_kernel(
   dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks / (B * n_tblk),
                   n_tblk, tile, b, tb);
   const int t0 = tb * (BS * R);
-  const int t_end = min(T, t0 + BS * R);
+  const int t_end = min(Tc, t0 + BS * R);
   const int64_t m_begin = tptr[tile], m_end = tptr[tile + 1];
   if (m_end <= m_begin) return;
   const int s0 = (int)(threadIdx.x / BS) * JW;  // first slot of this group
@@ -252,7 +253,7 @@ __global__ __launch_bounds__(256 * (JT / JW)) void tile_gather_kernel(
         const int n = min(__builtin_amdgcn_readlane(m.lag[k], idx) & kLagMask,
                           T);
         const __amdgpu_buffer_rsrc_t rs =
-            make_rsrc(src, n < t_end ? row_bytes : 0u);
+            make_rsrc(src, n < t_end ? (uint32_t)Tp * 4u : 0u);
 #pragma unroll
         for (int r = 0; r < R; ++r)
           v[c][k][r] = buffer_load(rs, bin_offset(tl + BS * r - n));
@@ -328,16 +329,17 @@ int launch_tile_shape(int64_t P, int64_t B, int64_t T, int64_t M,
                       const int64_t *tptr, const int64_t *grp_ptr,
                       const int32_t *mrow, const int32_t *mlag,
                       const double *mw, const float *prev, float *gsum,
-                      hipStream_t s) {
+                      const OrderStep *step, hipStream_t s) {
   constexpr int BS = 256;
+  const OrderSpan sp = span_of(step, T);
   const int64_t n_tiles = ceil_div(P, JT);
-  const int64_t nt = ceil_div(T, (int64_t)BS * R);
+  const int64_t nt = ceil_div((int64_t)sp.Tc, (int64_t)BS * R);
   const int64_t nb = n_tiles * B * nt;
   SPR_REQUIRE(nb < (int64_t)0x7fffffff, "exchange grid too large");
   SPR_REQUIRE(T < ((int64_t)1 << 29), "histogram too long (T >= 2^29)");
   hipLaunchKernelGGL((tile_gather_kernel<R, C, JT, JW, MB>),
                      dim3((unsigned)nb), dim3(BS * (JT / JW)), 0, s, P,
-                     (int)B, (int)T, (int)nt, nb, M, tptr, grp_ptr, mrow,
+                     (int)B, (int)T, sp.Tp, sp.Tc, (int)nt, nb, M, tptr, grp_ptr, mrow,
                      mlag, mw, prev, gsum);
   SPR_LAUNCH_CHECK();
   return SPR_OK;
@@ -347,12 +349,12 @@ int launch_tile_gather(int64_t P, int JT, int64_t B, int64_t T, int64_t M,
                        const int64_t *tptr, const int64_t *grp_ptr,
                        const int32_t *mrow, const int32_t *mlag,
                        const double *mw, const float *prev, float *gsum,
-                       hipStream_t s) {
+                       const OrderStep *step, hipStream_t s) {
   if (JT == 4)
     return launch_tile_shape<4, 1, 4, 4, 64>(P, B, T, M, tptr, grp_ptr, mrow,
-                                             mlag, mw, prev, gsum, s);
+                                             mlag, mw, prev, gsum, step, s);
   return launch_tile_shape<4, 1, 8, 4, 64>(P, B, T, M, tptr, grp_ptr, mrow,
-                                           mlag, mw, prev, gsum, s);
+                                           mlag, mw, prev, gsum, step, s);
 }
 
 // ---------------------------------------------------------------------
@@ -446,7 +448,7 @@ template <int R, int JT, int SMAX, bool DS>
 __global__ __launch_bounds__(64 * JT) __attribute__((
     amdgpu_waves_per_eu(lds_gather_waves_per_eu<R, DS>()))) void
 tile_lds_gather_kernel(
-    int64_t P, int B, int T, int n_tblk, int64_t nblocks, int64_t M,
+    int64_t P, int B, int T, int Tp, int n_tblk, int64_t nblocks, int64_t M,
     const int64_t *__restrict__ tptr, const int64_t *__restrict__ grp_ptr,
     const int64_t *__restrict__ gdiff, const int4 *__restrict__ mspan,
     const int32_t *__restrict__ mlag, const double *__restrict__ mw,
@@ -492,7 +494,8 @@ tile_lds_gather_kernel(
   const double *dw = DS ? mdw + ((int64_t)b * M + m_begin) * JT : nullptr;
   const int32_t *lagw = mlag + m_begin * JT;
   const int4 *span = mspan + m_begin;
-  const uint32_t row_bytes = (uint32_t)T * 4u;
+  const uint32_t row_bytes = (uint32_t)T * 4u;   // of a group's sums
+  const uint32_t src_bytes = (uint32_t)Tp * 4u;  // of a source row
   const int64_t bstride = (int64_t)B * T;
   auto n_at = [&](int mb) { return min(NB, n_tile - mb); };
 
@@ -517,7 +520,7 @@ tile_lds_gather_kernel(
     float *dst = &win(buf)[k][0];
     if (w0 >= 0) {
       const __amdgpu_buffer_rsrc_t rs = make_rsrc(
-          row + w0, w0 < T ? (uint32_t)(T - w0) * 4u : 0u);
+          row + w0, w0 < Tp ? (uint32_t)(Tp - w0) * 4u : 0u);
       const uint32_t vo = (uint32_t)lane * 4u;
       WindowDma<0, (NX < 16 ? NX : 16)>::run(rs, dst, vo);
 #pragma unroll
@@ -525,7 +528,7 @@ tile_lds_gather_kernel(
         if (x < TB / 64 || 64 * x < need)
           dma_dword(rs, dst + 64 * x, vo + 256u * (uint32_t)x);
     } else {
-      const __amdgpu_buffer_rsrc_t rs = make_rsrc(row, row_bytes);
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(row, src_bytes);
 #pragma unroll
       for (int x = 0; x < NX; ++x)
         if (x < TB / 64 || 64 * x < need)
@@ -636,7 +639,7 @@ tile_lds_gather_kernel(
       const int32_t row = __builtin_amdgcn_readfirstlane(meta[buf].row[idx]);
       const int32_t l = lagw[(int64_t)(mb + idx) * JT + k] & kLagMask;
       const __amdgpu_buffer_rsrc_t rs = make_rsrc(
-          prev + (int64_t)row * bstride + (int64_t)b * T, row_bytes);
+          prev + (int64_t)row * bstride + (int64_t)b * T, src_bytes);
       float v[R];
 #pragma unroll
       for (int r = 0; r < R; ++r)
@@ -749,15 +752,17 @@ int launch_tile_lds(int64_t P, int64_t B, int64_t T, int64_t M,
                     const int64_t *tptr, const int64_t *grp_ptr,
                     const int64_t *gdiff, const int32_t *mspan,
                     const int32_t *mlag, const double *mw, const double *mdw,
-                    const float *prev, float *gsum, hipStream_t s) {
+                    const float *prev, float *gsum, const OrderStep *step,
+                    hipStream_t s) {
+  const OrderSpan sp = span_of(step, T);
   const int64_t n_tiles = ceil_div(P, JT);
-  const int64_t nt = ceil_div(T, (int64_t)64 * R);
+  const int64_t nt = ceil_div((int64_t)sp.Tc, (int64_t)64 * R);
   const int64_t nb = n_tiles * B * nt;
   SPR_REQUIRE(nb < (int64_t)0x7fffffff, "exchange grid too large");
   SPR_REQUIRE(T < ((int64_t)1 << 29), "histogram too long (T >= 2^29)");
   hipLaunchKernelGGL((tile_lds_gather_kernel<R, JT, SMAX, DS>),
                      dim3((unsigned)nb), dim3(64 * JT), 0, s, P, (int)B,
-                     (int)T, (int)nt, nb, M, tptr, grp_ptr, gdiff,
+                     (int)T, sp.Tp, (int)nt, nb, M, tptr, grp_ptr, gdiff,
                      reinterpret_cast<const int4 *>(mspan), mlag, mw, mdw,
                      prev, gsum);
   SPR_LAUNCH_CHECK();
@@ -889,7 +894,7 @@ extern "C" int spr_exchange_gather_tiled(int64_t P, int64_t JT, int64_t B,
   SPR_REQUIRE(tptr && grp_ptr && mrow && mlag && mw && prev && gsum,
               "spr_exchange_gather_tiled: null pointer");
   return launch_tile_gather(P, (int)JT, B, T, M, tptr, grp_ptr, mrow, mlag,
-                            mw, prev, gsum, as_stream(stream));
+                            mw, prev, gsum, nullptr, as_stream(stream));
 }
 
 extern "C" int spr_exchange_gather_tiled_ds(
@@ -904,7 +909,7 @@ extern "C" int spr_exchange_gather_tiled_ds(
               "spr_exchange_gather_tiled_ds: null pointer");
   return launch_tile_lds<8, 16, 64, true>(P, B, T, M, tptr, gstart, gdiff,
                                           mspan, mlag, mw, mdw, prev, gsum,
-                                          as_stream(stream));
+                                          nullptr, as_stream(stream));
 }
 
 extern "C" int spr_exchange_gather_tiled_shape(
@@ -921,8 +926,26 @@ extern "C" int spr_exchange_gather_tiled_shape(
   if (R == 8)
     return launch_tile_lds<8, 16, 64, false>(P, B, T, M, tptr, grp_ptr,
                                              nullptr, mspan, mlag, mw,
-                                             nullptr, prev, gsum, s);
+                                             nullptr, prev, gsum, nullptr, s);
   return launch_tile_lds<16, 16, 64, false>(P, B, T, M, tptr, grp_ptr,
                                             nullptr, mspan, mlag, mw, nullptr,
-                                            prev, gsum, s);
+                                            prev, gsum, nullptr, s);
+}
+
+int spr::gather_tiles(const spr_exchange_plan &p, int64_t T, const float *prev,
+                      float *gsum, const OrderStep &step, hipStream_t s) {
+  if (p.kind == SPR_PLAN_DS)
+    return launch_tile_lds<8, 16, 64, true>(
+        p.tile_slots, p.B, T, p.M, p.tptr, p.gstart, p.gdiff, p.mspan, p.mlag,
+        p.mw, p.mdw, prev, gsum, &step, s);
+  if (p.tile_rows != 16)
+    return launch_tile_gather(p.tile_slots, (int)p.tile_rows, p.B, T, p.M,
+                              p.tptr, p.gstart, p.mrow, p.mlag, p.mw, prev,
+                              gsum, &step, s);
+  auto go = [&](auto launch) {
+    return launch(p.tile_slots, p.B, T, p.M, p.tptr, p.gstart, nullptr,
+                  p.mspan, p.mlag, p.mw, nullptr, prev, gsum, &step, s);
+  };
+  if (p.tile_r == 16) return go(launch_tile_lds<16, 16, 64, false>);
+  return go(launch_tile_lds<8, 16, 64, false>);
 }

@@ -8,6 +8,7 @@ them like ``DirectionalRadiosityFast``.
 """
 from __future__ import annotations
 
+import ctypes
 import dataclasses
 
 import numpy as np
@@ -22,7 +23,8 @@ __all__ = [
     "patch2patch_ff_universal", "direction_map", "point_direction_index",
     "form_factors_with_directivity_dim", "source_energy",
     "receiver_energy", "collect", "energy_exchange", "ExchangePlan",
-    "GroupedPlan", "ExchangeState",
+    "GroupedPlan", "ExchangeState", "exchange_orders",
+    "exchange_sum",
 ]
 
 
@@ -898,6 +900,88 @@ def gather_groups(plan, shape, prev, gsum):
     call("spr_exchange_gather_grouped", P, B, T, plan.Vd,
          ptr(plan.row_ptr), ptr(plan.grp_ptr), ptr(plan.rowid),
          ptr(plan.lag), ptr(plan.scal), ptr(prev), ptr(gsum), stream_ptr())
+
+
+def _plan_struct(plan):
+    """The plan as the C entry points take it (spr_exchange_plan); it holds
+    the plan's tensors' addresses, so it lives no longer than the plan."""
+    S = _hip.ExchangePlanStruct
+    st = S(P=plan.P, D=plan.D, B=plan.B, Vd=plan.Vd)
+    arrays = dict(row_ptr=plan.row_ptr, lag=plan.lag)
+    if isinstance(plan, ExchangePlan):
+        st.kind = S.PAIRS
+        arrays.update(src=plan.src, dir=plan.dir, coef=plan.coef)
+    else:
+        st.kind = S.DS if plan.diffuse_specular else S.GROUPED
+        arrays.update(grp_ptr=plan.grp_ptr, grp_key=plan.grp_key,
+                      rowid=plan.rowid, scal=plan.scal, dscal=plan.dscal,
+                      rtab=plan.rtab)
+        tp = plan.tiles
+        if tp is not None:
+            st.tile_slots, st.tile_rows, st.tile_r, st.M = \
+                tp.P, tp.JT, tp.R, tp.M
+            arrays.update(tptr=tp.tptr, gstart=tp.gstart, gdiff=tp.gdiff,
+                          mspan=tp.mspan, mrow=tp.mrow, mlag=tp.mlag,
+                          mw=tp.mw, mdw=tp.mdw)
+    for name, t in arrays.items():
+        if t is not None:
+            setattr(st, name, ptr(t).value)
+    return st
+
+
+def _exchange(plan, e0d, d0, speed_of_sound, time_resolution, n_samples,
+              max_order, recurrence):
+    e0d = _f64(e0d)
+    d0 = _f64(d0)
+    P, D, B = e0d.shape
+    T, K = int(n_samples), max(int(max_order), 0)
+    dev = e0d.device
+    if plan is None or not plan.Vd:
+        K = 0
+    st = _plan_struct(plan) if K else _hip.ExchangePlanStruct(P=P, D=D, B=B)
+
+    def state():
+        return torch.empty((P, D, B, T), dtype=torch.float32, device=dev)
+    out = state()
+    gsum = None
+    if K and isinstance(plan, GroupedPlan):
+        gsum = torch.empty((max(plan.n_groups, 1), B, T),
+                           dtype=torch.float32, device=dev)
+    n0 = torch.empty(P, dtype=torch.int32, device=dev)
+    err = torch.zeros(1, dtype=torch.int32, device=dev)
+    head = (ctypes.addressof(st), T, K, ptr(e0d), ptr(d0),
+            float(speed_of_sound), float(time_resolution), ptr(out))
+    tail = (ptr(gsum), ptr(n0), ptr(err), stream_ptr())
+    if recurrence:
+        call("spr_exchange_sum", *head, ptr(state()) if K else None, *tail)
+    else:
+        work = [ptr(state()) if K else None for _ in range(3)]
+        call("spr_exchange_orders", *head, *work, *tail)
+    if int(err.item()):
+        raise IndexError(
+            "source-to-patch delay exceeds the histogram length")
+    return out
+
+
+def exchange_orders(plan, energy_0_directivity, distance_0, speed_of_sound,
+                    time_resolution, n_samples, max_order):
+    """The sum of orders 0..max_order on a plan (the total of
+    RadiosityFast.py:1037-1145) -> float32 [P,D,B,T]: the bits of stepping
+    an :class:`ExchangeState` and finalizing it.
+
+    ``plan`` may be None for max_order < 1.  Raises IndexError if a source
+    delay falls beyond the histogram (RadiosityFast.py:1069)."""
+    return _exchange(plan, energy_0_directivity, distance_0, speed_of_sound,
+                     time_resolution, n_samples, max_order, False)
+
+
+def exchange_sum(plan, energy_0_directivity, distance_0, speed_of_sound,
+                 time_resolution, n_samples, max_order):
+    """As :func:`exchange_orders` by the recurrence x_{k+1} = x_0 + A x_k:
+    half the memory or less and no pass over the total, the same error
+    against float64, last bits of its own."""
+    return _exchange(plan, energy_0_directivity, distance_0, speed_of_sound,
+                     time_resolution, n_samples, max_order, True)
 
 
 class ExchangeState:

@@ -797,16 +797,13 @@ class DirectionalRadiosityFast:
                 raise ValueError(
                     "baked form factors and source energy disagree in "
                     "directions or bands")
-            state = ops.ExchangeState(P, D, B, n_samples)
-            state.init(e0d, d0, speed_of_sound, etc_time_resolution)
+            plan = None
             if max_reflection_order >= 1:
                 plan = self._exchange_plan(speed_of_sound,
                                            etc_time_resolution)
-                for _ in range(int(max_reflection_order)):
-                    state.step(plan)
-            etc = state.finalize(out=state.hi)
-            state.check()
-            del state
+            etc = ops.exchange_orders(plan, e0d, d0, speed_of_sound,
+                                      etc_time_resolution, n_samples,
+                                      max_reflection_order)
             self._etc = etc
         self._etc_time_resolution = float(etc_time_resolution)
         self._speed_of_sound = float(speed_of_sound)

@@ -513,6 +513,7 @@ int spr_energy_exchange(int64_t T, int64_t P, int64_t D, int64_t B,
 
 typedef struct spr_exchange_plan {
   int64_t kind, P, D, B, Vd;
+  int64_t max_lag; /* no entry's delay is longer (bins) */
   int64_t tile_slots, tile_rows, tile_r, M;
   const int64_t *row_ptr;
   const int32_t *src, *lag, *dir;
@@ -531,15 +532,18 @@ typedef struct spr_exchange_plan {
  * total is kept as a compensated pair and rounded once, the bits of
  * spr_exchange_init, K orders of gather and spread with the total updated
  * every other order (per-pair plans: every order) and spr_exchange_finalize.
- * e0dir [P,D,B] and d0 [P] as for spr_exchange_init; lo, prev, cur
- * [P,D,B,T] and gsum [groups,B,T] (grouped and diffuse + specular plans)
- * are workspaces, not read, needed for K >= 1; n0 [P] (int32) receives each
- * patch's source bin.  Bit 0 of *err_flag is set where a source delay lies
- * outside the histogram (the reference raises IndexError); such a patch
- * injects nothing.  Enqueues kernels only: no allocation, no
- * synchronisation, safe to capture. */
+ * reach: every source bin lies below it (T if nothing is known); an order
+ * runs on the bins that energy can have reached, reach + k * max_lag of
+ * them, the others being 0.  e0dir [P,D,B] and d0 [P] as for
+ * spr_exchange_init; lo, prev, cur [P,D,B,T] and gsum [groups,B,T] (grouped
+ * and diffuse + specular plans) are workspaces, not read, needed for
+ * K >= 1; n0 [P] (int32) receives each patch's source bin.  Bit 0 of
+ * *err_flag is set where a source delay lies outside the histogram (the
+ * reference raises IndexError), bit 1 where it lies inside but not below
+ * reach; such a patch injects nothing.  Enqueues kernels only: no
+ * allocation, no synchronisation, safe to capture. */
 int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T, int64_t K,
-                        const double *e0dir, const double *d0, double c,
+                        int64_t reach, const double *e0dir, const double *d0, double c,
                         double dt, float *out, float *lo, float *prev,
                         float *cur, float *gsum, int32_t *n0, int *err_flag,
                         void *stream);
@@ -550,7 +554,7 @@ int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T, int64_t K,
  * float64 is that of spr_exchange_orders, but not every last bit agrees
  * with it.  Other arguments as there. */
 int spr_exchange_sum(const spr_exchange_plan *plan, int64_t T, int64_t K,
-                     const double *e0dir, const double *d0, double c,
+                     int64_t reach, const double *e0dir, const double *d0, double c,
                      double dt, float *out, float *tmp, float *gsum,
                      int32_t *n0, int *err_flag, void *stream);
 

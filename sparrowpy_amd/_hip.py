@@ -151,9 +151,9 @@ SYMBOLS = {
     "spr_energy_exchange": (_int, [_i64, _i64, _i64, _i64, _vp, _vp, _vp,
                                    _vp, _vp, _dbl, _dbl, _i64, _i64, _vp,
                                    _vp, _vp, _i64, _vp]),
-    "spr_exchange_orders": (_int, [_vp, _i64, _i64, _vp, _vp, _dbl, _dbl,
+    "spr_exchange_orders": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _dbl, _dbl,
                                    _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
-    "spr_exchange_sum": (_int, [_vp, _i64, _i64, _vp, _vp, _dbl, _dbl, _vp,
+    "spr_exchange_sum": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _dbl, _dbl, _vp,
                                 _vp, _vp, _vp, _vp, _vp]),
     "spr_plan_dense_hash": (_int, [_i64, _i64, _i64, _vp, _vp, _vp, _vp,
                                    _vp]),
@@ -171,7 +171,7 @@ class ExchangePlanStruct(ctypes.Structure):
     """``spr_exchange_plan`` (sparrow_hip.h)."""
 
     PAIRS, GROUPED, DS = 0, 1, 2
-    SIZES = ("kind", "P", "D", "B", "Vd", "tile_slots", "tile_rows",
+    SIZES = ("kind", "P", "D", "B", "Vd", "max_lag", "tile_slots", "tile_rows",
              "tile_r", "M")
     ARRAYS = ("row_ptr", "src", "lag", "dir", "coef", "grp_ptr", "grp_key",
               "rowid", "scal", "dscal", "rtab", "tptr", "gstart", "gdiff",

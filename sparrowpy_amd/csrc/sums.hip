@@ -17,6 +17,13 @@
 // buffers instead of four.  x_k is rounded to float32 once per order like
 // E_k, and A averages that rounding over all sources, so the error against
 // float64 is the same; its bits are not those of the order-by-order sum.
+//
+// Both run an order only on the bins that energy can have reached: order 0
+// ends before bin `reach`, and an order reaches at most the plan's longest
+// delay further.  Bins beyond are exact zeros of the reference's loop too;
+// they are cleared once, at the end.  In a room the sound crosses in 60 bins
+// an order of 2,000 bins is a third of the work on average over 20 orders
+// (328 patches, 16 directions, 4 bands: 8.48 -> 5.27 ms).
 #include <algorithm>
 
 #include "spr_common.hpp"
@@ -47,12 +54,13 @@ __global__ __launch_bounds__(256) void row_fill_kernel(
     if (e0dir) {
       const int64_t i = row / DB;
       n = delay_floor(d0[i], c, dt);
-      // a delay outside the histogram injects nothing and is reported
-      const bool bad = n < 0 || n >= T;
+      // a delay outside the histogram, or beyond the caller's reach, injects
+      // nothing and is reported
+      const int bad = n < 0 || n >= T ? 1 : n >= t1 ? 2 : 0;
       if (bad) n = -1;
       if (chunk == 0 && lane == 0 && row % DB == 0) {
         n0[i] = (int32_t)n;
-        if (bad) atomicOr(err, 1);
+        if (bad) atomicOr(err, bad);
       }
       const double e = e0dir[row];
       v = (float)e;
@@ -115,13 +123,14 @@ int check_plan(const char *name, const spr_exchange_plan &p) {
 // The arguments both forms share; *K becomes 0 where there is no order to
 // run (none asked for, or no pair of patches sees another).
 int check_call(const char *name, const spr_exchange_plan &p, int64_t T,
-               int64_t *K, const double *e0dir, const double *d0, double c,
-               double dt, const float *out, const float *gsum,
+               int64_t *K, int64_t reach, const double *e0dir,
+               const double *d0, double c, double dt, const float *out, const float *gsum,
                const int32_t *n0, const int *err_flag) {
   SPR_REQUIRE(p.P > 0 && p.D > 0 && p.B > 0 && p.Vd >= 0 && T > 0 && c > 0 &&
                   dt > 0,
               "%s: bad sizes", name);
   SPR_REQUIRE(e0dir && d0 && out && n0 && err_flag, "%s: null pointer", name);
+  SPR_REQUIRE(reach > 0 && p.max_lag >= 0, "%s: bad reach", name);
   if (*K < 0 || p.Vd == 0) *K = 0;
   if (!*K) return SPR_OK;
   SPR_REQUIRE(T < 0x3fffffff, "%s: histogram too long", name);
@@ -144,23 +153,27 @@ int gather(const spr_exchange_plan &p, int64_t T, const float *x, float *gsum,
 using namespace spr;
 
 extern "C" int spr_exchange_sum(const spr_exchange_plan *plan, int64_t T,
-                                int64_t K, const double *e0dir,
-                                const double *d0, double c, double dt,
+                                int64_t K, int64_t reach,
+                                const double *e0dir, const double *d0,
+                                double c, double dt,
                                 float *out, float *tmp, float *gsum,
                                 int32_t *n0, int *err_flag, void *stream) {
   SPR_REQUIRE(plan, "spr_exchange_sum: null plan");
   const spr_exchange_plan &p = *plan;
-  int rc = check_call("spr_exchange_sum", p, T, &K, e0dir, d0, c, dt, out,
+  int rc = check_call("spr_exchange_sum", p, T, &K, reach, e0dir, d0, c, dt, out,
                       gsum, n0, err_flag);
   if (rc) return rc;
   SPR_REQUIRE(!K || (tmp && tmp != out), "spr_exchange_sum: null pointer");
   hipStream_t s = as_stream(stream);
   float *x = K % 2 ? tmp : out, *y = K % 2 ? out : tmp;
-  OrderStep step{{(int)T, (int)T, 0, 0, 0}, {e0dir, n0}};
-  if ((rc = fill_rows(p, T, 0, T, e0dir, d0, c, dt, x, nullptr, nullptr, n0,
+  int64_t Tc = K ? std::min(T, reach) : T;
+  if ((rc = fill_rows(p, T, 0, Tc, e0dir, d0, c, dt, x, nullptr, nullptr, n0,
                       err_flag, s)))
     return rc;
+  OrderStep step{{0, 0, 0, 0, 0}, {e0dir, n0}};
   for (int64_t k = 0; k < K; ++k) {
+    step.span.Tp = (int)Tc;
+    step.span.Tc = (int)(Tc = std::min(T, Tc + p.max_lag));
     if (p.kind == SPR_PLAN_PAIRS) {
       rc = step_pairs(p.P, p.D, p.B, T, p.row_ptr, p.src, p.lag, p.dir,
                       p.coef, x, y, nullptr, nullptr, &step, s);
@@ -172,30 +185,36 @@ extern "C" int spr_exchange_sum(const spr_exchange_plan *plan, int64_t T,
     if (rc) return rc;
     std::swap(x, y);
   }
-  return SPR_OK;
+  return fill_rows(p, T, Tc, T, nullptr, nullptr, c, dt, out, nullptr, nullptr,
+                   nullptr, nullptr, s);
 }
 
 extern "C" int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T,
-                                   int64_t K, const double *e0dir,
-                                   const double *d0, double c, double dt,
+                                   int64_t K, int64_t reach,
+                                   const double *e0dir, const double *d0,
+                                   double c, double dt,
                                    float *out, float *lo, float *prev,
                                    float *cur, float *gsum, int32_t *n0,
                                    int *err_flag, void *stream) {
   SPR_REQUIRE(plan, "spr_exchange_orders: null plan");
   const spr_exchange_plan &p = *plan;
-  int rc = check_call("spr_exchange_orders", p, T, &K, e0dir, d0, c, dt, out,
+  int rc = check_call("spr_exchange_orders", p, T, &K, reach, e0dir, d0, c, dt, out,
                       gsum, n0, err_flag);
   if (rc) return rc;
   SPR_REQUIRE(!K || (lo && prev && cur && prev != cur),
               "spr_exchange_orders: null pointer");
   hipStream_t s = as_stream(stream);
-  if ((rc = fill_rows(p, T, 0, T, e0dir, d0, c, dt, out, K ? lo : nullptr,
+  int64_t Tc = K ? std::min(T, reach) : T;
+  if ((rc = fill_rows(p, T, 0, Tc, e0dir, d0, c, dt, out, K ? lo : nullptr,
                       prev, n0, err_flag, s)))
     return rc;
-  OrderStep step{{(int)T, (int)T, (int)T, 0, 0}, {}};
+  OrderStep step{{0, 0, (int)Tc, 0, 0}, {}};
+  OrderSpan &sp = step.span;
   for (int64_t k = 1; k <= K; ++k) {
-    OrderSpan &sp = step.span;
+    sp.Tp = (int)Tc;
+    sp.Tc = (int)(Tc = std::min(T, Tc + p.max_lag));
     sp.last = k == K;
+    bool add = true;
     if (p.kind == SPR_PLAN_PAIRS) {
       rc = step_pairs(p.P, p.D, p.B, T, p.row_ptr, p.src, p.lag, p.dir,
                       p.coef, prev, cur, out, lo, &step, s);
@@ -203,14 +222,17 @@ extern "C" int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T,
       // the total takes two orders at a time (the even ones' spread); an
       // odd last order is added on its own, as rounded
       rc = gather(p, T, prev, gsum, step, s);
-      const bool pair = k % 2 == 0, add = pair || sp.last;
+      const bool pair = k % 2 == 0;
+      add = pair || sp.last;
       sp.round = add && !pair;
       if (!rc)
         rc = spread_rows(p, T, gsum, pair ? prev : nullptr, cur,
                          add ? out : nullptr, add ? lo : nullptr, step, s);
     }
     if (rc) return rc;
+    if (add) sp.Tv = sp.Tc;
     std::swap(prev, cur);
   }
-  return SPR_OK;
+  return fill_rows(p, T, Tc, T, nullptr, nullptr, c, dt, out, nullptr, nullptr,
+                   nullptr, nullptr, s);
 }

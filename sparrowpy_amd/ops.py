@@ -285,6 +285,7 @@ class ExchangePlan:
     lag: torch.Tensor
     dir: torch.Tensor
     coef: torch.Tensor
+    max_lag: int = None  # longest delay (once an exchange needed it)
 
     @property
     def Vd(self):
@@ -385,6 +386,7 @@ class GroupedPlan:
     rtab: torch.Tensor
     dscal: torch.Tensor = None  # diffuse weights (diffuse + specular plan)
     tiles: "TilePlan" = None    # merged destination tiles (tile_plan)
+    max_lag: int = None         # as ExchangePlan.max_lag
 
     @property
     def Vd(self):
@@ -906,7 +908,10 @@ def _plan_struct(plan):
     """The plan as the C entry points take it (spr_exchange_plan); it holds
     the plan's tensors' addresses, so it lives no longer than the plan."""
     S = _hip.ExchangePlanStruct
-    st = S(P=plan.P, D=plan.D, B=plan.B, Vd=plan.Vd)
+    if plan.max_lag is None:
+        plan.max_lag = int((plan.lag & (GroupedPlan.LAST_IN_GROUP - 1))
+                           .max().item())
+    st = S(P=plan.P, D=plan.D, B=plan.B, Vd=plan.Vd, max_lag=plan.max_lag)
     arrays = dict(row_ptr=plan.row_ptr, lag=plan.lag)
     if isinstance(plan, ExchangePlan):
         st.kind = S.PAIRS
@@ -930,7 +935,7 @@ def _plan_struct(plan):
 
 
 def _exchange(plan, e0d, d0, speed_of_sound, time_resolution, n_samples,
-              max_order, recurrence):
+              max_order, reach, recurrence):
     e0d = _f64(e0d)
     d0 = _f64(d0)
     P, D, B = e0d.shape
@@ -949,7 +954,8 @@ def _exchange(plan, e0d, d0, speed_of_sound, time_resolution, n_samples,
                            dtype=torch.float32, device=dev)
     n0 = torch.empty(P, dtype=torch.int32, device=dev)
     err = torch.zeros(1, dtype=torch.int32, device=dev)
-    head = (ctypes.addressof(st), T, K, ptr(e0d), ptr(d0),
+    reach = T if reach is None else min(max(int(reach), 1), T)
+    head = (ctypes.addressof(st), T, K, reach, ptr(e0d), ptr(d0),
             float(speed_of_sound), float(time_resolution), ptr(out))
     tail = (ptr(gsum), ptr(n0), ptr(err), stream_ptr())
     if recurrence:
@@ -957,31 +963,36 @@ def _exchange(plan, e0d, d0, speed_of_sound, time_resolution, n_samples,
     else:
         work = [ptr(state()) if K else None for _ in range(3)]
         call("spr_exchange_orders", *head, *work, *tail)
-    if int(err.item()):
+    flags = int(err.item())
+    if flags & 1:
         raise IndexError(
             "source-to-patch delay exceeds the histogram length")
+    if flags:
+        raise ValueError("a source delay is not below reach")
     return out
 
 
 def exchange_orders(plan, energy_0_directivity, distance_0, speed_of_sound,
-                    time_resolution, n_samples, max_order):
+                    time_resolution, n_samples, max_order, reach=None):
     """The sum of orders 0..max_order on a plan (the total of
     RadiosityFast.py:1037-1145) -> float32 [P,D,B,T]: the bits of stepping
     an :class:`ExchangeState` and finalizing it.
 
-    ``plan`` may be None for max_order < 1.  Raises IndexError if a source
+    ``plan`` may be None for max_order < 1.  ``reach``: every source delay
+    in bins lies below it (None: nothing is known); orders run only on the
+    bins that energy can have reached by then.  Raises IndexError if a source
     delay falls beyond the histogram (RadiosityFast.py:1069)."""
     return _exchange(plan, energy_0_directivity, distance_0, speed_of_sound,
-                     time_resolution, n_samples, max_order, False)
+                     time_resolution, n_samples, max_order, reach, False)
 
 
 def exchange_sum(plan, energy_0_directivity, distance_0, speed_of_sound,
-                 time_resolution, n_samples, max_order):
+                 time_resolution, n_samples, max_order, reach=None):
     """As :func:`exchange_orders` by the recurrence x_{k+1} = x_0 + A x_k:
     half the memory or less and no pass over the total, the same error
     against float64, last bits of its own."""
     return _exchange(plan, energy_0_directivity, distance_0, speed_of_sound,
-                     time_resolution, n_samples, max_order, True)
+                     time_resolution, n_samples, max_order, reach, True)
 
 
 class ExchangeState:

@@ -137,6 +137,7 @@ class DirectionalRadiosityFast:
         self._bake = None
         self._plan = None
         self._etc = None
+        self._source_far = None   # no patch is further from the source
         # saved arrays, validated by check() before they are uploaded
         self._form_factors_in = _as_array(form_factors)
         self._form_factors_tilde_in = _as_array(form_factors_tilde)
@@ -162,6 +163,8 @@ class DirectionalRadiosityFast:
             self._dev["distance_patches_to_source"] = ops.as_dev(
                 np.asarray(distance_patches_to_source, float),
                 torch.float64)
+            self._source_far = float(np.max(distance_patches_to_source,
+                                            initial=0.))
         if energy_exchange_etc is not None:
             self._etc = ops.as_dev(np.asarray(energy_exchange_etc),
                                    torch.float32)
@@ -636,6 +639,9 @@ class DirectionalRadiosityFast:
             pos[0], g["centers"], g["points"], vis, self._air_attenuation,
             self.n_bins, g["wall_ids"], sources, brdf, bidx,
             receivers.shape[1])
+        # the farthest corner of the patches' bounding box
+        far = np.abs(self._patches_points - pos[0]).max(axis=(0, 1))
+        self._source_far = float(np.sqrt((far * far).sum()))
         self._dev["source_visibility"] = vis
         self._dev["energy_0"] = e0
         self._dev["energy_init_source"] = e0d
@@ -763,6 +769,14 @@ class DirectionalRadiosityFast:
         if plan.tiles is not None:
             plan.tiles.R = self.TILE_R
 
+    def _reach(self, speed_of_sound, time_resolution):
+        """A bin beyond every source delay (None: unknown); one bin more
+        than the farthest patch's, for the delays' rounding."""
+        far = self._source_far
+        if far is None or not np.isfinite(far):
+            return None
+        return int(far / speed_of_sound / time_resolution) + 2
+
     def calculate_energy_exchange(self, speed_of_sound, etc_time_resolution,
                                   etc_duration, max_reflection_order=-1,
                                   recalculate=False):
@@ -803,7 +817,9 @@ class DirectionalRadiosityFast:
                                            etc_time_resolution)
             etc = ops.exchange_orders(plan, e0d, d0, speed_of_sound,
                                       etc_time_resolution, n_samples,
-                                      max_reflection_order)
+                                      max_reflection_order,
+                                      self._reach(speed_of_sound,
+                                                  etc_time_resolution))
             self._etc = etc
         self._etc_time_resolution = float(etc_time_resolution)
         self._speed_of_sound = float(speed_of_sound)

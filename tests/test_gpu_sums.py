@@ -51,7 +51,12 @@ def _check(ops, r, plan, T, dt, K):
     ref = orc.exchange(T, r.energy_init_source, r.distance_patches_to_source,
                        r.pair_distances(), r.fft, r.p2o, 343., dt, K,
                        r.visible_patches, nthreads=8)
-    outs = [_np(f(*args)) for f in (ops.exchange_orders, ops.exchange_sum)]
+    # with the tightest reach, and with none
+    far = int(np.max(r.distance_patches_to_source) / 343. / dt) + 1
+    outs = [_np(f(*args, far)) for f in (ops.exchange_orders,
+                                         ops.exchange_sum)]
+    for f, out in zip((ops.exchange_orders, ops.exchange_sum), outs):
+        np.testing.assert_array_equal(_np(f(*args)), out)
     for out in outs:
         assert np.isfinite(out).all()
         assert (out[ref == 0] == 0).all()
@@ -92,7 +97,8 @@ def test_orders_give_the_stepped_total(ops, rooms, form, K):
 
 
 @pytest.mark.parametrize("form", ["pairs", "grouped", "grouped-16-8", "ds"])
-@pytest.mark.parametrize("T,K", [(1, 0), (75, 1), (1500, 2), (4099, 3)])
+@pytest.mark.parametrize("T,K", [(1, 0), (75, 1), (1500, 2), (4099, 3),
+                                 (2049, 6)])
 def test_sum_lengths_and_orders(ops, rooms, form, T, K):
     """One bin and no order, one order, delays of hundreds of bins beyond
     the kernels' lane strides (48 kHz), many time blocks."""
@@ -104,7 +110,10 @@ def test_sum_lengths_and_orders(ops, rooms, form, T, K):
 def test_sum_reports_delay_beyond_histogram(ops, rooms):
     r = rooms[16]
     plan = _plan(ops, r, "grouped", 1 / 2000)
+    args = (plan, r.energy_init_source, r.distance_patches_to_source, 343.,
+            1 / 2000)
     for f in (ops.exchange_orders, ops.exchange_sum):
         with pytest.raises(IndexError):
-            f(plan, r.energy_init_source, r.distance_patches_to_source, 343.,
-              1 / 2000, 3, 2)
+            f(*args, 3, 2)
+        with pytest.raises(ValueError):
+            f(*args, 100, 2, reach=3)

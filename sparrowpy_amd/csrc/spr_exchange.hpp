@@ -70,12 +70,14 @@ __device__ __forceinline__ void buffer_store(float v,
                                         (int)off, 0, 0);
 }
 
-__device__ __forceinline__ double readlane_f64(double v, int k) {
-  const int64_t u = __builtin_bit_cast(int64_t, v);
+__device__ __forceinline__ int64_t readlane_i64(int64_t u, int k) {
   const int32_t lo = __builtin_amdgcn_readlane((int32_t)u, k);
   const int32_t hi = __builtin_amdgcn_readlane((int32_t)(u >> 32), k);
+  return ((int64_t)hi << 32) | (int64_t)(uint32_t)lo;
+}
+__device__ __forceinline__ double readlane_f64(double v, int k) {
   return __builtin_bit_cast(double,
-                            ((int64_t)hi << 32) | (int64_t)(uint32_t)lo);
+                            readlane_i64(__builtin_bit_cast(int64_t, v), k));
 }
 
 // BRDF row of entry e (source i -> destination j): brdf_index[w_i] * S +

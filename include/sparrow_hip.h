@@ -498,10 +498,11 @@ int spr_energy_exchange(int64_t T, int64_t P, int64_t D, int64_t B,
                         void *stream);
 
 /* An exchange plan of one scene, as the plan builders above fill it, for
- * spr_exchange_orders and spr_exchange_sum.  kind SPR_PLAN_PAIRS: row_ptr, src, lag, dir, coef
- * (spr_plan_from_geometry / _from_dense).  SPR_PLAN_GROUPED: row_ptr,
- * grp_ptr, grp_key, rowid, lag, scal, rtab (spr_plan_grouped_fill).
- * SPR_PLAN_DS: the same with dscal, rtab not read (spr_plan_ds_fill).  With
+ * spr_exchange_orders and spr_exchange_sum.  kind SPR_PLAN_PAIRS: row_ptr,
+ * src, lag, dir, coef (spr_plan_from_geometry / _from_dense).
+ * SPR_PLAN_GROUPED: row_ptr, grp_ptr, grp_start (NULL if grp_key holds each
+ * group's first entry), grp_key, rowid, lag, scal, rtab
+ * (spr_plan_grouped_fill).  SPR_PLAN_DS: the same with dscal, rtab not read (spr_plan_ds_fill).  With
  * M > 0 the last two gather on destination tiles of tile_rows rows
  * (spr_plan_tile_order / _fill / _span): tptr, gstart [tile_slots], mlag,
  * mw, and mspan for 16 rows (tile_r 8 or 16 bins per lane) or mrow for 4
@@ -513,12 +514,15 @@ int spr_energy_exchange(int64_t T, int64_t P, int64_t D, int64_t B,
 
 typedef struct spr_exchange_plan {
   int64_t kind, P, D, B, Vd;
-  int64_t max_lag; /* no entry's delay is longer (bins) */
+  int64_t max_lag;    /* no entry's delay is longer (bins) */
+  int64_t max_groups; /* no destination has more groups */
+  int64_t order_shape; /* an order's launches: 0 as the sizes suggest, 2 or 4
+                        * one launch (bins per lane), -1 gather and spread */
   int64_t tile_slots, tile_rows, tile_r, M;
   const int64_t *row_ptr;
   const int32_t *src, *lag, *dir;
   const double *coef;
-  const int64_t *grp_ptr;
+  const int64_t *grp_ptr, *grp_start;
   const int32_t *grp_key, *rowid;
   const double *scal, *dscal, *rtab;
   const int64_t *tptr, *gstart, *gdiff;

@@ -171,11 +171,11 @@ class ExchangePlanStruct(ctypes.Structure):
     """``spr_exchange_plan`` (sparrow_hip.h)."""
 
     PAIRS, GROUPED, DS = 0, 1, 2
-    SIZES = ("kind", "P", "D", "B", "Vd", "max_lag", "tile_slots", "tile_rows",
-             "tile_r", "M")
-    ARRAYS = ("row_ptr", "src", "lag", "dir", "coef", "grp_ptr", "grp_key",
-              "rowid", "scal", "dscal", "rtab", "tptr", "gstart", "gdiff",
-              "mspan", "mrow", "mlag", "mw", "mdw")
+    SIZES = ("kind", "P", "D", "B", "Vd", "max_lag", "max_groups",
+             "order_shape", "tile_slots", "tile_rows", "tile_r", "M")
+    ARRAYS = ("row_ptr", "src", "lag", "dir", "coef", "grp_ptr", "grp_start",
+              "grp_key", "rowid", "scal", "dscal", "rtab", "tptr", "gstart",
+              "gdiff", "mspan", "mrow", "mlag", "mw", "mdw")
     _fields_ = [(n, _i64) for n in SIZES] + [(n, _vp) for n in ARRAYS]
 
 

@@ -18,7 +18,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libsparrow_hip.so")
 SOURCES = ["util.hip", "bake.hip", "exchange.hip", "tiles.hip",
-           "sums.hip", "collect.hip", "adjoint.hip"]
+           "rows.hip", "sums.hip", "collect.hip", "adjoint.hip"]
 ARCH = os.environ.get("SPARROW_HIP_ARCH", "gfx950")
 
 HIPFLAGS = [

@@ -43,7 +43,7 @@ __global__ void receiver_energy_kernel(int64_t NQ,
 // flight at a time.  One workgroup walking all patches in turn, each term
 // formed by every thread, was a serial chain of loads: 238 us on 148
 // patches (1 receiver, 1 band, 1,000 bins), 3.3 ms on 1,500 (16 receivers,
-// 8 bands, 6,000 bins; now 18 us and 2.4 ms.
+// 8 bands, 6,000 bins); now 18 us and 2.4 ms.
 constexpr int kCollectWaves = 16;
 constexpr int kCollectR = 4;  // bins per lane
 constexpr int kCollectBins = 64 * kCollectR;

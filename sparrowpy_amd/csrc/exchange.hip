@@ -2266,23 +2266,25 @@ DenseLayout dense_layout(int64_t P, int64_t D, int64_t B, int64_t T,
   take(L.grp_key, sizeof(int32_t) * L.gcap);
   take(L.scal, sizeof(double) * B * Vd);
   take(L.gsum, sizeof(float) * L.gcap * B * T);
-  take(L.bad, 2 * sizeof(int32_t));
+  take(L.bad, 3 * sizeof(int32_t));
   L.total = off;
   return L;
 }
 
-// far[0] = the largest delay of the plan's entries, far[1] = the largest
-// source delay (0 for one outside int32, which the exchange reports); one
+// most[0] = the largest delay of the plan's entries, most[1] = the largest
+// source delay (0 for one outside int32, which the exchange reports),
+// most[2] = the most groups of a destination (grp_ptr not null); one
 // workgroup, its loads 8 entries per thread at a time.
-__global__ __launch_bounds__(1024) void delay_max_kernel(
+__global__ __launch_bounds__(1024) void plan_max_kernel(
     int64_t P, const int64_t *__restrict__ row_ptr,
-    const int32_t *__restrict__ lag, const double *__restrict__ d0, double c,
-    double dt, int32_t *__restrict__ far) {
-  __shared__ int32_t m[2];
-  if (threadIdx.x < 2) m[threadIdx.x] = 0;
+    const int32_t *__restrict__ lag, const int64_t *__restrict__ grp_ptr,
+    const double *__restrict__ d0, double c, double dt,
+    int32_t *__restrict__ most) {
+  __shared__ int32_t m[3];
+  if (threadIdx.x < 3) m[threadIdx.x] = 0;
   __syncthreads();
   const int64_t n = row_ptr[P];
-  int32_t a = 0, b = 0;
+  int32_t a = 0, b = 0, g = 0;
   for (int64_t e = threadIdx.x; e < n; e += 8 * 1024) {
     int32_t v[8];
 #pragma unroll
@@ -2294,11 +2296,13 @@ __global__ __launch_bounds__(1024) void delay_max_kernel(
   for (int64_t i = threadIdx.x; i < P; i += 1024) {
     const int64_t q = delay_floor(d0[i], c, dt);
     if (q > b && q < 0x3fffffff) b = (int32_t)q;
+    if (grp_ptr) g = max(g, (int32_t)(grp_ptr[i + 1] - grp_ptr[i]));
   }
   atomicMax(&m[0], a);
   atomicMax(&m[1], b);
+  atomicMax(&m[2], g);
   __syncthreads();
-  if (threadIdx.x < 2) far[threadIdx.x] = m[threadIdx.x];
+  if (threadIdx.x < 3) most[threadIdx.x] = m[threadIdx.x];
 }
 
 // Groups of the last spr_energy_exchange call on this thread (0: the
@@ -2445,17 +2449,17 @@ int energy_exchange_on(const char *name, int64_t T, int64_t P, int64_t D,
       p.dir = dir;
       p.coef = coef;
     }
-    // the longest delay of a visible pair and of the source
-    int32_t far[2];
-    auto *far_dev = reinterpret_cast<int32_t *>(ws + L.bad);
-    hipLaunchKernelGGL(delay_max_kernel, dim3(1), dim3(1024), 0, s, P, row_ptr,
-                       lag, d0, c, dt, far_dev);
+    int32_t most[3];
+    auto *most_dev = reinterpret_cast<int32_t *>(ws + L.bad);
+    hipLaunchKernelGGL(plan_max_kernel, dim3(1), dim3(1024), 0, s, P, row_ptr,
+                       lag, p.grp_ptr, d0, c, dt, most_dev);
     SPR_LAUNCH_CHECK();
-    SPR_HIP(hipMemcpyAsync(far, far_dev, sizeof(far), hipMemcpyDeviceToHost,
-                           s));
+    SPR_HIP(hipMemcpyAsync(most, most_dev, sizeof(most),
+                           hipMemcpyDeviceToHost, s));
     SPR_HIP(hipStreamSynchronize(s));
-    p.max_lag = far[0];
-    reach = std::min<int64_t>(T, (int64_t)far[1] + 1);
+    p.max_lag = most[0];
+    p.max_groups = most[2];
+    reach = std::min<int64_t>(T, (int64_t)most[1] + 1);
   }
   if ((rc = spr_exchange_sum(&p, T, K, reach, e0dir, d0, c, dt, etc, prev,
                              reinterpret_cast<float *>(ws + L.gsum), n0, err,

@@ -1,0 +1,426 @@
+// One reflection order in one launch: group sums and their spread over the
+// directions, a destination's group sums staying in LDS.
+//
+// Reference: the per-order loop of _energy_exchange
+// (sparrowpy/classes/RadiosityFast.py:1073-1145), as grouped by
+// spr_plan_grouped_sort / _fill and spr_plan_ds_sort / _fill.
+//
+// The two-pass order (gather on destination tiles, then spread) is made for
+// large scenes: a tile's workgroup walks the sources of 16 destinations in
+// turn, so a room of ten tiles keeps twenty workgroups busy for as long as
+// one of them takes.  Here a workgroup of 8 waves takes one destination,
+// band and block of 64 R bins, and its waves share the destination's groups:
+// a 148-patch room (16 directions, 1 band, 512 bins) takes 26 us per order
+// instead of 96, launches included, a 328-patch one (4 bands) 82 instead
+// of 175.  Large scenes stay with the tiles, which read a source row once for
+// 16 destinations (1,072 patches, 6 bands, 2,048 bins: 2.5 ms against 3.4).
+#include <algorithm>
+
+#include "spr_common.hpp"
+#include "spr_exchange.hpp"
+
+namespace spr {
+namespace {
+
+constexpr int kRowWaves = 8;
+
+struct RowArgs {
+  int D, B, T, n_tblk;
+  int64_t nblocks, Vd;
+  OrderSpan sp;
+  Injection inj;  // order of the running sum (n0 set), else none
+  int max_groups;
+  const int64_t *row_ptr, *grp_ptr, *grp_start;
+  const int32_t *grp_key, *rowid, *lag;
+  const double *scal, *dscal, *rtab;
+  const float *prev;      // source histograms
+  const float *pair;      // added to the total with this order, or null
+  float *cur, *tot_hi, *tot_lo;  // no total: null
+};
+
+// LDS bytes of a workgroup: the group sums, and, where the waves share a sum
+// (the diffuse sum, or a destination's only group), its parts; then the
+// groups' BRDF rows, or the direction map of the diffuse + specular plan.
+inline size_t row_lds(const spr_exchange_plan &p, int R) {
+  const bool ds = p.kind == SPR_PLAN_DS;
+  size_t n = (size_t)p.max_groups * 64 * R * sizeof(float);
+  if (ds || p.max_groups == 1) n += (size_t)kRowWaves * 64 * R * sizeof(double);
+  return n + (ds ? 64 * sizeof(int32_t)
+                 : (size_t)p.max_groups * spr_padded_directions(p.D) *
+                       sizeof(double));
+}
+
+// Phase 1: each wave sums a run of whole groups with about an eighth of the
+// entries, C entries' rows in flight at a time (metadata one entry per lane,
+// broadcast with v_readlane), in float64, and writes each group's sum to
+// LDS as float32 -- the sums the two-pass order stores, bit for bit (of the
+// diffuse + specular plan the diffuse sum is formed in 8 parts).  Phase 2:
+// each wave sums the groups times their BRDF rows for its directions, in
+// group order, in float64, and writes the order and the total.
+// Bound by the latency of the row reads and the float64 multiply-adds; four
+// waves per SIMD (two workgroups per CU) at up to 128 registers.
+template <int DP, int R, bool DS>
+__global__ __launch_bounds__(64 * kRowWaves)
+    __attribute__((amdgpu_waves_per_eu(4))) void row_order_kernel(RowArgs a) {
+  constexpr int NW = kRowWaves, TB = 64 * R, C = 16 / R;
+  extern __shared__ char smem[];
+  float *gs = reinterpret_cast<float *>(smem);  // [max_groups][TB]
+  double *part = reinterpret_cast<double *>(gs + (size_t)a.max_groups * TB);
+  const bool one = !DS && a.max_groups == 1;  // the waves share the group
+  double *ct = part + (one ? NW * TB : 0);    // [max_groups][DP], !DS
+  const int B = a.B, D = a.D;
+  const int64_t T = a.T;
+  int64_t j;
+  int b, tb;
+  dest_major_tile(xcd_tile(blockIdx.x, a.nblocks),
+                  a.nblocks / ((int64_t)B * a.n_tblk), a.n_tblk, j, b, tb);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int lane = (int)threadIdx.x & 63;
+  const int t0 = tb * TB, t_end = min(a.sp.Tc, t0 + TB);
+  const int tl = t0 + lane;
+  const int64_t e_begin = a.row_ptr[j], e_end = a.row_ptr[j + 1];
+  const int64_t g0 = a.grp_ptr[j];
+  const int ng = (int)(a.grp_ptr[j + 1] - g0);
+  const uint32_t src_bytes = (uint32_t)a.sp.Tp * 4u;
+  const double *w = a.scal + (int64_t)b * a.Vd;
+  const double *w2 = DS ? a.dscal + (int64_t)b * a.Vd : w;
+
+  // the wave's groups [c_lo, c_hi) and entries [e_lo, e_hi): whole groups
+  // whose start lies in the wave's eighth of the entries
+  const int64_t cut_lo = e_begin + (e_end - e_begin) * wave / NW;
+  const int64_t cut_hi = e_begin + (e_end - e_begin) * (wave + 1) / NW;
+  auto start_of = [&](int g) -> int64_t {
+    return a.grp_start ? a.grp_start[g0 + g] : a.grp_key[g0 + g];
+  };
+  int c_lo = 0, c_hi = 0;
+  for (int i = 0; i < ng; i += 64) {
+    const bool in = i + lane < ng;
+    const int64_t st = start_of(in ? i + lane : ng - 1);
+    c_lo += __popcll(__ballot(in && st < cut_lo));
+    c_hi += __popcll(__ballot(in && st < cut_hi));
+  }
+  if (wave == NW - 1) c_hi = ng;
+  const int64_t e_lo = one          ? cut_lo
+                       : c_lo < ng ? start_of(c_lo)
+                                   : e_end;
+  const int64_t e_hi = one                         ? cut_hi
+                       : c_hi < ng && wave < NW - 1 ? start_of(c_hi)
+                                                    : e_end;
+
+  if (!DS) {
+    for (int i = (int)threadIdx.x; i < ng * DP; i += 64 * NW)
+      ct[i] = a.rtab[((int64_t)a.grp_key[g0 + i / DP] * B + b) * DP + i % DP];
+  } else {
+    int32_t *gmap = reinterpret_cast<int32_t *>(part + (size_t)NW * TB);
+    for (int d = (int)threadIdx.x; d < DP; d += 64 * NW) gmap[d] = -1;
+    __syncthreads();
+    for (int g = (int)threadIdx.x; g < ng - 1; g += 64 * NW) {
+      const int32_t k = a.grp_key[g0 + g];
+      if (k >= 0 && k < D) gmap[k] = g;
+    }
+  }
+
+  double S[R], Sd[DS ? R : 1];
+#pragma unroll
+  for (int r = 0; r < R; ++r) S[r] = 0.0;
+#pragma unroll
+  for (int r = 0; r < (DS ? R : 1); ++r) Sd[r] = 0.0;
+  int gl = c_lo;
+  struct Meta {
+    int32_t row, lag;
+    double w, w2;
+  };
+  auto load_meta = [&](int64_t e0) {
+    const int64_t e = e0 + lane;
+    const bool in = e < e_hi;
+    const int64_t ec = in ? e : e_hi - 1;
+    Meta m;
+    m.row = a.rowid[ec];
+    m.lag = in ? a.lag[ec] : kLagMask;  // past the end: no bins, no flag
+    m.w = in ? w[ec] : 0.0;
+    m.w2 = DS && in ? w2[ec] : 0.0;
+    return m;
+  };
+  auto fetch = [&](const Meta &m, int q, float (&v)[C][R]) {
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int32_t rk = __builtin_amdgcn_readlane(m.row, q + c);
+      const int32_t lk = __builtin_amdgcn_readlane(m.lag, q + c);
+      const int n = min(lk & kLagMask, (int)T);
+      const __amdgpu_buffer_rsrc_t rs =
+          make_rsrc(a.prev + ((int64_t)rk * B + b) * T,
+                    n < t_end ? src_bytes : 0u);
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        v[c][r] = buffer_load(rs, bin_offset(tl + 64 * r - n));
+    }
+  };
+  auto consume = [&](const Meta &m, int q, const float (&v)[C][R]) {
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const double wk = readlane_f64(m.w, q + c);
+      const double dk = DS ? readlane_f64(m.w2, q + c) : 0.0;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const double x = (double)v[c][r];
+        S[r] = fma(wk, x, S[r]);
+        if (DS) Sd[DS ? r : 0] = fma(dk, x, Sd[DS ? r : 0]);
+      }
+      if (!one && __builtin_amdgcn_readlane(m.lag, q + c) & kLastInGroup) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          gs[gl * TB + 64 * r + lane] = (float)S[r];
+          S[r] = 0.0;
+        }
+        gl += 1;
+      }
+    }
+  };
+  if (e_hi > e_lo) {  // uniform
+    Meta cur = load_meta(e_lo);
+    float va[C][R], vb[C][R];
+    for (int64_t blk = e_lo; blk < e_hi; blk += 64) {
+      const Meta next = load_meta(blk + 64);
+      const int n = (int)min((int64_t)64, e_hi - blk);
+      fetch(cur, 0, va);
+      for (int q = 0; q < n; q += 2 * C) {
+        if (q + C < n) fetch(cur, q + C, vb);
+        consume(cur, q, va);
+        if (q + C >= n) break;
+        if (q + 2 * C < n) fetch(cur, q + 2 * C, va);
+        consume(cur, q + C, vb);
+      }
+      cur = next;
+    }
+  }
+  if (DS || one) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      part[wave * TB + 64 * r + lane] = DS ? Sd[DS ? r : 0] : S[r];
+  }
+  __syncthreads();
+  // the shared sum of a bin, in wave order, as the two-pass order stores it
+  auto shared_sum = [&](int r) {
+    double sum = 0.0;
+#pragma unroll
+    for (int q = 0; q < NW; ++q) sum += part[q * TB + 64 * r + lane];
+    return (double)(float)sum;
+  };
+
+  // directions d0 .. d0+DW-1 and bin rows r0 .. r0+RW-1 of this wave
+  constexpr int NWD = DP < NW ? DP : NW, DW = DP / NWD;
+  constexpr int NWT = NW / NWD, RW = R < NWT ? 1 : R / NWT;
+  const int d0 = wave % NWD * DW, r0 = wave / NWD * RW;
+  if (r0 >= R) return;  // uniform
+  double acc[DW][RW];
+#pragma unroll
+  for (int d = 0; d < DW; ++d)
+#pragma unroll
+    for (int r = 0; r < RW; ++r) acc[d][r] = 0.0;
+  if (!DS) {
+    // (the BRDF rows by LDS broadcast; by scalar loads 10 % slower)
+#pragma unroll 4
+    for (int g = 0; g < ng; ++g) {
+      double x[RW];
+#pragma unroll
+      for (int r = 0; r < RW; ++r)
+        x[r] = one ? shared_sum(r0 + r)
+                   : (double)gs[g * TB + 64 * (r0 + r) + lane];
+#pragma unroll
+      for (int d = 0; d < DW; ++d) {
+        const double cd = ct[g * DP + d0 + d];
+#pragma unroll
+        for (int r = 0; r < RW; ++r) acc[d][r] = fma(cd, x[r], acc[d][r]);
+      }
+    }
+  } else {
+    const int32_t *gmap =
+        reinterpret_cast<const int32_t *>(part + (size_t)NW * TB);
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+      const double sd = shared_sum(r0 + r);
+#pragma unroll
+      for (int d = 0; d < DW; ++d) {
+        const int g = gmap[d0 + d];
+        acc[d][r] =
+            (g >= 0 ? (double)gs[g * TB + 64 * (r0 + r) + lane] : 0.0) + sd;
+      }
+    }
+  }
+  const int64_t dstride = (int64_t)B * T;
+  const int64_t base = j * D * dstride + (int64_t)b * T;
+  const uint32_t span = (uint32_t)(((int64_t)(D - 1) * dstride + T) * 4);
+  auto offset = [&](int d, int t, int end) {
+    return d < D && t < end ? (uint32_t)((int64_t)d * dstride + t) * 4u
+                            : kNoOffset;
+  };
+  const __amdgpu_buffer_rsrc_t rc =
+      make_rsrc(a.cur + base, a.sp.last ? 0u : span);
+  if (!a.tot_hi) {  // uniform
+    const int nj = a.inj.n0 ? a.inj.n0[j] : -1;
+#pragma unroll
+    for (int d = 0; d < DW; ++d)
+#pragma unroll
+      for (int r = 0; r < RW; ++r) {
+        const int t = tl + 64 * (r0 + r);
+        double v = acc[d][r];
+        if (t == nj && d0 + d < D)
+          v += a.inj.e0[(j * D + d0 + d) * B + b];
+        buffer_store((float)v, rc, offset(d0 + d, t, a.sp.Tc));
+      }
+    return;
+  }
+  const __amdgpu_buffer_rsrc_t rh = make_rsrc(a.tot_hi + base, span);
+  const __amdgpu_buffer_rsrc_t rl = make_rsrc(a.tot_lo + base, span);
+  const __amdgpu_buffer_rsrc_t wl =
+      make_rsrc(a.tot_lo + base, a.sp.last ? 0u : span);
+  const __amdgpu_buffer_rsrc_t rp =
+      make_rsrc((a.pair ? a.pair : a.cur) + base, a.pair ? span : 0u);
+  constexpr int NP = DW * RW, K = NP < 8 ? NP : 8;  // (d, r) pairs
+#pragma unroll
+  for (int p0 = 0; p0 < NP; p0 += K) {
+    float h[K], l[K], e[K];
+#pragma unroll
+    for (int q = 0; q < K; ++q) {
+      const int d = d0 + (p0 + q) / RW, t = tl + 64 * (r0 + (p0 + q) % RW);
+      h[q] = buffer_load(rh, offset(d, t, a.sp.Tv));
+      l[q] = buffer_load(rl, offset(d, t, a.sp.Tv));
+      e[q] = buffer_load(rp, offset(d, t, a.sp.Tp));
+    }
+#pragma unroll
+    for (int q = 0; q < K; ++q) {
+      const int d = (p0 + q) / RW, r = (p0 + q) % RW;
+      const uint32_t off = offset(d0 + d, tl + 64 * (r0 + r), a.sp.Tc);
+      const double v = a.sp.round ? (double)(float)acc[d][r] : acc[d][r];
+      double sum = (double)h[q] + (double)l[q];
+      sum += (double)e[q];
+      sum += v;
+      const float hs = (float)sum;
+      buffer_store((float)v, rc, off);
+      buffer_store(hs, rh, off);
+      buffer_store((float)(sum - (double)hs), wl, off);
+    }
+  }
+}
+
+template <int DP, int R, bool DS>
+int launch_row_order(const spr_exchange_plan &p, RowArgs a, hipStream_t s) {
+  const size_t lds = row_lds(p, R);
+  a.n_tblk = (int)ceil_div(a.sp.Tc, 64 * R);
+  a.nblocks = p.P * p.B * a.n_tblk;
+  SPR_REQUIRE(a.nblocks < (int64_t)0x7fffffff, "exchange grid too large");
+  if (lds > 65536)
+    SPR_HIP(hipFuncSetAttribute((const void *)row_order_kernel<DP, R, DS>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds));
+  hipLaunchKernelGGL((row_order_kernel<DP, R, DS>), dim3((unsigned)a.nblocks),
+                     dim3(64 * kRowWaves), lds, s, a);
+  SPR_LAUNCH_CHECK();
+  return SPR_OK;
+}
+
+template <int R, bool DS>
+int launch_dp(const spr_exchange_plan &p, const RowArgs &a, hipStream_t s) {
+  switch (spr_padded_directions(p.D)) {
+    case 1: return launch_row_order<1, R, DS>(p, a, s);
+    case 2: return launch_row_order<2, R, DS>(p, a, s);
+    case 4: return launch_row_order<4, R, DS>(p, a, s);
+    case 8: return launch_row_order<8, R, DS>(p, a, s);
+    case 16: return launch_row_order<16, R, DS>(p, a, s);
+    case 32: return launch_row_order<32, R, DS>(p, a, s);
+    case 64: return launch_row_order<64, R, DS>(p, a, s);
+  }
+  return fail(SPR_ERR_UNSUPPORTED, "row order: bad D");
+}
+
+}  // namespace
+
+// The shape of an order: R bins per lane here, or 0 for the two passes.  The
+// two costs are estimated in ns from what was measured on shoeboxes of 94 to
+// 1,072 patches, 1, 16 and 64 directions, 1 to 8 bands, 128 to 2,048 bins
+// (R = 1 and 8 were tried too: at most 10 % faster anywhere):
+// * here a workgroup costs 6 for its start, 0.2 per direction and bin row
+//   written, and per entry 0.06 (R = 4) or 0.048 (R = 2), 1.6 times that with
+//   two weights (an eighth of it per wave; shared out over the chip), more
+//   where there are fewer groups than waves;
+// * a tile's workgroup walks its entries in 130 per merged entry and 12 per
+//   entry, whatever its bins; a workgroup per CU runs at that pace, the
+//   chip takes 410 in that time;
+// * without tiles a workgroup (512 bins, or 2,048 with two weights) walks
+//   its row in 900 per entry, at a rate of 0.2 (0.65) per entry;
+// * two passes write and read the group sums, 0.0018 per group and bin, and
+//   take a launch more, 8,000.
+// Over 810 such cases the choice is within 1.5 % of the better one on
+// average (at most 1.4 times slower) and 1.6 times faster than two passes.
+int row_shape(const spr_exchange_plan &p, int64_t T, const OrderSpan &sp) {
+  const int64_t DP = spr_padded_directions(p.D);
+  if (p.order_shape < 0 || T >= ((int64_t)1 << 29) ||
+      p.D * p.B * T >= ((int64_t)1 << 29))
+    return 0;
+  const bool ds = p.kind == SPR_PLAN_DS;
+  // 64 directions at R = 4 keep 32 float64 sums per lane (with two weights,
+  // none: one pick per direction)
+  int R = p.order_shape ? (int)p.order_shape
+                        : (DP <= 32 || ds) && sp.Tc > 128 ? 4 : 2;
+  constexpr size_t kLds = 160 * 1024;
+  if (!p.order_shape && row_lds(p, R) > kLds / 2) R = 2;
+  const int64_t n = p.P * p.B, nb = n * ceil_div(sp.Tc, 64 * R);
+  if (row_lds(p, R) > kLds || nb >= (int64_t)0x7fffffff) return 0;
+  if (p.order_shape) return R;
+  const double E = (double)p.Vd / (double)p.P;
+  const double idle =
+      p.max_groups == 1 ? 1.0 : std::max(1.0, 8.0 / (double)p.max_groups);
+  const double here = (double)nb * (6.0 + 0.2 * (double)(DP * R) +
+                                    (R == 4 ? 0.06 : 0.048) *
+                                        (ds ? 1.6 : 1.0) * idle * E);
+  double two = 8000.0 + (double)(n * sp.Tc) *
+                            (0.0018 * (double)p.max_groups +
+                             0.0033 * (double)DP);
+  if (p.M) {
+    const double tiles = (double)(p.tile_slots / p.tile_rows);
+    const double blocks = tiles * (double)(p.B * ceil_div(sp.Tc, 512));
+    two += (130.0 * (double)p.M + 12.0 * (double)p.Vd) / tiles *
+           std::max(1.0, 0.55 + blocks / 410.0);
+  } else {
+    const double blocks = (double)(n * ceil_div(sp.Tc, ds ? 2048 : 512));
+    two += E * std::max(900.0, blocks * (ds ? 0.65 : 0.2));
+  }
+  return here < two ? R : 0;
+}
+
+int row_order(const spr_exchange_plan &p, int R, int64_t T, const float *prev,
+              const float *pair, float *cur, float *tot_hi, float *tot_lo,
+              const OrderStep &step, hipStream_t s) {
+  RowArgs a{};
+  a.D = (int)p.D;
+  a.B = (int)p.B;
+  a.T = (int)T;
+  a.Vd = p.Vd;
+  a.sp = step.span;
+  a.inj = step.inj;
+  a.max_groups = (int)p.max_groups;
+  a.row_ptr = p.row_ptr;
+  a.grp_ptr = p.grp_ptr;
+  a.grp_start = p.grp_start;
+  a.grp_key = p.grp_key;
+  a.rowid = p.rowid;
+  a.lag = p.lag;
+  a.scal = p.scal;
+  a.dscal = p.dscal;
+  a.rtab = p.rtab;
+  a.prev = prev;
+  a.pair = pair;
+  a.cur = cur;
+  a.tot_hi = tot_hi;
+  a.tot_lo = tot_lo;
+  const bool ds = p.kind == SPR_PLAN_DS;
+  switch (R) {
+    case 2:
+      return ds ? launch_dp<2, true>(p, a, s) : launch_dp<2, false>(p, a, s);
+    case 4:
+      return ds ? launch_dp<4, true>(p, a, s) : launch_dp<4, false>(p, a, s);
+  }
+  return fail(SPR_ERR_UNSUPPORTED, "spr_exchange_plan: order_shape is -1, 0, 2 or 4");
+}
+
+}  // namespace spr

@@ -127,6 +127,12 @@ int gather_tiles(const spr_exchange_plan &p, int64_t T, const float *prev,
 int spread_rows(const spr_exchange_plan &p, int64_t T, const float *gsum,
                 const float *prev, float *cur, float *tot_hi, float *tot_lo,
                 const OrderStep &step, hipStream_t s);
+// A whole order of a grouped or diffuse + specular plan in one launch
+// (rows.hip) at R bins per lane, and the R to take (0: the two passes).
+int row_shape(const spr_exchange_plan &p, int64_t T, const OrderSpan &sp);
+int row_order(const spr_exchange_plan &p, int R, int64_t T, const float *prev,
+              const float *pair, float *cur, float *tot_hi, float *tot_lo,
+              const OrderStep &step, hipStream_t s);
 int step_pairs(int64_t P, int64_t D, int64_t B, int64_t T,
                const int64_t *row_ptr, const int32_t *src, const int32_t *lag,
                const int32_t *dir, const double *coef, const float *prev,

@@ -140,11 +140,16 @@ int check_call(const char *name, const spr_exchange_plan &p, int64_t T,
   return check_plan(name, p);
 }
 
-// Pass 1 of an order on a grouped or diffuse + specular plan.
-int gather(const spr_exchange_plan &p, int64_t T, const float *x, float *gsum,
-           const OrderStep &step, hipStream_t s) {
-  return p.M ? gather_tiles(p, T, x, gsum, step, s)
-             : gather_rows(p, T, x, gsum, step, s);
+// One order of a grouped or diffuse + specular plan: y = A x (plus the
+// step's injection), the total updated with it and with `pair`.
+int order(const spr_exchange_plan &p, int64_t T, const float *x,
+          const float *pair, float *y, float *hi, float *lo, float *gsum,
+          const OrderStep &step, hipStream_t s) {
+  if (const int R = row_shape(p, T, step.span))
+    return row_order(p, R, T, x, pair, y, hi, lo, step, s);
+  const int rc = p.M ? gather_tiles(p, T, x, gsum, step, s)
+                     : gather_rows(p, T, x, gsum, step, s);
+  return rc ? rc : spread_rows(p, T, gsum, pair, y, hi, lo, step, s);
 }
 
 }  // namespace
@@ -178,9 +183,7 @@ extern "C" int spr_exchange_sum(const spr_exchange_plan *plan, int64_t T,
       rc = step_pairs(p.P, p.D, p.B, T, p.row_ptr, p.src, p.lag, p.dir,
                       p.coef, x, y, nullptr, nullptr, &step, s);
     } else {
-      rc = gather(p, T, x, gsum, step, s);
-      if (!rc)
-        rc = spread_rows(p, T, gsum, nullptr, y, nullptr, nullptr, step, s);
+      rc = order(p, T, x, nullptr, y, nullptr, nullptr, gsum, step, s);
     }
     if (rc) return rc;
     std::swap(x, y);
@@ -221,13 +224,11 @@ extern "C" int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T,
     } else {
       // the total takes two orders at a time (the even ones' spread); an
       // odd last order is added on its own, as rounded
-      rc = gather(p, T, prev, gsum, step, s);
       const bool pair = k % 2 == 0;
       add = pair || sp.last;
       sp.round = add && !pair;
-      if (!rc)
-        rc = spread_rows(p, T, gsum, pair ? prev : nullptr, cur,
-                         add ? out : nullptr, add ? lo : nullptr, step, s);
+      rc = order(p, T, prev, pair ? prev : nullptr, cur, add ? out : nullptr,
+                 add ? lo : nullptr, gsum, step, s);
     }
     if (rc) return rc;
     if (add) sp.Tv = sp.Tc;

@@ -285,7 +285,7 @@ class ExchangePlan:
     lag: torch.Tensor
     dir: torch.Tensor
     coef: torch.Tensor
-    max_lag: int = None  # longest delay (once an exchange needed it)
+    limits: list = None  # [longest delay], once an exchange needed it
 
     @property
     def Vd(self):
@@ -386,7 +386,8 @@ class GroupedPlan:
     rtab: torch.Tensor
     dscal: torch.Tensor = None  # diffuse weights (diffuse + specular plan)
     tiles: "TilePlan" = None    # merged destination tiles (tile_plan)
-    max_lag: int = None         # as ExchangePlan.max_lag
+    limits: list = None  # [longest delay, most groups of a destination]
+    order_shape: int = 0  # an order's launches (spr_exchange_plan)
 
     @property
     def Vd(self):
@@ -908,18 +909,22 @@ def _plan_struct(plan):
     """The plan as the C entry points take it (spr_exchange_plan); it holds
     the plan's tensors' addresses, so it lives no longer than the plan."""
     S = _hip.ExchangePlanStruct
-    if plan.max_lag is None:
-        plan.max_lag = int((plan.lag & (GroupedPlan.LAST_IN_GROUP - 1))
-                           .max().item())
-    st = S(P=plan.P, D=plan.D, B=plan.B, Vd=plan.Vd, max_lag=plan.max_lag)
+    if plan.limits is None:
+        most = [(plan.lag & (GroupedPlan.LAST_IN_GROUP - 1)).max()]
+        if isinstance(plan, GroupedPlan):
+            most.append((plan.grp_ptr[1:] - plan.grp_ptr[:-1]).max())
+        plan.limits = [int(n) for n in torch.stack(
+            [n.to(torch.int64) for n in most]).tolist()]
+    st = S(P=plan.P, D=plan.D, B=plan.B, Vd=plan.Vd, max_lag=plan.limits[0])
     arrays = dict(row_ptr=plan.row_ptr, lag=plan.lag)
     if isinstance(plan, ExchangePlan):
         st.kind = S.PAIRS
         arrays.update(src=plan.src, dir=plan.dir, coef=plan.coef)
     else:
         st.kind = S.DS if plan.diffuse_specular else S.GROUPED
-        arrays.update(grp_ptr=plan.grp_ptr, grp_key=plan.grp_key,
-                      rowid=plan.rowid, scal=plan.scal, dscal=plan.dscal,
+        st.max_groups, st.order_shape = plan.limits[1], plan.order_shape
+        arrays.update(grp_ptr=plan.grp_ptr, grp_start=plan.grp_start,
+                      grp_key=plan.grp_key, rowid=plan.rowid, scal=plan.scal, dscal=plan.dscal,
                       rtab=plan.rtab)
         tp = plan.tiles
         if tp is not None:

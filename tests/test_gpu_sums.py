@@ -39,7 +39,10 @@ def _plan(ops, r, form, dt):
         return pairs
     plan = _ds_plan(ops, r, 343., dt) if form.startswith("ds") else grouped
     tiles = form.split("-")[1:]
-    if tiles:
+    plan.order_shape = -1
+    if tiles and tiles[0] == "row":
+        plan.order_shape = int(tiles[1])
+    elif tiles:
         plan.tiles = ops.tile_plan(plan, int(tiles[0]), min_merge=0)
         plan.tiles.R = int(tiles[1]) if len(tiles) > 1 else 8
     return plan
@@ -68,7 +71,9 @@ def _check(ops, r, plan, T, dt, K):
 
 @pytest.mark.parametrize("form", ["pairs", "grouped", "grouped-4",
                                   "grouped-8", "grouped-16-8",
-                                  "grouped-16-16", "ds", "ds-16"])
+                                  "grouped-16-16", "grouped-row-2",
+                                  "grouped-row-4", "ds", "ds-16", "ds-row-2",
+                                  "ds-row-4"])
 @pytest.mark.parametrize("D", [4, 16, 24, 64])
 def test_sum_matches_oracle(ops, rooms, form, D):
     """Every plan form and padded direction count; 301 bins (no whole
@@ -80,7 +85,8 @@ def test_sum_matches_oracle(ops, rooms, form, D):
         _check(ops, r, plan, 301, dt, K)
 
 
-@pytest.mark.parametrize("form", ["pairs", "grouped-16-8", "ds"])
+@pytest.mark.parametrize("form", ["pairs", "grouped-16-8", "grouped-row-2",
+                                  "grouped-row-4", "ds"])
 @pytest.mark.parametrize("K", [1, 2, 7])
 def test_orders_give_the_stepped_total(ops, rooms, form, K):
     """One call gives the bits of stepping an ExchangeState."""
@@ -92,11 +98,13 @@ def test_orders_give_the_stepped_total(ops, rooms, form, K):
     st.init(r.energy_init_source, r.distance_patches_to_source, 343.,
             1 / 2000)
     for _ in range(K):
-        st.step(plan)
+        st.step(plan)   # always two passes
     np.testing.assert_array_equal(out, _np(st.finalize()))
 
 
-@pytest.mark.parametrize("form", ["pairs", "grouped", "grouped-16-8", "ds"])
+@pytest.mark.parametrize("form", ["pairs", "grouped", "grouped-16-8",
+                                  "grouped-row-2", "grouped-row-4", "ds",
+                                  "ds-row-2", "ds-row-4"])
 @pytest.mark.parametrize("T,K", [(1, 0), (75, 1), (1500, 2), (4099, 3),
                                  (2049, 6)])
 def test_sum_lengths_and_orders(ops, rooms, form, T, K):
@@ -105,6 +113,25 @@ def test_sum_lengths_and_orders(ops, rooms, form, T, K):
     r = rooms[16]
     dt = 1. if T == 1 else 1 / 2000 if T == 75 else 1 / 48000
     _check(ops, r, _plan(ops, r, form, dt), T, dt, K)
+
+
+@pytest.mark.parametrize("shape", [-1, 0, 2, 4])
+@pytest.mark.parametrize("walls", [[0], [0, 1], [0, 2], [0, 1, 2, 3]])
+def test_rows_without_brdf(ops, walls, shape):
+    """One direction and one group per destination (the waves share it), and
+    destinations with no source at all (walls in one plane, or facing away)."""
+    from conftest import make_oracle
+    room = testing.shoebox_room_stub(*ROOM)
+    r = make_oracle([room[w] for w in walls], .25)
+    r.set_air_attenuation(np.array([1e-3]), np.array([1000.]))
+    r.bake_geometry()
+    r.init_source_energy(SRC)
+    args = (r.visibility_matrix, r.patches_center, r.patches_area,
+            r.form_factors, r.p2o, r.air, r.patch_to_wall_ids, None, None,
+            None, 1, 1, 343., 1 / 2000)
+    plan = ops.GroupedPlan.from_geometry(*args)
+    plan.order_shape = shape
+    _check(ops, r, plan, 200, 1 / 2000, 4)
 
 
 def test_sum_reports_delay_beyond_histogram(ops, rooms):

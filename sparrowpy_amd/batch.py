@@ -309,8 +309,10 @@ class BatchedExchange:
                 parts = []
                 for x, off in zip(xs, offsets[:-1]):
                     r = self.items[x].radiosity
-                    o = ops.block_order(r._patches_points,
-                                        r._patch_to_wall_ids, block)
+                    o = ops.block_order(
+                        r._patches_points,
+                        ops.tile_surfaces(r._walls_points, r._walls_normal,
+                                          r._patch_to_wall_ids), block)
                     parts.append(np.where(o >= 0, o + off, -1))
                 order = np.concatenate(parts)
             plan.tiles = ops.tile_plan(plan, rows, order=order)

@@ -15,6 +15,7 @@
 // of 175.  Large scenes stay with the tiles, which read a source row once for
 // 16 destinations (1,072 patches, 6 bands, 2,048 bins: 2.5 ms against 3.4).
 #include <algorithm>
+#include <cmath>
 
 #include "spr_common.hpp"
 #include "spr_exchange.hpp"
@@ -340,12 +341,12 @@ int launch_dp(const spr_exchange_plan &p, const RowArgs &a, hipStream_t s) {
 // 1,072 patches, 1, 16 and 64 directions, 1 to 8 bands, 128 to 2,048 bins
 // (R = 1 and 8 were tried too: at most 10 % faster anywhere):
 // * here a workgroup costs 6 for its start, 0.2 per direction and bin row
-//   written, and per entry 0.06 (R = 4) or 0.048 (R = 2), 1.6 times that with
+//   written (0.13 with two weights), and per entry 0.06 (R = 4) or 0.048 (R = 2), 1.6 times that with
 //   two weights (an eighth of it per wave; shared out over the chip), more
 //   where there are fewer groups than waves;
-// * a tile's workgroup walks its entries in 130 per merged entry and 12 per
-//   entry, whatever its bins; a workgroup per CU runs at that pace, the
-//   chip takes 410 in that time;
+// * a tile's workgroup (512 bins, or 256 with two weights) walks its entries
+//   in 130 per merged entry and 12 per entry, whatever its bins; a workgroup
+//   per CU runs at that pace, the chip takes 410 (530) in that time;
 // * without tiles a workgroup (512 bins, or 2,048 with two weights) walks
 //   its row in 900 per entry, at a rate of 0.2 (0.65) per entry;
 // * two passes write and read the group sums, 0.0018 per group and bin, and
@@ -368,9 +369,11 @@ int row_shape(const spr_exchange_plan &p, int64_t T, const OrderSpan &sp) {
   if (row_lds(p, R) > kLds || nb >= (int64_t)0x7fffffff) return 0;
   if (p.order_shape) return R;
   const double E = (double)p.Vd / (double)p.P;
-  const double idle =
-      p.max_groups == 1 ? 1.0 : std::max(1.0, 8.0 / (double)p.max_groups);
-  const double here = (double)nb * (6.0 + 0.2 * (double)(DP * R) +
+  const double groups = (double)(p.max_groups - (ds ? 1 : 0));
+  const double idle = p.max_groups > 1 && groups < 8.0
+                          ? std::pow(8.0 / std::max(groups, 1.0), 1.3)
+                          : 1.0;
+  const double here = (double)nb * (6.0 + (ds ? 0.13 : 0.2) * (double)(DP * R) +
                                     (R == 4 ? 0.06 : 0.048) *
                                         (ds ? 1.6 : 1.0) * idle * E);
   double two = 8000.0 + (double)(n * sp.Tc) *
@@ -378,9 +381,10 @@ int row_shape(const spr_exchange_plan &p, int64_t T, const OrderSpan &sp) {
                              0.0033 * (double)DP);
   if (p.M) {
     const double tiles = (double)(p.tile_slots / p.tile_rows);
-    const double blocks = tiles * (double)(p.B * ceil_div(sp.Tc, 512));
+    const double blocks =
+        tiles * (double)(p.B * ceil_div(sp.Tc, ds ? 256 : 512));
     two += (130.0 * (double)p.M + 12.0 * (double)p.Vd) / tiles *
-           std::max(1.0, 0.55 + blocks / 410.0);
+           std::max(1.0, 0.55 + blocks / (ds ? 530.0 : 410.0));
   } else {
     const double blocks = (double)(n * ceil_div(sp.Tc, ds ? 2048 : 512));
     two += E * std::max(900.0, blocks * (ds ? 0.65 : 0.2));

@@ -435,18 +435,18 @@ struct BatchMeta {
   int32_t maxlag[NB];         // largest delay of the entry's present slots
 };
 
-// R = 8 without the diffuse sums: 80 KiB of LDS and at most 64 VGPRs, so
-// two workgroups share a CU (8 waves per SIMD): the sums are latency-bound
-// (each entry's reads, conversions and FP64 FMAs form one chain per wave),
-// and twice the waves hide twice the latency.
-template <int R, bool DS>
+// R = 8, or R = 4 with the diffuse sums: 80 (52) KiB of LDS and at most 64
+// VGPRs, so two workgroups share a CU (8 waves per SIMD): the sums are
+// latency-bound (each entry's reads, conversions and FP64 FMAs form one chain
+// per wave), and twice the waves hide twice the latency.
+template <int R>
 constexpr int lds_gather_waves_per_eu() {
-  return R == 8 && !DS ? 8 : 1;
+  return R <= 8 ? 8 : 1;
 }
 
 template <int R, int JT, int SMAX, bool DS>
 __global__ __launch_bounds__(64 * JT) __attribute__((
-    amdgpu_waves_per_eu(lds_gather_waves_per_eu<R, DS>()))) void
+    amdgpu_waves_per_eu(lds_gather_waves_per_eu<R>()))) void
 tile_lds_gather_kernel(
     int64_t P, int B, int T, int Tp, int n_tblk, int64_t nblocks, int64_t M,
     const int64_t *__restrict__ tptr, const int64_t *__restrict__ grp_ptr,
@@ -745,8 +745,11 @@ tile_lds_gather_kernel(
 // canyon (T = 6,000, 4 x 4 blocks, 1.71 M merged entries): R = 8 98 ms,
 // R = 16 108 ms; with the metadata broadcast by v_readlane from per-lane
 // loads instead of staged in LDS, and the windows staged through
-// registers, R = 16 took 131 ms.  The diffuse + specular plan runs R = 8
-// with one workgroup per CU (its second sums need 95 VGPRs).
+// registers, R = 16 took 131 ms.  The diffuse + specular plan runs R = 4:
+// with its second sums R = 8 needs 95 VGPRs, one workgroup per CU.  Shoebox
+// with a BRDF per patch (1,072 patches, 16 directions, 6 bands, whole orders):
+// 6,000 bins row by row 12.1 ms, R = 8 10.1 ms, R = 4 9.8 ms; 300 bins 3.35,
+// 0.89, 0.90 ms; with 64 directions 20.2, 18.8, 18.6 and 3.75, 1.45, 1.46 ms.
 template <int R, int JT, int SMAX, bool DS>
 int launch_tile_lds(int64_t P, int64_t B, int64_t T, int64_t M,
                     const int64_t *tptr, const int64_t *grp_ptr,
@@ -907,7 +910,7 @@ extern "C" int spr_exchange_gather_tiled_ds(
   SPR_REQUIRE(tptr && gstart && gdiff && mspan && mlag && mw && mdw && prev &&
                   gsum,
               "spr_exchange_gather_tiled_ds: null pointer");
-  return launch_tile_lds<8, 16, 64, true>(P, B, T, M, tptr, gstart, gdiff,
+  return launch_tile_lds<4, 16, 64, true>(P, B, T, M, tptr, gstart, gdiff,
                                           mspan, mlag, mw, mdw, prev, gsum,
                                           nullptr, as_stream(stream));
 }
@@ -935,7 +938,7 @@ extern "C" int spr_exchange_gather_tiled_shape(
 int spr::gather_tiles(const spr_exchange_plan &p, int64_t T, const float *prev,
                       float *gsum, const OrderStep &step, hipStream_t s) {
   if (p.kind == SPR_PLAN_DS)
-    return launch_tile_lds<8, 16, 64, true>(
+    return launch_tile_lds<4, 16, 64, true>(
         p.tile_slots, p.B, T, p.M, p.tptr, p.gstart, p.gdiff, p.mspan, p.mlag,
         p.mw, p.mdw, prev, gsum, &step, s);
   if (p.tile_rows != 16)

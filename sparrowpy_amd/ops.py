@@ -712,9 +712,11 @@ def block_order(patch_points, patch_to_wall_ids, block=(4, 4), pad=True):
     """Destination order in which every run of block[0]*block[1] slots is
     one block of neighbouring patches of one wall (the patches of a wall
     form a regular grid; blocks at a wall's edge are padded with empty
-    slots, -1).  With ``pad=False`` the blocks follow each other without
-    padding (a tile may then hold the end of one block and the start of
-    the next, but no empty slot).  For tile_plan(..., order=...)."""
+    slots, -1; where patches of several sizes share a cell of the grid, a
+    block takes several runs).  With ``pad=False`` the blocks follow each
+    other without padding (a tile may then hold the end of one block and
+    the start of the next, but no empty slot).  For tile_plan(...,
+    order=...)."""
     pts = np.asarray(patch_points, float)
     wall = np.asarray(patch_to_wall_ids)
     ctr = pts.mean(axis=1)
@@ -728,17 +730,33 @@ def block_order(patch_points, patch_to_wall_ids, block=(4, 4), pad=True):
         # grid coordinates along the wall's two in-plane axes
         size = np.abs(pts[idx, 2] - pts[idx, 0]).max(0)
         size = np.where(size > 0, size, 1.0)
-        u = np.rint((c[:, ax[0]] - c[:, ax[0]].min()) / size[ax[0]])
-        v = np.rint((c[:, ax[1]] - c[:, ax[1]].min()) / size[ax[1]])
-        u, v = u.astype(np.int64), v.astype(np.int64)
-        bu, bv = u // a, v // b
-        for key in sorted(set(zip(bu.tolist(), bv.tolist()))):
-            mask = (bu == key[0]) & (bv == key[1])
-            sel = idx[mask][np.lexsort((v[mask], u[mask]))]
-            out.extend(sel.tolist())
+        u, v = (np.rint((c[:, x] - c[:, x].min()) / size[x]).astype(np.int64)
+                for x in ax)
+        sel = np.lexsort((v, u, v // b, u // a))   # blocks, rows, patches
+        cell = (u // a)[sel] * (v.max() // b + 1) + (v // b)[sel]
+        cuts = np.flatnonzero(np.diff(cell)) + 1
+        for blk in np.split(idx[sel], cuts):
+            out.append(blk)
             if pad:
-                out.extend([-1] * (a * b - len(sel)))
-    return np.array(out, np.int64)
+                out.append(np.full(-len(blk) % (a * b), -1))
+    return np.concatenate(out).astype(np.int64)
+
+
+def tile_surfaces(walls_points, walls_normal, patch_to_wall_ids):
+    """Per patch the surface whose grid of patches block_order cuts into
+    blocks: its wall, or, where walls have fewer than 4 patches on average (a
+    surface split into one wall per patch, so that every patch has its own
+    BRDF: a block of 16 slots would be mostly empty), the first wall of its
+    plane: the same normal and offset, to 1e-6."""
+    wall = np.asarray(patch_to_wall_ids)
+    n = np.asarray(walls_normal, float)
+    if len(wall) >= 4 * len(n):
+        return wall
+    off = (n * np.asarray(walls_points, float)[:, 0]).sum(-1)
+    plane = np.round(np.concatenate([n, off[:, None]], 1) * 1e6) + 0.0
+    _, first, inv = np.unique(plane, axis=0, return_index=True,
+                              return_inverse=True)
+    return first[inv.reshape(-1)][wall]
 
 
 def diffuse_specular_tables(scattering, n_directions, n_bins, n_rows):

@@ -683,9 +683,11 @@ class DirectionalRadiosityFast:
         a, bb = blk
         if a * bb != self.TILE_ROWS:
             raise ValueError("TILE_BLOCK must hold TILE_ROWS patches")
-        return ops.block_order(self._patches_points,
-                               self._patch_to_wall_ids, (a, bb),
-                               pad=self.TILE_PAD)
+        return ops.block_order(
+            self._patches_points,
+            ops.tile_surfaces(self._walls_points, self._walls_normal,
+                              self._patch_to_wall_ids), (a, bb),
+            pad=self.TILE_PAD)
 
     def _exchange_plan(self, speed_of_sound, time_resolution, kind=None):
         """Plan of the exchange (cached per speed of sound and bin width).

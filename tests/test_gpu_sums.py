@@ -144,3 +144,35 @@ def test_sum_reports_delay_beyond_histogram(ops, rooms):
             f(*args, 3, 2)
         with pytest.raises(ValueError):
             f(*args, 100, 2, reach=3)
+
+
+def test_split_walls_give_the_rows_orders(ops):
+    """A BRDF per patch (one wall each): tiles across the walls of a plane,
+    the bits of the row-by-row plan."""
+    from sparrowpy_amd import DirectionalRadiosityFast, samplings
+    from sparrowpy_amd import brdf as B
+    from sparrowpy_amd.coordinates import Coordinates, FrequencyData
+    from sparrowpy_amd.geometry import Polygon, create_patches
+    rng = np.random.default_rng(0)
+    dirs = samplings.hemisphere(samplings.sph_gaussian(sh_order=3))
+    f = np.array([500.])
+    walls = [Polygon(p, w.up_vector, w.normal)
+             for w in testing.shoebox_room_stub(3, 2.5, 2)
+             for p in create_patches(w.pts, .5)]
+    r = DirectionalRadiosityFast.from_polygon(walls, .5)
+    for i in range(len(walls)):
+        r.set_wall_brdf([i], B.create_from_scattering(
+            dirs, dirs, FrequencyData(rng.uniform(.2, .8, (1, 1)), f),
+            FrequencyData(rng.uniform(.1, .3, (1, 1)), f)), dirs, dirs)
+    r.bake_geometry()
+    r.init_source_energy(Coordinates(*SRC))
+    plan = r._exchange_plan(343., 1 / 2000)
+    assert plan.diffuse_specular and plan.tiles is not None
+    plan.order_shape = -1
+    outs = []
+    for tiles in (plan.tiles, None):
+        plan.tiles = tiles
+        outs.append(_np(ops.exchange_orders(
+            plan, r._energy_init_source, r._distance_patches_to_source, 343.,
+            1 / 2000, 333, 5)))
+    np.testing.assert_array_equal(*outs)

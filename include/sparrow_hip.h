@@ -539,18 +539,20 @@ typedef struct spr_exchange_plan {
  * reach: every source bin lies below it (T if nothing is known); an order
  * runs on the bins that energy can have reached, reach + k * max_lag of
  * them, the others being 0.  e0dir [P,D,B] and d0 [P] as for
- * spr_exchange_init; lo, prev, cur [P,D,B,T] and gsum [groups,B,T] (grouped
- * and diffuse + specular plans) are workspaces, not read, needed for
- * K >= 1; n0 [P] (int32) receives each patch's source bin.  Bit 0 of
+ * spr_exchange_init; states: host array of K buffers [P,D,B,T], states[k]
+ * receiving order k's reached bins (two buffers in turn will do, or one of
+ * its own for every order to be kept); lo [P,D,B,T] and gsum [groups,B,T]
+ * (grouped and diffuse + specular plans) are workspaces, not read; all
+ * needed for K >= 1; n0 [P] (int32) receives each patch's source bin.  Bit 0 of
  * *err_flag is set where a source delay lies outside the histogram (the
  * reference raises IndexError), bit 1 where it lies inside but not below
  * reach; such a patch injects nothing.  Enqueues kernels only: no
  * allocation, no synchronisation, safe to capture. */
 int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T, int64_t K,
                         int64_t reach, const double *e0dir, const double *d0, double c,
-                        double dt, float *out, float *lo, float *prev,
-                        float *cur, float *gsum, int32_t *n0, int *err_flag,
-                        void *stream);
+                        double dt, float *out, float *lo,
+                        float *const *states, float *gsum, int32_t *n0,
+                        int *err_flag, void *stream);
 
 /* The same sum by the recurrence x_{k+1} = x_0 + A x_k, x_0 the injected
  * energy: two state buffers (out and tmp [P,D,B,T]) and no total.  Each x_k
@@ -561,6 +563,36 @@ int spr_exchange_sum(const spr_exchange_plan *plan, int64_t T, int64_t K,
                      int64_t reach, const double *e0dir, const double *d0, double c,
                      double dt, float *out, float *tmp, float *gsum,
                      int32_t *n0, int *err_flag, void *stream);
+
+/* Backward orders k0 + n - 1 .. k0 of the diffuse + specular adjoint:
+ * orders k0 + 1 .. k0 + n - 1 are recomputed from states[0] = order k0 into
+ * states[1 ..], then per order spr_direction_sum and spr_exchange_adjoint_ds,
+ * each on the bins that energy can have reached (reach as in
+ * spr_exchange_orders; only those bins of the mu's are formed and read).
+ * mu_next = dL/dE_{k0+n}; mu of order k goes to mu_even or mu_odd by k's
+ * parity; gsum as there, musum [P,B,T] a workspace. */
+int spr_adjoint_segment_ds(const spr_exchange_plan *plan, int64_t T,
+                           int64_t k0, int64_t n, int64_t reach,
+                           float *const *states, float *gsum,
+                           const int64_t *tgptr, const int32_t *tkey,
+                           const int32_t *tlag, const int32_t *tm,
+                           const double *twa, const double *twc,
+                           const float *lam, const float *mu_next,
+                           float *mu_even, float *mu_odd, float *musum,
+                           double *ga, void *stream);
+
+/* The same on a grouped plan (spr_grouped_table_grad, _spread_adjoint,
+ * _gather_adjoint): gsums: host array of n buffers [groups,B,T] for the
+ * orders' group sums, kept from the recomputing where they are n different
+ * ones, formed again where they are one; nu [groups,B,T] a workspace. */
+int spr_adjoint_segment_grouped(const spr_exchange_plan *plan, int64_t T,
+                                int64_t k0, int64_t n, int64_t reach,
+                                float *const *states, float *const *gsums,
+                                const int64_t *trow_ptr, const int32_t *tgrp,
+                                const int32_t *tlag, const double *tscal,
+                                const float *lam, const float *mu_next,
+                                float *mu_even, float *mu_odd, float *nu,
+                                double *gg, void *stream);
 
 /* hkey[e] (uint64, Vd entries) = hash of entry e's F~ row fft[src[e], j]
  * (destination j of row_ptr's row holding e) with every band divided by its

@@ -151,8 +151,14 @@ SYMBOLS = {
     "spr_energy_exchange": (_int, [_i64, _i64, _i64, _i64, _vp, _vp, _vp,
                                    _vp, _vp, _dbl, _dbl, _i64, _i64, _vp,
                                    _vp, _vp, _i64, _vp]),
-    "spr_exchange_orders": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _dbl, _dbl,
-                                   _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "spr_exchange_orders": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _dbl,
+                                   _dbl, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "spr_adjoint_segment_ds": (_int, [_vp, _i64, _i64, _i64, _i64, _vp, _vp,
+                                      _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                      _vp, _vp, _vp, _vp, _vp]),
+    "spr_adjoint_segment_grouped": (_int, [_vp, _i64, _i64, _i64, _i64, _vp,
+                                           _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                           _vp, _vp, _vp, _vp, _vp]),
     "spr_exchange_sum": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _dbl, _dbl, _vp,
                                 _vp, _vp, _vp, _vp, _vp]),
     "spr_plan_dense_hash": (_int, [_i64, _i64, _i64, _vp, _vp, _vp, _vp,
@@ -243,6 +249,13 @@ def ptr(t):
     if t.numel() == 0:
         return DevicePointer(_anchor(t.device))
     return DevicePointer(t)
+
+
+def ptr_array(tensors):
+    """Host array of the tensors' device pointers (a C ``float *const *``);
+    the caller keeps the tensors alive."""
+    return (ctypes.c_void_p * max(len(tensors), 1))(
+        *(ptr(t).value for t in tensors))
 
 
 def stream_ptr(stream=None):

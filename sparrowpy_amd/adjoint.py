@@ -27,6 +27,8 @@ forward order histograms recomputed from checkpoints kept every
 """
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
@@ -65,6 +67,55 @@ def _source_and_receivers(adj, r, source, receivers):
     adj.air = ops.as_dev(b["air"] if b["air"] is not None
                          else np.zeros(adj.B), torch.float64)
     adj.R = adj.rpts.shape[0]
+    # a bin beyond every source delay (the farthest corner of the patches'
+    # bounding box, and one bin for the delays' rounding)
+    far = np.abs(r._patches_points - pos).max(axis=(0, 1))
+    adj.reach = min(adj.T, int(np.sqrt((far * far).sum()) / adj.c / adj.dt)
+                    + 2)
+
+
+def _forward(adj):
+    """Receiver histograms [R, B, T] at the injection adj.e0dir on adj.plan,
+    and the orders kept every adj.every orders."""
+    total, checkpoints = ops._exchange(
+        adj.plan, adj.e0dir, adj.d0, adj.c, adj.dt, adj.T, adj.K, adj.reach,
+        lambda k: k % adj.every == 0)
+    # (without an order to run nothing reads it, but a record has order 0)
+    checkpoints.setdefault(0, total)
+    return ops.collect(total, adj.rpts, adj._geom["centers"], adj.ridx,
+                       adj.rfactor, adj.air, adj.c, adj.dt), checkpoints
+
+
+def _backward(adj, grad_hist, checkpoints, segment):
+    """mu_0 = dL/dE_0 (its bins below adj.reach) for dL/dH = ``grad_hist``:
+    ``segment(s, states, lam, mu, mu_even, mu_odd)`` runs the backward orders
+    of one checkpoint segment, states[0] being the checkpoint, the others
+    scratch."""
+    starts = sorted(checkpoints)
+    if not adj.plan.Vd:
+        starts = []                          # no pair: mu_0 = lambda
+    elif starts != list(range(0, max(adj.K, 1), adj.every)):
+        raise RuntimeError(f"{type(adj).__name__}.backward: the record's "
+                           "checkpoints do not cover the orders")
+    P, D, B, T = adj.P, adj.D, adj.B, adj.T
+
+    def state():
+        return torch.empty((P, D, B, T), dtype=torch.float32, device=adj.dev)
+    gH = ops.as_dev(grad_hist, torch.float32).contiguous()
+    lam = state()
+    call("spr_collect_adjoint", adj.R, P, D, B, T, ptr(gH), ptr(adj.rpts),
+         ptr(adj._geom["centers"]), ptr(adj.ridx), ptr(adj.rfactor),
+         ptr(adj.air), adj.c, adj.dt, ptr(lam), stream_ptr())
+    mu = lam                                 # mu_K
+    if not starts or not adj.K:
+        return mu
+    mus = (state(), state())                 # even orders, odd orders
+    scratch = [state() for _ in range(min(adj.every, adj.K) - 1)]
+    for s in reversed(starts):
+        n = min(s + adj.every, adj.K) - s
+        segment(s, [checkpoints[s]] + scratch[:n - 1], lam, mu, *mus)
+        mu = mus[s % 2]
+    return mu
 
 
 class ExchangeAdjoint:
@@ -148,17 +199,6 @@ class ExchangeAdjoint:
              ptr(self.e0dir), stream_ptr())
 
     # -- forward ----------------------------------------------------------------
-    def _order(self, state_prev, out, gsum):
-        """One order without the running total: out = A state_prev."""
-        p = self.plan
-        call("spr_exchange_gather_ds", self.P, self.B, self.T, p.Vd,
-             ptr(p.row_ptr), ptr(p.grp_ptr), ptr(p.rowid), ptr(p.lag),
-             ptr(p.scal), ptr(p.dscal), ptr(state_prev), ptr(gsum),
-             stream_ptr())
-        call("spr_exchange_spread_ds", self.P, self.D, self.B, self.T,
-             ptr(p.grp_ptr), ptr(p.grp_key), ptr(gsum), None, ptr(out),
-             None, None, stream_ptr())
-
     def forward(self, A, C):
         """Receiver histograms (float32 [R, B, T]) for tables (A, C).
 
@@ -169,22 +209,8 @@ class ExchangeAdjoint:
         A = ops.as_dev(A, torch.float64).detach().clone()
         C = ops.as_dev(C, torch.float64).detach().clone()
         self._set_tables(A, C)
-        st = ops.ExchangeState(self.P, self.D, self.B, self.T, self.dev)
-        st.init(self.e0dir, self.d0, self.c, self.dt)
-        checkpoints = {0: st.prev.clone()}
-        for k in range(self.K):
-            st.step(self.plan)
-            if (k + 1) % self.every == 0 and k + 1 < self.K:
-                checkpoints[k + 1] = st.prev.clone()
-        st.check()
+        H, checkpoints = _forward(self)
         self.last = ForwardRecord(A, C, checkpoints)
-        total = st.finalize(out=st.hi)
-        self._gsum = st.gsum if st.gsum is not None else torch.empty(
-            (max(self.plan.n_groups, 1), self.B, self.T), dtype=torch.float32,
-            device=self.dev)
-        H = ops.collect(total, self.rpts, self._geom["centers"], self.ridx,
-                        self.rfactor, self.air, self.c, self.dt)
-        del st, total
         return H
 
     # -- backward ---------------------------------------------------------------
@@ -200,45 +226,26 @@ class ExchangeAdjoint:
                                "(forward() was not called, or its record "
                                "was released)")
         self._set_tables(record.A, record.C)
-        checkpoints = record.checkpoints
         P, D, B, T, Vd = self.P, self.D, self.B, self.T, self.plan.Vd
         dev, p, adj = self.dev, self.plan, self.plan.adjoint
-        gH = ops.as_dev(grad_hist, torch.float32).contiguous()
-        shape = (P, D, B, T)
-        lam = torch.empty(shape, dtype=torch.float32, device=dev)
-        call("spr_collect_adjoint", self.R, P, D, B, T, ptr(gH),
-             ptr(self.rpts), ptr(self._geom["centers"]), ptr(self.ridx),
-             ptr(self.rfactor), ptr(self.air), self.c, self.dt, ptr(lam),
-             stream_ptr())
         twa = torch.empty((B, max(Vd, 1)), dtype=torch.float64, device=dev)
         twc = torch.empty_like(twa)
         call("spr_ds_transposed_weights", B, Vd, ptr(self.te), ptr(p.scal),
              ptr(p.dscal), ptr(twa), ptr(twc), stream_ptr())
         ga = torch.zeros((2, B, max(Vd, 1)), dtype=torch.float64, device=dev)
         musum = torch.empty((P, B, T), dtype=torch.float32, device=dev)
-        mu = lam.clone()                     # mu_K
-        mu_out = torch.empty_like(lam)
-        starts = sorted(checkpoints)
-        if starts != list(range(0, max(self.K, 1), self.every)):
-            raise RuntimeError("ExchangeAdjoint.backward: the record's "
-                               "checkpoints do not cover the orders")
-        for s in reversed(starts):
-            end = min(s + self.every, self.K)
-            states = [checkpoints[s]]   # E_s .. E_{end-1}
-            for k in range(s, end - 1):
-                nxt = torch.empty_like(lam)
-                self._order(states[-1], nxt, self._gsum)
-                states.append(nxt)
-            for k in range(end - 1, s - 1, -1):
-                call("spr_direction_sum", P, D, B, T, ptr(mu), ptr(musum),
-                     stream_ptr())
-                call("spr_exchange_adjoint_ds", P, D, B, T, Vd,
-                     ptr(self.tgptr), ptr(self.tkey), ptr(self.tlag),
-                     ptr(self.tm), ptr(twa), ptr(twc), ptr(lam), ptr(musum),
-                     ptr(mu), ptr(states[k - s]), ptr(mu_out), ptr(ga),
-                     stream_ptr())
-                mu, mu_out = mu_out, mu
-            del states
+        gsum = torch.empty((max(p.n_groups, 1), B, T), dtype=torch.float32,
+                           device=dev)
+        plan = ops._plan_struct(p) if Vd else None
+
+        def segment(s, states, lam, mu, mu_even, mu_odd):
+            call("spr_adjoint_segment_ds", ctypes.addressof(plan), T, s,
+                 len(states), self.reach, _hip.ptr_array(states), ptr(gsum),
+                 ptr(self.tgptr), ptr(self.tkey), ptr(self.tlag),
+                 ptr(self.tm), ptr(twa), ptr(twc), ptr(lam), ptr(mu),
+                 ptr(mu_even), ptr(mu_odd), ptr(musum), ptr(ga),
+                 stream_ptr())
+        mu = _backward(self, grad_hist, record.checkpoints, segment)
         gA = torch.zeros((self.NK, B), dtype=torch.float64, device=dev)
         gC = torch.zeros_like(gA)
         call("spr_ds_injection_grad", P, D, B, T, ptr(self.energy0),
@@ -377,37 +384,14 @@ class BRDFExchangeAdjoint:
         self.plan.rtab[:, :, :self.D] = t.permute(0, 2, 1)
         self.e0dir = (self.energy0[:, None, :] * t[self._k0]).contiguous()
 
-    def _gather(self, state, gsum):
-        ops.gather_groups(self.plan, (self.P, self.D, self.B, self.T), state,
-                          gsum)
-
-    def _order(self, state_prev, out, gsum):
-        """One order without the running total: out = A state_prev."""
-        p = self.plan
-        self._gather(state_prev, gsum)
-        call("spr_exchange_spread_grouped", self.P, self.D, self.B, self.T,
-             ptr(p.grp_ptr), ptr(p.grp_key), ptr(p.rtab), ptr(gsum),
-             ptr(out), None, None, stream_ptr())
-
     def forward(self, table):
         """Receiver histograms (float32 [R, B, T]) for ``table``; the call's
         checkpoints and table are kept as ``self.last`` (see
         :meth:`ExchangeAdjoint.forward`)."""
         table = ops.as_dev(table, torch.float64).detach().clone()
         self._set_table(table)
-        st = ops.ExchangeState(self.P, self.D, self.B, self.T, self.dev)
-        st.init(self.e0dir, self.d0, self.c, self.dt)
-        checkpoints = {0: st.prev.clone()}
-        for k in range(self.K):
-            st.step(self.plan)
-            if (k + 1) % self.every == 0 and k + 1 < self.K:
-                checkpoints[k + 1] = st.prev.clone()
-        st.check()
+        H, checkpoints = _forward(self)
         self.last = TableRecord(table, checkpoints)
-        total = st.finalize(out=st.hi)
-        H = ops.collect(total, self.rpts, self._geom["centers"], self.ridx,
-                        self.rfactor, self.air, self.c, self.dt)
-        del st, total
         return H
 
     def backward(self, grad_hist, record=None):
@@ -420,60 +404,29 @@ class BRDFExchangeAdjoint:
                                "record (forward() was not called, or its "
                                "record was released)")
         self._set_table(record.table)
-        checkpoints = record.checkpoints
-        starts = sorted(checkpoints)
-        if starts != list(range(0, max(self.K, 1), self.every)):
-            raise RuntimeError("BRDFExchangeAdjoint.backward: the record's "
-                               "checkpoints do not cover the orders")
         P, D, B, T = self.P, self.D, self.B, self.T
         p, dev = self.plan, self.dev
         G = p.n_groups
-        gH = ops.as_dev(grad_hist, torch.float32).contiguous()
-        shape = (P, D, B, T)
-        lam = torch.empty(shape, dtype=torch.float32, device=dev)
-        call("spr_collect_adjoint", self.R, P, D, B, T, ptr(gH),
-             ptr(self.rpts), ptr(self._geom["centers"]), ptr(self.ridx),
-             ptr(self.rfactor), ptr(self.air), self.c, self.dt, ptr(lam),
-             stream_ptr())
         DP = p.rtab.shape[2]
         gg = torch.zeros((max(G, 1), B, DP), dtype=torch.float64, device=dev)
-        gsum = torch.empty((max(G, 1), B, T), dtype=torch.float32, device=dev)
-        nu = torch.empty_like(gsum)
-        mu = lam.clone()                     # mu_K
-        mu_out = torch.empty_like(lam)
-        for s in reversed(starts):
-            end = min(s + self.every, self.K)
-            states = [checkpoints[s]]        # E_s .. E_{end-1}
-            # the group sums of orders s .. end-2 come out of recomputing
-            # the segment; kept (when there is room) instead of gathered
-            # again for the backward orders
-            keep = _fits(gsum, end - s - 1)
-            sums = {}
-            for k in range(s, end - 1):
-                nxt = torch.empty_like(lam)
-                gk = torch.empty_like(gsum) if keep else gsum
-                self._order(states[-1], nxt, gk)
-                if keep:
-                    sums[k] = gk
-                states.append(nxt)
-            for k in range(end - 1, s - 1, -1):
-                # mu = dL/dE_{k+1}; the group sums of order k -> k+1
-                gk = sums.pop(k, None)
-                if gk is None:
-                    gk = gsum
-                    self._gather(states[k - s], gk)
-                call("spr_grouped_table_grad", P, D, B, T, ptr(p.grp_ptr),
-                     ptr(mu), ptr(gk), ptr(gg), stream_ptr())
-                del gk
-                call("spr_grouped_spread_adjoint", P, D, B, T,
-                     ptr(p.grp_ptr), ptr(p.grp_key), ptr(p.rtab), ptr(mu),
-                     ptr(nu), stream_ptr())
-                call("spr_grouped_gather_adjoint", P, D, B, T, p.Vd,
-                     ptr(self.trow_ptr), ptr(self.tgrp), ptr(self.tlag),
-                     ptr(self.tscal), ptr(nu), ptr(lam), ptr(mu_out),
-                     stream_ptr())
-                mu, mu_out = mu_out, mu
-            del states
+        nu = torch.empty((max(G, 1), B, T), dtype=torch.float32, device=dev)
+        # the orders' group sums come out of recomputing a segment; kept
+        # (when there is room) instead of formed again for the backward
+        # orders
+        n = min(self.every, max(self.K, 1))
+        sums = [torch.empty_like(nu)
+                for _ in range(n if _fits(nu, n - 1) else 1)]
+        plan = ops._plan_struct(p) if p.Vd else None
+
+        def segment(s, states, lam, mu, mu_even, mu_odd):
+            m = len(states)
+            call("spr_adjoint_segment_grouped", ctypes.addressof(plan), T, s,
+                 m, self.reach, _hip.ptr_array(states),
+                 _hip.ptr_array((sums * m)[:m]), ptr(self.trow_ptr),
+                 ptr(self.tgrp), ptr(self.tlag), ptr(self.tscal), ptr(lam),
+                 ptr(mu), ptr(mu_even), ptr(mu_odd), ptr(nu), ptr(gg),
+                 stream_ptr())
+        mu = _backward(self, grad_hist, record.checkpoints, segment)
         gt = torch.zeros((self.NK, D, B), dtype=torch.float64, device=dev)
         call("spr_grouped_key_grad", G, D, B, ptr(p.grp_key), ptr(gg),
              ptr(gt), stream_ptr())

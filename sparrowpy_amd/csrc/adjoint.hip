@@ -83,14 +83,16 @@ __global__ void ds_injection_kernel(
   }
 }
 
-// musum[j,b,t] = sum_d mu[j,d,b,t] (float64 sum in direction order,
-// float32 result); 8 directions' loads are issued before they are added.
+// musum[j,b,t] = sum_d mu[j,d,b,t] for bins t < Tn (float64 sum in direction
+// order, float32 result); 8 directions' loads are issued before they are
+// added.
 __global__ void direction_sum_kernel(int64_t P, int64_t D, int64_t B,
-                                     int64_t T, const float *__restrict__ mu,
+                                     int64_t T, int64_t Tn,
+                                     const float *__restrict__ mu,
                                      float *__restrict__ musum) {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= P * B * T) return;
-  const int64_t t = q % T, b = (q / T) % B, j = q / (B * T);
+  if (q >= P * B * Tn) return;
+  const int64_t t = q % Tn, b = (q / Tn) % B, j = q / (B * Tn);
   const float *p = mu + (j * D * B + b) * T + t;  // element (j, 0, b, t)
   const int64_t stride = B * T;                  // next direction
   double s = 0.0;
@@ -103,7 +105,7 @@ __global__ void direction_sum_kernel(int64_t P, int64_t D, int64_t B,
     for (int k = 0; k < 8; ++k) s += (double)v[k];
   }
   for (; d < D; ++d) s += (double)p[d * stride];
-  musum[q] = (float)s;
+  musum[(j * B + b) * T + t] = (float)s;
 }
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -125,10 +127,12 @@ __device__ __forceinline__ double wave_sum(double v) {
 // add, so the result does not depend on their order).  A bin t + n beyond
 // the histogram is an out-of-range buffer offset and reads 0.  The
 // per-entry dot products are reduced over each wave and added (float64
-// atomics) by lanes 0 .. 2C-1.  Requires T < 2^29.
+// atomics) by lanes 0 .. 2C-1.  Requires T < 2^29.  Only bins that E_k can
+// hold energy in (t < Tk) are formed, from mu_next's bins below Tn (those of
+// E_{k+1}, at least Tk plus the longest delay or T).
 template <int R, int C>
 __global__ __launch_bounds__(256) void adjoint_ds_kernel(
-    int D, int B, int T, int n_tblk, int64_t nblocks, int64_t Vd,
+    int D, int B, int T, int Tk, int Tn, int n_tblk, int64_t nblocks, int64_t Vd,
     const int64_t *__restrict__ tgptr, const int32_t *__restrict__ tkey,
     const int32_t *__restrict__ tlag, const int32_t *__restrict__ tm,
     const double *__restrict__ twa, const double *__restrict__ twc,
@@ -145,7 +149,7 @@ __global__ __launch_bounds__(256) void adjoint_ds_kernel(
   if (q1 == q0) return;
   const int tl = tb * (BS * R) + (int)threadIdx.x;
   const int lane = (int)threadIdx.x & 63;
-  const uint32_t row_bytes = (uint32_t)T * 4u;
+  const uint32_t mu_bytes = (uint32_t)Tn * 4u, ek_bytes = (uint32_t)Tk * 4u;
   const double *wa = twa + (int64_t)b * Vd, *wc = twc + (int64_t)b * Vd;
   double *gda = ga + (int64_t)b * Vd, *gdc = ga + ((int64_t)B + b) * Vd;
   const int64_t srow = i * D;  // row (i, d') = srow + d'
@@ -159,13 +163,14 @@ __global__ __launch_bounds__(256) void adjoint_ds_kernel(
       const int32_t key = tkey[qc];
       const int64_t j = key & kDstMask, d = key >> 25, m = tm[qc];
       const int n = min(tlag[qc] & kLagMask, T);  // >= T: reads 0
-      const uint32_t sz = in ? row_bytes : 0u;
+      const uint32_t sz = in ? mu_bytes : 0u;
       const __amdgpu_buffer_rsrc_t rx =
           make_rsrc(musum + (j * B + b) * (int64_t)T, sz);
       const __amdgpu_buffer_rsrc_t ry =
           make_rsrc(munext + ((j * D + m) * B + b) * (int64_t)T, sz);
       const __amdgpu_buffer_rsrc_t re =
-          make_rsrc(ek + ((srow + d) * B + b) * (int64_t)T, sz);
+          make_rsrc(ek + ((srow + d) * B + b) * (int64_t)T,
+                    in ? ek_bytes : 0u);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int t = tl + BS * r;
@@ -201,7 +206,7 @@ __global__ __launch_bounds__(256) void adjoint_ds_kernel(
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             const int t = tl + BS * r;
-            if (t < T) unsafeAtomicAdd(o + t, (float)acc[r]);
+            if (t < Tk) unsafeAtomicAdd(o + t, (float)acc[r]);
             acc[r] = 0.0;
           }
         }
@@ -298,7 +303,7 @@ __global__ void injection_grad_kernel(
 // took 12.2 ms per call on the directional shoebox.)
 template <int DPT>
 __global__ __launch_bounds__(256) void grouped_spread_adjoint_kernel(
-    int D, int B, int T, int DP, int n_tblk,
+    int D, int B, int T, int Tn, int DP, int n_tblk,
     const int64_t *__restrict__ grp_ptr, const int32_t *__restrict__ grp_key,
     const double *__restrict__ rtab, const float *__restrict__ mu,
     float *__restrict__ nu) {
@@ -311,7 +316,7 @@ __global__ __launch_bounds__(256) void grouped_spread_adjoint_kernel(
   const int64_t g0 = grp_ptr[j], g1 = grp_ptr[j + 1];
   if (g0 == g1) return;  // uniform
   const int t = tb * 256 + (int)threadIdx.x;
-  const bool in = t < T;
+  const bool in = t < Tn;
   const int64_t dstride = (int64_t)B * T;
   const float *m = mu + (j * D * B + b) * (int64_t)T + (in ? t : 0);
   double v[DPT];
@@ -355,7 +360,7 @@ typedef double mfma_d4 __attribute__((ext_vector_type(4)));
 
 template <int NQ, int NR>
 __device__ __forceinline__ void table_grad_tile(
-    int D, int B, int T, int DP, int b, int64_t gt, int64_t g1,
+    int D, int B, int T, int Tn, int DP, int b, int64_t gt, int64_t g1,
     const float *__restrict__ mrow, const float *__restrict__ gsum,
     double *__restrict__ gg, float (&sg)[64][kTgChunk + 1],
     float (&sm)[64][kTgChunk + 1]) {
@@ -376,22 +381,22 @@ __device__ __forceinline__ void table_grad_tile(
 #pragma unroll
     for (int s = 0; s < 2 * NQ; ++s) {
       const int64_t g = gt + tid / TC + 8 * s;
-      pg[s] = (g < g1 && t < T) ? gsum[(g * B + b) * (int64_t)T + t] : 0.f;
+      pg[s] = (g < g1 && t < Tn) ? gsum[(g * B + b) * (int64_t)T + t] : 0.f;
     }
 #pragma unroll
     for (int s = 0; s < 2 * NR; ++s) {
       const int d = tid / TC + 8 * s;
-      pm[s] = (d < D && t < T) ? mrow[d * dstride + t] : 0.f;
+      pm[s] = (d < D && t < Tn) ? mrow[d * dstride + t] : 0.f;
     }
   };
   fetch(0);
-  for (int t0 = 0; t0 < T; t0 += TC) {
+  for (int t0 = 0; t0 < Tn; t0 += TC) {
 #pragma unroll
     for (int s = 0; s < 2 * NQ; ++s) sg[tid / TC + 8 * s][col] = pg[s];
 #pragma unroll
     for (int s = 0; s < 2 * NR; ++s) sm[tid / TC + 8 * s][col] = pm[s];
     __syncthreads();
-    if (t0 + TC < T) fetch(t0 + TC);  // uniform
+    if (t0 + TC < Tn) fetch(t0 + TC);  // uniform
     if (wave < NQ) {  // uniform per wave
 #pragma unroll 4
       for (int c = 0; c < TC; c += 4) {
@@ -417,7 +422,7 @@ __device__ __forceinline__ void table_grad_tile(
 
 template <int NR>
 __global__ __launch_bounds__(256) void grouped_table_grad_kernel(
-    int D, int B, int T, int DP, const int64_t *__restrict__ grp_ptr,
+    int D, int B, int T, int Tn, int DP, const int64_t *__restrict__ grp_ptr,
     const float *__restrict__ mu, const float *__restrict__ gsum,
     double *__restrict__ gg) {
   __shared__ float sg[64][kTgChunk + 1];
@@ -429,13 +434,17 @@ __global__ __launch_bounds__(256) void grouped_table_grad_kernel(
   for (int64_t gt = g0; gt < g1; gt += 64) {
     const int64_t left = g1 - gt;  // uniform
     if (left > 48)
-      table_grad_tile<4, NR>(D, B, T, DP, b, gt, g1, mrow, gsum, gg, sg, sm);
+      table_grad_tile<4, NR>(D, B, T, Tn, DP, b, gt, g1, mrow, gsum, gg, sg,
+                             sm);
     else if (left > 32)
-      table_grad_tile<3, NR>(D, B, T, DP, b, gt, g1, mrow, gsum, gg, sg, sm);
+      table_grad_tile<3, NR>(D, B, T, Tn, DP, b, gt, g1, mrow, gsum, gg, sg,
+                             sm);
     else if (left > 16)
-      table_grad_tile<2, NR>(D, B, T, DP, b, gt, g1, mrow, gsum, gg, sg, sm);
+      table_grad_tile<2, NR>(D, B, T, Tn, DP, b, gt, g1, mrow, gsum, gg, sg,
+                             sm);
     else
-      table_grad_tile<1, NR>(D, B, T, DP, b, gt, g1, mrow, gsum, gg, sg, sm);
+      table_grad_tile<1, NR>(D, B, T, Tn, DP, b, gt, g1, mrow, gsum, gg, sg,
+                             sm);
   }
 }
 
@@ -457,7 +466,7 @@ struct SpreadAdjMfma {
 
 template <int DP>
 __global__ __launch_bounds__(256) void grouped_spread_adjoint_mfma_kernel(
-    int D, int B, int T, int n_tblk, const int64_t *__restrict__ grp_ptr,
+    int D, int B, int T, int Tn, int n_tblk, const int64_t *__restrict__ grp_ptr,
     const int32_t *__restrict__ grp_key, const double *__restrict__ rtab,
     const float *__restrict__ mu, float *__restrict__ nu) {
   constexpr int KS = DP / 4, NT = SpreadAdjMfma<DP>::NT;
@@ -479,7 +488,7 @@ __global__ __launch_bounds__(256) void grouped_spread_adjoint_mfma_kernel(
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       const int d = 4 * s + kk, t = tw + 16 * nt + cc;
-      const bool ok = d < D && t < T;
+      const bool ok = d < D && t < Tn;
       const float v = m[ok ? d * dstride + t : 0];
       mv[s][nt] = ok ? v : 0.f;
     }
@@ -508,27 +517,29 @@ __global__ __launch_bounds__(256) void grouped_spread_adjoint_mfma_kernel(
       for (int r = 0; r < 4; ++r) {
         const int64_t g = gt + kk + 4 * r;
         const int t = tw + 16 * nt + cc;
-        if (g < g1 && t < T) nu[(g * B + b) * (int64_t)T + t] = (float)acc[nt][r];
+        if (g < g1 && t < Tn)
+          nu[(g * B + b) * (int64_t)T + t] = (float)acc[nt][r];
       }
     __syncthreads();
   }
 }
 
 // muout[r,b,t] = lam[r,b,t] + sum_{q in T(r)} tscal[b,q] nu[tgrp_q,b,t+n_q]
-// (float64 sum in transposed-entry order; a bin t + n beyond the histogram
-// reads 0 through the row's buffer descriptor and adds nothing).  A
-// workgroup per (source row r, band, 1,024 bins), 4 bins per lane, rows
+// for bins t < Tk (float64 sum in transposed-entry order; a bin t + n from Tn
+// on reads 0 through the row's buffer descriptor and adds nothing).  A
+// workgroup per (source row r, band, 256 R bins), R bins per lane, rows
 // taken direction-major (r = i*D + d for d slow, i fast: neighbouring
 // patches sending in one direction feed the same groups, whose nu rows
 // they then share through L2); the entries are taken C at a time, every
 // load of the chunk issued before any is summed.
+template <int R>
 __global__ __launch_bounds__(256) void grouped_gather_adjoint_kernel(
-    int64_t P, int D, int B, int T, int n_tblk, int64_t Vd,
+    int64_t P, int D, int B, int T, int Tk, int Tn, int n_tblk, int64_t Vd,
     const int64_t *__restrict__ trow_ptr,
     const int32_t *__restrict__ tgrp, const int32_t *__restrict__ tlag,
     const double *__restrict__ tscal, const float *__restrict__ nu,
     const float *__restrict__ lam, float *__restrict__ muout) {
-  constexpr int R = 4, C = 4;
+  constexpr int C = 4;
   const int64_t blk = blockIdx.x;
   const int tb = (int)(blk % n_tblk);
   const int b = (int)((blk / n_tblk) % B);
@@ -536,13 +547,13 @@ __global__ __launch_bounds__(256) void grouped_gather_adjoint_kernel(
   const int64_t r = (rd % P) * D + rd / P;
   const int64_t q0 = trow_ptr[r], q1 = trow_ptr[r + 1];
   const int64_t base = (r * B + b) * (int64_t)T;
-  const uint32_t row_bytes = (uint32_t)T * 4u;
+  const uint32_t row_bytes = (uint32_t)Tn * 4u;
   int t[R];
   double s[R];
 #pragma unroll
   for (int i = 0; i < R; ++i) {
     t[i] = tb * 256 * R + (int)threadIdx.x + 256 * i;
-    s[i] = t[i] < T ? (double)lam[base + t[i]] : 0.0;
+    s[i] = t[i] < Tk ? (double)lam[base + t[i]] : 0.0;
   }
   for (int64_t q = q0; q < q1; q += C) {
     float v[C][R];
@@ -567,7 +578,7 @@ __global__ __launch_bounds__(256) void grouped_gather_adjoint_kernel(
   }
 #pragma unroll
   for (int i = 0; i < R; ++i)
-    if (t[i] < T) muout[base + t[i]] = (float)s[i];
+    if (t[i] < Tk) muout[base + t[i]] = (float)s[i];
 }
 
 // gt[key_g,d,b] += gg[g,b,d] (float64 atomics: the groups of one BRDF row
@@ -601,12 +612,149 @@ __global__ void injection_table_grad_kernel(
                   energy0[p * B + b] * (double)mu0[q * T + n]);
 }
 
+// dst = src on bins [0, Tk) of every histogram row; a wave takes 256 bins of
+// one row.
+__global__ __launch_bounds__(256) void copy_rows_kernel(
+    int64_t rows, int64_t T, int64_t Tk, int64_t chunks,
+    const float *__restrict__ src, float *__restrict__ dst) {
+  const int lane = (int)threadIdx.x & 63;
+  const int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (q >= rows * chunks) return;
+  const int64_t row = q / chunks, t0 = q % chunks * 256 + lane;
+  float v[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int64_t t = t0 + 64 * r;
+    v[r] = src[row * T + (t < Tk ? t : 0)];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int64_t t = t0 + 64 * r;
+    if (t < Tk) dst[row * T + t] = v[r];
+  }
+}
+
 }  // namespace
+
+int direction_sum(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tn,
+                  const float *mu, float *musum, hipStream_t s) {
+  hipLaunchKernelGGL(direction_sum_kernel,
+                     dim3((unsigned)ceil_div(P * B * Tn, 256)), dim3(256), 0,
+                     s, P, D, B, T, Tn, mu, musum);
+  SPR_LAUNCH_CHECK();
+  return SPR_OK;
+}
+
+int adjoint_ds(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tk,
+               int64_t Tn, int64_t Vd, const int64_t *tgptr,
+               const int32_t *tkey, const int32_t *tlag, const int32_t *tm,
+               const double *twa, const double *twc, const float *lam,
+               const float *musum, const float *munext, const float *ek,
+               float *muout, double *ga, hipStream_t s) {
+  const int64_t chunks = ceil_div(Tk, 256), copies = P * D * B * chunks;
+  SPR_REQUIRE(ceil_div(copies, 4) < (int64_t)0x7fffffff,
+              "spr_exchange_adjoint_ds: grid too large");
+  hipLaunchKernelGGL(copy_rows_kernel, dim3((unsigned)ceil_div(copies, 4)),
+                     dim3(256), 0, s, P * D * B, T, Tk, chunks, lam, muout);
+  SPR_LAUNCH_CHECK();
+  // 8 bins per lane, 2 entries per chunk: each entry's two wave
+  // reductions (its table-gradient dot products) then cover 512 bins.
+  // Directional shoebox, order 30: backward 1.49 s with this shape; 1.66 s
+  // with R = 4, C = 4, 1.76 s with R = 8, C = 1, 1.78 s with R = 16, C = 1
+  // or R = 4, C = 2, 1.95 s with R = 16, C = 2, 2.68 s with R = 2, C = 4.
+  // Fewer bins per lane where 256 R would reach past Tk.
+  auto go = [&](auto kernel, int R) {
+    const int64_t nt = ceil_div(Tk, (int64_t)256 * R);
+    const int64_t nb = P * B * nt;
+    SPR_REQUIRE(nb < (int64_t)0x7fffffff,
+                "spr_exchange_adjoint_ds: grid too large");
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(256), 0, s, (int)D,
+                       (int)B, (int)T, (int)Tk, (int)Tn, (int)nt, nb, Vd,
+                       tgptr, tkey, tlag, tm, twa, twc, musum, munext, ek,
+                       muout, ga);
+    SPR_LAUNCH_CHECK();
+    return SPR_OK;
+  };
+  if (Tk <= 256) return go(adjoint_ds_kernel<1, 4>, 1);
+  if (Tk <= 512) return go(adjoint_ds_kernel<2, 4>, 2);
+  if (Tk <= 1024) return go(adjoint_ds_kernel<4, 2>, 4);
+  return go(adjoint_ds_kernel<8, 2>, 8);
+}
+
+int spread_adjoint(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tn,
+                   const int64_t *grp_ptr, const int32_t *grp_key,
+                   const double *rtab, const float *mu, float *nu,
+                   hipStream_t s) {
+  const int64_t DP = spr_padded_directions(D);
+  const int64_t nt = ceil_div(Tn, (int64_t)256);
+  const int64_t nb = P * B * nt;
+  SPR_REQUIRE(2 * nb < (int64_t)0x7fffffff,  // 128-bin blocks at D = 64
+              "spr_grouped_spread_adjoint: grid too large");
+  auto mfma = [&](auto kernel, int64_t bins) {
+    const int64_t n = ceil_div(Tn, bins);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(P * B * n)), dim3(256), 0, s,
+                       (int)D, (int)B, (int)T, (int)Tn, (int)n, grp_ptr,
+                       grp_key, rtab, mu, nu);
+  };
+  if (DP == 16)
+    mfma(grouped_spread_adjoint_mfma_kernel<16>, SpreadAdjMfma<16>::BINS);
+  else if (DP == 32)
+    mfma(grouped_spread_adjoint_mfma_kernel<32>, SpreadAdjMfma<32>::BINS);
+  else if (DP == 64)
+    mfma(grouped_spread_adjoint_mfma_kernel<64>, SpreadAdjMfma<64>::BINS);
+  else  // up to 8 directions: the vector kernel
+    hipLaunchKernelGGL((grouped_spread_adjoint_kernel<8>), dim3((unsigned)nb),
+                       dim3(256), 0, s, (int)D, (int)B, (int)T, (int)Tn,
+                       (int)DP, (int)nt, grp_ptr, grp_key, rtab, mu, nu);
+  SPR_LAUNCH_CHECK();
+  return SPR_OK;
+}
+
+int table_grad(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tn,
+               const int64_t *grp_ptr, const float *mu, const float *gsum,
+               double *gg, hipStream_t s) {
+  const int64_t DP = spr_padded_directions(D);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(P * B)), dim3(256), 0, s,
+                       (int)D, (int)B, (int)T, (int)Tn, (int)DP, grp_ptr, mu,
+                       gsum, gg);
+  };
+  if (D <= 16)
+    go(grouped_table_grad_kernel<1>);
+  else if (D <= 32)
+    go(grouped_table_grad_kernel<2>);
+  else if (D <= 48)
+    go(grouped_table_grad_kernel<3>);
+  else
+    go(grouped_table_grad_kernel<4>);
+  SPR_LAUNCH_CHECK();
+  return SPR_OK;
+}
+
+int gather_adjoint(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tk,
+                   int64_t Tn, int64_t Vd, const int64_t *trow_ptr,
+                   const int32_t *tgrp, const int32_t *tlag,
+                   const double *tscal, const float *nu, const float *lam,
+                   float *muout, hipStream_t s) {
+  auto go = [&](auto kernel, int R) {
+    const int64_t nt = ceil_div(Tk, (int64_t)256 * R);
+    const int64_t nb = P * D * B * nt;
+    SPR_REQUIRE(nb < (int64_t)0x7fffffff,
+                "spr_grouped_gather_adjoint: grid too large");
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(256), 0, s, P, (int)D,
+                       (int)B, (int)T, (int)Tk, (int)Tn, (int)nt, Vd, trow_ptr,
+                       tgrp, tlag, tscal, nu, lam, muout);
+    SPR_LAUNCH_CHECK();
+    return SPR_OK;
+  };
+  if (Tk <= 256) return go(grouped_gather_adjoint_kernel<1>, 1);
+  if (Tk <= 512) return go(grouped_gather_adjoint_kernel<2>, 2);
+  return go(grouped_gather_adjoint_kernel<4>, 4);
+}
+
 }  // namespace spr
 
 using namespace spr;
-
-extern "C" int64_t spr_padded_directions(int64_t D);  // exchange.hip
 
 extern "C" int spr_ds_weights(int64_t B, int64_t Vd, const int32_t *krow,
                               const double *wgt, const double *a,
@@ -667,11 +815,7 @@ extern "C" int spr_direction_sum(int64_t P, int64_t D, int64_t B, int64_t T,
   SPR_REQUIRE(P > 0 && D > 0 && B > 0 && T > 0,
               "spr_direction_sum: bad sizes");
   SPR_REQUIRE(mu && musum, "spr_direction_sum: null pointer");
-  hipLaunchKernelGGL(direction_sum_kernel,
-                     dim3((unsigned)ceil_div(P * B * T, 256)), dim3(256), 0,
-                     as_stream(stream), P, D, B, T, mu, musum);
-  SPR_LAUNCH_CHECK();
-  return SPR_OK;
+  return direction_sum(P, D, B, T, T, mu, musum, as_stream(stream));
 }
 
 extern "C" int spr_exchange_adjoint_ds(
@@ -689,24 +833,8 @@ extern "C" int spr_exchange_adjoint_ds(
               "spr_exchange_adjoint_ds: null pointer");
   SPR_REQUIRE(muout != munext && muout != lam && muout != ek,
               "spr_exchange_adjoint_ds: muout aliases an input");
-  // 8 bins per lane, 2 entries per chunk: each entry's two wave
-  // reductions (its table-gradient dot products) then cover 512 bins.
-  // Directional shoebox, order 30: backward 1.49 s with this shape; 1.66 s
-  // with R = 4, C = 4, 1.76 s with R = 8, C = 1, 1.78 s with R = 16, C = 1
-  // or R = 4, C = 2, 1.95 s with R = 16, C = 2, 2.68 s with R = 2, C = 4.
-  constexpr int R = 8, C = 2;
-  const int64_t nt = ceil_div(T, (int64_t)256 * R);
-  const int64_t nb = P * B * nt;
-  SPR_REQUIRE(nb < (int64_t)0x7fffffff, "spr_exchange_adjoint_ds: grid too "
-                                        "large");
-  hipStream_t s = as_stream(stream);
-  SPR_HIP(hipMemcpyAsync(muout, lam, sizeof(float) * P * D * B * T,
-                         hipMemcpyDeviceToDevice, s));
-  hipLaunchKernelGGL((adjoint_ds_kernel<R, C>), dim3((unsigned)nb), dim3(256),
-                     0, s, (int)D, (int)B, (int)T, (int)nt, nb, Vd, tgptr,
-                     tkey, tlag, tm, twa, twc, musum, munext, ek, muout, ga);
-  SPR_LAUNCH_CHECK();
-  return SPR_OK;
+  return adjoint_ds(P, D, B, T, T, T, Vd, tgptr, tkey, tlag, tm, twa, twc, lam,
+                    musum, munext, ek, muout, ga, as_stream(stream));
 }
 
 extern "C" int spr_ds_table_grad(int64_t B, int64_t Vd, const int32_t *te,
@@ -753,31 +881,8 @@ extern "C" int spr_grouped_spread_adjoint(int64_t P, int64_t D, int64_t B,
               "spr_grouped_spread_adjoint: bad sizes");
   SPR_REQUIRE(grp_ptr && grp_key && rtab && mu && nu,
               "spr_grouped_spread_adjoint: null pointer");
-  const int64_t nt = ceil_div(T, (int64_t)256);
-  const int64_t nb = P * B * nt;
-  SPR_REQUIRE(2 * nb < (int64_t)0x7fffffff,  // 128-bin blocks at D = 64
-              "spr_grouped_spread_adjoint: grid too large");
-  hipStream_t s = as_stream(stream);
-#define SPR_NU_MFMA(DPV)                                                      \
-  hipLaunchKernelGGL(                                                         \
-      (grouped_spread_adjoint_mfma_kernel<DPV>),                              \
-      dim3((unsigned)(P * B * ceil_div(T, (int64_t)SpreadAdjMfma<DPV>::BINS))), \
-      dim3(256), 0, s, (int)D, (int)B, (int)T,                                \
-      (int)ceil_div(T, (int64_t)SpreadAdjMfma<DPV>::BINS), grp_ptr, grp_key,  \
-      rtab, mu, nu)
-  if (DP == 16)
-    SPR_NU_MFMA(16);
-  else if (DP == 32)
-    SPR_NU_MFMA(32);
-  else if (DP == 64)
-    SPR_NU_MFMA(64);
-  else  // up to 8 directions: the vector kernel
-    hipLaunchKernelGGL((grouped_spread_adjoint_kernel<8>), dim3((unsigned)nb),
-                       dim3(256), 0, s, (int)D, (int)B, (int)T, (int)DP,
-                       (int)nt, grp_ptr, grp_key, rtab, mu, nu);
-#undef SPR_NU_MFMA
-  SPR_LAUNCH_CHECK();
-  return SPR_OK;
+  return spread_adjoint(P, D, B, T, T, grp_ptr, grp_key, rtab, mu, nu,
+                        as_stream(stream));
 }
 
 extern "C" int spr_grouped_table_grad(int64_t P, int64_t D, int64_t B,
@@ -791,22 +896,7 @@ extern "C" int spr_grouped_table_grad(int64_t P, int64_t D, int64_t B,
               "spr_grouped_table_grad: null pointer");
   SPR_REQUIRE(P * B < (int64_t)0x7fffffff,
               "spr_grouped_table_grad: grid too large");
-  hipStream_t s = as_stream(stream);
-#define SPR_TG(NRV)                                                           \
-  hipLaunchKernelGGL((grouped_table_grad_kernel<NRV>),                        \
-                     dim3((unsigned)(P * B)), dim3(256), 0, s, (int)D,        \
-                     (int)B, (int)T, (int)DP, grp_ptr, mu, gsum, gg)
-  if (D <= 16)
-    SPR_TG(1);
-  else if (D <= 32)
-    SPR_TG(2);
-  else if (D <= 48)
-    SPR_TG(3);
-  else
-    SPR_TG(4);
-#undef SPR_TG
-  SPR_LAUNCH_CHECK();
-  return SPR_OK;
+  return table_grad(P, D, B, T, T, grp_ptr, mu, gsum, gg, as_stream(stream));
 }
 
 extern "C" int spr_grouped_gather_adjoint(
@@ -820,16 +910,8 @@ extern "C" int spr_grouped_gather_adjoint(
   SPR_REQUIRE(trow_ptr && tgrp && tlag && tscal && nu && lam && muout,
               "spr_grouped_gather_adjoint: null pointer");
   SPR_REQUIRE(muout != lam, "spr_grouped_gather_adjoint: muout aliases lam");
-  const int64_t nt = ceil_div(T, (int64_t)1024);
-  const int64_t nb = P * D * B * nt;
-  SPR_REQUIRE(nb < (int64_t)0x7fffffff,
-              "spr_grouped_gather_adjoint: grid too large");
-  hipLaunchKernelGGL(grouped_gather_adjoint_kernel, dim3((unsigned)nb),
-                     dim3(256), 0, as_stream(stream), P, (int)D, (int)B,
-                     (int)T, (int)nt, Vd, trow_ptr, tgrp, tlag, tscal, nu,
-                     lam, muout);
-  SPR_LAUNCH_CHECK();
-  return SPR_OK;
+  return gather_adjoint(P, D, B, T, T, T, Vd, trow_ptr, tgrp, tlag, tscal, nu,
+                        lam, muout, as_stream(stream));
 }
 
 extern "C" int spr_grouped_key_grad(int64_t G, int64_t D, int64_t B,

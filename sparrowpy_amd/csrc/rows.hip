@@ -36,7 +36,8 @@ struct RowArgs {
   const double *scal, *dscal, *rtab;
   const float *prev;      // source histograms
   const float *pair;      // added to the total with this order, or null
-  float *cur, *tot_hi, *tot_lo;  // no total: null
+  float *cur, *tot_hi, *tot_lo;  // no total: null; group sums only: all null
+  float *gsum;                   // the group sums for the adjoint, or null
 };
 
 // LDS bytes of a workgroup: the group sums, and, where the waves share a sum
@@ -156,6 +157,14 @@ __global__ __launch_bounds__(64 * kRowWaves)
         v[c][r] = buffer_load(rs, bin_offset(tl + 64 * r - n));
     }
   };
+  // a group's sums to memory too, as the two-pass order stores them
+  auto keep_sums = [&](int g, const double (&x)[R]) {
+    const __amdgpu_buffer_rsrc_t os = make_rsrc(
+        a.gsum + ((g0 + g) * B + b) * T, (uint32_t)a.sp.Tc * 4u);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      buffer_store((float)x[r], os, (uint32_t)(tl + 64 * r) * 4u);
+  };
   auto consume = [&](const Meta &m, int q, const float (&v)[C][R]) {
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -169,10 +178,11 @@ __global__ __launch_bounds__(64 * kRowWaves)
       }
       if (!one && __builtin_amdgcn_readlane(m.lag, q + c) & kLastInGroup) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
+        for (int r = 0; r < R; ++r)
           gs[gl * TB + 64 * r + lane] = (float)S[r];
-          S[r] = 0.0;
-        }
+        if (a.gsum) keep_sums(gl, S);
+#pragma unroll
+        for (int r = 0; r < R; ++r) S[r] = 0.0;
         gl += 1;
       }
     }
@@ -199,6 +209,7 @@ __global__ __launch_bounds__(64 * kRowWaves)
     for (int r = 0; r < R; ++r)
       part[wave * TB + 64 * r + lane] = DS ? Sd[DS ? r : 0] : S[r];
   }
+  if (!a.cur && !one) return;  // uniform
   __syncthreads();
   // the shared sum of a bin, in wave order, as the two-pass order stores it
   auto shared_sum = [&](int r) {
@@ -207,6 +218,14 @@ __global__ __launch_bounds__(64 * kRowWaves)
     for (int q = 0; q < NW; ++q) sum += part[q * TB + 64 * r + lane];
     return (double)(float)sum;
   };
+
+  if (one && a.gsum && ng && wave == 0) {
+    double x[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) x[r] = shared_sum(r);
+    keep_sums(0, x);
+  }
+  if (!a.cur) return;  // uniform
 
   // directions d0 .. d0+DW-1 and bin rows r0 .. r0+RW-1 of this wave
   constexpr int NWD = DP < NW ? DP : NW, DW = DP / NWD;
@@ -394,7 +413,7 @@ int row_shape(const spr_exchange_plan &p, int64_t T, const OrderSpan &sp) {
 
 int row_order(const spr_exchange_plan &p, int R, int64_t T, const float *prev,
               const float *pair, float *cur, float *tot_hi, float *tot_lo,
-              const OrderStep &step, hipStream_t s) {
+              float *gsum, const OrderStep &step, hipStream_t s) {
   RowArgs a{};
   a.D = (int)p.D;
   a.B = (int)p.B;
@@ -417,6 +436,7 @@ int row_order(const spr_exchange_plan &p, int R, int64_t T, const float *prev,
   a.cur = cur;
   a.tot_hi = tot_hi;
   a.tot_lo = tot_lo;
+  a.gsum = gsum;
   const bool ds = p.kind == SPR_PLAN_DS;
   switch (R) {
     case 2:

@@ -132,11 +132,34 @@ int spread_rows(const spr_exchange_plan &p, int64_t T, const float *gsum,
 int row_shape(const spr_exchange_plan &p, int64_t T, const OrderSpan &sp);
 int row_order(const spr_exchange_plan &p, int R, int64_t T, const float *prev,
               const float *pair, float *cur, float *tot_hi, float *tot_lo,
-              const OrderStep &step, hipStream_t s);
+              float *gsum, const OrderStep &step, hipStream_t s);
 int step_pairs(int64_t P, int64_t D, int64_t B, int64_t T,
                const int64_t *row_ptr, const int32_t *src, const int32_t *lag,
                const int32_t *dir, const double *coef, const float *prev,
                float *cur, float *tot_hi, float *tot_lo, const OrderStep *step,
                hipStream_t s);
+
+// The passes of a backward order (adjoint.hip) on the bins below Tk that
+// E_k can hold energy in, and below Tn for E_{k+1}.
+int direction_sum(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tn,
+                  const float *mu, float *musum, hipStream_t s);
+int adjoint_ds(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tk,
+               int64_t Tn, int64_t Vd, const int64_t *tgptr,
+               const int32_t *tkey, const int32_t *tlag, const int32_t *tm,
+               const double *twa, const double *twc, const float *lam,
+               const float *musum, const float *munext, const float *ek,
+               float *muout, double *ga, hipStream_t s);
+int spread_adjoint(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tn,
+                   const int64_t *grp_ptr, const int32_t *grp_key,
+                   const double *rtab, const float *mu, float *nu,
+                   hipStream_t s);
+int table_grad(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tn,
+               const int64_t *grp_ptr, const float *mu, const float *gsum,
+               double *gg, hipStream_t s);
+int gather_adjoint(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tk,
+                   int64_t Tn, int64_t Vd, const int64_t *trow_ptr,
+                   const int32_t *tgrp, const int32_t *tlag,
+                   const double *tscal, const float *nu, const float *lam,
+                   float *muout, hipStream_t s);
 
 }  // namespace spr

@@ -141,15 +141,56 @@ int check_call(const char *name, const spr_exchange_plan &p, int64_t T,
 }
 
 // One order of a grouped or diffuse + specular plan: y = A x (plus the
-// step's injection), the total updated with it and with `pair`.
+// step's injection), the total updated with it and with `pair`.  gsum is
+// left with the group sums if keep is set (with y null: only they are formed).
 int order(const spr_exchange_plan &p, int64_t T, const float *x,
           const float *pair, float *y, float *hi, float *lo, float *gsum,
-          const OrderStep &step, hipStream_t s) {
+          bool keep, const OrderStep &step, hipStream_t s) {
   if (const int R = row_shape(p, T, step.span))
-    return row_order(p, R, T, x, pair, y, hi, lo, step, s);
+    return row_order(p, R, T, x, pair, y, hi, lo, keep ? gsum : nullptr, step,
+                     s);
   const int rc = p.M ? gather_tiles(p, T, x, gsum, step, s)
                      : gather_rows(p, T, x, gsum, step, s);
-  return rc ? rc : spread_rows(p, T, gsum, pair, y, hi, lo, step, s);
+  return rc || !y ? rc : spread_rows(p, T, gsum, pair, y, hi, lo, step, s);
+}
+
+// Bins that order k can hold energy in.
+int64_t reached(const spr_exchange_plan &p, int64_t T, int64_t reach,
+                int64_t k) {
+  return std::min(T, std::min(T, reach) + k * std::min(T, p.max_lag));
+}
+
+// The step from order k to k + 1, without a total.
+OrderStep step_from(const spr_exchange_plan &p, int64_t T, int64_t reach,
+                    int64_t k) {
+  return {{(int)reached(p, T, reach, k), (int)reached(p, T, reach, k + 1), 0, 0,
+           0},
+          {}};
+}
+
+// What both backward segments check; recomputes orders k0 + 1 .. k0 + n - 1
+// from states[0] = E_k0, gsums (if not null) receiving the group sums of the
+// orders k0 .. k0 + n - 2.
+int recompute(const char *name, const spr_exchange_plan *plan, int64_t kind,
+              int64_t T, int64_t k0, int64_t n, int64_t reach,
+              float *const *states, float *gsum, float *const *gsums,
+              hipStream_t s) {
+  SPR_REQUIRE(plan && plan->kind == kind, "%s: bad plan", name);
+  const spr_exchange_plan &p = *plan;
+  SPR_REQUIRE(p.P > 0 && p.P < ((int64_t)1 << 25) && p.D > 0 && p.D <= 64 &&
+                  p.B > 0 && p.Vd > 0 && T > 0 && T < ((int64_t)1 << 29) &&
+                  k0 >= 0 && n > 0 && reach > 0 && p.max_lag >= 0,
+              "%s: bad sizes", name);
+  int rc = check_plan(name, p);
+  if (rc) return rc;
+  for (int64_t i = 0; i < n; ++i)
+    SPR_REQUIRE(states[i] && (!gsums || gsums[i]), "%s: null pointer", name);
+  for (int64_t i = 0; i + 1 < n; ++i)
+    if ((rc = order(p, T, states[i], nullptr, states[i + 1], nullptr, nullptr,
+                    gsums ? gsums[i] : gsum, gsums != nullptr,
+                    step_from(p, T, reach, k0 + i), s)))
+      return rc;
+  return SPR_OK;
 }
 
 }  // namespace
@@ -183,7 +224,7 @@ extern "C" int spr_exchange_sum(const spr_exchange_plan *plan, int64_t T,
       rc = step_pairs(p.P, p.D, p.B, T, p.row_ptr, p.src, p.lag, p.dir,
                       p.coef, x, y, nullptr, nullptr, &step, s);
     } else {
-      rc = order(p, T, x, nullptr, y, nullptr, nullptr, gsum, step, s);
+      rc = order(p, T, x, nullptr, y, nullptr, nullptr, gsum, false, step, s);
     }
     if (rc) return rc;
     std::swap(x, y);
@@ -196,20 +237,23 @@ extern "C" int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T,
                                    int64_t K, int64_t reach,
                                    const double *e0dir, const double *d0,
                                    double c, double dt,
-                                   float *out, float *lo, float *prev,
-                                   float *cur, float *gsum, int32_t *n0,
-                                   int *err_flag, void *stream) {
+                                   float *out, float *lo,
+                                   float *const *states, float *gsum,
+                                   int32_t *n0, int *err_flag, void *stream) {
   SPR_REQUIRE(plan, "spr_exchange_orders: null plan");
   const spr_exchange_plan &p = *plan;
   int rc = check_call("spr_exchange_orders", p, T, &K, reach, e0dir, d0, c, dt, out,
                       gsum, n0, err_flag);
   if (rc) return rc;
-  SPR_REQUIRE(!K || (lo && prev && cur && prev != cur),
-              "spr_exchange_orders: null pointer");
+  SPR_REQUIRE(!K || (lo && states), "spr_exchange_orders: null pointer");
+  for (int64_t k = 0; k < K; ++k)
+    SPR_REQUIRE(states[k] && (k == 0 || states[k] != states[k - 1]),
+                "spr_exchange_orders: orders need a buffer each, two in turn "
+                "at least");
   hipStream_t s = as_stream(stream);
   int64_t Tc = K ? std::min(T, reach) : T;
   if ((rc = fill_rows(p, T, 0, Tc, e0dir, d0, c, dt, out, K ? lo : nullptr,
-                      prev, n0, err_flag, s)))
+                      K ? states[0] : nullptr, n0, err_flag, s)))
     return rc;
   OrderStep step{{0, 0, (int)Tc, 0, 0}, {}};
   OrderSpan &sp = step.span;
@@ -217,6 +261,8 @@ extern "C" int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T,
     sp.Tp = (int)Tc;
     sp.Tc = (int)(Tc = std::min(T, Tc + p.max_lag));
     sp.last = k == K;
+    const float *prev = states[k - 1];
+    float *cur = sp.last ? lo : states[k];  // (the last order is not stored)
     bool add = true;
     if (p.kind == SPR_PLAN_PAIRS) {
       rc = step_pairs(p.P, p.D, p.B, T, p.row_ptr, p.src, p.lag, p.dir,
@@ -228,12 +274,84 @@ extern "C" int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T,
       add = pair || sp.last;
       sp.round = add && !pair;
       rc = order(p, T, prev, pair ? prev : nullptr, cur, add ? out : nullptr,
-                 add ? lo : nullptr, gsum, step, s);
+                 add ? lo : nullptr, gsum, false, step, s);
     }
     if (rc) return rc;
     if (add) sp.Tv = sp.Tc;
-    std::swap(prev, cur);
   }
   return fill_rows(p, T, Tc, T, nullptr, nullptr, c, dt, out, nullptr, nullptr,
                    nullptr, nullptr, s);
+}
+
+extern "C" int spr_adjoint_segment_ds(
+    const spr_exchange_plan *plan, int64_t T, int64_t k0, int64_t n,
+    int64_t reach, float *const *states, float *gsum, const int64_t *tgptr,
+    const int32_t *tkey, const int32_t *tlag, const int32_t *tm,
+    const double *twa, const double *twc, const float *lam,
+    const float *mu_next, float *mu_even, float *mu_odd, float *musum,
+    double *ga, void *stream) {
+  SPR_REQUIRE(states && gsum && tgptr && tkey && tlag && tm && twa && twc &&
+                  lam && mu_next && mu_even && mu_odd && musum && ga,
+              "spr_adjoint_segment_ds: null pointer");
+  hipStream_t s = as_stream(stream);
+  int rc = recompute("spr_adjoint_segment_ds", plan, SPR_PLAN_DS, T, k0, n,
+                     reach, states, gsum, nullptr, s);
+  if (rc) return rc;
+  const spr_exchange_plan &p = *plan;
+  const float *mu = mu_next;
+  for (int64_t k = k0 + n - 1; k >= k0; --k) {
+    const int64_t Tk = reached(p, T, reach, k);
+    const int64_t Tn = reached(p, T, reach, k + 1);
+    float *out = k % 2 ? mu_odd : mu_even;
+    SPR_REQUIRE(out != mu && out != lam, "spr_adjoint_segment_ds: aliased mu");
+    if ((rc = direction_sum(p.P, p.D, p.B, T, Tn, mu, musum, s))) return rc;
+    if ((rc = adjoint_ds(p.P, p.D, p.B, T, Tk, Tn, p.Vd, tgptr, tkey, tlag, tm,
+                         twa, twc, lam, musum, mu, states[k - k0], out, ga,
+                         s)))
+      return rc;
+    mu = out;
+  }
+  return SPR_OK;
+}
+
+extern "C" int spr_adjoint_segment_grouped(
+    const spr_exchange_plan *plan, int64_t T, int64_t k0, int64_t n,
+    int64_t reach, float *const *states, float *const *gsums,
+    const int64_t *trow_ptr, const int32_t *tgrp, const int32_t *tlag,
+    const double *tscal, const float *lam, const float *mu_next,
+    float *mu_even, float *mu_odd, float *nu, double *gg, void *stream) {
+  SPR_REQUIRE(states && gsums && trow_ptr && tgrp && tlag && tscal && lam &&
+                  mu_next && mu_even && mu_odd && nu && gg,
+              "spr_adjoint_segment_grouped: null pointer");
+  hipStream_t s = as_stream(stream);
+  int rc = recompute("spr_adjoint_segment_grouped", plan, SPR_PLAN_GROUPED, T,
+                     k0, n, reach, states, nullptr, gsums, s);
+  if (rc) return rc;
+  const spr_exchange_plan &p = *plan;
+  const float *mu = mu_next;
+  for (int64_t k = k0 + n - 1; k >= k0; --k) {
+    const int64_t i = k - k0;
+    const int64_t Tk = reached(p, T, reach, k);
+    const int64_t Tn = reached(p, T, reach, k + 1);
+    float *out = k % 2 ? mu_odd : mu_even;
+    SPR_REQUIRE(out != mu && out != lam,
+                "spr_adjoint_segment_grouped: aliased mu");
+    // the last order's group sums are still to be formed, and those whose
+    // buffer a later order took
+    if ((i == n - 1 || gsums[i] == gsums[n - 1]) &&
+        (rc = order(p, T, states[i], nullptr, nullptr, nullptr, nullptr,
+                    gsums[i], true, step_from(p, T, reach, k), s)))
+      return rc;
+    if ((rc = table_grad(p.P, p.D, p.B, T, Tn, p.grp_ptr, mu, gsums[i], gg,
+                         s)))
+      return rc;
+    if ((rc = spread_adjoint(p.P, p.D, p.B, T, Tn, p.grp_ptr, p.grp_key,
+                             p.rtab, mu, nu, s)))
+      return rc;
+    if ((rc = gather_adjoint(p.P, p.D, p.B, T, Tk, Tn, p.Vd, trow_ptr, tgrp,
+                             tlag, tscal, nu, lam, out, s)))
+      return rc;
+    mu = out;
+  }
+  return SPR_OK;
 }

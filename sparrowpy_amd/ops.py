@@ -958,7 +958,10 @@ def _plan_struct(plan):
 
 
 def _exchange(plan, e0d, d0, speed_of_sound, time_resolution, n_samples,
-              max_order, reach, recurrence):
+              max_order, reach, keep=None):
+    """The sum of the orders: by the recurrence (keep None), or order by
+    order, keep(k) naming the orders whose histograms are returned too
+    ({k: float32 [P,D,B,T], its reached bins})."""
     e0d = _f64(e0d)
     d0 = _f64(d0)
     P, D, B = e0d.shape
@@ -981,18 +984,28 @@ def _exchange(plan, e0d, d0, speed_of_sound, time_resolution, n_samples,
     head = (ctypes.addressof(st), T, K, reach, ptr(e0d), ptr(d0),
             float(speed_of_sound), float(time_resolution), ptr(out))
     tail = (ptr(gsum), ptr(n0), ptr(err), stream_ptr())
-    if recurrence:
+    kept = {}
+    if keep is None:
         call("spr_exchange_sum", *head, ptr(state()) if K else None, *tail)
     else:
-        work = [ptr(state()) if K else None for _ in range(3)]
-        call("spr_exchange_orders", *head, *work, *tail)
+        lo = state() if K else None
+        turn = {}
+        states = []
+        for k in range(K):
+            if keep(k):
+                kept[k] = state()
+            elif k % 2 not in turn:
+                turn[k % 2] = state()
+            states.append(kept[k] if k in kept else turn[k % 2])
+        call("spr_exchange_orders", *head, ptr(lo), _hip.ptr_array(states),
+             *tail)
     flags = int(err.item())
     if flags & 1:
         raise IndexError(
             "source-to-patch delay exceeds the histogram length")
     if flags:
         raise ValueError("a source delay is not below reach")
-    return out
+    return out, kept
 
 
 def exchange_orders(plan, energy_0_directivity, distance_0, speed_of_sound,
@@ -1003,10 +1016,11 @@ def exchange_orders(plan, energy_0_directivity, distance_0, speed_of_sound,
 
     ``plan`` may be None for max_order < 1.  ``reach``: every source delay
     in bins lies below it (None: nothing is known); orders run only on the
-    bins that energy can have reached by then.  Raises IndexError if a source
-    delay falls beyond the histogram (RadiosityFast.py:1069)."""
+    bins that energy can have reached by then.  Raises IndexError if a
+    source delay falls beyond the histogram (RadiosityFast.py:1069)."""
     return _exchange(plan, energy_0_directivity, distance_0, speed_of_sound,
-                     time_resolution, n_samples, max_order, reach, False)
+                     time_resolution, n_samples, max_order, reach,
+                     lambda k: False)[0]
 
 
 def exchange_sum(plan, energy_0_directivity, distance_0, speed_of_sound,
@@ -1015,7 +1029,7 @@ def exchange_sum(plan, energy_0_directivity, distance_0, speed_of_sound,
     half the memory or less and no pass over the total, the same error
     against float64, last bits of its own."""
     return _exchange(plan, energy_0_directivity, distance_0, speed_of_sound,
-                     time_resolution, n_samples, max_order, reach, True)
+                     time_resolution, n_samples, max_order, reach)[0]
 
 
 class ExchangeState:

@@ -147,8 +147,7 @@ class BatchedExchange:
             g = r._geometry()
             self._receivers[x] = (ops.as_dev(pts, torch.float64), factor,
                                   idx, g["centers"],
-                                  ops.as_dev(r._air_attenuation,
-                                             torch.float64))
+                                  r._air())
 
     @staticmethod
     def _tiling(rows, block, r):
@@ -420,7 +419,7 @@ def run_per_instance(items, speed_of_sound, time_resolution, duration,
         r = it.radiosity
         pts, _, factor, idx = r._receiver_terms(it.receivers)
         g = r._geometry()
-        air = ops.as_dev(r._air_attenuation, torch.float64)
+        air = r._air()
         for s, src in enumerate(it.sources):
             r.init_source_energy(src)
             r.calculate_energy_exchange(speed_of_sound, time_resolution,

@@ -134,6 +134,8 @@ class DirectionalRadiosityFast:
             float(etc_duration)
         self._source = None
         self._dev = {}
+        self._tables = None
+        self._air_dev = None
         self._bake = None
         self._plan = None
         self._etc = None
@@ -520,12 +522,14 @@ class DirectionalRadiosityFast:
                                             self._walls_up_vector[i], out))
         self._brdf.append(np.real(np.asarray(brdf.freq)) * np.pi)
         self._brdf_index[np.atleast_1d(wall_indexes)] = len(self._brdf) - 1
+        self._tables = None
 
     def set_air_attenuation(self, air_attenuation):
         """Air attenuation in Np/m (reference ``RadiosityFast.py:754-764``)."""
         self._check_set_frequency(air_attenuation.frequencies)
         self._air_attenuation = np.atleast_1d(
             np.asarray(air_attenuation.freq, float).squeeze())
+        self._air_dev = None
 
     def _check_set_frequency(self, frequencies):
         frequencies = np.atleast_1d(np.asarray(frequencies, float))
@@ -538,10 +542,14 @@ class DirectionalRadiosityFast:
                 "Frequencies do not match"
 
     def _brdf_tables(self):
-        """Stacked BRDF tables and per-wall direction arrays (host).
+        """Stacked BRDF tables, BRDF indices and per-wall direction arrays
+        (device tensors, uploaded once until :meth:`set_wall_brdf` changes
+        them: they are megabytes where every patch has its own BRDF).
 
         Every wall needs a BRDF here (the kernels index the tables by
         wall); the reference fails there too, on its unset walls."""
+        if self._tables is not None:
+            return self._tables
         if (any(s is None for s in self._brdf_incoming_directions)
                 or any(s is None for s in self._brdf_outgoing_directions)
                 or (np.asarray(self._brdf_index) < 0).any()):
@@ -555,8 +563,17 @@ class DirectionalRadiosityFast:
                             self._brdf_incoming_directions])
         receivers = np.array([s.cartesian for s in
                               self._brdf_outgoing_directions])
-        return (np.array(self._brdf), np.array(self._brdf_index), sources,
-                receivers)
+        self._tables = (ops.as_dev(np.array(self._brdf), torch.float64),
+                        ops.as_dev(np.array(self._brdf_index), torch.int64),
+                        ops.as_dev(sources, torch.float64),
+                        ops.as_dev(receivers, torch.float64))
+        return self._tables
+
+    def _air(self):
+        """The air attenuation on the device (None if unset)."""
+        if self._air_dev is None and self._air_attenuation is not None:
+            self._air_dev = ops.as_dev(self._air_attenuation, torch.float64)
+        return self._air_dev
 
     # -- device geometry --------------------------------------------------
     def _geometry(self):
@@ -633,10 +650,11 @@ class DirectionalRadiosityFast:
             self._frequencies = freqs
         g = self._geometry()
         brdf, bidx, sources, receivers = self._brdf_tables()
+        pos_dev = ops.as_dev(pos, torch.float64)
         vis = ops.check_point2patch_visibility(
-            pos, g["centers"], g["walls_normal"], g["walls_points"])[0]
+            pos_dev, g["centers"], g["walls_normal"], g["walls_points"])[0]
         e0, e0d, d0 = ops.source_energy(
-            pos[0], g["centers"], g["points"], vis, self._air_attenuation,
+            pos_dev[0], g["centers"], g["points"], vis, self._air(),
             self.n_bins, g["wall_ids"], sources, brdf, bidx,
             receivers.shape[1])
         # the farthest corner of the patches' bounding box
@@ -830,7 +848,7 @@ class DirectionalRadiosityFast:
     # -- receivers ------------------------------------------------------------
     def _receiver_terms(self, receivers):
         g = self._geometry()
-        pts = _cartesian(receivers)
+        pts = ops.as_dev(_cartesian(receivers), torch.float64)
         vis = ops.check_point2patch_visibility(
             pts, g["centers"], g["walls_normal"], g["walls_points"])
         factor = ops.receiver_energy(pts, g["points"], vis)
@@ -848,7 +866,7 @@ class DirectionalRadiosityFast:
         pts, _, factor, idx = self._receiver_terms(receivers)
         g = self._geometry()
         out = ops.collect(self._etc, pts, g["centers"], idx, factor,
-                          self._air_attenuation, self._speed_of_sound,
+                          self._air(), self._speed_of_sound,
                           self._etc_time_resolution, patchwise=True)
         data = out.double().cpu().numpy()
         times = np.arange(data.shape[-1]) * self._etc_time_resolution
@@ -865,7 +883,7 @@ class DirectionalRadiosityFast:
         pts, _, factor, idx = self._receiver_terms(receivers)
         g = self._geometry()
         out = ops.collect(self._etc, pts, g["centers"], idx, factor,
-                          self._air_attenuation, self._speed_of_sound,
+                          self._air(), self._speed_of_sound,
                           self._etc_time_resolution, patchwise=False)
         data = out.double().cpu().numpy()
         if direct_sound:

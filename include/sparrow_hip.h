@@ -55,7 +55,8 @@ int spr_p2p_visibility(int64_t P, const double *centers, int64_t NS,
                        void *stream);
 
 /* Workspace bytes of spr_p2p_visibility / spr_point_visibility for NS
- * blocking surfaces (one precomputed record per surface).
+ * blocking surfaces (one precomputed record per surface, and the groups of
+ * coplanar ones).
  * Sizing helper; no counterpart in the reference. */
 int64_t spr_visibility_workspace(int64_t NS);
 

@@ -16,27 +16,177 @@ namespace {
 // ---------------------------------------------------------------------
 // visibility
 // ---------------------------------------------------------------------
-__global__ void blocker_kernel(int64_t NS, const double *__restrict__ normals,
-                               const double *__restrict__ pts,
-                               BlockerRec *__restrict__ out) {
-  int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= NS) return;
-  BlockerRec r;
-  make_blocker(pts + 12 * k, normals + 3 * k, r);
-  out[k] = r;
+// Members of the group that starts at bit m, of n_here blockers in its run.
+__device__ inline int count_of_group(uint32_t head, int m, int n_here) {
+  const uint32_t later = m + 1 < kGroup ? head >> (m + 1) : 0u;
+  return later ? __ffs((int)later) : n_here - m;
+}
+
+// Component q of the box (xmin, xmax, ymin, ymax) of corners from..to-1.
+__device__ inline double extent(const double *sx, const double *sy, int from,
+                                int to, int q) {
+  const double *v = q < 2 ? sx : sy;
+  double e = v[from];
+#pragma unroll 4
+  for (int t = from + 1; t < to; ++t)
+    e = (q & 1) ? fmax(e, v[t]) : fmin(e, v[t]);
+  return e;
+}
+
+// Blocker records, and the groups of coplanar blockers among each kGroup
+// consecutive ones: bit m of heads[k / kGroup] is set where blocker k's run
+// of kGroup starts a group, and groups[] holds the group at the index of its
+// first member.  A workgroup per run, a lane per corner: most calls have a
+// handful of blockers and wait for the kernel's own code to come in from
+// memory, so every step is written once and not unrolled over corners (6
+// walls 4.4 us, 208 patches 10 us; a lane per blocker 19 us for either).
+__global__ __launch_bounds__(4 * kGroup) void blocker_kernel(
+    int64_t NS, const double *__restrict__ normals,
+    const double *__restrict__ pts, BlockerRec *__restrict__ recs,
+    BlockerGroup *__restrict__ groups, uint32_t *__restrict__ heads) {
+  __shared__ double sx[4 * kGroup], sy[4 * kGroup];
+  __shared__ uint32_t s_head, s_long, s_lines[kGroup];
+  const int t = (int)threadIdx.x, m = t >> 2, q = t & 3;
+  const int64_t k0 = (int64_t)blockIdx.x * kGroup, k = k0 + m;
+  const int n_here = (int)(NS - k0 < kGroup ? NS - k0 : kGroup);
+  const bool valid = m < n_here;
+  if (t < kGroup) s_lines[t] = 0;
+  if (t == 0) s_head = s_long = 0;
+  double m0[3], m1[3];
+  d3 n{0.0, 0.0, 0.0}, p0{0.0, 0.0, 0.0};
+  double c = 0.0;
+  bool same = false;  // in the plane of the blocker before
+  if (valid) {
+    n = load3(normals + 3 * k);
+    p0 = load3(pts + 12 * k);
+    c = dot(n, p0);
+    if (m > 0) {
+      const d3 o = load3(normals + 3 * (k - 1));
+      const double co = dot(n, load3(pts + 12 * (k - 1)));
+      same = __double_as_longlong(o.x) == __double_as_longlong(n.x) &&
+             __double_as_longlong(o.y) == __double_as_longlong(n.y) &&
+             __double_as_longlong(o.z) == __double_as_longlong(n.z) &&
+             fabs(c - co) <= kPlaneStep * (1.0 + fabs(c));
+    }
+    rotation_rows(normals + 3 * k, m0, m1);
+    const d3 p = load3(pts + 12 * k + 3 * q);
+    sx[t] = dot(load3(m0), p);
+    sy[t] = dot(load3(m1), p);
+  }
+  __syncthreads();
+  if (valid) {
+    BlockerRec &r = recs[k];
+    const int t1 = (t & ~3) | ((q + 1) & 3);
+    const d2 side = d2{sx[t1], sy[t1]} - d2{sx[t], sy[t]};
+    const double ns = norm(side);
+    r.px[q] = sx[t], r.py[q] = sy[t];
+    r.nlx[q] = -side.y / ns;
+    r.nly[q] = side.x / ns;
+    r.elen[q] = ns;
+    // n, p0, m0, m1: three components each, a row to a lane
+    double *row = q == 0 ? r.n : q == 1 ? r.p0 : q == 2 ? r.m0 : r.m1;
+    row[0] = q == 0 ? n.x : q == 1 ? p0.x : q == 2 ? m0[0] : m1[0];
+    row[1] = q == 0 ? n.y : q == 1 ? p0.y : q == 2 ? m0[1] : m1[1];
+    row[2] = q == 0 ? n.z : q == 1 ? p0.z : q == 2 ? m0[2] : m1[2];
+    r.box[q] = extent(sx, sy, t & ~3, (t & ~3) + 4, q);
+    if (!(ns <= kLongEdge)) atomicOr(&s_long, 1u << m);
+    if (q == 0 && !same) atomicOr(&s_head, 1u << m);
+  }
+  __syncthreads();
+  const uint32_t head = s_head;
+  if (t == 0) heads[blockIdx.x] = head;
+  const int start =
+      31 - __clz((int)(head & (uint32_t)((2ull << m) - 1ull)));
+  const int count = count_of_group(head, start, n_here);
+  if (valid) {
+    // a line for a corner whose y no earlier corner of the group has
+    bool first = true;
+#pragma unroll 4
+    for (int e = 4 * start; e < t; ++e)
+      first &= !(fabs(sy[t] - sy[e]) <= kLineStep);
+    if (first) {
+      const uint32_t l = atomicAdd(&s_lines[start], 1u);
+      if (l < kLines) groups[k0 + start].lines[l] = sy[t];
+    }
+  }
+  __syncthreads();
+  if (!valid || same) return;
+  BlockerGroup &g = groups[k];
+  g.box[q] = extent(sx, sy, 4 * m, 4 * (m + count), q);
+  if (q != 0) return;
+  g.n[0] = n.x, g.n[1] = n.y, g.n[2] = n.z;
+  for (int e = 0; e < 3; ++e) g.m0[e] = m0[e], g.m1[e] = m1[e];
+  g.c = c;
+  g.dc = kGroup * kPlaneStep * (2.0 + fabs(c));
+  g.count = count;
+  g.left = (s_long >> m & ((2u << (count - 1)) - 1u)) == 0;
+  g.n_lines = s_lines[m] <= kLines ? (int)s_lines[m] : 0;
+}
+
+// Whether any member of the group that starts at blocker k0 blocks this
+// lane's segment a-b.  Every lane marks the members that its segment can meet
+// (records through scalar loads), then evaluates the predicate for its own
+// marks: nearly always one or two, so a wave takes a few turns instead of one
+// for each member that any of its lanes meets.
+__device__ inline bool group_blocks(d3 a, d3 b, bool alive, int64_t k0,
+                                    const BlockerGroup &grp,
+                                    const BlockerRec *__restrict__ recs) {
+  Sight s;
+  bool meets = alive && sight(a, b, grp, s);
+  if (!__any(meets)) return false;
+  if (!meets) s = Sight{0.0, 0.0, 0.0, 0.0, 0.0, false};
+  if (!s.two) s.x2 = s.x, s.y2 = s.y;
+  const bool any_two = __any(s.two);
+  meets = meets && (in_reach(s.x, s.y, s.g, grp.box) ||
+                    in_reach(s.x2, s.y2, s.g, grp.box));
+  const bool left = meets && left_of(s.x, s.g, grp.box[0]) &&
+                    left_of(s.x2, s.g, grp.box[0]);
+  if (grp.left != 0 && grp.n_lines > 0 && __any(left)) {
+    const double m = kCullBox + kLineSlack + s.g;
+    bool near = false;
+    for (int l = 0; l < grp.n_lines; ++l)
+      near |= !(fabs(s.y - grp.lines[l]) > m);
+    if (any_two)
+      for (int l = 0; l < grp.n_lines; ++l)
+        near |= !(fabs(s.y2 - grp.lines[l]) > m);
+    meets = meets && (near || !left);
+  }
+  if (!__any(meets)) return false;
+  uint32_t mine = 0;
+#pragma unroll 4
+  for (int m = 0; m < grp.count; ++m) {
+    const BlockerRec &r = recs[k0 + m];
+    mine |= (uint32_t)may_block(s.x, s.y, s.g, grp.left, r) << m;
+  }
+  if (any_two)
+    for (int m = 0; m < grp.count; ++m)
+      mine |= (uint32_t)may_block(s.x2, s.y2, s.g, grp.left, recs[k0 + m])
+              << m;
+  if (!meets) mine = 0;
+  bool blocked = false;
+  while (mine != 0 && !blocked) {
+    blocked = !basic_visibility(a, b, recs[k0 + __ffs((int)mine) - 1]);
+    mine &= mine - 1;
+  }
+  return blocked;
 }
 
 // Thread per pair (i, j) of a 16x16 tile.  The workgroup first culls the
-// blockers for the whole tile (may_block_tile over the boxes of its 16 row
-// and 16 column patch centres) into a candidate list in LDS, 256 blockers
-// at a time; every lane then walks the candidates (a uniform loop, so
-// records arrive through scalar loads) until its pair is blocked.  The cull
-// only drops blockers that cannot block any pair of the tile, so the flags
-// are those of the full scan (canyon, 5,122 patches as blockers: ~1,500
-// candidates per tile, 105 ms instead of 277 ms).
-__global__ __launch_bounds__(256) void p2p_visibility_kernel(
+// groups of blockers for the whole tile (may_block_tile over the boxes of its
+// 16 row and 16 column patch centres) into a candidate list in LDS; every
+// lane then walks the candidates (a uniform loop) until its pair is blocked.
+// Culls and marks only drop blockers that cannot block the pair, so the flags
+// are those of the full scan.
+// Bound by sight()'s float64 arithmetic and by the wait for each group's
+// record: in a canyon of 5,122 patches, all of them blockers, a wave looks at
+// 86 groups, meets the box of 2.6 and takes 1.7 turns of the predicate, in
+// 8.0 ms for 13.1 M pairs; testing the predicate for every blocker that the
+// tile's cull leaves (about 1,500) took 105 ms.
+__global__ __launch_bounds__(256, 4) void p2p_visibility_kernel(
     int64_t P, const double *__restrict__ centers, int64_t NS,
-    const BlockerRec *__restrict__ recs, uint8_t *__restrict__ vis) {
+    const BlockerRec *__restrict__ recs,
+    const BlockerGroup *__restrict__ groups,
+    const uint32_t *__restrict__ heads, uint8_t *__restrict__ vis) {
   __shared__ int32_t cand[256];
   __shared__ int32_t wave_count[4];
   __shared__ double box[12];
@@ -75,7 +225,9 @@ __global__ __launch_bounds__(256) void p2p_visibility_kernel(
   const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
   for (int64_t k0 = 0; k0 < NS; k0 += 256) {
     const int64_t kk = k0 + (int64_t)threadIdx.x;
-    const bool keep = kk < NS && may_block_tile(ilo, ihi, jlo, jhi, recs[kk]);
+    const bool keep =
+        kk < NS && (heads[kk / kGroup] >> (kk % kGroup) & 1u) != 0 &&
+        may_block_tile(ilo, ihi, jlo, jhi, groups[kk]);
     const uint64_t m = __ballot(keep);
     if (lane == 0) wave_count[wave] = __popcll(m);
     __syncthreads();
@@ -90,28 +242,53 @@ __global__ __launch_bounds__(256) void p2p_visibility_kernel(
     for (int c = 0; c < n_cand; ++c) {
       if (!__any(alive)) break;
       const int k = __builtin_amdgcn_readfirstlane(cand[c]);
-      if (alive) alive = basic_visibility(a, b, recs[k]);
+      if (group_blocks(a, b, alive, k, groups[k], recs)) alive = false;
     }
     if (!__syncthreads_or(alive)) break;
   }
   if (valid) vis[i * P + j] = (uint8_t)alive;
 }
 
-// Thread per (query point q, patch k); walls as blockers.
-__global__ __launch_bounds__(256) void point_visibility_kernel(
+// Workgroup per query point and 64 patches; its kSightWaves waves share the
+// blockers, a run of kGroup at a time, and leave a patch that another wave has
+// found blocked.  One or two query points leave most of the chip idle, so the
+// length of the walk is what a call waits for: 208 patches as blockers 17 us
+// (one thread walking all of them: 221 us), 1,072 21 us (944 us), 6 walls
+// 15 us, most of it the kernel's code coming in.
+constexpr int kSightWaves = 8;
+__global__ __launch_bounds__(64 * kSightWaves) void point_visibility_kernel(
     int64_t NQ, const double *__restrict__ points, int64_t P,
     const double *__restrict__ centers, int64_t NS,
-    const BlockerRec *__restrict__ recs, uint8_t *__restrict__ vis) {
+    const BlockerRec *__restrict__ recs,
+    const BlockerGroup *__restrict__ groups,
+    const uint32_t *__restrict__ heads, uint8_t *__restrict__ vis) {
+  __shared__ int32_t blocked[64];
+  const int lane = (int)threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int64_t q = blockIdx.y;
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t k = (int64_t)blockIdx.x * 64 + lane;
+  if (wave == 0) blocked[lane] = 0;
+  __syncthreads();
   bool alive = k < P;
-  d3 a = load3(points + 3 * q), b{0, 0, 0};
+  const d3 a = load3(points + 3 * q);
+  d3 b{0, 0, 0};
   if (alive) b = load3(centers + 3 * k);
-  for (int64_t s = 0; s < NS; ++s) {
+  const int64_t runs = (NS + kGroup - 1) / kGroup;
+  for (int64_t run = wave; run < runs; run += kSightWaves) {
+    alive = alive && __hip_atomic_load(blocked + lane, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP) == 0;
     if (!__any(alive)) break;
-    if (alive) alive = basic_visibility(a, b, recs[s]);
+    for (uint32_t h = heads[run]; h != 0; h &= h - 1) {
+      const int64_t s = run * kGroup + __ffs((int)h) - 1;
+      if (group_blocks(a, b, alive, s, groups[s], recs)) {
+        alive = false;
+        __hip_atomic_store(blocked + lane, 1, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+    }
   }
-  if (k < P) vis[q * P + k] = (uint8_t)alive;
+  __syncthreads();
+  if (wave == 0 && k < P) vis[q * P + k] = (uint8_t)(blocked[lane] == 0);
 }
 
 // ---------------------------------------------------------------------
@@ -531,21 +708,36 @@ __global__ void source_energy_kernel(
 
 using namespace spr;
 
+// Blocker records, groups (at most one per blocker) and group starts.
+namespace {
+struct Blockers {
+  const BlockerRec *recs;
+  const BlockerGroup *groups;
+  const uint32_t *heads;
+};
+}  // namespace
+
 extern "C" int64_t spr_visibility_workspace(int64_t NS) {
-  return NS < 0 ? -1 : (int64_t)sizeof(BlockerRec) * (NS > 0 ? NS : 1);
+  if (NS < 0) return -1;
+  const int64_t n = NS > 0 ? NS : 1;
+  return (int64_t)(sizeof(BlockerRec) + sizeof(BlockerGroup)) * n +
+         (int64_t)sizeof(uint32_t) * ceil_div(n, kGroup);
 }
 
 static int build_blockers(int64_t NS, const double *normals,
                           const double *pts, void *ws, int64_t ws_bytes,
-                          hipStream_t s) {
+                          hipStream_t s, Blockers &out) {
   if (ws_bytes < spr_visibility_workspace(NS))
     return fail(SPR_ERR_WORKSPACE, "visibility workspace of %lld bytes, "
                 "need %lld", (long long)ws_bytes,
                 (long long)spr_visibility_workspace(NS));
+  auto *recs = static_cast<BlockerRec *>(ws);
+  auto *groups = reinterpret_cast<BlockerGroup *>(recs + NS);
+  auto *heads = reinterpret_cast<uint32_t *>(groups + NS);
+  out = Blockers{recs, groups, heads};
   if (NS == 0) return SPR_OK;
-  hipLaunchKernelGGL(blocker_kernel, dim3((unsigned)ceil_div(NS, 128)),
-                     dim3(128), 0, s, NS, normals, pts,
-                     static_cast<BlockerRec *>(ws));
+  hipLaunchKernelGGL(blocker_kernel, dim3((unsigned)ceil_div(NS, kGroup)),
+                     dim3(4 * kGroup), 0, s, NS, normals, pts, recs, groups, heads);
   SPR_LAUNCH_CHECK();
   return SPR_OK;
 }
@@ -561,13 +753,13 @@ extern "C" int spr_p2p_visibility(int64_t P, const double *centers,
                                                           surf_points)),
               "spr_p2p_visibility: null pointer");
   hipStream_t s = as_stream(stream);
+  Blockers bl;
   int rc = build_blockers(NS, surf_normals, surf_points, workspace,
-                          workspace_bytes, s);
+                          workspace_bytes, s, bl);
   if (rc) return rc;
   unsigned nt = (unsigned)ceil_div(P, 16);
   hipLaunchKernelGGL(p2p_visibility_kernel, dim3(nt, nt), dim3(256), 0, s, P,
-                     centers, NS, static_cast<const BlockerRec *>(workspace),
-                     vis);
+                     centers, NS, bl.recs, bl.groups, bl.heads, vis);
   SPR_LAUNCH_CHECK();
   return SPR_OK;
 }
@@ -584,13 +776,14 @@ extern "C" int spr_point_visibility(int64_t NQ, const double *points,
                   (NS == 0 || (surf_normals && surf_points)),
               "spr_point_visibility: null pointer");
   hipStream_t s = as_stream(stream);
+  Blockers bl;
   int rc = build_blockers(NS, surf_normals, surf_points, workspace,
-                          workspace_bytes, s);
+                          workspace_bytes, s, bl);
   if (rc) return rc;
   hipLaunchKernelGGL(point_visibility_kernel,
-                     dim3((unsigned)ceil_div(P, 256), (unsigned)NQ), dim3(256),
-                     0, s, NQ, points, P, centers, NS,
-                     static_cast<const BlockerRec *>(workspace), vis);
+                     dim3((unsigned)ceil_div(P, 64), (unsigned)NQ),
+                     dim3(64 * kSightWaves), 0, s, NQ, points, P, centers, NS,
+                     bl.recs, bl.groups, bl.heads, vis);
   SPR_LAUNCH_CHECK();
   return SPR_OK;
 }

@@ -17,8 +17,10 @@
 //    "segment crosses the polygon" test evaluates the cheap
 //    (pt - a).(pt - b) < 0 condition before the winding test (both are pure
 //    and are combined with AND).
-//  * Blockers that cannot block any segment between two boxes of points
-//    (may_block_tile) are not evaluated for those segments.
+//  * Blockers that cannot block a segment are not evaluated for it: groups
+//    of coplanar blockers are dropped for a tile of segments
+//    (may_block_tile) and for one segment (sight, may_block), and so are
+//    the members of a group.
 #pragma once
 
 #include "spr_common.hpp"
@@ -86,38 +88,28 @@ __host__ __device__ inline void rotation_rows(const double *n_in,
   }
 }
 
-__host__ __device__ inline void make_blocker(const double *pts,
-                                             const double *normal,
-                                             BlockerRec &r) {
-  for (int c = 0; c < 3; ++c) {
-    r.n[c] = normal[c];
-    r.p0[c] = pts[c];
-  }
-  rotation_rows(normal, r.m0, r.m1);
-  for (int i = 0; i < 4; ++i) {
-    d3 p = load3(pts + 3 * i);
-    r.px[i] = dot(load3(r.m0), p);
-    r.py[i] = dot(load3(r.m1), p);
-  }
-  r.box[0] = r.box[1] = r.px[0];
-  r.box[2] = r.box[3] = r.py[0];
-  for (int i = 0; i < 4; ++i) {
-    d2 a1{r.px[(i + 1) % 4], r.py[(i + 1) % 4]};
-    d2 a0{r.px[i], r.py[i]};
-    d2 side = a1 - a0;
-    double ns = norm(side);
-    r.nlx[i] = -side.y / ns;
-    r.nly[i] = side.x / ns;
-    r.elen[i] = ns;
-    r.box[0] = fmin(r.box[0], r.px[i]);
-    r.box[1] = fmax(r.box[1], r.px[i]);
-    r.box[2] = fmin(r.box[2], r.py[i]);
-    r.box[3] = fmax(r.box[3], r.py[i]);
-  }
-}
+// Up to kGroup consecutive blockers in one plane: their normals, and with
+// them the rotation rows, are the same bits, and their planes' offsets
+// follow one another within kPlaneStep (1 + |c|).
+constexpr int kGroup = 32;
+constexpr double kPlaneStep = 1e-12;
+constexpr double kLongEdge = 1e3;  // see may_block
+constexpr int kLines = 36;         // 33 rows of corners, with some to spare
+constexpr double kLineStep = 1e-6;
+struct BlockerGroup {
+  double n[3], m0[3], m1[3];
+  double c;         // n . p0 of the first member
+  double dc;        // no member's offset is further from c
+  double box[4];    // union of the members' boxes
+  int32_t count;
+  int32_t left;     // 1: no edge longer than kLongEdge (see may_block)
+  int32_t n_lines;  // 0: more than kLines
+  // rotated y of the members' corners, those within kLineStep once
+  double lines[kLines];
+};
 
 // geometry.py:614-686 _point_in_polygon for a 4-corner blocker.
-__device__ inline bool point_in_blocker(d3 p, const BlockerRec &r) {
+__host__ __device__ inline bool point_in_blocker(d3 p, const BlockerRec &r) {
   if (fabs(dot(p - load3(r.p0), load3(r.n))) > kEta) return false;
   d2 pt{dot(load3(r.m0), p), dot(load3(r.m1), p)};
   // Bounding-box early out (see header comment): count stays 0.
@@ -182,9 +174,9 @@ __device__ inline double form_max(d3 c, d3 lo, d3 hi) {
 // only that neighbourhood of the box is tested; otherwise the whole union
 // box is.
 __device__ inline bool may_block_tile(d3 ilo, d3 ihi, d3 jlo, d3 jhi,
-                                      const BlockerRec &r) {
+                                      const BlockerGroup &r) {
   const d3 n = load3(r.n), m0 = load3(r.m0), m1 = load3(r.m1);
-  const double np0 = dot(n, load3(r.p0));
+  const double np0 = r.c;
   const double di0 = form_min(n, ilo, ihi) - np0;
   const double di1 = form_max(n, ilo, ihi) - np0;
   const double dj0 = form_min(n, jlo, jhi) - np0;
@@ -211,8 +203,91 @@ __device__ inline bool may_block_tile(d3 ilo, d3 ihi, d3 jlo, d3 jhi,
            form_min(m1, lo, hi) - grow > r.box[3] + kCullBox);
 }
 
+// Where one segment can meet the plane of a group: every point of it that
+// the predicate could find in a member lies within g of (x, y) in the
+// rotated frame, or of (x2, y2) if two is set.
+struct Sight {
+  double x, y, g, x2, y2;
+  bool two;
+};
+
+// False if the segment a-b cannot be blocked by any member: both ends lie
+// beyond kCullPlane on one side, so that neither is in the plane and the
+// crossing point lies outside the segment.  With the ends beyond kCullPlane
+// on either side only the crossing point counts (a member's plane, up to dc off
+// this one, moves it by g); with one end near the plane
+// only that end's neighbourhood (as in may_block_tile); with both ends near
+// the plane and the segment as good as parallel to it (the reference takes no
+// crossing point below 1e-6) only the two ends; otherwise the whole segment.
+// A NaN anywhere makes the later comparisons false, and members are kept.
+__host__ __device__ inline bool sight(d3 a, d3 b, const BlockerGroup &r,
+                                      Sight &s) {
+  const d3 n = load3(r.n), m0 = load3(r.m0), m1 = load3(r.m1);
+  const double da = dot(n, a) - r.c, db = dot(n, b) - r.c;
+  if ((da > kCullPlane && db > kCullPlane) ||
+      (da < -kCullPlane && db < -kCullPlane))
+    return false;
+  const double xa = dot(m0, a), ya = dot(m1, a);
+  const double xb = dot(m0, b), yb = dot(m1, b);
+  const bool na = fabs(da) <= kCullPlane, nb = fabs(db) <= kCullPlane;
+  s.two = false;
+  s.g = 0.0;
+  if (!na && !nb) {
+    const double inv = 1.0 / (da - db), t = da * inv;
+    s.x = xa + t * (xb - xa);
+    s.y = ya + t * (yb - ya);
+    s.g = r.dc * (fabs(xb - xa) + fabs(yb - ya)) * fabs(inv);
+    return true;
+  }
+  if (na && fabs(db) > 2 * kCullPlane) {
+    s.x = xa, s.y = ya;
+    s.g = 2 * kCullPlane / (fabs(db) - kCullPlane) * norm(b - a);
+  } else if (nb && fabs(da) > 2 * kCullPlane) {
+    s.x = xb, s.y = yb;
+    s.g = 2 * kCullPlane / (fabs(da) - kCullPlane) * norm(b - a);
+  } else if (fabs(da - db) < 5e-7) {
+    s.x = xa, s.y = ya, s.x2 = xb, s.y2 = yb;
+    s.two = true;
+  } else {
+    s.x = xa, s.y = ya;
+    s.g = norm(b - a);
+  }
+  return true;
+}
+
+// Corners left out of a group's lines follow from one to the next within
+// kLineStep, so one of the lines is within this of each.
+constexpr double kLineSlack = 4 * kGroup * kLineStep;
+
+// Whether a point within g of (x, y) may pass point_in_blocker with this box:
+// it needs x <= box[1] and y in box[2..3], up to the margin.
+__host__ __device__ inline bool in_reach(double x, double y, double g,
+                                         const double *box) {
+  return ((int)(x - g > box[1] + kCullBox) | (int)(y + g < box[2] - kCullBox) |
+          (int)(y - g > box[3] + kCullBox)) == 0;
+}
+
+// The same for one member, which also drops points left of its box: their
+// ray (to +x) crosses as many edges upwards as downwards, so the count is 0,
+// unless it passes a corner so closely that the edge test's tolerance
+// decides.  More than kCullBox in y from every corner, a crossed edge spans
+// at least twice that in y, so with edges up to kLongEdge its normal's x is
+// above the 1e-6 at which the reference skips an edge, and both the edge
+// test and the sign of each crossing are decided far above rounding.
+// near: whether y is that close to a corner.
+__host__ __device__ inline bool left_of(double x, double g, double x_min) {
+  return x + (kCullBox + g) < x_min;
+}
+__host__ __device__ inline bool may_block(double x, double y, double g,
+                                          int left, const BlockerRec &r) {
+  const double m = kCullBox + g;
+  int near = left == 0 || !left_of(x, g, r.box[0]);
+  for (int q = 0; q < 4; ++q) near |= !(fabs(y - r.py[q]) > m);
+  return (in_reach(x, y, g, r.box) & near) != 0;
+}
+
 // geometry.py:841-909 _basic_visibility(vis_point=a, eval_point=b).
-__device__ inline bool basic_visibility(d3 a, d3 b, const BlockerRec &r) {
+__host__ __device__ inline bool basic_visibility(d3 a, d3 b, const BlockerRec &r) {
   const bool vin = point_in_blocker(a, r);
   const bool ein = point_in_blocker(b, r);
   const d3 n = load3(r.n);

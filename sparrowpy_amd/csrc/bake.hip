@@ -320,11 +320,16 @@ __global__ __launch_bounds__(256) void visible_pairs_kernel(
 // universal form factor (universal.py:54-96)
 // ---------------------------------------------------------------------
 
-// geometry.py:719-748 _coincidence_check(receiver, source), threshold 1e-6
+// geometry.py:719-748 _coincidence_check(receiver, source), threshold 1e-6:
+// whether any corner of p0 meets any of p1.
+__device__ inline bool corners_meet(const double *p0, const double *p1, int a,
+                                    int b) {
+  return norm(load3(p0 + 3 * a) - load3(p1 + 3 * b)) < 1e-6;
+}
 __device__ inline bool coincident(const double *p0, const double *p1) {
   for (int a = 0; a < 4; ++a)
     for (int b = 0; b < 4; ++b)
-      if (norm(load3(p0 + 3 * a) - load3(p1 + 3 * b)) < 1e-6) return true;
+      if (corners_meet(p0, p1, a, b)) return true;
   return false;
 }
 
@@ -338,65 +343,96 @@ __device__ inline d3 boundary_point(const double *el, int q, int n_div) {
             a.z + (t * (b.z - a.z)) / nd};
 }
 
-__device__ inline double coord(d3 p, int dim) {
-  return dim == 0 ? p.x : (dim == 1 ? p.y : p.z);
+// integration.py:462-486 _newton_cotes_4th (Boole's rule) in its two factors:
+// the step's, and the sum over the five values.
+__device__ inline double boole_step(double x0, double x1) {
+  return (2.0 * (x1 - x0)) / 45.0;
+}
+__device__ inline double boole_sum(const double *y) {
+  return (((7.0 * y[0] + 32.0 * y[1]) + 12.0 * y[2]) + 32.0 * y[3]) +
+         7.0 * y[4];
 }
 
-// integration.py:462-486 _newton_cotes_4th (Boole's rule)
-__device__ inline double boole(const double *x, const double *y) {
-  double h = x[1] - x[0];
-  return ((2.0 * h) / 45.0) *
-         ((((7.0 * y[0] + 32.0 * y[1]) + 12.0 * y[2]) + 32.0 * y[3]) +
-          7.0 * y[4]);
-}
-
-// integration.py:38-114 stokes_integration, one wavefront per pair:
-// lanes fill the 16x16 ln|r| table, 48 lanes integrate over patch j's
-// boundary (one per sample point of i and coordinate), lane 0 integrates
-// over patch i's boundary in the reference's (dim, segment) order.
-__global__ __launch_bounds__(64) void stokes_kernel(
+// integration.py:38-114 stokes_integration, one wavefront per pair (four
+// pairs per workgroup: one pair per workgroup is bound by how fast workgroups
+// start).  Whatever several terms share is formed once, by one lane each: the
+// 2x16 boundary points, the step factor of each segment and coordinate (NaN
+// where the reference skips the segment), Boole's sum over the 16x16 ln|r|
+// table, which is the same for the three coordinates.  Lane 0 only adds the
+// twelve outer terms, in the reference's (dim, segment) order.
+// Bound by the float64 logarithms and square roots of the table: 7.4 M pairs
+// of a canyon in 9.8 ms.  With 48 lanes forming each segment's nodes anew and
+// lane 0 alone all outer terms it was 21 ms.
+__global__ __launch_bounds__(256) void stokes_kernel(
     int64_t P, const double *__restrict__ pts, const double *__restrict__ areas,
     int64_t V, const int32_t *__restrict__ pairs, double *__restrict__ ff) {
-  __shared__ double form[16][16];
-  __shared__ double inner[16][3];
-  const int64_t v = blockIdx.x;
-  const int64_t i = pairs[2 * v], j = pairs[2 * v + 1];
-  if (i < 0 || j < 0 || i >= P || j >= P) return;  // invalid pair: skip
-  const double *pi = pts + 12 * i, *pj = pts + 12 * j;
-  if (coincident(pj, pi)) return;  // handled by nusselt_kernel
-  const int lane = threadIdx.x;
-  for (int q = lane; q < 256; q += 64) {
-    int a = q >> 4, b = q & 15;
-    form[a][b] = log(norm(boundary_point(pi, a, 4) - boundary_point(pj, b, 4)));
+  constexpr double kSkip = __builtin_nan("");
+  struct Pair {
+    double point[2][3][16];  // patch i's and j's boundary points, by dim
+    double step[2][3][4];
+    double form[16][17];
+    double sum[16][4];
+    double inner[3][16];
+    double outer[12];
+  };
+  __shared__ Pair sh[4];
+  const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+  const int64_t v = (int64_t)blockIdx.x * 4 + wave;
+  Pair &w = sh[wave];
+  int64_t i = -1, j = -1;
+  if (v < V) i = pairs[2 * v], j = pairs[2 * v + 1];
+  bool ok = i >= 0 && j >= 0 && i < P && j < P;  // else an invalid pair: skip
+  const double *pi = pts + (ok ? 12 * i : 0), *pj = pts + (ok ? 12 * j : 0);
+  // coincident pairs are nusselt_kernel's
+  ok = ok && !__any(lane < 16 && corners_meet(pj, pi, lane >> 2, lane & 3));
+  if (ok && lane < 32) {
+    const d3 p = boundary_point(lane < 16 ? pi : pj, lane & 15, 4);
+    double(*o)[16] = w.point[lane >> 4];
+    o[0][lane & 15] = p.x, o[1][lane & 15] = p.y, o[2][lane & 15] = p.z;
   }
   __syncthreads();
-  if (lane < 48) {
-    int a = lane / 3, dim = lane % 3;
-    double acc = 0.0, x[5], y[5];
-    for (int s = 0; s < 4; ++s) {
-      for (int k = 0; k < 5; ++k) {
-        int q = (4 * s + k) & 15;
-        x[k] = coord(boundary_point(pj, q, 4), dim);
-      }
-      if (fabs(x[4] - x[0]) > 1e-3) {
-        for (int k = 0; k < 5; ++k) y[k] = form[a][(4 * s + k) & 15];
-        acc += boole(x, y);
-      }
+  if (ok) {
+    if (lane < 24) {
+      const int dim = (lane % 12) >> 2, s = lane & 3;
+      const double *x = w.point[lane / 12][dim];
+      const bool take = fabs(x[(4 * s + 4) & 15] - x[4 * s]) > 1e-3;
+      w.step[lane / 12][dim][s] =
+          take ? boole_step(x[4 * s], x[4 * s + 1]) : kSkip;
     }
-    inner[a][dim] = acc;
+    const int q = lane & 15;
+    const d3 b{w.point[1][0][q], w.point[1][1][q], w.point[1][2][q]};
+    for (int a = lane >> 4; a < 16; a += 4)
+      w.form[a][q] = log(norm(
+          d3{w.point[0][0][a], w.point[0][1][a], w.point[0][2][a]} - b));
   }
   __syncthreads();
-  if (lane == 0) {
-    double outer = 0.0, x[5], y[5];
-    for (int dim = 0; dim < 3; ++dim)
-      for (int s = 0; s < 4; ++s) {
-        for (int k = 0; k < 5; ++k)
-          x[k] = coord(boundary_point(pi, (4 * s + k) & 15, 4), dim);
-        if (fabs(x[4] - x[0]) > 1e-3) {
-          for (int k = 0; k < 5; ++k) y[k] = inner[(4 * s + k) & 15][dim];
-          outer += boole(x, y);
-        }
-      }
+  double y[5];
+  if (ok) {
+    const int a = lane >> 2, s = lane & 3;
+    for (int k = 0; k < 5; ++k) y[k] = w.form[a][(4 * s + k) & 15];
+    w.sum[a][s] = boole_sum(y);
+  }
+  __syncthreads();
+  if (ok && lane < 48) {
+    const int a = lane / 3, dim = lane % 3;
+    double acc = 0.0;
+    for (int s = 0; s < 4; ++s) {
+      const double h = w.step[1][dim][s];
+      if (h == h) acc += h * w.sum[a][s];
+    }
+    w.inner[dim][a] = acc;
+  }
+  __syncthreads();
+  if (ok && lane < 12) {
+    const int dim = lane >> 2, s = lane & 3;
+    const double h = w.step[0][dim][s];
+    for (int k = 0; k < 5; ++k) y[k] = w.inner[dim][(4 * s + k) & 15];
+    w.outer[lane] = h == h ? h * boole_sum(y) : 0.0;
+  }
+  __syncthreads();
+  if (ok && lane == 0) {
+    double outer = 0.0;
+    for (int t = 0; t < 12; ++t) outer += w.outer[t];
     ff[i * P + j] = fabs(outer / ((2.0 * M_PI) * areas[i]));
   }
 }
@@ -546,53 +582,65 @@ __device__ inline double linspace0(double stop, int num, int k) {
 }
 
 // integration.py:232-289 nusselt_integration over the regular grid of
-// integration.py:533-605; one wavefront per pair, one lane per sample,
-// samples summed in the reference's order by lane 0.
+// integration.py:533-605 for the pairs that share a corner.  Each lane (of
+// the first per_wave) looks at one pair; the wavefront then takes the pairs found, one after the other,
+// with one lane per sample and the samples summed in the reference's order by
+// lane 0.  A pair in a few hundred shares a corner, so a wavefront for each
+// pair is bound by starting them: 7.4 M pairs of a canyon in 0.6 ms instead
+// of 9.7 ms.
 __global__ __launch_bounds__(64) void nusselt_kernel(
     int64_t P, const double *__restrict__ pts,
-    const double *__restrict__ normals, int64_t V,
+    const double *__restrict__ normals, int64_t V, int per_wave,
     const int32_t *__restrict__ pairs, double *__restrict__ ff) {
   __shared__ double vals[64];
   __shared__ double m[6];
-  const int64_t v = blockIdx.x;
-  const int64_t i = pairs[2 * v], j = pairs[2 * v + 1];
-  if (i < 0 || j < 0 || i >= P || j >= P) return;  // invalid pair: skip
-  const double *pi = pts + 12 * i, *pj = pts + 12 * j;
-  if (!coincident(pj, pi)) return;  // handled by stokes_kernel
   const int lane = threadIdx.x;
-  if (lane == 0) rotation_rows(normals + 3 * i, m, m + 3);
-  d3 u = load3(pi + 3) - load3(pi), w = load3(pi + 9) - load3(pi);
-  double nu = norm(u), nw = norm(w);
-  double sq = sqrt(1.0 * 64.0);
-  int npx = (int)rint(nu / nw * sq);
-  int npz = (int)rint(nw / nu * sq);
-  if (npz == 0) npz = 1;
-  if (npx == 0) npx = 1;
-  const int n = npx * npz;
-  const double stx = 1.0 - 1.0 / (double)npx, stz = 1.0 - 1.0 / (double)npz;
-  const double ssx = 1.0 / (double)(npx * 2), ssz = 1.0 / (double)(npz * 2);
-  __syncthreads();
-  double out = 0.0;
-  for (int base = 0; base < n; base += 64) {
-    int q = base + lane;
-    if (q < n) {
-      int a = q / npz, b = q % npz;
-      double s = linspace0(stx, npx, a) + ssx;
-      double t = linspace0(stz, npz, b) + ssz;
-      d3 p0{(s * u.x + t * w.x) + pi[0], (s * u.y + t * w.y) + pi[1],
-            (s * u.z + t * w.z) + pi[2]};
-      vals[lane] = nusselt_analog(p0, m, m + 3, pj, normals + 3 * j);
-    }
-    __syncthreads();
-    if (lane == 0) {
-      int cnt = n - base < 64 ? n - base : 64;
-      for (int k = 0; k < cnt; ++k) out += vals[k];
-    }
-    __syncthreads();
+  int64_t i = -1, j = -1;
+  {
+    const int64_t v = (int64_t)blockIdx.x * per_wave + lane;
+    if (lane < per_wave && v < V) i = pairs[2 * v], j = pairs[2 * v + 1];
   }
-  if (lane == 0) {
-    out *= 1.0 / (M_PI * (double)n);
-    ff[i * P + j] = out;
+  uint64_t found =
+      __ballot(i >= 0 && j >= 0 && i < P && j < P &&
+               coincident(pts + 12 * j, pts + 12 * i));
+  for (; found != 0; found &= found - 1) {
+    const int from = __ffsll((unsigned long long)found) - 1;
+    const int64_t fi = __shfl((int)i, from), fj = __shfl((int)j, from);
+    const double *pi = pts + 12 * fi, *pj = pts + 12 * fj;
+    if (lane == 0) rotation_rows(normals + 3 * fi, m, m + 3);
+    d3 u = load3(pi + 3) - load3(pi), w = load3(pi + 9) - load3(pi);
+    double nu = norm(u), nw = norm(w);
+    double sq = sqrt(1.0 * 64.0);
+    int npx = (int)rint(nu / nw * sq);
+    int npz = (int)rint(nw / nu * sq);
+    if (npz == 0) npz = 1;
+    if (npx == 0) npx = 1;
+    const int n = npx * npz;
+    const double stx = 1.0 - 1.0 / (double)npx, stz = 1.0 - 1.0 / (double)npz;
+    const double ssx = 1.0 / (double)(npx * 2), ssz = 1.0 / (double)(npz * 2);
+    __syncthreads();
+    double out = 0.0;
+    for (int base = 0; base < n; base += 64) {
+      int q = base + lane;
+      if (q < n) {
+        int a = q / npz, b = q % npz;
+        double s = linspace0(stx, npx, a) + ssx;
+        double t = linspace0(stz, npz, b) + ssz;
+        d3 p0{(s * u.x + t * w.x) + pi[0], (s * u.y + t * w.y) + pi[1],
+              (s * u.z + t * w.z) + pi[2]};
+        vals[lane] = nusselt_analog(p0, m, m + 3, pj, normals + 3 * fj);
+      }
+      __syncthreads();
+      if (lane == 0) {
+        int cnt = n - base < 64 ? n - base : 64;
+        for (int k = 0; k < cnt; ++k) out += vals[k];
+      }
+      __syncthreads();
+    }
+    if (lane == 0) {
+      out *= 1.0 / (M_PI * (double)n);
+      ff[fi * P + fj] = out;
+    }
   }
 }
 
@@ -817,11 +865,16 @@ extern "C" int spr_form_factors(int64_t P, const double *points,
   hipStream_t s = as_stream(stream);
   int rc = fill<double>(ff, P * P, 0.0, s);
   if (rc || V == 0) return rc;
-  hipLaunchKernelGGL(stokes_kernel, dim3((unsigned)V), dim3(64), 0, s, P,
-                     points, areas, V, pairs, ff);
+  hipLaunchKernelGGL(stokes_kernel, dim3((unsigned)ceil_div(V, 4)), dim3(256),
+                     0, s, P, points, areas, V, pairs, ff);
   SPR_LAUNCH_CHECK();
-  hipLaunchKernelGGL(nusselt_kernel, dim3((unsigned)V), dim3(64), 0, s, P,
-                     points, normals, V, pairs, ff);
+  // As few pairs to a wavefront as 16,384 of them allow: in a small scene many
+  // pairs share a corner, and those of one wavefront are one after the other.
+  int per_wave = 1;
+  while (per_wave < 64 && ceil_div(V, per_wave) > 16384) per_wave *= 2;
+  hipLaunchKernelGGL(nusselt_kernel, dim3((unsigned)ceil_div(V, per_wave)),
+                     dim3(64), 0, s, P, points, normals, V, per_wave, pairs,
+                     ff);
   SPR_LAUNCH_CHECK();
   return SPR_OK;
 }

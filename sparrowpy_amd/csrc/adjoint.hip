@@ -143,8 +143,8 @@ __global__ __launch_bounds__(256) void adjoint_ds_kernel(
   constexpr int32_t kDstMask = (1 << 25) - 1;
   int64_t i;
   int b, tb;
-  dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks / (B * n_tblk),
-                  n_tblk, i, b, tb);
+  dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks, B, n_tblk, i, b,
+                  tb);
   const int64_t q0 = tgptr[i * D], q1 = tgptr[i * D + D];
   if (q1 == q0) return;
   const int tl = tb * (BS * R) + (int)threadIdx.x;

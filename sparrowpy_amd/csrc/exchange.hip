@@ -285,11 +285,11 @@ __global__ __launch_bounds__(BS) void exchange_step_kernel(
   constexpr int NLD = (NW + BS - 1) / BS;      // of them per thread
   static_assert(NBE % C == 0, "chunks tile a batch");
   __shared__ double cfs[2][NW];
-  const int64_t tile = xcd_tile(blockIdx.x, nblocks);
-  const int tb = (int)(tile % n_tblk);
-  const int64_t jb = tile / n_tblk;
-  const int b = (int)(jb % B);
-  const int64_t j = jb / B;
+  const uint32_t tile = xcd_tile(blockIdx.x, nblocks);
+  const int tb = (int)(tile % (uint32_t)n_tblk);
+  const uint32_t jb = tile / (uint32_t)n_tblk;
+  const int b = (int)(jb % (uint32_t)B);
+  const int64_t j = jb / (uint32_t)B;
   const int t0 = tb * (BS * R);
   const int t_end = min(sp.Tc, t0 + BS * R);
 
@@ -407,11 +407,11 @@ __global__ __launch_bounds__(256) void exchange_mfma_kernel(
   constexpr int MT = DP / 16;
   constexpr int WBINS = 16 * NT;  // bins per wave
   static_assert(MT * NT == 8, "eight accumulator tiles per wave");
-  const int64_t tile = xcd_tile(blockIdx.x, nblocks);
-  const int tb = (int)(tile % n_tblk);
-  const int64_t jb = tile / n_tblk;
-  const int b = (int)(jb % B);
-  const int64_t j = jb / B;
+  const uint32_t tile = xcd_tile(blockIdx.x, nblocks);
+  const int tb = (int)(tile % (uint32_t)n_tblk);
+  const uint32_t jb = tile / (uint32_t)n_tblk;
+  const int b = (int)(jb % (uint32_t)B);
+  const int64_t j = jb / (uint32_t)B;
   const int lane = (int)threadIdx.x & 63;
   const int kk = lane >> 4, cc = lane & 15;
   const int tw = (tb * 4 + ((int)threadIdx.x >> 6)) * WBINS;
@@ -568,8 +568,8 @@ __global__ __launch_bounds__(BS) void group_gather_kernel(
   constexpr int NQ = kMetaBlock / C;  // chunks per block
   int64_t j;
   int b, tb;
-  dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks / (B * n_tblk),
-                  n_tblk, j, b, tb);
+  dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks, B, n_tblk, j, b,
+                  tb);
   const int t0 = tb * (BS * R);
   const int t_end = min(T, t0 + BS * R);
   const int64_t e_begin = row_ptr[j], e_end = row_ptr[j + 1];
@@ -656,8 +656,8 @@ __global__ __launch_bounds__(BS) void ds_gather_kernel(
     const float *__restrict__ prev, float *__restrict__ gsum) {
   int64_t j;
   int b, tb;
-  dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks / (B * n_tblk),
-                  n_tblk, j, b, tb);
+  dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks, B, n_tblk, j, b,
+                  tb);
   const int t0 = tb * (BS * R);
   const int t_end = min(T, t0 + BS * R);
   const int64_t e_begin = row_ptr[j], e_end = row_ptr[j + 1];
@@ -764,11 +764,9 @@ __global__ __launch_bounds__(256) void group_spread_kernel(
   // runs of each direction row (no reuse across destinations to keep here;
   // 41.6 ms instead of 47.1 ms with the destination-major order on the
   // street canyon)
-  const int64_t tile = xcd_tile(blockIdx.x, nblocks);
-  const int64_t P = nblocks / (B * n_tblk);
-  const int tb = (int)(tile % n_tblk);
-  const int64_t j = (tile / n_tblk) % P;
-  const int b = (int)(tile / (n_tblk * P));
+  int64_t j;
+  int b, tb;
+  time_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks, B, n_tblk, j, b, tb);
   // the wave index as a scalar (readfirstlane): the BRDF-row reads below
   // then stay scalar loads shared by the wave, not per-lane loads
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -919,11 +917,9 @@ __global__ __launch_bounds__(256) void ds_spread_kernel(
     float *__restrict__ tot_lo, Injection inj) {
   constexpr int K = 8;
   __shared__ int32_t gmap[DP];  // direction -> specular group offset, or -1
-  const int64_t tile = xcd_tile(blockIdx.x, nblocks);
-  const int64_t P = nblocks / (B * n_tblk);
-  const int tb = (int)(tile % n_tblk);
-  const int64_t j = (tile / n_tblk) % P;
-  const int b = (int)(tile / (n_tblk * P));
+  int64_t j;
+  int b, tb;
+  time_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks, B, n_tblk, j, b, tb);
   const int t = tb * 256 + (int)threadIdx.x;
   const uint32_t row_bytes = (uint32_t)sp.Tc * 4u;
   const int64_t g0 = grp_ptr[j], g1 = grp_ptr[j + 1];

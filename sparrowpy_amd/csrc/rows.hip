@@ -10,10 +10,11 @@
 // turn, so a room of ten tiles keeps twenty workgroups busy for as long as
 // one of them takes.  Here a workgroup of 8 waves takes one destination,
 // band and block of 64 R bins, and its waves share the destination's groups:
-// a 148-patch room (16 directions, 1 band, 512 bins) takes 26 us per order
-// instead of 96, launches included, a 328-patch one (4 bands) 82 instead
-// of 175.  Large scenes stay with the tiles, which read a source row once for
-// 16 destinations (1,072 patches, 6 bands, 2,048 bins: 2.5 ms against 3.4).
+// a 228-patch room (16 directions, 1 band, 700 bins) takes 35 us per order
+// instead of 127, launches included, a 508-patch one (3 bands, 1,500 bins)
+// 350 instead of 449.  Large scenes stay with the tiles, which read a source
+// row once for 16 destinations (1,072 patches, 8 bands, 1,500 bins: 2.6 ms
+// against 3.0).
 #include <algorithm>
 #include <cmath>
 
@@ -59,8 +60,15 @@ inline size_t row_lds(const spr_exchange_plan &p, int R) {
 // diffuse + specular plan the diffuse sum is formed in 8 parts).  Phase 2:
 // each wave sums the groups times their BRDF rows for its directions, in
 // group order, in float64, and writes the order and the total.
-// Bound by the latency of the row reads and the float64 multiply-adds; four
-// waves per SIMD (two workgroups per CU) at up to 128 registers.
+// Bound by the row reads: an entry's R = 4 loads take 16 clocks of the CU's
+// first-level cache, its 13 vector instructions as many.  Forming each
+// entry's row address and offsets in the wave (23 scalar and 6 vector
+// instructions more) a 426-patch, 4-band order took 139 us instead of 119.
+// With two weights and 64 directions the second phase is half of it; its
+// values are picked where they are written, 16 totals' loads in flight
+// (1,072 patches, 6 bands: 7.0 ms, with the values held in registers and 8
+// loads in flight 7.3).  Four waves per SIMD (two workgroups per CU) at up to
+// 128 registers.
 template <int DP, int R, bool DS>
 __global__ __launch_bounds__(64 * kRowWaves)
     __attribute__((amdgpu_waves_per_eu(4))) void row_order_kernel(RowArgs a) {
@@ -74,8 +82,8 @@ __global__ __launch_bounds__(64 * kRowWaves)
   const int64_t T = a.T;
   int64_t j;
   int b, tb;
-  dest_major_tile(xcd_tile(blockIdx.x, a.nblocks),
-                  a.nblocks / ((int64_t)B * a.n_tblk), a.n_tblk, j, b, tb);
+  dest_major_tile(xcd_tile(blockIdx.x, a.nblocks), a.nblocks, B, a.n_tblk, j,
+                  b, tb);
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lane = (int)threadIdx.x & 63;
   const int t0 = tb * TB, t_end = min(a.sp.Tc, t0 + TB);
@@ -83,7 +91,6 @@ __global__ __launch_bounds__(64 * kRowWaves)
   const int64_t e_begin = a.row_ptr[j], e_end = a.row_ptr[j + 1];
   const int64_t g0 = a.grp_ptr[j];
   const int ng = (int)(a.grp_ptr[j + 1] - g0);
-  const uint32_t src_bytes = (uint32_t)a.sp.Tp * 4u;
   const double *w = a.scal + (int64_t)b * a.Vd;
   const double *w2 = DS ? a.dscal + (int64_t)b * a.Vd : w;
 
@@ -128,9 +135,21 @@ __global__ __launch_bounds__(64 * kRowWaves)
 #pragma unroll
   for (int r = 0; r < (DS ? R : 1); ++r) Sd[r] = 0.0;
   int gl = c_lo;
+  // One entry per lane, 64 at a time: as loaded (a block ahead), and made
+  // ready: where the entry's bins for this block start in memory and how
+  // many bytes from there are the row's, so that an entry costs the wave
+  // three v_readlane and its loads, with immediate offsets.  An entry whose
+  // first bin lies before the row's (`early`: the first blocks only) starts
+  // at the row, and its lanes' offsets are formed whole.
   struct Meta {
     int32_t row, lag;
     double w, w2;
+  };
+  struct Ready {
+    int64_t addr;
+    int32_t bytes, w0;
+    double w, w2;
+    uint64_t ends, early;
   };
   auto load_meta = [&](int64_t e0) {
     const int64_t e = e0 + lane;
@@ -143,18 +162,41 @@ __global__ __launch_bounds__(64 * kRowWaves)
     m.w2 = DS && in ? w2[ec] : 0.0;
     return m;
   };
-  auto fetch = [&](const Meta &m, int q, float (&v)[C][R]) {
+  auto ready = [&](const Meta &m) {
+    Ready x;
+    const int n = min(m.lag & kLagMask, (int)T);
+    x.w0 = t0 - n;
+    const int skip = max(x.w0, 0), left = max(a.sp.Tp - skip, 0);
+    x.addr = (int64_t)(a.prev + ((int64_t)m.row * B + b) * T + skip);
+    x.bytes = n < t_end ? left * 4 : 0;
+    x.w = m.w;
+    x.w2 = m.w2;
+    x.ends = __ballot((m.lag & kLastInGroup) != 0);
+    x.early = __ballot(x.w0 < 0 && x.bytes != 0);
+    return x;
+  };
+  auto fetch = [&](const Ready &m, int q, float (&v)[C][R]) {
+    if ((m.early >> q & ((1ull << C) - 1ull)) == 0) {  // uniform
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const __amdgpu_buffer_rsrc_t rs =
+            make_rsrc((const void *)readlane_i64(m.addr, q + c),
+                      (uint32_t)__builtin_amdgcn_readlane(m.bytes, q + c));
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          v[c][r] = buffer_load(rs, (uint32_t)lane * 4u + 256u * (uint32_t)r);
+      }
+      return;
+    }
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-      const int32_t rk = __builtin_amdgcn_readlane(m.row, q + c);
-      const int32_t lk = __builtin_amdgcn_readlane(m.lag, q + c);
-      const int n = min(lk & kLagMask, (int)T);
       const __amdgpu_buffer_rsrc_t rs =
-          make_rsrc(a.prev + ((int64_t)rk * B + b) * T,
-                    n < t_end ? src_bytes : 0u);
+          make_rsrc((const void *)readlane_i64(m.addr, q + c),
+                    (uint32_t)__builtin_amdgcn_readlane(m.bytes, q + c));
+      const int w0 = min(__builtin_amdgcn_readlane(m.w0, q + c), 0);
 #pragma unroll
       for (int r = 0; r < R; ++r)
-        v[c][r] = buffer_load(rs, bin_offset(tl + 64 * r - n));
+        v[c][r] = buffer_load(rs, bin_offset(w0 + lane + 64 * r));
     }
   };
   // a group's sums to memory too, as the two-pass order stores them
@@ -165,7 +207,7 @@ __global__ __launch_bounds__(64 * kRowWaves)
     for (int r = 0; r < R; ++r)
       buffer_store((float)x[r], os, (uint32_t)(tl + 64 * r) * 4u);
   };
-  auto consume = [&](const Meta &m, int q, const float (&v)[C][R]) {
+  auto consume = [&](const Ready &m, int q, const float (&v)[C][R]) {
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       const double wk = readlane_f64(m.w, q + c);
@@ -176,7 +218,7 @@ __global__ __launch_bounds__(64 * kRowWaves)
         S[r] = fma(wk, x, S[r]);
         if (DS) Sd[DS ? r : 0] = fma(dk, x, Sd[DS ? r : 0]);
       }
-      if (!one && __builtin_amdgcn_readlane(m.lag, q + c) & kLastInGroup) {
+      if (!one && (m.ends >> (q + c) & 1ull) != 0) {  // uniform
 #pragma unroll
         for (int r = 0; r < R; ++r)
           gs[gl * TB + 64 * r + lane] = (float)S[r];
@@ -188,10 +230,11 @@ __global__ __launch_bounds__(64 * kRowWaves)
     }
   };
   if (e_hi > e_lo) {  // uniform
-    Meta cur = load_meta(e_lo);
+    Meta next = load_meta(e_lo);
     float va[C][R], vb[C][R];
     for (int64_t blk = e_lo; blk < e_hi; blk += 64) {
-      const Meta next = load_meta(blk + 64);
+      const Ready cur = ready(next);
+      next = load_meta(blk + 64);
       const int n = (int)min((int64_t)64, e_hi - blk);
       fetch(cur, 0, va);
       for (int q = 0; q < n; q += 2 * C) {
@@ -201,7 +244,6 @@ __global__ __launch_bounds__(64 * kRowWaves)
         if (q + 2 * C < n) fetch(cur, q + 2 * C, va);
         consume(cur, q + C, vb);
       }
-      cur = next;
     }
   }
   if (DS || one) {
@@ -232,12 +274,12 @@ __global__ __launch_bounds__(64 * kRowWaves)
   constexpr int NWT = NW / NWD, RW = R < NWT ? 1 : R / NWT;
   const int d0 = wave % NWD * DW, r0 = wave / NWD * RW;
   if (r0 >= R) return;  // uniform
-  double acc[DW][RW];
-#pragma unroll
-  for (int d = 0; d < DW; ++d)
-#pragma unroll
-    for (int r = 0; r < RW; ++r) acc[d][r] = 0.0;
+  double acc[DS ? 1 : DW][RW];
   if (!DS) {
+#pragma unroll
+    for (int d = 0; d < DW; ++d)
+#pragma unroll
+      for (int r = 0; r < RW; ++r) acc[DS ? 0 : d][r] = 0.0;
     // (the BRDF rows by LDS broadcast; by scalar loads 10 % slower)
 #pragma unroll 4
     for (int g = 0; g < ng; ++g) {
@@ -250,23 +292,24 @@ __global__ __launch_bounds__(64 * kRowWaves)
       for (int d = 0; d < DW; ++d) {
         const double cd = ct[g * DP + d0 + d];
 #pragma unroll
-        for (int r = 0; r < RW; ++r) acc[d][r] = fma(cd, x[r], acc[d][r]);
+        for (int r = 0; r < RW; ++r)
+          acc[DS ? 0 : d][r] = fma(cd, x[r], acc[DS ? 0 : d][r]);
       }
     }
   } else {
-    const int32_t *gmap =
-        reinterpret_cast<const int32_t *>(part + (size_t)NW * TB);
 #pragma unroll
-    for (int r = 0; r < RW; ++r) {
-      const double sd = shared_sum(r0 + r);
-#pragma unroll
-      for (int d = 0; d < DW; ++d) {
-        const int g = gmap[d0 + d];
-        acc[d][r] =
-            (g >= 0 ? (double)gs[g * TB + 64 * (r0 + r) + lane] : 0.0) + sd;
-      }
-    }
+    for (int r = 0; r < RW; ++r) acc[0][r] = shared_sum(r0 + r);
   }
+  // the order's value: of the diffuse + specular plan the diffuse sum and
+  // the direction's specular group, picked where it is written
+  const int32_t *gmap =
+      reinterpret_cast<const int32_t *>(part + (size_t)NW * TB);
+  auto value = [&](int d, int r) {
+    if (!DS) return acc[DS ? 0 : d][r];
+    const int g = gmap[d0 + d];
+    return (g >= 0 ? (double)gs[g * TB + 64 * (r0 + r) + lane] : 0.0) +
+           acc[0][r];
+  };
   const int64_t dstride = (int64_t)B * T;
   const int64_t base = j * D * dstride + (int64_t)b * T;
   const uint32_t span = (uint32_t)(((int64_t)(D - 1) * dstride + T) * 4);
@@ -283,7 +326,7 @@ __global__ __launch_bounds__(64 * kRowWaves)
 #pragma unroll
       for (int r = 0; r < RW; ++r) {
         const int t = tl + 64 * (r0 + r);
-        double v = acc[d][r];
+        double v = value(d, r);
         if (t == nj && d0 + d < D)
           v += a.inj.e0[(j * D + d0 + d) * B + b];
         buffer_store((float)v, rc, offset(d0 + d, t, a.sp.Tc));
@@ -296,7 +339,8 @@ __global__ __launch_bounds__(64 * kRowWaves)
       make_rsrc(a.tot_lo + base, a.sp.last ? 0u : span);
   const __amdgpu_buffer_rsrc_t rp =
       make_rsrc((a.pair ? a.pair : a.cur) + base, a.pair ? span : 0u);
-  constexpr int NP = DW * RW, K = NP < 8 ? NP : 8;  // (d, r) pairs
+  constexpr int NP = DW * RW, KM = DS ? 16 : 8;  // (d, r) pairs
+  constexpr int K = NP < KM ? NP : KM;           // loaded at a time
 #pragma unroll
   for (int p0 = 0; p0 < NP; p0 += K) {
     float h[K], l[K], e[K];
@@ -311,7 +355,8 @@ __global__ __launch_bounds__(64 * kRowWaves)
     for (int q = 0; q < K; ++q) {
       const int d = (p0 + q) / RW, r = (p0 + q) % RW;
       const uint32_t off = offset(d0 + d, tl + 64 * (r0 + r), a.sp.Tc);
-      const double v = a.sp.round ? (double)(float)acc[d][r] : acc[d][r];
+      const double x = value(d, r);
+      const double v = a.sp.round ? (double)(float)x : x;
       double sum = (double)h[q] + (double)l[q];
       sum += (double)e[q];
       sum += v;
@@ -357,12 +402,12 @@ int launch_dp(const spr_exchange_plan &p, const RowArgs &a, hipStream_t s) {
 
 // The shape of an order: R bins per lane here, or 0 for the two passes.  The
 // two costs are estimated in ns from what was measured on shoeboxes of 94 to
-// 1,072 patches, 1, 16 and 64 directions, 1 to 8 bands, 128 to 2,048 bins
+// 1,170 patches, 1, 16 and 64 directions, 1 to 8 bands, 100 to 4,000 bins
 // (R = 1 and 8 were tried too: at most 10 % faster anywhere):
 // * here a workgroup costs 6 for its start, 0.2 per direction and bin row
-//   written (0.13 with two weights), and per entry 0.06 (R = 4) or 0.048 (R = 2), 1.6 times that with
-//   two weights (an eighth of it per wave; shared out over the chip), more
-//   where there are fewer groups than waves;
+//   written (0.13 with two weights), and per entry 0.06 (R = 4) or 0.048
+//   (R = 2), 1.6 times that with two weights (an eighth of it per wave;
+//   shared out over the chip), more where there are fewer groups than waves;
 // * a tile's workgroup (512 bins, or 256 with two weights) walks its entries
 //   in 130 per merged entry and 12 per entry, whatever its bins; a workgroup
 //   per CU runs at that pace, the chip takes 410 (530) in that time;
@@ -370,8 +415,8 @@ int launch_dp(const spr_exchange_plan &p, const RowArgs &a, hipStream_t s) {
 //   its row in 900 per entry, at a rate of 0.2 (0.65) per entry;
 // * two passes write and read the group sums, 0.0018 per group and bin, and
 //   take a launch more, 8,000.
-// Over 810 such cases the choice is within 1.5 % of the better one on
-// average (at most 1.4 times slower) and 1.6 times faster than two passes.
+// Over 881 such cases the choice is within 1.3 % of the best one on average
+// (at most 1.5 times slower) and 1.5 times faster than two passes.
 int row_shape(const spr_exchange_plan &p, int64_t T, const OrderSpan &sp) {
   const int64_t DP = spr_padded_directions(p.D);
   if (p.order_shape < 0 || T >= ((int64_t)1 << 29) ||

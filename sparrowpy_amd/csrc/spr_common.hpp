@@ -48,10 +48,12 @@ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // modulo 8 picks the XCD).  xcd_tile maps block ids so that each XCD works
 // through one contiguous range of logical tiles: neighbouring tiles (same
 // destination patch, neighbouring time blocks) then share that XCD's L2.
-__device__ __forceinline__ int64_t xcd_tile(int64_t bid, int64_t nblocks) {
-  const int64_t n_xcd = 8;
-  int64_t per = nblocks / n_xcd, rem = nblocks % n_xcd;
-  int64_t x = bid % n_xcd, k = bid / n_xcd;
+// Grids hold fewer than 2^31 blocks; 32-bit arithmetic, as a 64-bit division
+// is over a hundred scalar instructions before a block's first load.
+__device__ __forceinline__ uint32_t xcd_tile(uint32_t bid, int64_t nblocks) {
+  const uint32_t n_xcd = 8, n = (uint32_t)nblocks;
+  const uint32_t per = n / n_xcd, rem = n % n_xcd;
+  const uint32_t x = bid % n_xcd, k = bid / n_xcd;
   return x < rem ? x * (per + 1) + k : rem * (per + 1) + (x - rem) * per + k;
 }
 

@@ -20,13 +20,29 @@ constexpr int32_t kLagMask = 0x3fffffff;
 // one XCD at a time are neighbouring destinations (neighbouring patches of
 // a wall) in the same band and time window, which read nearly the same
 // source histogram segments -- so those reads are shared through L2/MALL.
-__device__ __forceinline__ void dest_major_tile(int64_t tile, int64_t P,
+__device__ __forceinline__ void dest_major_tile(uint32_t tile,
+                                                int64_t nblocks, int B,
                                                 int n_tblk, int64_t &j,
                                                 int &b, int &tb) {
+  const uint32_t nt = (uint32_t)n_tblk;
+  const uint32_t P = (uint32_t)nblocks / ((uint32_t)B * nt);
+  const uint32_t rest = tile / P;
   j = tile % P;
-  const int64_t rest = tile / P;
-  tb = (int)(rest % n_tblk);
-  b = (int)(rest / n_tblk);
+  tb = (int)(rest % nt);
+  b = (int)(rest / nt);
+}
+
+// Time-major: consecutive tiles are the time blocks of one destination.
+__device__ __forceinline__ void time_major_tile(uint32_t tile,
+                                                int64_t nblocks, int B,
+                                                int n_tblk, int64_t &j,
+                                                int &b, int &tb) {
+  const uint32_t nt = (uint32_t)n_tblk;
+  const uint32_t P = (uint32_t)nblocks / ((uint32_t)B * nt);
+  const uint32_t jb = tile / nt;
+  tb = (int)(tile % nt);
+  j = jb % P;
+  b = (int)(jb / P);
 }
 
 // Raw buffer access with a gfx9 buffer descriptor: a load whose byte

@@ -225,8 +225,8 @@ __global__ __launch_bounds__(256 * (JT / JW)) void tile_gather_kernel(
   constexpr int NQ = MB / C, BS = 256;
   int64_t tile;
   int b, tb;
-  dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks / (B * n_tblk),
-                  n_tblk, tile, b, tb);
+  dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks, B, n_tblk, tile, b,
+                  tb);
   const int t0 = tb * (BS * R);
   const int t_end = min(Tc, t0 + BS * R);
   const int64_t m_begin = tptr[tile], m_end = tptr[tile + 1];
@@ -474,8 +474,8 @@ tile_lds_gather_kernel(
   auto win = [&](int buf) -> float(*)[W] { return buf ? lds_b : lds_a; };
   int64_t tile;
   int b, tb;
-  dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks / (B * n_tblk),
-                  n_tblk, tile, b, tb);
+  dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks, B, n_tblk, tile, b,
+                  tb);
   const int64_t m_begin = tptr[tile];
   // entries of the tile (< 2^31): batch positions are 32-bit offsets from
   // m_begin, so every loop bound is a scalar 32-bit compare

@@ -108,131 +108,262 @@ __global__ void direction_sum_kernel(int64_t P, int64_t D, int64_t B,
   musum[(j * B + b) * T + t] = (float)s;
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+// Lane exchanges of a float64 for the reductions below.  swap32 gives a the
+// low halves (lanes 0-31) of a and b and b their high halves; swap16 gives a
+// the even 16-lane rows and b the odd ones; ror turns each 16-lane row.
+__device__ __forceinline__ void swap32(double &a, double &b) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, a),
+                 y = __builtin_bit_cast(uint64_t, b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)y,
+                                                   false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(
+      (uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
+  a = __builtin_bit_cast(double, (uint64_t)lo[0] | (uint64_t)hi[0] << 32);
+  b = __builtin_bit_cast(double, (uint64_t)lo[1] | (uint64_t)hi[1] << 32);
+}
+__device__ __forceinline__ void swap16(double &a, double &b) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, a),
+                 y = __builtin_bit_cast(uint64_t, b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)y,
+                                                   false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(
+      (uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
+  a = __builtin_bit_cast(double, (uint64_t)lo[0] | (uint64_t)hi[0] << 32);
+  b = __builtin_bit_cast(double, (uint64_t)lo[1] | (uint64_t)hi[1] << 32);
+}
+template <int N>
+__device__ __forceinline__ double ror(double v) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(
+      0, (int)(uint32_t)x, 0x120 | N, 0xf, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(
+      0, (int)(uint32_t)(x >> 32), 0x120 | N, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, (uint64_t)lo | (uint64_t)hi << 32);
 }
 
-// One backward order: mu_out += A^T mu_next (mu_out holds lambda on entry),
-// and the entries' table gradients ga[0,b,q] += sum_t musum[j,b,t+n]
-// ek[i,d',b,t], ga[1,b,q] += sum_t mu_next[j,m,b,t+n] ek[i,d',b,t]
-// (q: transposed entry, d' its source direction).  A workgroup takes one
-// (source i, band, block of 256*R bins), sources fastest, and streams all
-// entries of source i -- sorted by direction, a flag on the last entry of
-// each direction -- in chunks of C, the next chunk's loads (mu-sum row,
-// specular mu row, the source's own order-k row) in flight while the
-// current one is summed.  At a direction's last entry the sum is added to
-// its mu_out row with float atomics (each element receives exactly one
-// add, so the result does not depend on their order).  A bin t + n beyond
-// the histogram is an out-of-range buffer offset and reads 0.  The
-// per-entry dot products are reduced over each wave and added (float64
-// atomics) by lanes 0 .. 2C-1.  Requires T < 2^29.  Only bins that E_k can
-// hold energy in (t < Tk) are formed, from mu_next's bins below Tn (those of
-// E_{k+1}, at least Tk plus the longest delay or T).
-template <int R, int C>
-__global__ __launch_bounds__(256) void adjoint_ds_kernel(
-    int D, int B, int T, int Tk, int Tn, int n_tblk, int64_t nblocks, int64_t Vd,
-    const int64_t *__restrict__ tgptr, const int32_t *__restrict__ tkey,
-    const int32_t *__restrict__ tlag, const int32_t *__restrict__ tm,
-    const double *__restrict__ twa, const double *__restrict__ twc,
-    const float *__restrict__ musum, const float *__restrict__ munext,
-    const float *__restrict__ ek, float *__restrict__ muout,
-    double *__restrict__ ga) {
-  constexpr int BS = 256;
+// The wave's sums of four values: lanes 0-15 get v0's, 16-31 v2's, 32-47
+// v1's, 48-63 v3's (16 vector instructions for each two values; a butterfly
+// over the wave for each is 36, 12 of them through LDS).
+__device__ __forceinline__ double wave_sums(double v0, double v1, double v2,
+                                            double v3) {
+  swap32(v0, v1);
+  swap32(v2, v3);
+  double a = v0 + v1, b = v2 + v3;
+  swap16(a, b);
+  double s = a + b;
+  s += ror<8>(s);
+  s += ror<4>(s);
+  s += ror<2>(s);
+  return s + ror<1>(s);
+}
+
+// One backward order: mu_out = lambda + A^T mu_next, and the entries' table
+// gradients ga[0,b,q] += sum_t musum[j,b,t+n] ek[i,d',b,t], ga[1,b,q] +=
+// sum_t mu_next[j,m,b,t+n] ek[i,d',b,t] (q: transposed entry, d' its source
+// direction).  A workgroup of 8 waves takes one (source i, band, block of
+// 64 R bins), sources fastest.  It sets its part of mu_out to lambda; then
+// each wave sums a run of whole directions with about an eighth of the
+// source's entries (sorted by direction, a flag on the last entry of each),
+// two at a time, the next two's loads (mu-sum row, specular mu row, the
+// source's own order-k row) in flight while the current ones are summed.
+// Each lane makes one entry of 64 ready (addresses and bytes left in the
+// rows), which the wave then takes by v_readlane.  At a direction's last
+// entry the sum is added to its mu_out row with float atomics (each element
+// receives exactly one add, so the result does not depend on their order).
+// A bin t + n beyond the histogram is an out-of-range buffer offset and reads
+// 0.  The dot products of two entries are reduced over the wave at once and
+// added (float64 atomics) by four lanes.  Requires T < 2^29.  Only bins that
+// E_k can hold energy in (t < Tk) are formed, from mu_next's bins below Tn
+// (those of E_{k+1}, at least Tk plus the longest delay or T).
+// Bound by the vector instructions of an entry, about 50 of which 28 are its
+// sums, and by latency where there are few sources.  232 patches, 64
+// directions, 3 bands: 107 us on average over orders of up to 1,400 bins;
+// with four waves of 64 R bins that each walked all entries, a butterfly for
+// each dot product and lambda copied by a launch of its own 206 + 24 us.
+// Gradient of a directional shoebox (1,072 patches, 6 bands, 2,000 bins, 10
+// orders) 91 ms instead of 124.
+constexpr int kAdjointWaves = 8;
+
+template <int R>
+__global__ __launch_bounds__(64 * kAdjointWaves)
+    __attribute__((amdgpu_waves_per_eu(4))) void adjoint_ds_kernel(
+        int D, int B, int T, int Tk, int Tn, int n_tblk, int64_t nblocks,
+        int64_t Vd, const int64_t *__restrict__ tgptr,
+        const int32_t *__restrict__ tkey, const int32_t *__restrict__ tlag,
+        const int32_t *__restrict__ tm, const double *__restrict__ twa,
+        const double *__restrict__ twc, const float *__restrict__ lam,
+        const float *__restrict__ musum, const float *__restrict__ munext,
+        const float *__restrict__ ek, float *__restrict__ muout,
+        double *__restrict__ ga) {
+  constexpr int NW = kAdjointWaves, TB = 64 * R, C = 2;
   constexpr int32_t kDstMask = (1 << 25) - 1;
   int64_t i;
   int b, tb;
   dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks, B, n_tblk, i, b,
                   tb);
-  const int64_t q0 = tgptr[i * D], q1 = tgptr[i * D + D];
-  if (q1 == q0) return;
-  const int tl = tb * (BS * R) + (int)threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lane = (int)threadIdx.x & 63;
-  const uint32_t mu_bytes = (uint32_t)Tn * 4u, ek_bytes = (uint32_t)Tk * 4u;
+  const int t0 = tb * TB;
+  const int64_t srow = i * D;  // row (i, d') = srow + d'
+  const int64_t stride = (int64_t)B * T;
+
+  // mu_out = lambda: the waves take the directions in turn
+  const int64_t own = srow * stride + (int64_t)b * T + t0;
+  const uint32_t own_bytes = (uint32_t)min(Tk - t0, TB) * 4u;
+  constexpr int CP = 4;  // rows' loads in flight
+  for (int d = wave; d < D; d += NW * CP) {
+    float v[CP][R];
+#pragma unroll
+    for (int c = 0; c < CP; ++c) {
+      const int dd = d + c * NW;
+      const __amdgpu_buffer_rsrc_t rs =
+          make_rsrc(lam + own + min(dd, D - 1) * stride,
+                    dd < D ? own_bytes : 0u);
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        v[c][r] = buffer_load(rs, (uint32_t)(lane + 64 * r) * 4u);
+    }
+#pragma unroll
+    for (int c = 0; c < CP; ++c) {
+      const int dd = d + c * NW;
+      const __amdgpu_buffer_rsrc_t rs =
+          make_rsrc(muout + own + min(dd, D - 1) * stride,
+                    dd < D ? own_bytes : 0u);
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        buffer_store(v[c][r], rs, (uint32_t)(lane + 64 * r) * 4u);
+    }
+  }
+
+  // the wave's entries [e_lo, e_hi): whole directions whose first entry lies
+  // in the wave's eighth
+  const int64_t *starts = tgptr + srow;
+  const int64_t q0 = starts[0], q1 = starts[D];
+  const int64_t cut_lo = q0 + (q1 - q0) * wave / NW;
+  const int64_t cut_hi = q0 + (q1 - q0) * (wave + 1) / NW;
+  int64_t e_lo = q1, e_hi = q1;
+  for (int d = 0; d < D; d += 64) {
+    const bool in = d + lane < D;
+    const int64_t st = starts[in ? d + lane : D];
+    const uint64_t lo = __ballot(in && st >= cut_lo);
+    const uint64_t hi = __ballot(in && st >= cut_hi);
+    if (lo != 0 && e_lo == q1) e_lo = readlane_i64(st, __builtin_ctzll(lo));
+    if (hi != 0 && e_hi == q1) e_hi = readlane_i64(st, __builtin_ctzll(hi));
+  }
+  // the stores above are complete (vmcnt(0): in the L2 that this workgroup's
+  // atomics work in) before any wave adds to them
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  __syncthreads();
+  if (e_hi <= e_lo) return;  // uniform, after the barrier
+
   const double *wa = twa + (int64_t)b * Vd, *wc = twc + (int64_t)b * Vd;
   double *gda = ga + (int64_t)b * Vd, *gdc = ga + ((int64_t)B + b) * Vd;
-  const int64_t srow = i * D;  // row (i, d') = srow + d'
-
-  auto fetch = [&](int64_t qq, float (&x)[C][R], float (&y)[C][R],
+  struct Meta {
+    int32_t key, lag, m;
+    double a, c;
+  };
+  struct Ready {
+    int64_t x, y, row;  // addresses; the source's row from ek's first element
+    int32_t bytes;
+    double a, c;
+    uint64_t ends;
+  };
+  auto load_meta = [&](int64_t e0) {
+    const int64_t q = e0 + lane;
+    const bool in = q < e_hi;
+    const int64_t qc = in ? q : e_hi - 1;
+    Meta v;
+    v.key = tkey[qc];
+    v.m = tm[qc];
+    v.lag = in ? tlag[qc] : kLagMask;  // past the end: no bins, no flag
+    v.a = in ? wa[qc] : 0.0;
+    v.c = in ? wc[qc] : 0.0;
+    return v;
+  };
+  auto ready = [&](const Meta &v) {
+    Ready x;
+    const int64_t j = v.key & kDstMask, d = v.key >> 25;
+    const int n = min(v.lag & kLagMask, T), first = t0 + n;
+    x.x = (int64_t)(musum + (j * B + b) * (int64_t)T + first);
+    x.y = (int64_t)(munext + ((j * D + v.m) * B + b) * (int64_t)T + first);
+    x.row = ((srow + d) * B + b) * (int64_t)T + t0;
+    x.bytes = max(Tn - first, 0) * 4;
+    x.a = v.a;
+    x.c = v.c;
+    x.ends = __ballot((v.lag & kLastInGroup) != 0);
+    return x;
+  };
+  auto fetch = [&](const Ready &v, int q, float (&x)[C][R], float (&y)[C][R],
                    float (&e)[C][R]) {
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-      const bool in = qq + c < q1;
-      const int64_t qc = in ? qq + c : q1 - 1;
-      const int32_t key = tkey[qc];
-      const int64_t j = key & kDstMask, d = key >> 25, m = tm[qc];
-      const int n = min(tlag[qc] & kLagMask, T);  // >= T: reads 0
-      const uint32_t sz = in ? mu_bytes : 0u;
+      const uint32_t sz =
+          (uint32_t)__builtin_amdgcn_readlane(v.bytes, q + c);
       const __amdgpu_buffer_rsrc_t rx =
-          make_rsrc(musum + (j * B + b) * (int64_t)T, sz);
+          make_rsrc((const void *)readlane_i64(v.x, q + c), sz);
       const __amdgpu_buffer_rsrc_t ry =
-          make_rsrc(munext + ((j * D + m) * B + b) * (int64_t)T, sz);
+          make_rsrc((const void *)readlane_i64(v.y, q + c), sz);
       const __amdgpu_buffer_rsrc_t re =
-          make_rsrc(ek + ((srow + d) * B + b) * (int64_t)T,
-                    in ? ek_bytes : 0u);
+          make_rsrc(ek + readlane_i64(v.row, q + c), own_bytes);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const int t = tl + BS * r;
-        x[c][r] = buffer_load(rx, (uint32_t)(t + n) * 4u);
-        y[c][r] = buffer_load(ry, (uint32_t)(t + n) * 4u);
-        e[c][r] = buffer_load(re, (uint32_t)t * 4u);
+        const uint32_t off = (uint32_t)lane * 4u + 256u * (uint32_t)r;
+        x[c][r] = buffer_load(rx, off);
+        y[c][r] = buffer_load(ry, off);
+        e[c][r] = buffer_load(re, off);
       }
     }
   };
   double acc[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) acc[r] = 0.0;
-  auto consume = [&](int64_t qq, const float (&x)[C][R],
-                     const float (&y)[C][R], const float (&e)[C][R]) {
+  auto consume = [&](const Ready &v, int64_t blk, int q,
+                     const float (&x)[C][R], const float (&y)[C][R],
+                     const float (&e)[C][R]) {
     double pa[C], pc[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       pa[c] = pc[c] = 0.0;
-      if (qq + c < q1) {
-        const double a = wa[qq + c], s = wc[qq + c];
+      const double wx = readlane_f64(v.a, q + c);
+      const double wy = readlane_f64(v.c, q + c);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const double xd = (double)x[c][r], yd = (double)y[c][r];
+        const double ed = (double)e[c][r];
+        acc[r] = fma(wx, xd, acc[r]);
+        acc[r] = fma(wy, yd, acc[r]);
+        pa[c] = fma(ed, xd, pa[c]);
+        pc[c] = fma(ed, yd, pc[c]);
+      }
+      if ((v.ends >> (q + c) & 1ull) != 0) {  // uniform
+        float *o = muout + readlane_i64(v.row, q + c) + lane;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-          const double xd = (double)x[c][r], yd = (double)y[c][r];
-          const double ed = (double)e[c][r];
-          acc[r] = fma(a, xd, acc[r]);
-          acc[r] = fma(s, yd, acc[r]);
-          pa[c] = fma(ed, xd, pa[c]);
-          pc[c] = fma(ed, yd, pc[c]);
-        }
-        if (tlag[qq + c] & kLastInGroup) {
-          const int64_t d = tkey[qq + c] >> 25;
-          float *o = muout + ((srow + d) * B + b) * (int64_t)T;
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            const int t = tl + BS * r;
-            if (t < Tk) unsafeAtomicAdd(o + t, (float)acc[r]);
-            acc[r] = 0.0;
-          }
+          if (t0 + lane + 64 * r < Tk)
+            unsafeAtomicAdd(o + 64 * r, (float)acc[r]);
+          acc[r] = 0.0;
         }
       }
     }
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-      pa[c] = wave_sum(pa[c]);
-      pc[c] = wave_sum(pc[c]);
-    }
-    if (lane < 2 * C) {
-      const int c = lane % C;
-      double v = 0.0;
-#pragma unroll
-      for (int cc = 0; cc < C; ++cc)
-        if (cc == c) v = lane < C ? pa[cc] : pc[cc];
-      if (qq + c < q1) unsafeAtomicAdd((lane < C ? gda : gdc) + qq + c, v);
-    }
+    const double sum = wave_sums(pa[0], pa[1], pc[0], pc[1]);
+    const int64_t qq = blk + q + (lane >> 5);
+    if ((lane & 15) == 0 && qq < e_hi)
+      unsafeAtomicAdd((lane & 16 ? gdc : gda) + qq, sum);
   };
+  Meta next = load_meta(e_lo);
   float xa[C][R], ya[C][R], ea[C][R], xb[C][R], yb[C][R], eb[C][R];
-  fetch(q0, xa, ya, ea);
-  for (int64_t q = q0; q < q1; q += 2 * C) {
-    fetch(q + C, xb, yb, eb);
-    consume(q, xa, ya, ea);
-    fetch(q + 2 * C, xa, ya, ea);
-    consume(q + C, xb, yb, eb);
+  for (int64_t blk = e_lo; blk < e_hi; blk += 64) {
+    const Ready cur = ready(next);
+    next = load_meta(blk + 64);
+    const int n = (int)min((int64_t)64, e_hi - blk);
+    fetch(cur, 0, xa, ya, ea);
+    for (int q = 0; q < n; q += 2 * C) {
+      if (q + C < n) fetch(cur, q + C, xb, yb, eb);
+      consume(cur, blk, q, xa, ya, ea);
+      if (q + C >= n) break;
+      if (q + 2 * C < n) fetch(cur, q + 2 * C, xa, ya, ea);
+      consume(cur, blk, q + C, xb, yb, eb);
+    }
   }
 }
 
@@ -612,28 +743,6 @@ __global__ void injection_table_grad_kernel(
                   energy0[p * B + b] * (double)mu0[q * T + n]);
 }
 
-// dst = src on bins [0, Tk) of every histogram row; a wave takes 256 bins of
-// one row.
-__global__ __launch_bounds__(256) void copy_rows_kernel(
-    int64_t rows, int64_t T, int64_t Tk, int64_t chunks,
-    const float *__restrict__ src, float *__restrict__ dst) {
-  const int lane = (int)threadIdx.x & 63;
-  const int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (q >= rows * chunks) return;
-  const int64_t row = q / chunks, t0 = q % chunks * 256 + lane;
-  float v[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int64_t t = t0 + 64 * r;
-    v[r] = src[row * T + (t < Tk ? t : 0)];
-  }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int64_t t = t0 + 64 * r;
-    if (t < Tk) dst[row * T + t] = v[r];
-  }
-}
-
 }  // namespace
 
 int direction_sum(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tn,
@@ -651,34 +760,23 @@ int adjoint_ds(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tk,
                const double *twa, const double *twc, const float *lam,
                const float *musum, const float *munext, const float *ek,
                float *muout, double *ga, hipStream_t s) {
-  const int64_t chunks = ceil_div(Tk, 256), copies = P * D * B * chunks;
-  SPR_REQUIRE(ceil_div(copies, 4) < (int64_t)0x7fffffff,
-              "spr_exchange_adjoint_ds: grid too large");
-  hipLaunchKernelGGL(copy_rows_kernel, dim3((unsigned)ceil_div(copies, 4)),
-                     dim3(256), 0, s, P * D * B, T, Tk, chunks, lam, muout);
-  SPR_LAUNCH_CHECK();
-  // 8 bins per lane, 2 entries per chunk: each entry's two wave
-  // reductions (its table-gradient dot products) then cover 512 bins.
-  // Directional shoebox, order 30: backward 1.49 s with this shape; 1.66 s
-  // with R = 4, C = 4, 1.76 s with R = 8, C = 1, 1.78 s with R = 16, C = 1
-  // or R = 4, C = 2, 1.95 s with R = 16, C = 2, 2.68 s with R = 2, C = 4.
-  // Fewer bins per lane where 256 R would reach past Tk.
   auto go = [&](auto kernel, int R) {
-    const int64_t nt = ceil_div(Tk, (int64_t)256 * R);
+    const int64_t nt = ceil_div(Tk, (int64_t)64 * R);
     const int64_t nb = P * B * nt;
     SPR_REQUIRE(nb < (int64_t)0x7fffffff,
                 "spr_exchange_adjoint_ds: grid too large");
-    hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(256), 0, s, (int)D,
-                       (int)B, (int)T, (int)Tk, (int)Tn, (int)nt, nb, Vd,
-                       tgptr, tkey, tlag, tm, twa, twc, musum, munext, ek,
-                       muout, ga);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(64 * kAdjointWaves),
+                       0, s, (int)D, (int)B, (int)T, (int)Tk, (int)Tn,
+                       (int)nt, nb, Vd, tgptr, tkey, tlag, tm, twa, twc, lam,
+                       musum, munext, ek, muout, ga);
     SPR_LAUNCH_CHECK();
     return SPR_OK;
   };
-  if (Tk <= 256) return go(adjoint_ds_kernel<1, 4>, 1);
-  if (Tk <= 512) return go(adjoint_ds_kernel<2, 4>, 2);
-  if (Tk <= 1024) return go(adjoint_ds_kernel<4, 2>, 4);
-  return go(adjoint_ds_kernel<8, 2>, 8);
+  // 4 bins per lane, or 2 where 4 would reach past Tk for nothing: an entry's
+  // reductions and lane reads then serve 256 bins (8 do not fit the
+  // registers).
+  if (Tk <= 128) return go(adjoint_ds_kernel<2>, 2);
+  return go(adjoint_ds_kernel<4>, 4);
 }
 
 int spread_adjoint(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tn,

@@ -27,7 +27,7 @@ __device__ inline double extent(const double *sx, const double *sy, int from,
                                 int to, int q) {
   const double *v = q < 2 ? sx : sy;
   double e = v[from];
-#pragma unroll 4
+#pragma unroll 8
   for (int t = from + 1; t < to; ++t)
     e = (q & 1) ? fmax(e, v[t]) : fmin(e, v[t]);
   return e;
@@ -39,7 +39,7 @@ __device__ inline double extent(const double *sx, const double *sy, int from,
 // first member.  A workgroup per run, a lane per corner: most calls have a
 // handful of blockers and wait for the kernel's own code to come in from
 // memory, so every step is written once and not unrolled over corners (6
-// walls 4.4 us, 208 patches 10 us; a lane per blocker 19 us for either).
+// walls 5 us, 208 patches 11 us; a lane per blocker 19 us for either).
 __global__ __launch_bounds__(4 * kGroup) void blocker_kernel(
     int64_t NS, const double *__restrict__ normals,
     const double *__restrict__ pts, BlockerRec *__restrict__ recs,
@@ -110,9 +110,22 @@ __global__ __launch_bounds__(4 * kGroup) void blocker_kernel(
     }
   }
   __syncthreads();
+  const int n_lines = (int)s_lines[m] <= kLines ? (int)s_lines[m] : 0;
   if (!valid || same) return;
   BlockerGroup &g = groups[k];
-  g.box[q] = extent(sx, sy, 4 * m, 4 * (m + count), q);
+  const double u = extent(sx, sy, 4 * m, 4 * (m + count), q);
+  g.box[q] = u;
+  // evenly spaced lines?  (the member's four lanes look at a corner each)
+  const double y0 = __shfl(u, (t & 60) | 2), y1 = __shfl(u, (t & 60) | 3);
+  const double step = n_lines > 1 ? (y1 - y0) / (n_lines - 1) : kFarStep;
+  const double inv = 1.0 / step;
+  bool even = n_lines > 0;
+#pragma unroll 4
+  for (int e = m; e < m + count; ++e) {
+    const double l = (sy[4 * e + q] - y0) * inv;
+    even &= fabs(l - rint(l)) * step <= kLineSlack;
+  }
+  even = (__ballot(even) >> (t & 60) & 15u) == 15u;
   if (q != 0) return;
   g.n[0] = n.x, g.n[1] = n.y, g.n[2] = n.z;
   for (int e = 0; e < 3; ++e) g.m0[e] = m0[e], g.m1[e] = m1[e];
@@ -120,7 +133,10 @@ __global__ __launch_bounds__(4 * kGroup) void blocker_kernel(
   g.dc = kGroup * kPlaneStep * (2.0 + fabs(c));
   g.count = count;
   g.left = (s_long >> m & ((2u << (count - 1)) - 1u)) == 0;
-  g.n_lines = s_lines[m] <= kLines ? (int)s_lines[m] : 0;
+  g.n_lines = n_lines;
+  g.y0 = y0;
+  g.inv_step = inv;
+  g.step = even ? step : 0.0;
 }
 
 // Whether any member of the group that starts at blocker k0 blocks this
@@ -142,13 +158,8 @@ __device__ inline bool group_blocks(d3 a, d3 b, bool alive, int64_t k0,
   const bool left = meets && left_of(s.x, s.g, grp.box[0]) &&
                     left_of(s.x2, s.g, grp.box[0]);
   if (grp.left != 0 && grp.n_lines > 0 && __any(left)) {
-    const double m = kCullBox + kLineSlack + s.g;
-    bool near = false;
-    for (int l = 0; l < grp.n_lines; ++l)
-      near |= !(fabs(s.y - grp.lines[l]) > m);
-    if (any_two)
-      for (int l = 0; l < grp.n_lines; ++l)
-        near |= !(fabs(s.y2 - grp.lines[l]) > m);
+    bool near = near_line(s.y, s.g, grp);
+    if (any_two) near |= near_line(s.y2, s.g, grp);
     meets = meets && (near || !left);
   }
   if (!__any(meets)) return false;
@@ -180,7 +191,8 @@ __device__ inline bool group_blocks(d3 a, d3 b, bool alive, int64_t k0,
 // Bound by sight()'s float64 arithmetic and by the wait for each group's
 // record: in a canyon of 5,122 patches, all of them blockers, a wave looks at
 // 86 groups, meets the box of 2.6 and takes 1.7 turns of the predicate, in
-// 8.0 ms for 13.1 M pairs; testing the predicate for every blocker that the
+// 5.6 ms for 13.1 M pairs (8.0 with unfused products, a division per group
+// and each line of corners compared); testing the predicate for every blocker that the
 // tile's cull leaves (about 1,500) took 105 ms.
 __global__ __launch_bounds__(256, 4) void p2p_visibility_kernel(
     int64_t P, const double *__restrict__ centers, int64_t NS,

@@ -96,6 +96,10 @@ constexpr double kPlaneStep = 1e-12;
 constexpr double kLongEdge = 1e3;  // see may_block
 constexpr int kLines = 36;         // 33 rows of corners, with some to spare
 constexpr double kLineStep = 1e-6;
+// Corners left out of a group's lines follow from one to the next within
+// kLineStep, so one of the lines is within this of each.
+constexpr double kLineSlack = 4 * kGroup * kLineStep;
+constexpr double kFarStep = 1e30;
 struct BlockerGroup {
   double n[3], m0[3], m1[3];
   double c;         // n . p0 of the first member
@@ -104,6 +108,9 @@ struct BlockerGroup {
   int32_t count;
   int32_t left;     // 1: no edge longer than kLongEdge (see may_block)
   int32_t n_lines;  // 0: more than kLines
+  // The lines as y0 + k step (k whole), each within kLineSlack: most walls'
+  // patches.  step 0: they are not; a single line has a step out of reach.
+  double y0, step, inv_step;
   // rotated y of the members' corners, those within kLineStep once
   double lines[kLines];
 };
@@ -211,6 +218,23 @@ struct Sight {
   bool two;
 };
 
+// a . b as the culls form it, two fused steps (their margins cover rounding;
+// the predicate's dot() is the reference's).
+__host__ __device__ inline double cull_dot(d3 a, d3 b) {
+  return fma(a.z, b.z, fma(a.y, b.y, a.x * b.x));
+}
+
+// 1 / x to about 1e-15 of it (hardware reciprocal and a Newton step); what
+// overflows or is 0 gives an infinity or NaN, which no cull drops.
+__host__ __device__ inline double cull_inverse(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double r = __builtin_amdgcn_rcp(x);
+  return fma(fma(-x, r, 1.0), r, r);
+#else
+  return 1.0 / x;
+#endif
+}
+
 // False if the segment a-b cannot be blocked by any member: both ends lie
 // beyond kCullPlane on one side, so that neither is in the plane and the
 // crossing point lies outside the segment.  With the ends beyond kCullPlane
@@ -223,19 +247,19 @@ struct Sight {
 __host__ __device__ inline bool sight(d3 a, d3 b, const BlockerGroup &r,
                                       Sight &s) {
   const d3 n = load3(r.n), m0 = load3(r.m0), m1 = load3(r.m1);
-  const double da = dot(n, a) - r.c, db = dot(n, b) - r.c;
+  const double da = cull_dot(n, a) - r.c, db = cull_dot(n, b) - r.c;
   if ((da > kCullPlane && db > kCullPlane) ||
       (da < -kCullPlane && db < -kCullPlane))
     return false;
-  const double xa = dot(m0, a), ya = dot(m1, a);
-  const double xb = dot(m0, b), yb = dot(m1, b);
+  const double xa = cull_dot(m0, a), ya = cull_dot(m1, a);
+  const double xb = cull_dot(m0, b), yb = cull_dot(m1, b);
   const bool na = fabs(da) <= kCullPlane, nb = fabs(db) <= kCullPlane;
   s.two = false;
   s.g = 0.0;
   if (!na && !nb) {
-    const double inv = 1.0 / (da - db), t = da * inv;
-    s.x = xa + t * (xb - xa);
-    s.y = ya + t * (yb - ya);
+    const double inv = cull_inverse(da - db), t = da * inv;
+    s.x = fma(t, xb - xa, xa);
+    s.y = fma(t, yb - ya, ya);
     s.g = r.dc * (fabs(xb - xa) + fabs(yb - ya)) * fabs(inv);
     return true;
   }
@@ -255,10 +279,6 @@ __host__ __device__ inline bool sight(d3 a, d3 b, const BlockerGroup &r,
   return true;
 }
 
-// Corners left out of a group's lines follow from one to the next within
-// kLineStep, so one of the lines is within this of each.
-constexpr double kLineSlack = 4 * kGroup * kLineStep;
-
 // Whether a point within g of (x, y) may pass point_in_blocker with this box:
 // it needs x <= box[1] and y in box[2..3], up to the margin.
 __host__ __device__ inline bool in_reach(double x, double y, double g,
@@ -274,9 +294,20 @@ __host__ __device__ inline bool in_reach(double x, double y, double g,
 // at least twice that in y, so with edges up to kLongEdge its normal's x is
 // above the 1e-6 at which the reference skips an edge, and both the edge
 // test and the sign of each crossing are decided far above rounding.
-// near: whether y is that close to a corner.
 __host__ __device__ inline bool left_of(double x, double g, double x_min) {
   return x + (kCullBox + g) < x_min;
+}
+// Whether y is that close to one of the group's lines of corners.
+__host__ __device__ inline bool near_line(double y, double g,
+                                          const BlockerGroup &r) {
+  const double m = kCullBox + 2 * kLineSlack + g;
+  if (r.step > 0) {  // uniform
+    const double u = (y - r.y0) * r.inv_step;
+    return !(fabs(u - rint(u)) * r.step > m);
+  }
+  bool near = false;
+  for (int l = 0; l < r.n_lines; ++l) near |= !(fabs(y - r.lines[l]) > m);
+  return near;
 }
 __host__ __device__ inline bool may_block(double x, double y, double g,
                                           int left, const BlockerRec &r) {
@@ -287,7 +318,8 @@ __host__ __device__ inline bool may_block(double x, double y, double g,
 }
 
 // geometry.py:841-909 _basic_visibility(vis_point=a, eval_point=b).
-__host__ __device__ inline bool basic_visibility(d3 a, d3 b, const BlockerRec &r) {
+__host__ __device__ inline bool basic_visibility(d3 a, d3 b,
+                                                 const BlockerRec &r) {
   const bool vin = point_in_blocker(a, r);
   const bool ein = point_in_blocker(b, r);
   const d3 n = load3(r.n);

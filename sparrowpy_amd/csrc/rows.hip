@@ -407,7 +407,10 @@ int launch_dp(const spr_exchange_plan &p, const RowArgs &a, hipStream_t s) {
 // * here a workgroup costs 6 for its start, 0.2 per direction and bin row
 //   written (0.13 with two weights), and per entry 0.06 (R = 4) or 0.048
 //   (R = 2), 1.6 times that with two weights (an eighth of it per wave;
-//   shared out over the chip), more where there are fewer groups than waves;
+//   shared out over the chip), more where there are fewer groups than waves
+//   (with one group they share it, and an entry costs 0.03 with R = 4: with
+//   0.06 the two passes were taken for a 1,170-patch diffuse room, 3 bands,
+//   700 bins: 612 us against 433);
 // * a tile's workgroup (512 bins, or 256 with two weights) walks its entries
 //   in 130 per merged entry and 12 per entry, whatever its bins; a workgroup
 //   per CU runs at that pace, the chip takes 410 (530) in that time;
@@ -415,8 +418,8 @@ int launch_dp(const spr_exchange_plan &p, const RowArgs &a, hipStream_t s) {
 //   its row in 900 per entry, at a rate of 0.2 (0.65) per entry;
 // * two passes write and read the group sums, 0.0018 per group and bin, and
 //   take a launch more, 8,000.
-// Over 881 such cases the choice is within 1.3 % of the best one on average
-// (at most 1.5 times slower) and 1.5 times faster than two passes.
+// Over 881 such cases the choice is within 1.2 % of the best one on average
+// (at most 1.3 times slower, 1.7 with two weights) and 1.5 times faster than two passes.
 int row_shape(const spr_exchange_plan &p, int64_t T, const OrderSpan &sp) {
   const int64_t DP = spr_padded_directions(p.D);
   if (p.order_shape < 0 || T >= ((int64_t)1 << 29) ||
@@ -438,7 +441,9 @@ int row_shape(const spr_exchange_plan &p, int64_t T, const OrderSpan &sp) {
                           ? std::pow(8.0 / std::max(groups, 1.0), 1.3)
                           : 1.0;
   const double here = (double)nb * (6.0 + (ds ? 0.13 : 0.2) * (double)(DP * R) +
-                                    (R == 4 ? 0.06 : 0.048) *
+                                    (R == 2            ? 0.048
+                                     : p.max_groups > 1 ? 0.06
+                                                        : 0.03) *
                                         (ds ? 1.6 : 1.0) * idle * E);
   double two = 8000.0 + (double)(n * sp.Tc) *
                             (0.0018 * (double)p.max_groups +

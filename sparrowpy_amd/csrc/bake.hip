@@ -365,16 +365,26 @@ __device__ inline double boole_sum(const double *y) {
          7.0 * y[4];
 }
 
-// integration.py:38-114 stokes_integration, one wavefront per pair (four
-// pairs per workgroup: one pair per workgroup is bound by how fast workgroups
-// start).  Whatever several terms share is formed once, by one lane each: the
-// 2x16 boundary points, the step factor of each segment and coordinate (NaN
-// where the reference skips the segment), Boole's sum over the 16x16 ln|r|
-// table, which is the same for the three coordinates.  Lane 0 only adds the
-// twelve outer terms, in the reference's (dim, segment) order.
+// What the lanes of one wave write to LDS before is read after.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// integration.py:38-114 stokes_integration, two pairs per wavefront (eight
+// per workgroup: one pair per workgroup is bound by how fast workgroups
+// start), a half of the wave for each where a pair has no more than 32 values
+// to form.  Whatever several terms share is formed once, by one lane each:
+// the 2x16 boundary points, the step factor of each segment and coordinate
+// (NaN where the reference skips the segment), Boole's sum over the 16x16
+// ln|r| table, which is the same for the three coordinates.  One lane only
+// adds the twelve outer terms, in the reference's (dim, segment) order.
 // Bound by the float64 logarithms and square roots of the table: 7.4 M pairs
-// of a canyon in 9.8 ms.  With 48 lanes forming each segment's nodes anew and
-// lane 0 alone all outer terms it was 21 ms.
+// of a canyon in 9.0 ms; one pair per wavefront 9.8; with 48 lanes forming
+// each segment's nodes anew and one all outer terms 21.
+constexpr int kStokesPairs = 2;  // of a wave
+
 __global__ __launch_bounds__(256) void stokes_kernel(
     int64_t P, const double *__restrict__ pts, const double *__restrict__ areas,
     int64_t V, const int32_t *__restrict__ pairs, double *__restrict__ ff) {
@@ -387,46 +397,55 @@ __global__ __launch_bounds__(256) void stokes_kernel(
     double inner[3][16];
     double outer[12];
   };
-  __shared__ Pair sh[4];
+  __shared__ Pair sh[4 * kStokesPairs];
   const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
-  const int64_t v = (int64_t)blockIdx.x * 4 + wave;
-  Pair &w = sh[wave];
+  const int half = lane >> 5, l = lane & 31;
+  const int64_t v = ((int64_t)blockIdx.x * 4 + wave) * kStokesPairs + half;
+  Pair *const two = sh + wave * kStokesPairs;
+  Pair &own = two[half];  // this half's pair
   int64_t i = -1, j = -1;
   if (v < V) i = pairs[2 * v], j = pairs[2 * v + 1];
   bool ok = i >= 0 && j >= 0 && i < P && j < P;  // else an invalid pair: skip
   const double *pi = pts + (ok ? 12 * i : 0), *pj = pts + (ok ? 12 * j : 0);
   // coincident pairs are nusselt_kernel's
-  ok = ok && !__any(lane < 16 && corners_meet(pj, pi, lane >> 2, lane & 3));
-  if (ok && lane < 32) {
-    const d3 p = boundary_point(lane < 16 ? pi : pj, lane & 15, 4);
-    double(*o)[16] = w.point[lane >> 4];
-    o[0][lane & 15] = p.x, o[1][lane & 15] = p.y, o[2][lane & 15] = p.z;
-  }
-  __syncthreads();
+  const uint64_t meet = __ballot(l < 16 && corners_meet(pj, pi, l >> 2, l & 3));
+  ok = ok && (uint32_t)(meet >> (32 * half)) == 0;
+  const uint64_t live = __ballot(ok);
+  if (live == 0) return;  // uniform; no workgroup barrier follows
   if (ok) {
-    if (lane < 24) {
-      const int dim = (lane % 12) >> 2, s = lane & 3;
-      const double *x = w.point[lane / 12][dim];
-      const bool take = fabs(x[(4 * s + 4) & 15] - x[4 * s]) > 1e-3;
-      w.step[lane / 12][dim][s] =
-          take ? boole_step(x[4 * s], x[4 * s + 1]) : kSkip;
-    }
+    const d3 p = boundary_point(l < 16 ? pi : pj, l & 15, 4);
+    double(*o)[16] = own.point[l >> 4];
+    o[0][l & 15] = p.x, o[1][l & 15] = p.y, o[2][l & 15] = p.z;
+  }
+  wave_lds_sync();
+  if (ok && l < 24) {
+    const int dim = (l % 12) >> 2, s = l & 3;
+    const double *x = own.point[l / 12][dim];
+    const bool take = fabs(x[(4 * s + 4) & 15] - x[4 * s]) > 1e-3;
+    own.step[l / 12][dim][s] =
+        take ? boole_step(x[4 * s], x[4 * s + 1]) : kSkip;
+  }
+  double y[5];
+  for (int h = 0; h < kStokesPairs; ++h) {
+    if ((live >> (32 * h) & 1) == 0) continue;  // uniform
+    Pair &w = two[h];
     const int q = lane & 15;
     const d3 b{w.point[1][0][q], w.point[1][1][q], w.point[1][2][q]};
     for (int a = lane >> 4; a < 16; a += 4)
       w.form[a][q] = log(norm(
           d3{w.point[0][0][a], w.point[0][1][a], w.point[0][2][a]} - b));
   }
-  __syncthreads();
-  double y[5];
-  if (ok) {
+  wave_lds_sync();
+  for (int h = 0; h < kStokesPairs; ++h) {
+    Pair &w = two[h];
     const int a = lane >> 2, s = lane & 3;
     for (int k = 0; k < 5; ++k) y[k] = w.form[a][(4 * s + k) & 15];
     w.sum[a][s] = boole_sum(y);
   }
-  __syncthreads();
-  if (ok && lane < 48) {
-    const int a = lane / 3, dim = lane % 3;
+  wave_lds_sync();
+  for (int t = lane; t < 48 * kStokesPairs; t += 64) {
+    Pair &w = two[t / 48];
+    const int a = t % 48 / 3, dim = t % 3;
     double acc = 0.0;
     for (int s = 0; s < 4; ++s) {
       const double h = w.step[1][dim][s];
@@ -434,17 +453,17 @@ __global__ __launch_bounds__(256) void stokes_kernel(
     }
     w.inner[dim][a] = acc;
   }
-  __syncthreads();
-  if (ok && lane < 12) {
-    const int dim = lane >> 2, s = lane & 3;
-    const double h = w.step[0][dim][s];
-    for (int k = 0; k < 5; ++k) y[k] = w.inner[dim][(4 * s + k) & 15];
-    w.outer[lane] = h == h ? h * boole_sum(y) : 0.0;
+  wave_lds_sync();
+  if (ok && l < 12) {
+    const int dim = l >> 2, s = l & 3;
+    const double h = own.step[0][dim][s];
+    for (int k = 0; k < 5; ++k) y[k] = own.inner[dim][(4 * s + k) & 15];
+    own.outer[l] = h == h ? h * boole_sum(y) : 0.0;
   }
-  __syncthreads();
-  if (ok && lane == 0) {
+  wave_lds_sync();
+  if (ok && l == 0) {
     double outer = 0.0;
-    for (int t = 0; t < 12; ++t) outer += w.outer[t];
+    for (int t = 0; t < 12; ++t) outer += own.outer[t];
     ff[i * P + j] = fabs(outer / ((2.0 * M_PI) * areas[i]));
   }
 }
@@ -877,7 +896,8 @@ extern "C" int spr_form_factors(int64_t P, const double *points,
   hipStream_t s = as_stream(stream);
   int rc = fill<double>(ff, P * P, 0.0, s);
   if (rc || V == 0) return rc;
-  hipLaunchKernelGGL(stokes_kernel, dim3((unsigned)ceil_div(V, 4)), dim3(256),
+  hipLaunchKernelGGL(stokes_kernel,
+                     dim3((unsigned)ceil_div(V, 4 * kStokesPairs)), dim3(256),
                      0, s, P, points, areas, V, pairs, ff);
   SPR_LAUNCH_CHECK();
   // As few pairs to a wavefront as 16,384 of them allow: in a small scene many

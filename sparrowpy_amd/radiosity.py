@@ -334,10 +334,8 @@ class DirectionalRadiosityFast:
             raise ValueError(
                 "form_factors need to be of shape (n_patches, n_patches)")
         if self._brdf_outgoing_directions is not None:
-            brdf, bidx, sources, receivers = self._brdf_tables()
-            D = receivers.shape[1]
+            D = self._wall_directions()[1].shape[1]
         else:
-            brdf = bidx = sources = receivers = None
             D = 1
         n_bins = 1 if self._frequencies is None else self.n_bins
         if pairs is not None:
@@ -364,6 +362,8 @@ class DirectionalRadiosityFast:
             raise ValueError(
                 "form_factors_tilde need to be of shape "
                 "(n_patches, n_patches, n_outgoing_directions, n_bins)")
+        brdf, bidx, sources, receivers = (None,) * 4 if \
+            self._brdf_outgoing_directions is None else self._brdf_tables()
         self._bake = dict(
             vis=ops.as_dev(vis, torch.uint8),
             pairs=ops.as_dev(np.asarray(pairs, dtype=np.int32).reshape(-1, 2)
@@ -541,15 +541,11 @@ class DirectionalRadiosityFast:
             assert (self._frequencies == frequencies).all(), \
                 "Frequencies do not match"
 
-    def _brdf_tables(self):
-        """Stacked BRDF tables, BRDF indices and per-wall direction arrays
-        (device tensors, uploaded once until :meth:`set_wall_brdf` changes
-        them: they are megabytes where every patch has its own BRDF).
+    def _wall_directions(self):
+        """Per-wall incoming and outgoing direction arrays (host).
 
         Every wall needs a BRDF here (the kernels index the tables by
         wall); the reference fails there too, on its unset walls."""
-        if self._tables is not None:
-            return self._tables
         if (any(s is None for s in self._brdf_incoming_directions)
                 or any(s is None for s in self._brdf_outgoing_directions)
                 or (np.asarray(self._brdf_index) < 0).any()):
@@ -559,14 +555,22 @@ class DirectionalRadiosityFast:
                 self._brdf_incoming_directions}) != 1:
             raise ValueError("brdf_incoming_directions need the same number "
                              "of directions on every wall")
-        sources = np.array([s.cartesian for s in
-                            self._brdf_incoming_directions])
-        receivers = np.array([s.cartesian for s in
-                              self._brdf_outgoing_directions])
-        self._tables = (ops.as_dev(np.array(self._brdf), torch.float64),
-                        ops.as_dev(np.array(self._brdf_index), torch.int64),
-                        ops.as_dev(sources, torch.float64),
-                        ops.as_dev(receivers, torch.float64))
+        return (np.array([s.cartesian for s in
+                          self._brdf_incoming_directions]),
+                np.array([s.cartesian for s in
+                          self._brdf_outgoing_directions]))
+
+    def _brdf_tables(self):
+        """Stacked BRDF tables, BRDF indices and per-wall direction arrays
+        (device tensors, uploaded once until :meth:`set_wall_brdf` changes
+        them: they are megabytes where every patch has its own BRDF)."""
+        if self._tables is None:
+            sources, receivers = self._wall_directions()
+            self._tables = (ops.as_dev(np.array(self._brdf), torch.float64),
+                            ops.as_dev(np.array(self._brdf_index),
+                                       torch.int64),
+                            ops.as_dev(sources, torch.float64),
+                            ops.as_dev(receivers, torch.float64))
         return self._tables
 
     def _air(self):

@@ -550,7 +550,8 @@ typedef struct spr_exchange_plan {
  * reach; such a patch injects nothing.  Enqueues kernels only: no
  * allocation, no synchronisation, safe to capture. */
 int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T, int64_t K,
-                        int64_t reach, const double *e0dir, const double *d0, double c,
+                        int64_t reach, const double *e0dir, const double *d0,
+                        double c,
                         double dt, float *out, float *lo,
                         float *const *states, float *gsum, int32_t *n0,
                         int *err_flag, void *stream);
@@ -561,7 +562,8 @@ int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T, int64_t K,
  * float64 is that of spr_exchange_orders, but not every last bit agrees
  * with it.  Other arguments as there. */
 int spr_exchange_sum(const spr_exchange_plan *plan, int64_t T, int64_t K,
-                     int64_t reach, const double *e0dir, const double *d0, double c,
+                     int64_t reach, const double *e0dir, const double *d0,
+                     double c,
                      double dt, float *out, float *tmp, float *gsum,
                      int32_t *n0, int *err_flag, void *stream);
 

@@ -63,7 +63,7 @@ inline size_t row_lds(const spr_exchange_plan &p, int R) {
 // Bound by the row reads: an entry's R = 4 loads take 16 clocks of the CU's
 // first-level cache, its 13 vector instructions as many.  Forming each
 // entry's row address and offsets in the wave (23 scalar and 6 vector
-// instructions more) a 426-patch, 4-band order took 139 us instead of 119.
+// instructions more) a 328-patch, 4-band order took 139 us instead of 126.
 // With two weights and 64 directions the second phase is half of it; its
 // values are picked where they are written, 16 totals' loads in flight
 // (1,072 patches, 6 bands: 7.0 ms, with the values held in registers and 8

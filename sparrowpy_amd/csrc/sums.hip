@@ -23,7 +23,8 @@
 // delay further.  Bins beyond are exact zeros of the reference's loop too;
 // they are cleared once, at the end.  In a room the sound crosses in 60 bins
 // an order of 2,000 bins is a third of the work on average over 20 orders
-// (328 patches, 16 directions, 4 bands: 8.48 -> 5.27 ms).
+// (328 patches, 16 directions, 4 bands: 8.48 -> 5.27 ms when orders took two
+// launches; 2.7 with one).
 #include <algorithm>
 
 #include "spr_common.hpp"

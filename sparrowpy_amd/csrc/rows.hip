@@ -76,8 +76,6 @@ __global__ __launch_bounds__(64 * kRowWaves)
   extern __shared__ char smem[];
   float *gs = reinterpret_cast<float *>(smem);  // [max_groups][TB]
   double *part = reinterpret_cast<double *>(gs + (size_t)a.max_groups * TB);
-  const bool one = !DS && a.max_groups == 1;  // the waves share the group
-  double *ct = part + (one ? NW * TB : 0);    // [max_groups][DP], !DS
   const int B = a.B, D = a.D;
   const int64_t T = a.T;
   int64_t j;
@@ -91,6 +89,11 @@ __global__ __launch_bounds__(64 * kRowWaves)
   const int64_t e_begin = a.row_ptr[j], e_end = a.row_ptr[j + 1];
   const int64_t g0 = a.grp_ptr[j];
   const int ng = (int)(a.grp_ptr[j + 1] - g0);
+  // the waves share the only group: of the plan, or the diffuse one of a
+  // destination whose entries all lack a specular direction (it starts at the
+  // row's end, so no wave would find entries by group starts)
+  const bool one = DS ? ng == 1 : a.max_groups == 1;  // uniform
+  double *ct = part + (one ? NW * TB : 0);            // [max_groups][DP], !DS
   const double *w = a.scal + (int64_t)b * a.Vd;
   const double *w2 = DS ? a.dscal + (int64_t)b * a.Vd : w;
 

@@ -2230,13 +2230,14 @@ extern "C" int spr_exchange_step_grouped(
 }
 
 namespace {
-// Workspace of spr_energy_exchange.  Besides the per-pair plan and the
-// state buffers (prev, beside the caller's etc, for the running sum; lo
-// holds the source bins) it holds the grouped plan built from the dense F~
-// (hashes alias coef, which is filled after the sort) with group sums for
-// at most gcap = min(ceil(Vd / 4), 2 P D) groups: beyond a quarter of the
-// entries the per-pair plan is used, and the group sums never take more
-// than two state buffers.
+// Workspace of spr_energy_exchange.  Besides the per-pair plan and the three
+// state buffers (two orders in turn and the total's low part; its high part is
+// the caller's etc) it holds the grouped plan built from the dense F~ (hashes
+// alias coef, which is filled after the sort) with group sums for at most
+// gcap = min(ceil(Vd / 4), 2 P D) groups: beyond a quarter of the entries the
+// per-pair plan is used, and the group sums never take more than two state
+// buffers.  The source bins (P int32) alias vis (P * P bytes, 256 at least),
+// which only the row lists are built from.
 struct DenseLayout {
   size_t vis, row_ptr, src, lag, dir, coef, prev, cur, lo, err, start, rowid,
       grp_ptr, grp_key, scal, gsum, bad, total;
@@ -2277,7 +2278,8 @@ DenseLayout dense_layout(int64_t P, int64_t D, int64_t B, int64_t T,
 }
 
 // most[0] = the largest delay of the plan's entries, most[1] = the largest
-// source delay (0 for one outside int32, which the exchange reports),
+// source delay (0 for one of 0x3fffffff bins or more, which is beyond any
+// histogram: the exchange reports it),
 // most[2] = the most groups of a destination (grp_ptr not null); one
 // workgroup, its loads 8 entries per thread at a time.
 __global__ __launch_bounds__(1024) void plan_max_kernel(
@@ -2394,8 +2396,8 @@ int dense_grouped_plan(int64_t T, int64_t P, int64_t D, int64_t B,
 }
 
 // The body of spr_energy_exchange on a workspace `ws` of the dense layout
-// (sizes already checked by the caller): the grouped two-pass exchange
-// when the F~ rows factorise, else the per-pair plan.
+// (sizes already checked by the caller): the orders on the grouped plan
+// when the F~ rows factorise, else on the per-pair plan.
 int energy_exchange_on(const char *name, int64_t T, int64_t P, int64_t D,
                        int64_t B, const double *e0dir, const double *d0,
                        const double *dist, const double *fft,
@@ -2409,8 +2411,10 @@ int energy_exchange_on(const char *name, int64_t T, int64_t P, int64_t D,
   auto *lag = reinterpret_cast<int32_t *>(ws + L.lag);
   auto *dir = reinterpret_cast<int32_t *>(ws + L.dir);
   auto *coef = reinterpret_cast<double *>(ws + L.coef);
-  auto *prev = reinterpret_cast<float *>(ws + L.prev);
-  auto *n0 = reinterpret_cast<int32_t *>(ws + L.lo);
+  float *states[2] = {reinterpret_cast<float *>(ws + L.prev),
+                      reinterpret_cast<float *>(ws + L.cur)};
+  auto *lo = reinterpret_cast<float *>(ws + L.lo);
+  auto *n0 = reinterpret_cast<int32_t *>(ws + L.vis);
   auto *err = reinterpret_cast<int *>(ws + L.err);
   last_dense_groups = 0;
   int rc;
@@ -2466,9 +2470,10 @@ int energy_exchange_on(const char *name, int64_t T, int64_t P, int64_t D,
     p.max_groups = most[2];
     reach = std::min<int64_t>(T, (int64_t)most[1] + 1);
   }
-  if ((rc = spr_exchange_sum(&p, T, K, reach, e0dir, d0, c, dt, etc, prev,
-                             reinterpret_cast<float *>(ws + L.gsum), n0, err,
-                             stream)))
+  if ((rc = exchange_orders(name, p, T, K, reach, e0dir, d0, c, dt, etc, lo,
+                            states, 2,
+                            reinterpret_cast<float *>(ws + L.gsum), n0, err,
+                            s)))
     return rc;
   int h_err = 0;
   SPR_HIP(hipMemcpyAsync(&h_err, err, sizeof(int), hipMemcpyDeviceToHost, s));

@@ -155,6 +155,13 @@ int step_pairs(int64_t P, int64_t D, int64_t B, int64_t T,
                float *cur, float *tot_hi, float *tot_lo, const OrderStep *step,
                hipStream_t s);
 
+// spr_exchange_orders on n_states order buffers taken in turn (sums.hip).
+int exchange_orders(const char *name, const spr_exchange_plan &p, int64_t T,
+                    int64_t K, int64_t reach, const double *e0dir,
+                    const double *d0, double c, double dt, float *out,
+                    float *lo, float *const *states, int64_t n_states,
+                    float *gsum, int32_t *n0, int *err_flag, hipStream_t s);
+
 // The passes of a backward order (adjoint.hip) on the bins below Tk that
 // E_k can hold energy in, and below Tn for E_{k+1}.
 int direction_sum(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tn,

@@ -1026,8 +1026,9 @@ def exchange_orders(plan, energy_0_directivity, distance_0, speed_of_sound,
 def exchange_sum(plan, energy_0_directivity, distance_0, speed_of_sound,
                  time_resolution, n_samples, max_order, reach=None):
     """As :func:`exchange_orders` by the recurrence x_{k+1} = x_0 + A x_k:
-    half the memory or less and no pass over the total, the same error
-    against float64, last bits of its own."""
+    half the memory or less and no pass over the total, but the sum is one
+    float32 rounded every order, so its error against float64 grows with the
+    orders (figures at ``spr_exchange_sum``)."""
     return _exchange(plan, energy_0_directivity, distance_0, speed_of_sound,
                      time_resolution, n_samples, max_order, reach)[0]
 

@@ -9,6 +9,8 @@
 // patch the direction index, factor, delay and air factor are uniform across
 // a wave and the histogram row etc[k, idx, b, :] is read contiguously
 // (circularly shifted by the delay).
+#include <algorithm>
+
 #include "spr_common.hpp"
 #include "spr_exchange.hpp"
 #include "spr_geom.hpp"
@@ -49,15 +51,16 @@ constexpr int kCollectR = 4;  // bins per lane
 constexpr int kCollectBins = 64 * kCollectR;
 
 __global__ __launch_bounds__(64 * kCollectWaves) void collect_mono_kernel(
-    int64_t P, int64_t D, int64_t B, int64_t T, int n_tblk,
+    int64_t P, int64_t D, int64_t B, int64_t T, int n_tblk, uint32_t first,
     const float *__restrict__ etc, const double *__restrict__ points,
     const double *__restrict__ centers, const int64_t *__restrict__ idx,
     const double *__restrict__ factor, const double *__restrict__ air,
     double c, double dt, float *__restrict__ out) {
   constexpr int R = kCollectR, C = 4;
   __shared__ double part[kCollectWaves][kCollectBins];
-  const int tb = blockIdx.x % n_tblk;
-  const int64_t rb = blockIdx.x / n_tblk;
+  const uint32_t blk = first + blockIdx.x;
+  const int tb = (int)(blk % (uint32_t)n_tblk);
+  const int64_t rb = blk / (uint32_t)n_tblk;
   const int64_t b = rb % B, r = rb / B;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lane = (int)threadIdx.x & 63;
@@ -206,10 +209,13 @@ extern "C" int spr_collect(int64_t NR, int64_t P, int64_t D, int64_t B,
     const int64_t n_tblk = ceil_div(T, (int64_t)kCollectBins);
     const int64_t nb = NR * B * n_tblk;
     SPR_REQUIRE(nb < 0x7fffffff, "spr_collect: grid too large");
-    hipLaunchKernelGGL(collect_mono_kernel, dim3((unsigned)nb),
-                       dim3(64 * kCollectWaves), 0, s, P, D, B, T,
-                       (int)n_tblk, etc, points, centers, idx, factor, air, c,
-                       dt, out);
+    // 16 waves for 256 bins: 4.2 M blocks reach a launch's limit
+    const int64_t most = max_blocks(64 * kCollectWaves);
+    for (int64_t first = 0; first < nb; first += most)
+      hipLaunchKernelGGL(
+          collect_mono_kernel, dim3((unsigned)std::min(most, nb - first)),
+          dim3(64 * kCollectWaves), 0, s, P, D, B, T, (int)n_tblk,
+          (uint32_t)first, etc, points, centers, idx, factor, air, c, dt, out);
   } else {
     const int64_t n_tblk = ceil_div(T, 256);
     const int64_t nb = NR * P * B * n_tblk;

@@ -44,6 +44,9 @@ inline hipStream_t as_stream(void *s) { return static_cast<hipStream_t>(s); }
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// Blocks of `threads` that one launch takes in x: fewer than 2^32 work items.
+inline int64_t max_blocks(int64_t threads) { return 0xffffffffll / threads; }
+
 // Blocks are dispatched round-robin over the 8 XCDs of an MI355X (block id
 // modulo 8 picks the XCD).  xcd_tile maps block ids so that each XCD works
 // through one contiguous range of logical tiles: neighbouring tiles (same

@@ -376,7 +376,8 @@ int launch_row_order(const spr_exchange_plan &p, RowArgs a, hipStream_t s) {
   const size_t lds = row_lds(p, R);
   a.n_tblk = (int)ceil_div(a.sp.Tc, 64 * R);
   a.nblocks = p.P * p.B * a.n_tblk;
-  SPR_REQUIRE(a.nblocks < (int64_t)0x7fffffff, "exchange grid too large");
+  SPR_REQUIRE(a.nblocks <= max_blocks(64 * kRowWaves),
+              "exchange grid too large");
   if (lds > 65536)
     SPR_HIP(hipFuncSetAttribute((const void *)row_order_kernel<DP, R, DS>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -436,7 +437,8 @@ int row_shape(const spr_exchange_plan &p, int64_t T, const OrderSpan &sp) {
   constexpr size_t kLds = 160 * 1024;
   if (!p.order_shape && row_lds(p, R) > kLds / 2) R = 2;
   const int64_t n = p.P * p.B, nb = n * ceil_div(sp.Tc, 64 * R);
-  if (row_lds(p, R) > kLds || nb >= (int64_t)0x7fffffff) return 0;
+  // (the two passes have half the threads or fewer for as many bins)
+  if (row_lds(p, R) > kLds || nb > max_blocks(64 * kRowWaves)) return 0;
   if (p.order_shape) return R;
   const double E = (double)p.Vd / (double)p.P;
   const double groups = (double)(p.max_groups - (ds ? 1 : 0));

@@ -26,3 +26,33 @@ def test_mono_collection_of_many_receivers():
     want = .75 * factor * torch.exp(-.01 * dist)
     assert float((out.double().reshape(n, 1) / want - 1).abs().max()) \
         <= 2 ** -23
+
+
+@pytest.mark.parametrize("shape", [-1, 0, 2, 4])
+def test_orders_of_many_destinations_and_bands(shape):
+    """512 work items a destination and band in the one-launch order, which
+    the two passes take over.  Each destination hears the next patch at once:
+    every bin of the sum is a product chain, two roundings an order."""
+    import torch
+    from sparrowpy_amd import ops
+    P, B, K = 8200, 1024, 2
+    gen = torch.Generator("cuda").manual_seed(1)
+    f64 = dict(dtype=torch.float64, device="cuda")
+    n = torch.arange(P + 1, device="cuda")
+    rowid = ((n[:-1] + 1) % P).to(torch.int32)
+    lag = torch.full((P,), ops.GroupedPlan.LAST_IN_GROUP, dtype=torch.int32,
+                     device="cuda")
+    scal = torch.rand(B, P, generator=gen, **f64) + .5
+    rtab = torch.rand(1, B, 1, generator=gen, **f64) + .5
+    plan = ops.GroupedPlan(P, 1, B, n, n, n, torch.zeros_like(rowid), rowid,
+                           lag, scal, rtab)
+    plan.order_shape = shape
+    e0 = torch.rand(P, 1, B, generator=gen, **f64) + .5
+    out = ops.exchange_orders(plan, e0, torch.zeros(P, **f64), 343., 1., 1,
+                              K)
+    term, want = e0[:, 0], e0[:, 0].clone()
+    for _ in range(K):
+        term = term.roll(-1, 0) * scal.T * rtab[0, :, 0]
+        want += term
+    err = float((out.double().reshape(P, B) / want - 1).abs().max())
+    assert err <= (2 * K + 2) * 2.0 ** -24

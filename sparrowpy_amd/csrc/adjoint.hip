@@ -14,6 +14,7 @@
 // E_0dir[i,:,b] = E0[i,b] (A + C e_m)[k0_i, b] (RadiosityFast.py:988-1034).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "spr_common.hpp"
@@ -188,7 +189,8 @@ template <int R>
 __global__ __launch_bounds__(64 * kAdjointWaves)
     __attribute__((amdgpu_waves_per_eu(4))) void adjoint_ds_kernel(
         int D, int B, int T, int Tk, int Tn, int n_tblk, int64_t nblocks,
-        int64_t Vd, const int64_t *__restrict__ tgptr,
+        uint32_t first, uint32_t count, int64_t Vd,
+        const int64_t *__restrict__ tgptr,
         const int32_t *__restrict__ tkey, const int32_t *__restrict__ tlag,
         const int32_t *__restrict__ tm, const double *__restrict__ twa,
         const double *__restrict__ twc, const float *__restrict__ lam,
@@ -199,8 +201,8 @@ __global__ __launch_bounds__(64 * kAdjointWaves)
   constexpr int32_t kDstMask = (1 << 25) - 1;
   int64_t i;
   int b, tb;
-  dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks, B, n_tblk, i, b,
-                  tb);
+  dest_major_tile(first + xcd_tile(blockIdx.x, count), nblocks, B, n_tblk,
+                  i, b, tb);
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lane = (int)threadIdx.x & 63;
   const int t0 = tb * TB;
@@ -765,10 +767,15 @@ int adjoint_ds(int64_t P, int64_t D, int64_t B, int64_t T, int64_t Tk,
     const int64_t nb = P * B * nt;
     SPR_REQUIRE(nb < (int64_t)0x7fffffff,
                 "spr_exchange_adjoint_ds: grid too large");
-    hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(64 * kAdjointWaves),
-                       0, s, (int)D, (int)B, (int)T, (int)Tk, (int)Tn,
-                       (int)nt, nb, Vd, tgptr, tkey, tlag, tm, twa, twc, lam,
-                       musum, munext, ek, muout, ga);
+    // 8 waves for 128 or 256 bins: 8.4 M blocks reach a launch's limit
+    const int64_t most = max_blocks(64 * kAdjointWaves);
+    for (int64_t first = 0; first < nb; first += most) {
+      const uint32_t count = (uint32_t)std::min(most, nb - first);
+      hipLaunchKernelGGL(kernel, dim3(count), dim3(64 * kAdjointWaves), 0, s,
+                         (int)D, (int)B, (int)T, (int)Tk, (int)Tn, (int)nt, nb,
+                         (uint32_t)first, count, Vd, tgptr, tkey, tlag, tm,
+                         twa, twc, lam, musum, munext, ek, muout, ga);
+    }
     SPR_LAUNCH_CHECK();
     return SPR_OK;
   };

@@ -56,3 +56,33 @@ def test_orders_of_many_destinations_and_bands(shape):
         want += term
     err = float((out.double().reshape(P, B) / want - 1).abs().max())
     assert err <= (2 * K + 2) * 2.0 ** -24
+
+
+def test_adjoint_of_many_sources_and_bands():
+    """512 work items a source and band: one entry each, so mu is lambda plus
+    two products, rounded to float32 and added to it."""
+    import torch
+    from sparrowpy_amd import _hip
+    P, B = 8200, 1024
+    gen = torch.Generator("cuda").manual_seed(2)
+
+    def rand(*shape, dtype=torch.float32):
+        return torch.rand(*shape, dtype=dtype, generator=gen,
+                          device="cuda") + .5
+    lam, mu, ek = (rand(P, B) for _ in range(3))
+    wa, wc = (rand(B, P, dtype=torch.float64) for _ in range(2))
+    n = torch.arange(P + 1, device="cuda")
+    i32 = dict(dtype=torch.int32, device="cuda")
+    tkey = ((n[:-1] + 1) % P).to(torch.int32)
+    tlag = torch.full((P,), 0x40000000, **i32)
+    out = torch.full((P, B), float("nan"), device="cuda")
+    ga = torch.zeros(2, B, P, dtype=torch.float64, device="cuda")
+    _hip.call("spr_exchange_adjoint_ds", P, 1, B, 1, P,
+              *(_hip.ptr(t) for t in (n, tkey, tlag, torch.zeros(P, **i32),
+                                      wa, wc, lam, mu, mu, ek, out, ga)),
+              _hip.stream_ptr())
+    heard = mu.double().roll(-1, 0)
+    want = lam.double() + heard * (wa + wc).T
+    assert float((out.double() / want - 1).abs().max()) <= 2 ** -23
+    want = heard * ek.double()
+    assert float((ga.transpose(1, 2) / want - 1).abs().max()) <= 1e-12

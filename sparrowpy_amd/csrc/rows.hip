@@ -89,11 +89,8 @@ __global__ __launch_bounds__(64 * kRowWaves)
   const int64_t e_begin = a.row_ptr[j], e_end = a.row_ptr[j + 1];
   const int64_t g0 = a.grp_ptr[j];
   const int ng = (int)(a.grp_ptr[j + 1] - g0);
-  // the waves share the only group: of the plan, or the diffuse one of a
-  // destination whose entries all lack a specular direction (it starts at the
-  // row's end, so no wave would find entries by group starts)
-  const bool one = DS ? ng == 1 : a.max_groups == 1;  // uniform
-  double *ct = part + (one ? NW * TB : 0);            // [max_groups][DP], !DS
+  const bool one = !DS && a.max_groups == 1;  // the waves share the group
+  double *ct = part + (one ? NW * TB : 0);    // [max_groups][DP], !DS
   const double *w = a.scal + (int64_t)b * a.Vd;
   const double *w2 = DS ? a.dscal + (int64_t)b * a.Vd : w;
 
@@ -112,10 +109,13 @@ __global__ __launch_bounds__(64 * kRowWaves)
     c_hi += __popcll(__ballot(in && st < cut_hi));
   }
   if (wave == NW - 1) c_hi = ng;
-  const int64_t e_lo = one          ? cut_lo
+  // (the diffuse group starts at the row's end: where a destination's entries
+  // all lack a specular direction it is the only one, and shared as well)
+  const bool share = one || (DS && ng == 1);
+  const int64_t e_lo = share       ? cut_lo
                        : c_lo < ng ? start_of(c_lo)
                                    : e_end;
-  const int64_t e_hi = one                         ? cut_hi
+  const int64_t e_hi = share                        ? cut_hi
                        : c_hi < ng && wave < NW - 1 ? start_of(c_hi)
                                                     : e_end;
 

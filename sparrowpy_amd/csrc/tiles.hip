@@ -18,6 +18,8 @@
 // order of the entries of each group in the grouped plan, so every slot sums
 // its group in exactly the grouped plan's order: the per-group sums are
 // bit-identical to spr_exchange_gather_grouped's.
+#include <algorithm>
+
 #include "spr_common.hpp"
 #include "spr_exchange.hpp"
 #include "spr_util.hpp"
@@ -448,7 +450,8 @@ template <int R, int JT, int SMAX, bool DS>
 __global__ __launch_bounds__(64 * JT) __attribute__((
     amdgpu_waves_per_eu(lds_gather_waves_per_eu<R>()))) void
 tile_lds_gather_kernel(
-    int64_t P, int B, int T, int Tp, int n_tblk, int64_t nblocks, int64_t M,
+    int64_t P, int B, int T, int Tp, int n_tblk, int64_t nblocks,
+    uint32_t first, uint32_t count, int64_t M,
     const int64_t *__restrict__ tptr, const int64_t *__restrict__ grp_ptr,
     const int64_t *__restrict__ gdiff, const int4 *__restrict__ mspan,
     const int32_t *__restrict__ mlag, const double *__restrict__ mw,
@@ -474,8 +477,8 @@ tile_lds_gather_kernel(
   auto win = [&](int buf) -> float(*)[W] { return buf ? lds_b : lds_a; };
   int64_t tile;
   int b, tb;
-  dest_major_tile(xcd_tile(blockIdx.x, nblocks), nblocks, B, n_tblk, tile, b,
-                  tb);
+  dest_major_tile(first + xcd_tile(blockIdx.x, count), nblocks, B, n_tblk,
+                  tile, b, tb);
   const int64_t m_begin = tptr[tile];
   // entries of the tile (< 2^31): batch positions are 32-bit offsets from
   // m_begin, so every loop bound is a scalar 32-bit compare
@@ -763,11 +766,16 @@ int launch_tile_lds(int64_t P, int64_t B, int64_t T, int64_t M,
   const int64_t nb = n_tiles * B * nt;
   SPR_REQUIRE(nb < (int64_t)0x7fffffff, "exchange grid too large");
   SPR_REQUIRE(T < ((int64_t)1 << 29), "histogram too long (T >= 2^29)");
-  hipLaunchKernelGGL((tile_lds_gather_kernel<R, JT, SMAX, DS>),
-                     dim3((unsigned)nb), dim3(64 * JT), 0, s, P, (int)B,
-                     (int)T, sp.Tp, (int)nt, nb, M, tptr, grp_ptr, gdiff,
-                     reinterpret_cast<const int4 *>(mspan), mlag, mw, mdw,
-                     prev, gsum);
+  // 16 waves for 256 to 1,024 bins: 4.2 M blocks reach a launch's limit
+  const int64_t most = max_blocks(64 * JT);
+  for (int64_t first = 0; first < nb; first += most) {
+    const uint32_t count = (uint32_t)std::min(most, nb - first);
+    hipLaunchKernelGGL((tile_lds_gather_kernel<R, JT, SMAX, DS>), dim3(count),
+                       dim3(64 * JT), 0, s, P, (int)B, (int)T, sp.Tp, (int)nt,
+                       nb, (uint32_t)first, count, M, tptr, grp_ptr, gdiff,
+                       reinterpret_cast<const int4 *>(mspan), mlag, mw, mdw,
+                       prev, gsum);
+  }
   SPR_LAUNCH_CHECK();
   return SPR_OK;
 }

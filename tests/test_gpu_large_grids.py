@@ -86,3 +86,33 @@ def test_adjoint_of_many_sources_and_bands():
     assert float((out.double() / want - 1).abs().max()) <= 2 ** -23
     want = heard * ek.double()
     assert float((ga.transpose(1, 2) / want - 1).abs().max()) <= 1e-12
+
+
+def test_gather_on_many_diffuse_specular_tiles():
+    """1,024 work items a tile, band and 256 bins: a scene's tiles behind half
+    a million empty ones give the sums they give by themselves."""
+    import dataclasses
+
+    import torch
+    from sparrowpy_amd import ops, testing
+    from test_gpu_parity import _ds_plan, _oracle_directional
+    r = _oracle_directional(testing.shoebox_room_stub(2.5, 2., 1.5), .5,
+                            n_bands=4, seed=3)
+    plan = _ds_plan(ops, r, 343., 1 / 2000)
+    tiles = ops.tile_plan(plan, 16, min_merge=0)
+    empty, T = 1 << 19, 300
+    before = torch.zeros(empty, dtype=torch.int64, device="cuda")
+    many = dataclasses.replace(
+        tiles, P=tiles.P + 16 * empty, tptr=torch.cat([before, tiles.tptr]),
+        **{k: torch.cat([before.repeat(16), getattr(tiles, k)])
+           for k in ("gstart", "gdiff")})
+    shape = (plan.P, plan.D, plan.B, T)
+    gen = torch.Generator("cuda").manual_seed(4)
+    prev = torch.rand(shape, device="cuda", generator=gen)
+    sums = []
+    for plan.tiles in (tiles, many):
+        out = torch.zeros(plan.n_groups, plan.B, T, device="cuda")
+        ops.gather_groups(plan, shape, prev, out)
+        sums.append(out)
+    assert float(sums[0].max()) > 0
+    assert torch.equal(*sums)

@@ -410,16 +410,20 @@ class BRDFExchangeAdjoint:
         DP = p.rtab.shape[2]
         gg = torch.zeros((max(G, 1), B, DP), dtype=torch.float64, device=dev)
         nu = torch.empty((max(G, 1), B, T), dtype=torch.float32, device=dev)
-        # the orders' group sums come out of recomputing a segment; kept
-        # (when there is room) instead of formed again for the backward
-        # orders
-        n = min(self.every, max(self.K, 1))
-        sums = [torch.empty_like(nu)
-                for _ in range(n if _fits(nu, n - 1) else 1)]
         plan = ops._plan_struct(p) if p.Vd else None
+        sums = []
 
         def segment(s, states, lam, mu, mu_even, mu_odd):
             m = len(states)
+            if not sums:
+                # the orders' group sums come out of recomputing a segment;
+                # kept (when there is room beside every other buffer, all in
+                # place by now) instead of formed again for the backward
+                # orders
+                sums.append(torch.empty_like(nu))
+                more = min(self.every, self.K) - 1
+                if _fits(nu, more):
+                    sums.extend(torch.empty_like(nu) for _ in range(more))
             call("spr_adjoint_segment_grouped", ctypes.addressof(plan), T, s,
                  m, self.reach, _hip.ptr_array(states),
                  _hip.ptr_array((sums * m)[:m]), ptr(self.trow_ptr),

@@ -503,7 +503,8 @@ int spr_energy_exchange(int64_t T, int64_t P, int64_t D, int64_t B,
  * src, lag, dir, coef (spr_plan_from_geometry / _from_dense).
  * SPR_PLAN_GROUPED: row_ptr, grp_ptr, grp_start (NULL if grp_key holds each
  * group's first entry), grp_key, rowid, lag, scal, rtab
- * (spr_plan_grouped_fill).  SPR_PLAN_DS: the same with dscal, rtab not read (spr_plan_ds_fill).  With
+ * (spr_plan_grouped_fill).  SPR_PLAN_DS: the same with grp_start and dscal,
+ * rtab not read (spr_plan_ds_fill).  Both need max_groups > 0.  With
  * M > 0 the last two gather on destination tiles of tile_rows rows
  * (spr_plan_tile_order / _fill / _span): tptr, gstart [tile_slots], mlag,
  * mw, and mspan for 16 rows (tile_r 8 or 16 bins per lane) or mrow for 4

@@ -107,8 +107,12 @@ int check_plan(const char *name, const spr_exchange_plan &p) {
               "%s: unknown plan kind %lld", name, (long long)p.kind);
   SPR_REQUIRE(p.grp_ptr && p.grp_key && p.rowid && p.scal,
               "%s: null plan array", name);
-  SPR_REQUIRE(p.kind == SPR_PLAN_DS ? p.dscal != nullptr : p.rtab != nullptr,
+  // (without grp_start a grouped plan's keys are its groups' first entries;
+  // a diffuse + specular plan's keys are directions)
+  SPR_REQUIRE(p.kind == SPR_PLAN_DS ? p.dscal && p.grp_start
+                                    : p.rtab != nullptr,
               "%s: null plan array", name);
+  SPR_REQUIRE(p.max_groups > 0, "%s: max_groups must be positive", name);
   if (!p.M) return SPR_OK;
   SPR_REQUIRE(p.tile_slots > 0 && p.tptr && p.gstart && p.mlag && p.mw,
               "%s: null tile array", name);

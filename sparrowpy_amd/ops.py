@@ -967,6 +967,14 @@ def _exchange(plan, e0d, d0, speed_of_sound, time_resolution, n_samples,
     P, D, B = e0d.shape
     T, K = int(n_samples), max(int(max_order), 0)
     dev = e0d.device
+    if d0.numel() < P:
+        raise ValueError("distance_0 needs a value for every patch")
+    if K and plan is None:
+        raise ValueError("reflection orders need a plan")
+    if plan is not None and (plan.P, plan.D, plan.B) != (P, D, B):
+        raise ValueError(
+            f"the plan has {plan.P} patches, {plan.D} directions and {plan.B} "
+            f"bands, the source energy {P}, {D} and {B}")
     if plan is None or not plan.Vd:
         K = 0
     st = _plan_struct(plan) if K else _hip.ExchangePlanStruct(P=P, D=D, B=B)

@@ -508,6 +508,9 @@ class DirectionalRadiosityFast:
             raise AssertionError(
                 "Receivers must be in the positive half space")
         self._check_set_frequency(brdf.frequencies)
+        # first: a wall that does not exist raises below, after others have
+        # changed
+        self._tables = None
         if self._brdf_incoming_directions is None:
             self._brdf_incoming_directions = np.empty(self.n_walls, object)
             self._brdf_outgoing_directions = np.empty(self.n_walls, object)
@@ -522,7 +525,6 @@ class DirectionalRadiosityFast:
                                             self._walls_up_vector[i], out))
         self._brdf.append(np.real(np.asarray(brdf.freq)) * np.pi)
         self._brdf_index[np.atleast_1d(wall_indexes)] = len(self._brdf) - 1
-        self._tables = None
 
     def set_air_attenuation(self, air_attenuation):
         """Air attenuation in Np/m (reference ``RadiosityFast.py:754-764``)."""

@@ -548,8 +548,10 @@ typedef struct spr_exchange_plan {
  * needed for K >= 1; n0 [P] (int32) receives each patch's source bin.  Bit 0 of
  * *err_flag is set where a source delay lies outside the histogram (the
  * reference raises IndexError), bit 1 where it lies inside but not below
- * reach; such a patch injects nothing.  Enqueues kernels only: no
- * allocation, no synchronisation, safe to capture. */
+ * reach; such a patch injects nothing.  Bit 2 is set where reach < T and a
+ * factor of the plan is infinite or NaN: times the zeros of the bins left out
+ * it would give NaN, so the call is to be repeated with reach = T.  Enqueues
+ * kernels only: no allocation, no synchronisation, safe to capture. */
 int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T, int64_t K,
                         int64_t reach, const double *e0dir, const double *d0,
                         double c,
@@ -570,11 +572,17 @@ int spr_exchange_sum(const spr_exchange_plan *plan, int64_t T, int64_t K,
                      double dt, float *out, float *tmp, float *gsum,
                      int32_t *n0, int *err_flag, void *stream);
 
+/* *flag (device or pinned host memory) = 0 if one of x[n] is infinite or NaN,
+ * else left as it is.  For the backward orders below: a gradient that is not
+ * finite needs whole orders.  No counterpart in the reference. */
+int spr_all_finite(int64_t n, const float *x, int32_t *flag, void *stream);
+
 /* Backward orders k0 + n - 1 .. k0 of the diffuse + specular adjoint:
  * orders k0 + 1 .. k0 + n - 1 are recomputed from states[0] = order k0 into
  * states[1 ..], then per order spr_direction_sum and spr_exchange_adjoint_ds,
  * each on the bins that energy can have reached (reach as in
- * spr_exchange_orders; only those bins of the mu's are formed and read).
+ * spr_exchange_orders; only those bins of the mu's are formed and read: T
+ * where a factor of the plan, a gradient or a table is infinite or NaN).
  * mu_next = dL/dE_{k0+n}; mu of order k goes to mu_even or mu_odd by k's
  * parity; gsum as there, musum [P,B,T] a workspace. */
 int spr_adjoint_segment_ds(const spr_exchange_plan *plan, int64_t T,

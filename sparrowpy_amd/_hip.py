@@ -161,6 +161,7 @@ SYMBOLS = {
                                            _vp, _vp, _vp, _vp, _vp]),
     "spr_exchange_sum": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _dbl, _dbl, _vp,
                                 _vp, _vp, _vp, _vp, _vp]),
+    "spr_all_finite": (_int, [_i64, _vp, _vp, _vp]),
     "spr_plan_dense_hash": (_int, [_i64, _i64, _i64, _vp, _vp, _vp, _vp,
                                    _vp]),
     "spr_energy_exchange_groups": (_i64, []),

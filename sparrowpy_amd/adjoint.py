@@ -67,6 +67,7 @@ def _source_and_receivers(adj, r, source, receivers):
     adj.air = ops.as_dev(b["air"] if b["air"] is not None
                          else np.zeros(adj.B), torch.float64)
     adj.R = adj.rpts.shape[0]
+    adj.finite = _Finite()
     # a bin beyond every source delay (the farthest corner of the patches'
     # bounding box, and one bin for the delays' rounding)
     far = np.abs(r._patches_points - pos).max(axis=(0, 1))
@@ -76,21 +77,57 @@ def _source_and_receivers(adj, r, source, receivers):
 
 def _forward(adj):
     """Receiver histograms [R, B, T] at the injection adj.e0dir on adj.plan,
-    and the orders kept every adj.every orders."""
-    total, checkpoints = ops._exchange(
+    the orders kept every adj.every orders, and the reach of their bins."""
+    total, checkpoints, reach = ops._exchange(
         adj.plan, adj.e0dir, adj.d0, adj.c, adj.dt, adj.T, adj.K, adj.reach,
         lambda k: k % adj.every == 0)
     # (without an order to run nothing reads it, but a record has order 0)
     checkpoints.setdefault(0, total)
     return ops.collect(total, adj.rpts, adj._geom["centers"], adj.ridx,
-                       adj.rfactor, adj.air, adj.c, adj.dt), checkpoints
+                       adj.rfactor, adj.air, adj.c, adj.dt), checkpoints, reach
 
 
-def _backward(adj, grad_hist, checkpoints, segment):
-    """mu_0 = dL/dE_0 (its bins below adj.reach) for dL/dH = ``grad_hist``:
-    ``segment(s, states, lam, mu, mu_even, mu_odd)`` runs the backward orders
-    of one checkpoint segment, states[0] being the checkpoint, the others
-    scratch."""
+class _Finite:
+    """Whether a device array is finite, asked of the device and answered on
+    the host without waiting for what was enqueued in between."""
+
+    def __init__(self):
+        self._flag = torch.empty(1, dtype=torch.int32, pin_memory=True)
+        self._host = self._flag.numpy()
+        self._done = torch.cuda.Event()
+        self._asked = False
+
+    def ask(self, x):
+        # (while a graph is captured nothing can be known)
+        self._asked = not torch.cuda.is_current_stream_capturing()
+        if self._asked:
+            self._host[0] = 1
+            call("spr_all_finite", x.numel(), ptr(x), self._flag.data_ptr(),
+                 stream_ptr())
+            self._done.record()
+
+    def answer(self):
+        if not self._asked:
+            return False
+        self._done.synchronize()
+        return bool(self._host[0])
+
+
+def _gradient(adj, grad_hist, record):
+    """dL/dH on the device; asks whether it is finite where the backward
+    orders are to be limited to reached bins."""
+    gH = ops.as_dev(grad_hist, torch.float32).contiguous()
+    if record.reach < adj.T:
+        adj.finite.ask(gH)
+    return gH
+
+
+def _backward(adj, gH, record, segment):
+    """mu_0 = dL/dE_0 (its reached bins) for dL/dH = ``gH``:
+    ``segment(s, states, reach, lam, mu, mu_even, mu_odd)`` runs the backward
+    orders of one checkpoint segment, states[0] being the checkpoint, the
+    others scratch."""
+    checkpoints = record.checkpoints
     starts = sorted(checkpoints)
     if not adj.plan.Vd:
         starts = []                          # no pair: mu_0 = lambda
@@ -101,7 +138,6 @@ def _backward(adj, grad_hist, checkpoints, segment):
 
     def state():
         return torch.empty((P, D, B, T), dtype=torch.float32, device=adj.dev)
-    gH = ops.as_dev(grad_hist, torch.float32).contiguous()
     lam = state()
     call("spr_collect_adjoint", adj.R, P, D, B, T, ptr(gH), ptr(adj.rpts),
          ptr(adj._geom["centers"]), ptr(adj.ridx), ptr(adj.rfactor),
@@ -111,9 +147,16 @@ def _backward(adj, grad_hist, checkpoints, segment):
         return mu
     mus = (state(), state())                 # even orders, odd orders
     scratch = [state() for _ in range(min(adj.every, adj.K) - 1)]
+    reach = record.reach
+    if reach < T and not adj.finite.answer():
+        # an infinite or NaN gradient times the zeros of an unreached bin is
+        # NaN: whole orders
+        for k, x in checkpoints.items():     # (set on their reached bins)
+            x[..., min(T, reach + k * adj.plan.limits[0]):] = 0
+        reach = T
     for s in reversed(starts):
         n = min(s + adj.every, adj.K) - s
-        segment(s, [checkpoints[s]] + scratch[:n - 1], lam, mu, *mus)
+        segment(s, [checkpoints[s]] + scratch[:n - 1], reach, lam, mu, *mus)
         mu = mus[s % 2]
     return mu
 
@@ -209,8 +252,8 @@ class ExchangeAdjoint:
         A = ops.as_dev(A, torch.float64).detach().clone()
         C = ops.as_dev(C, torch.float64).detach().clone()
         self._set_tables(A, C)
-        H, checkpoints = _forward(self)
-        self.last = ForwardRecord(A, C, checkpoints)
+        H, checkpoints, reach = _forward(self)
+        self.last = ForwardRecord(A, C, checkpoints, reach)
         return H
 
     # -- backward ---------------------------------------------------------------
@@ -225,6 +268,7 @@ class ExchangeAdjoint:
             raise RuntimeError("ExchangeAdjoint.backward: no forward record "
                                "(forward() was not called, or its record "
                                "was released)")
+        gH = _gradient(self, grad_hist, record)
         self._set_tables(record.A, record.C)
         P, D, B, T, Vd = self.P, self.D, self.B, self.T, self.plan.Vd
         dev, p, adj = self.dev, self.plan, self.plan.adjoint
@@ -238,14 +282,14 @@ class ExchangeAdjoint:
                            device=dev)
         plan = ops._plan_struct(p) if Vd else None
 
-        def segment(s, states, lam, mu, mu_even, mu_odd):
+        def segment(s, states, reach, lam, mu, mu_even, mu_odd):
             call("spr_adjoint_segment_ds", ctypes.addressof(plan), T, s,
-                 len(states), self.reach, _hip.ptr_array(states), ptr(gsum),
+                 len(states), reach, _hip.ptr_array(states), ptr(gsum),
                  ptr(self.tgptr), ptr(self.tkey), ptr(self.tlag),
                  ptr(self.tm), ptr(twa), ptr(twc), ptr(lam), ptr(mu),
                  ptr(mu_even), ptr(mu_odd), ptr(musum), ptr(ga),
                  stream_ptr())
-        mu = _backward(self, grad_hist, record.checkpoints, segment)
+        mu = _backward(self, gH, record, segment)
         gA = torch.zeros((self.NK, B), dtype=torch.float64, device=dev)
         gC = torch.zeros_like(gA)
         call("spr_ds_injection_grad", P, D, B, T, ptr(self.energy0),
@@ -261,11 +305,13 @@ class ExchangeAdjoint:
 
 
 class ForwardRecord:
-    """What the adjoint of one forward call needs: its tables (A, C) and
-    the order histograms kept every ``checkpoint_every`` orders."""
+    """What the adjoint of one forward call needs: its tables (A, C), the
+    order histograms kept every ``checkpoint_every`` orders, and the reach of
+    their bins (order k's are set below reach + k times the longest delay)."""
 
-    def __init__(self, A, C, checkpoints):
+    def __init__(self, A, C, checkpoints, reach):
         self.A, self.C, self.checkpoints = A, C, checkpoints
+        self.reach = reach
 
 
 class _Histograms(torch.autograd.Function):
@@ -390,8 +436,8 @@ class BRDFExchangeAdjoint:
         :meth:`ExchangeAdjoint.forward`)."""
         table = ops.as_dev(table, torch.float64).detach().clone()
         self._set_table(table)
-        H, checkpoints = _forward(self)
-        self.last = TableRecord(table, checkpoints)
+        H, checkpoints, reach = _forward(self)
+        self.last = TableRecord(table, checkpoints, reach)
         return H
 
     def backward(self, grad_hist, record=None):
@@ -403,6 +449,7 @@ class BRDFExchangeAdjoint:
             raise RuntimeError("BRDFExchangeAdjoint.backward: no forward "
                                "record (forward() was not called, or its "
                                "record was released)")
+        gH = _gradient(self, grad_hist, record)
         self._set_table(record.table)
         P, D, B, T = self.P, self.D, self.B, self.T
         p, dev = self.plan, self.dev
@@ -413,7 +460,7 @@ class BRDFExchangeAdjoint:
         plan = ops._plan_struct(p) if p.Vd else None
         sums = []
 
-        def segment(s, states, lam, mu, mu_even, mu_odd):
+        def segment(s, states, reach, lam, mu, mu_even, mu_odd):
             m = len(states)
             if not sums:
                 # the orders' group sums come out of recomputing a segment;
@@ -425,12 +472,12 @@ class BRDFExchangeAdjoint:
                 if _fits(nu, more):
                     sums.extend(torch.empty_like(nu) for _ in range(more))
             call("spr_adjoint_segment_grouped", ctypes.addressof(plan), T, s,
-                 m, self.reach, _hip.ptr_array(states),
+                 m, reach, _hip.ptr_array(states),
                  _hip.ptr_array((sums * m)[:m]), ptr(self.trow_ptr),
                  ptr(self.tgrp), ptr(self.tlag), ptr(self.tscal), ptr(lam),
                  ptr(mu), ptr(mu_even), ptr(mu_odd), ptr(nu), ptr(gg),
                  stream_ptr())
-        mu = _backward(self, grad_hist, record.checkpoints, segment)
+        mu = _backward(self, gH, record, segment)
         gt = torch.zeros((self.NK, D, B), dtype=torch.float64, device=dev)
         call("spr_grouped_key_grad", G, D, B, ptr(p.grp_key), ptr(gg),
              ptr(gt), stream_ptr())
@@ -456,11 +503,13 @@ def _fits(like, n):
 
 
 class TableRecord:
-    """What the adjoint of one BRDFExchangeAdjoint forward needs: its table
-    and the order histograms kept every ``checkpoint_every`` orders."""
+    """What the adjoint of one BRDFExchangeAdjoint forward needs: its table,
+    the order histograms kept every ``checkpoint_every`` orders, and the reach
+    of their bins (as in :class:`ForwardRecord`)."""
 
-    def __init__(self, table, checkpoints):
+    def __init__(self, table, checkpoints, reach):
         self.table, self.checkpoints = table, checkpoints
+        self.reach = reach
 
 
 class _TableHistograms(torch.autograd.Function):

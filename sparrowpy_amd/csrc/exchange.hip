@@ -475,7 +475,9 @@ __global__ __launch_bounds__(256) void exchange_mfma_kernel(
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) a[mt] = o.in ? o.a[mt] : 0.0;
     // 16 bins that none of the step's four entries reaches (before their
-    // delays, or past the source's reached bins) would add zeros: with the
+    // delays, or past the source's reached bins) would add zeros (NaN, for a
+    // factor that is not finite: such a factor marks the bins from its delay
+    // on, as in the reference, and those of its step's 16 before): with the
     // waves past Tc ending at once, 208 patches, 32 directions, 10 orders of
     // 96 to 528 bins take 1.40 ms instead of 1.55, whole orders of 1,072
     // patches (64 directions, 6,000 bins) 94.3 ms instead of 96.7
@@ -2470,14 +2472,22 @@ int energy_exchange_on(const char *name, int64_t T, int64_t P, int64_t D,
     p.max_groups = most[2];
     reach = std::min<int64_t>(T, (int64_t)most[1] + 1);
   }
-  if ((rc = exchange_orders(name, p, T, K, reach, e0dir, d0, c, dt, etc, lo,
-                            states, 2,
-                            reinterpret_cast<float *>(ws + L.gsum), n0, err,
-                            s)))
-    return rc;
-  int h_err = 0;
-  SPR_HIP(hipMemcpyAsync(&h_err, err, sizeof(int), hipMemcpyDeviceToHost, s));
-  SPR_HIP(hipStreamSynchronize(s));
+  int h_err = 4;
+  while (h_err == 4) {
+    if ((rc = exchange_orders(name, p, T, K, reach, e0dir, d0, c, dt, etc, lo,
+                              states, 2,
+                              reinterpret_cast<float *>(ws + L.gsum), n0, err,
+                              s)))
+      return rc;
+    SPR_HIP(hipMemcpyAsync(&h_err, err, sizeof(int), hipMemcpyDeviceToHost,
+                           s));
+    SPR_HIP(hipStreamSynchronize(s));
+    if (h_err == 4) {  // factors that are not finite: whole orders
+      SPR_REQUIRE(reach < T, "%s: bad factors", name);
+      reach = T;
+      if ((rc = fill<int32_t>(err, 1, 0, s))) return rc;
+    }
+  }
   if (h_err)
     return fail(SPR_ERR_RANGE,
                 "%s: a source delay is beyond the histogram length", name);

@@ -27,7 +27,9 @@
 // they are cleared once, at the end.  In a room the sound crosses in 60 bins
 // an order of 2,000 bins is a third of the work on average over 20 orders
 // (328 patches, 16 directions, 4 bands: 8.48 -> 5.27 ms when orders took two
-// launches; 2.7 with one).
+// launches; 2.7 with one).  That holds for finite factors only: an infinite or
+// NaN one times those zeros is NaN, in the reference's loop from the pair's
+// delay on.  Such factors are reported, and the caller runs whole orders.
 #include <algorithm>
 
 #include "spr_common.hpp"
@@ -37,20 +39,73 @@
 namespace spr {
 namespace {
 
+// The factors of a plan: arrays read whole, and of a grouped plan the BRDF
+// rows (width values each, 2^lanes threads to a row) of its groups.
+struct Factors {
+  const double *whole[2] = {};
+  int64_t n[2] = {};
+  const double *rows = nullptr;
+  const int32_t *key = nullptr;
+  const int64_t *groups = nullptr;  // how many
+  int64_t width = 0;
+  int lanes = 0;
+};
+
+Factors factors_of(const spr_exchange_plan &p) {
+  const int64_t DP = spr_padded_directions(p.D);
+  Factors f;
+  if (p.kind == SPR_PLAN_PAIRS) {
+    f.whole[0] = p.coef, f.n[0] = p.Vd * p.B * DP;
+    return f;
+  }
+  f.whole[0] = p.scal, f.n[0] = p.B * p.Vd;
+  if (p.kind == SPR_PLAN_DS) {
+    f.whole[1] = p.dscal, f.n[1] = p.B * p.Vd;
+  } else {
+    f.rows = p.rtab, f.key = p.grp_key, f.groups = p.grp_ptr + p.P;
+    f.width = p.B * DP;
+    while (f.lanes < 6 && 1 << f.lanes < f.width) ++f.lanes;
+  }
+  return f;
+}
+
 // Bins [t0, t1) of every histogram row: E_0 (with e0dir), or 0; with lo, x
 // and lo as a compensated pair and x's rounded value in prev too.  A wave
-// takes kFillBins bins of one row at a time; bound by the writes.
+// takes kFillBins bins of one row at a time; bound by the writes.  The first
+// `looks` blocks look over `factors` instead and report infinities and NaN:
+// once per call, beside the bins cleared at its end, as a launch of its own
+// would wait for loads alone.
 constexpr int kFillBins = 1024;
 
 __global__ __launch_bounds__(256) void row_fill_kernel(
     int64_t P, int64_t DB, int64_t T, int64_t t0, int64_t t1, int64_t chunks,
     const double *__restrict__ e0dir, const double *__restrict__ d0, double c,
     double dt, float *__restrict__ x, float *__restrict__ lo,
-    float *__restrict__ prev, int32_t *__restrict__ n0,
-    int *__restrict__ err) {
+    float *__restrict__ prev, int32_t *__restrict__ n0, Factors factors,
+    uint32_t looks, int *__restrict__ err) {
   const int lane = (int)threadIdx.x & 63;
-  const int64_t waves = (int64_t)gridDim.x * 4;
-  for (int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (blockIdx.x < looks) {  // uniform
+    bool finite = true;
+    const int64_t me = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t threads = 256 * (int64_t)looks;
+    for (int a = 0; a < 2; ++a)
+#pragma unroll 4
+      for (int64_t i = me; i < factors.n[a]; i += threads)
+        finite &= fabs(factors.whole[a][i]) < __builtin_inf();
+    if (factors.rows) {
+      const int64_t n = *factors.groups, w = factors.width;
+      const int lanes = factors.lanes;
+      for (int64_t g = me >> lanes; g < n; g += threads >> lanes) {
+        const double *row = factors.rows + factors.key[g] * w;
+        for (int64_t i = me & ((1 << lanes) - 1); i < w; i += 1 << lanes)
+          finite &= fabs(row[i]) < __builtin_inf();
+      }
+    }
+    if (!finite) atomicOr(err, 4);
+    return;
+  }
+  const int64_t waves = (int64_t)(gridDim.x - looks) * 4;
+  for (int64_t q = (int64_t)(blockIdx.x - looks) * 4 + (threadIdx.x >> 6);
        q < P * DB * chunks; q += waves) {
     const int64_t row = q / chunks, chunk = q % chunks;
     int64_t n = -1;
@@ -85,14 +140,21 @@ __global__ __launch_bounds__(256) void row_fill_kernel(
 int fill_rows(const spr_exchange_plan &p, int64_t T, int64_t t0, int64_t t1,
               const double *e0dir, const double *d0, double c, double dt,
               float *x, float *lo, float *prev, int32_t *n0, int *err,
-              hipStream_t s) {
-  if (t1 <= t0) return SPR_OK;
-  const int64_t chunks = ceil_div(t1 - t0, kFillBins);
+              hipStream_t s, bool look = false) {
+  const Factors factors = look ? factors_of(p) : Factors{};
+  // 2 values or rows to a thread, as far as 2,048 blocks go
+  const int64_t values = std::max(
+      factors.n[0], factors.rows ? p.P * p.max_groups << factors.lanes : 0);
+  const int64_t looks =
+      look ? std::min<int64_t>(ceil_div(values, 512), 2048) : 0;
+  const int64_t chunks = t1 > t0 ? ceil_div(t1 - t0, kFillBins) : 0;
   const int64_t nb = ceil_div(p.P * p.D * p.B * chunks, 4);
+  if (!looks && !nb) return SPR_OK;
   hipLaunchKernelGGL(row_fill_kernel,
-                     dim3((unsigned)std::min<int64_t>(nb, 1 << 20)),
+                     dim3((unsigned)(looks + std::min<int64_t>(nb, 1 << 20))),
                      dim3(256), 0, s, p.P, p.D * p.B, T, t0, t1, chunks,
-                     e0dir, d0, c, dt, x, lo, prev, n0, err);
+                     e0dir, d0, c, dt, x, lo, prev, n0, factors,
+                     (uint32_t)looks, err);
   SPR_LAUNCH_CHECK();
   return SPR_OK;
 }
@@ -224,6 +286,7 @@ extern "C" int spr_exchange_sum(const spr_exchange_plan *plan, int64_t T,
   if ((rc = fill_rows(p, T, 0, Tc, e0dir, d0, c, dt, x, nullptr, nullptr, n0,
                       err_flag, s)))
     return rc;
+  const bool limited = Tc < T;
   OrderStep step{{0, 0, 0, 0, 0}, {e0dir, n0}};
   for (int64_t k = 0; k < K; ++k) {
     step.span.Tp = (int)Tc;
@@ -238,7 +301,7 @@ extern "C" int spr_exchange_sum(const spr_exchange_plan *plan, int64_t T,
     std::swap(x, y);
   }
   return fill_rows(p, T, Tc, T, nullptr, nullptr, c, dt, out, nullptr, nullptr,
-                   nullptr, nullptr, s);
+                   nullptr, err_flag, s, limited);
 }
 
 int spr::exchange_orders(const char *name, const spr_exchange_plan &p,
@@ -258,6 +321,7 @@ int spr::exchange_orders(const char *name, const spr_exchange_plan &p,
   if ((rc = fill_rows(p, T, 0, Tc, e0dir, d0, c, dt, out, K ? lo : nullptr,
                       K ? states[0] : nullptr, n0, err_flag, s)))
     return rc;
+  const bool limited = Tc < T;
   OrderStep step{{0, 0, (int)Tc, 0, 0}, {}};
   OrderSpan &sp = step.span;
   for (int64_t k = 1; k <= K; ++k) {
@@ -284,7 +348,7 @@ int spr::exchange_orders(const char *name, const spr_exchange_plan &p,
     if (add) sp.Tv = sp.Tc;
   }
   return fill_rows(p, T, Tc, T, nullptr, nullptr, c, dt, out, nullptr, nullptr,
-                   nullptr, nullptr, s);
+                   nullptr, err_flag, s, limited);
 }
 
 extern "C" int spr_exchange_orders(const spr_exchange_plan *plan, int64_t T,

@@ -961,7 +961,8 @@ def _exchange(plan, e0d, d0, speed_of_sound, time_resolution, n_samples,
               max_order, reach, keep=None):
     """The sum of the orders: by the recurrence (keep None), or order by
     order, keep(k) naming the orders whose histograms are returned too
-    ({k: float32 [P,D,B,T], its reached bins})."""
+    ({k: float32 [P,D,B,T], its reached bins}); and the reach it ran with, T
+    where a factor is not finite."""
     e0d = _f64(e0d)
     d0 = _f64(d0)
     P, D, B = e0d.shape
@@ -989,12 +990,9 @@ def _exchange(plan, e0d, d0, speed_of_sound, time_resolution, n_samples,
     n0 = torch.empty(P, dtype=torch.int32, device=dev)
     err = torch.zeros(1, dtype=torch.int32, device=dev)
     reach = T if reach is None else min(max(int(reach), 1), T)
-    head = (ctypes.addressof(st), T, K, reach, ptr(e0d), ptr(d0),
-            float(speed_of_sound), float(time_resolution), ptr(out))
-    tail = (ptr(gsum), ptr(n0), ptr(err), stream_ptr())
     kept = {}
     if keep is None:
-        call("spr_exchange_sum", *head, ptr(state()) if K else None, *tail)
+        tmp = state() if K else None
     else:
         lo = state() if K else None
         turn = {}
@@ -1005,15 +1003,25 @@ def _exchange(plan, e0d, d0, speed_of_sound, time_resolution, n_samples,
             elif k % 2 not in turn:
                 turn[k % 2] = state()
             states.append(kept[k] if k in kept else turn[k % 2])
-        call("spr_exchange_orders", *head, ptr(lo), _hip.ptr_array(states),
-             *tail)
-    flags = int(err.item())
-    if flags & 1:
-        raise IndexError(
-            "source-to-patch delay exceeds the histogram length")
-    if flags:
-        raise ValueError("a source delay is not below reach")
-    return out, kept
+    while True:
+        head = (ctypes.addressof(st), T, K, reach, ptr(e0d), ptr(d0),
+                float(speed_of_sound), float(time_resolution), ptr(out))
+        tail = (ptr(gsum), ptr(n0), ptr(err), stream_ptr())
+        if keep is None:
+            call("spr_exchange_sum", *head, ptr(tmp), *tail)
+        else:
+            call("spr_exchange_orders", *head, ptr(lo),
+                 _hip.ptr_array(states), *tail)
+        flags = int(err.item())
+        if flags & 1:
+            raise IndexError(
+                "source-to-patch delay exceeds the histogram length")
+        if flags & 2:
+            raise ValueError("a source delay is not below reach")
+        if not flags:
+            return out, kept, reach
+        reach = T    # factors that are not finite: whole orders
+        err.zero_()
 
 
 def exchange_orders(plan, energy_0_directivity, distance_0, speed_of_sound,

@@ -68,11 +68,10 @@ def _source_and_receivers(adj, r, source, receivers):
                          else np.zeros(adj.B), torch.float64)
     adj.R = adj.rpts.shape[0]
     adj.finite = _Finite()
-    # a bin beyond every source delay (the farthest corner of the patches'
-    # bounding box, and one bin for the delays' rounding)
+    # the farthest corner of the patches' bounding box
     far = np.abs(r._patches_points - pos).max(axis=(0, 1))
-    adj.reach = min(adj.T, int(np.sqrt((far * far).sum()) / adj.c / adj.dt)
-                    + 2)
+    reach = ops.source_reach(np.sqrt((far * far).sum()), adj.c, adj.dt)
+    adj.reach = adj.T if reach is None else min(adj.T, reach)
 
 
 def _forward(adj):

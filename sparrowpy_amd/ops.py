@@ -1024,6 +1024,16 @@ def _exchange(plan, e0d, d0, speed_of_sound, time_resolution, n_samples,
         err.zero_()
 
 
+def source_reach(distance, speed_of_sound, time_resolution):
+    """A bin beyond the delay of every patch up to ``distance`` from the
+    source, with one for the delays' rounding; None where nothing is known
+    (no distance, or arguments that the exchange itself refuses)."""
+    if distance is None or not (speed_of_sound > 0 and time_resolution > 0):
+        return None
+    bins = float(distance) / float(speed_of_sound) / float(time_resolution)
+    return int(bins) + 2 if np.isfinite(bins) else None
+
+
 def exchange_orders(plan, energy_0_directivity, distance_0, speed_of_sound,
                     time_resolution, n_samples, max_order, reach=None):
     """The sum of orders 0..max_order on a plan (the total of

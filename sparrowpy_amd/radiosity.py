@@ -795,14 +795,6 @@ class DirectionalRadiosityFast:
         if plan.tiles is not None:
             plan.tiles.R = self.TILE_R
 
-    def _reach(self, speed_of_sound, time_resolution):
-        """A bin beyond every source delay (None: unknown); one bin more
-        than the farthest patch's, for the delays' rounding."""
-        far = self._source_far
-        if far is None or not np.isfinite(far):
-            return None
-        return int(far / speed_of_sound / time_resolution) + 2
-
     def calculate_energy_exchange(self, speed_of_sound, etc_time_resolution,
                                   etc_duration, max_reflection_order=-1,
                                   recalculate=False):
@@ -844,8 +836,9 @@ class DirectionalRadiosityFast:
             etc = ops.exchange_orders(plan, e0d, d0, speed_of_sound,
                                       etc_time_resolution, n_samples,
                                       max_reflection_order,
-                                      self._reach(speed_of_sound,
-                                                  etc_time_resolution))
+                                      ops.source_reach(self._source_far,
+                                                       speed_of_sound,
+                                                       etc_time_resolution))
             self._etc = etc
         self._etc_time_resolution = float(etc_time_resolution)
         self._speed_of_sound = float(speed_of_sound)

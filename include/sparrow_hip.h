@@ -535,9 +535,14 @@ typedef struct spr_exchange_plan {
 /* out[P,D,B,T] (float32) = the sum of orders 0..K (RadiosityFast.py:
  * 1037-1145; the histogram energy_exchange_etc): every bin of out is
  * written.  Each order is summed in float64 and rounded to float32; the
- * total is kept as a compensated pair and rounded once, the bits of
+ * total is kept as a compensated pair and rounded once, as by
  * spr_exchange_init, K orders of gather and spread with the total updated
  * every other order (per-pair plans: every order) and spr_exchange_finalize.
+ * The bits are those of that sequence too, save where an order takes one
+ * launch whose waves share a float64 sum and add it up in parts: the diffuse
+ * sums of a diffuse + specular plan, and the group of a grouped plan with
+ * max_groups 1.  Those agree to float32 rounding, and as the launches are
+ * chosen from each order's reached bins, their last bits may depend on reach.
  * reach: every source bin lies below it (T if nothing is known); an order
  * runs on the bins that energy can have reached, reach + k * max_lag of
  * them, the others being 0.  e0dir [P,D,B] and d0 [P] as for

@@ -56,8 +56,9 @@ inline size_t row_lds(const spr_exchange_plan &p, int R) {
 // Phase 1: each wave sums a run of whole groups with about an eighth of the
 // entries, C entries' rows in flight at a time (metadata one entry per lane,
 // broadcast with v_readlane), in float64, and writes each group's sum to
-// LDS as float32 -- the sums the two-pass order stores, bit for bit (of the
-// diffuse + specular plan the diffuse sum is formed in 8 parts).  Phase 2:
+// LDS as float32 -- the sums the two-pass order stores, bit for bit, save
+// those that the waves share (the diffuse sum, a plan's only group): 8 parts
+// in float64, whose sum may round to the other neighbour.  Phase 2:
 // each wave sums the groups times their BRDF rows for its directions, in
 // group order, in float64, and writes the order and the total.
 // Bound by the row reads: an entry's R = 4 loads take 16 clocks of the CU's
@@ -256,7 +257,7 @@ __global__ __launch_bounds__(64 * kRowWaves)
   }
   if (!a.cur && !one) return;  // uniform
   __syncthreads();
-  // the shared sum of a bin, in wave order, as the two-pass order stores it
+  // the shared sum of a bin, in wave order, rounded as a group's sum is
   auto shared_sum = [&](int r) {
     double sum = 0.0;
 #pragma unroll

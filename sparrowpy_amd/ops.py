@@ -1037,8 +1037,10 @@ def source_reach(distance, speed_of_sound, time_resolution):
 def exchange_orders(plan, energy_0_directivity, distance_0, speed_of_sound,
                     time_resolution, n_samples, max_order, reach=None):
     """The sum of orders 0..max_order on a plan (the total of
-    RadiosityFast.py:1037-1145) -> float32 [P,D,B,T]: the bits of stepping
-    an :class:`ExchangeState` and finalizing it.
+    RadiosityFast.py:1037-1145) -> float32 [P,D,B,T]: the total that stepping
+    an :class:`ExchangeState` and finalizing it gives, bit for bit save on
+    diffuse + specular plans and plans with one group per destination, whose
+    sums may be formed in parts (``spr_exchange_orders``).
 
     ``plan`` may be None for max_order < 1.  ``reach``: every source delay
     in bins lies below it (None: nothing is known); orders run only on the

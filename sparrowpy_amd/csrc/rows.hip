@@ -406,9 +406,9 @@ int launch_dp(const spr_exchange_plan &p, const RowArgs &a, hipStream_t s) {
 }  // namespace
 
 // The shape of an order: R bins per lane here, or 0 for the two passes.  The
-// two costs are estimated in ns from what was measured on shoeboxes of 94 to
-// 1,170 patches, 1, 16 and 64 directions, 1 to 8 bands, 100 to 4,000 bins
-// (R = 1 and 8 were tried too: at most 10 % faster anywhere):
+// two costs are estimated in ns, fitted to 881 orders of shoeboxes of 42 to
+// 1,170 patches, 1 to 64 directions, 1 to 8 bands, 100 to 4,000 bins (R = 1
+// and 8 were tried too: at most 10 % faster anywhere):
 // * here a workgroup costs 6 for its start, 0.2 per direction and bin row
 //   written (0.13 with two weights), and per entry 0.06 (R = 4) or 0.048
 //   (R = 2), 1.6 times that with two weights (an eighth of it per wave;
@@ -423,8 +423,11 @@ int launch_dp(const spr_exchange_plan &p, const RowArgs &a, hipStream_t s) {
 //   its row in 900 per entry, at a rate of 0.2 (0.65) per entry;
 // * two passes write and read the group sums, 0.0018 per group and bin, and
 //   take a launch more, 8,000.
-// Over 881 such cases the choice is within 1.2 % of the best one on average
-// (at most 1.3 times slower, 1.7 with two weights) and 1.5 times faster than two passes.
+// Measured on 1,250 others (42 to 1,998 patches, 1, 2, 4, 8, 16, 24, 32 and 64
+// directions, 100 to 3,000 bins) the choice is within 1.1 % of the best one on
+// average with one weight and 0.7 % with two, at most 1.27 times slower
+// (24 and 32 directions, one band: R = 2 would be better), and 1.55 and 1.29
+// times faster than two passes.
 int row_shape(const spr_exchange_plan &p, int64_t T, const OrderSpan &sp) {
   const int64_t DP = spr_padded_directions(p.D);
   if (p.order_shape < 0 || T >= ((int64_t)1 << 29) ||

@@ -112,17 +112,8 @@ class _Finite:
         return bool(self._host[0])
 
 
-def _gradient(adj, grad_hist, record):
-    """dL/dH on the device; asks whether it is finite where the backward
-    orders are to be limited to reached bins."""
-    gH = ops.as_dev(grad_hist, torch.float32).contiguous()
-    if record.reach < adj.T:
-        adj.finite.ask(gH)
-    return gH
-
-
-def _backward(adj, gH, record, segment):
-    """mu_0 = dL/dE_0 (its reached bins) for dL/dH = ``gH``:
+def _backward(adj, grad_hist, record, segment):
+    """mu_0 = dL/dE_0 (its reached bins) for dL/dH = ``grad_hist``:
     ``segment(s, states, reach, lam, mu, mu_even, mu_odd)`` runs the backward
     orders of one checkpoint segment, states[0] being the checkpoint, the
     others scratch."""
@@ -137,6 +128,11 @@ def _backward(adj, gH, record, segment):
 
     def state():
         return torch.empty((P, D, B, T), dtype=torch.float32, device=adj.dev)
+    gH = ops.as_dev(grad_hist, torch.float32).contiguous()
+    reach = record.reach
+    limited = starts and adj.K and reach < T
+    if limited:
+        adj.finite.ask(gH)
     lam = state()
     call("spr_collect_adjoint", adj.R, P, D, B, T, ptr(gH), ptr(adj.rpts),
          ptr(adj._geom["centers"]), ptr(adj.ridx), ptr(adj.rfactor),
@@ -146,8 +142,7 @@ def _backward(adj, gH, record, segment):
         return mu
     mus = (state(), state())                 # even orders, odd orders
     scratch = [state() for _ in range(min(adj.every, adj.K) - 1)]
-    reach = record.reach
-    if reach < T and not adj.finite.answer():
+    if limited and not adj.finite.answer():
         # an infinite or NaN gradient times the zeros of an unreached bin is
         # NaN: whole orders
         for k, x in checkpoints.items():     # (set on their reached bins)
@@ -267,7 +262,6 @@ class ExchangeAdjoint:
             raise RuntimeError("ExchangeAdjoint.backward: no forward record "
                                "(forward() was not called, or its record "
                                "was released)")
-        gH = _gradient(self, grad_hist, record)
         self._set_tables(record.A, record.C)
         P, D, B, T, Vd = self.P, self.D, self.B, self.T, self.plan.Vd
         dev, p, adj = self.dev, self.plan, self.plan.adjoint
@@ -288,7 +282,7 @@ class ExchangeAdjoint:
                  ptr(self.tm), ptr(twa), ptr(twc), ptr(lam), ptr(mu),
                  ptr(mu_even), ptr(mu_odd), ptr(musum), ptr(ga),
                  stream_ptr())
-        mu = _backward(self, gH, record, segment)
+        mu = _backward(self, grad_hist, record, segment)
         gA = torch.zeros((self.NK, B), dtype=torch.float64, device=dev)
         gC = torch.zeros_like(gA)
         call("spr_ds_injection_grad", P, D, B, T, ptr(self.energy0),
@@ -448,7 +442,6 @@ class BRDFExchangeAdjoint:
             raise RuntimeError("BRDFExchangeAdjoint.backward: no forward "
                                "record (forward() was not called, or its "
                                "record was released)")
-        gH = _gradient(self, grad_hist, record)
         self._set_table(record.table)
         P, D, B, T = self.P, self.D, self.B, self.T
         p, dev = self.plan, self.dev
@@ -476,7 +469,7 @@ class BRDFExchangeAdjoint:
                  ptr(self.tgrp), ptr(self.tlag), ptr(self.tscal), ptr(lam),
                  ptr(mu), ptr(mu_even), ptr(mu_odd), ptr(nu), ptr(gg),
                  stream_ptr())
-        mu = _backward(self, gH, record, segment)
+        mu = _backward(self, grad_hist, record, segment)
         gt = torch.zeros((self.NK, D, B), dtype=torch.float64, device=dev)
         call("spr_grouped_key_grad", G, D, B, ptr(p.grp_key), ptr(gg),
              ptr(gt), stream_ptr())

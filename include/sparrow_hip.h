@@ -577,11 +577,6 @@ int spr_exchange_sum(const spr_exchange_plan *plan, int64_t T, int64_t K,
                      double dt, float *out, float *tmp, float *gsum,
                      int32_t *n0, int *err_flag, void *stream);
 
-/* *flag (device or pinned host memory) = 0 if one of x[n] is infinite or NaN,
- * else left as it is.  For the backward orders below: a gradient that is not
- * finite needs whole orders.  No counterpart in the reference. */
-int spr_all_finite(int64_t n, const float *x, int32_t *flag, void *stream);
-
 /* Backward orders k0 + n - 1 .. k0 of the diffuse + specular adjoint:
  * orders k0 + 1 .. k0 + n - 1 are recomputed from states[0] = order k0 into
  * states[1 ..], then per order spr_direction_sum and spr_exchange_adjoint_ds,
@@ -743,6 +738,16 @@ int spr_collect_adjoint(int64_t NR, int64_t P, int64_t D, int64_t B,
                         const double *centers, const int64_t *idx,
                         const double *factor, const double *air, double c,
                         double dt, float *lam, void *stream);
+
+/* The same, and *finite (device or pinned host memory) = 0 if a
+ * value of lam is infinite or NaN, else left as it is: the backward orders
+ * then need reach = T.  No counterpart in the reference. */
+int spr_collect_adjoint_finite(int64_t NR, int64_t P, int64_t D, int64_t B,
+                               int64_t T, const float *grad,
+                               const double *points, const double *centers,
+                               const int64_t *idx, const double *factor,
+                               const double *air, double c, double dt,
+                               float *lam, int32_t *finite, void *stream);
 
 /* musum[P,B,T] = sum over d of mu[P,D,B,T] (float64 sum).
  * Adjoint support; no counterpart in the reference. */

@@ -129,6 +129,8 @@ SYMBOLS = {
                                          _vp]),
     "spr_collect_adjoint": (_int, [_i64, _i64, _i64, _i64, _i64, _vp, _vp,
                                    _vp, _vp, _vp, _vp, _dbl, _dbl, _vp, _vp]),
+    "spr_collect_adjoint_finite": (_int, [_i64] * 5 + [_vp] * 6
+                                   + [_dbl] * 2 + [_vp] * 3),
     "spr_direction_sum": (_int, [_i64, _i64, _i64, _i64, _vp, _vp, _vp]),
     "spr_exchange_adjoint_ds": (_int, [_i64, _i64, _i64, _i64, _i64, _vp, _vp,
                                        _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
@@ -161,7 +163,6 @@ SYMBOLS = {
                                            _vp, _vp, _vp, _vp, _vp]),
     "spr_exchange_sum": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _dbl, _dbl, _vp,
                                 _vp, _vp, _vp, _vp, _vp]),
-    "spr_all_finite": (_int, [_i64, _vp, _vp, _vp]),
     "spr_plan_dense_hash": (_int, [_i64, _i64, _i64, _vp, _vp, _vp, _vp,
                                    _vp]),
     "spr_energy_exchange_groups": (_i64, []),

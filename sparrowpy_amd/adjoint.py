@@ -87,36 +87,32 @@ def _forward(adj):
 
 
 class _Finite:
-    """Whether a device array is finite, asked of the device and answered on
-    the host without waiting for what was enqueued in between."""
+    """A flag that the device clears where a value is not finite, read on the
+    host without waiting for what was enqueued since."""
 
     def __init__(self):
         self._flag = torch.empty(1, dtype=torch.int32, pin_memory=True)
         self._host = self._flag.numpy()
         self._done = torch.cuda.Event()
-        self._asked = False
 
-    def ask(self, x):
-        # (while a graph is captured nothing can be known)
-        self._asked = not torch.cuda.is_current_stream_capturing()
-        if self._asked:
-            self._host[0] = 1
-            call("spr_all_finite", x.numel(), ptr(x), self._flag.data_ptr(),
-                 stream_ptr())
-            self._done.record()
+    def ask(self):
+        """The flag's address, set, for an entry point to clear."""
+        self._host[0] = 1
+        return self._flag.data_ptr()
+
+    def asked(self):
+        self._done.record()
 
     def answer(self):
-        if not self._asked:
-            return False
         self._done.synchronize()
         return bool(self._host[0])
 
 
-def _backward(adj, grad_hist, record, segment):
+def _backward(adj, grad_hist, record, segment, sums):
     """mu_0 = dL/dE_0 (its reached bins) for dL/dH = ``grad_hist``:
     ``segment(s, states, reach, lam, mu, mu_even, mu_odd)`` runs the backward
     orders of one checkpoint segment, states[0] being the checkpoint, the
-    others scratch."""
+    others scratch, and adds to ``sums`` (zeros)."""
     checkpoints = record.checkpoints
     starts = sorted(checkpoints)
     if not adj.plan.Vd:
@@ -129,30 +125,40 @@ def _backward(adj, grad_hist, record, segment):
     def state():
         return torch.empty((P, D, B, T), dtype=torch.float32, device=adj.dev)
     gH = ops.as_dev(grad_hist, torch.float32).contiguous()
-    reach = record.reach
-    limited = starts and adj.K and reach < T
-    if limited:
-        adj.finite.ask(gH)
     lam = state()
-    call("spr_collect_adjoint", adj.R, P, D, B, T, ptr(gH), ptr(adj.rpts),
-         ptr(adj._geom["centers"]), ptr(adj.ridx), ptr(adj.rfactor),
-         ptr(adj.air), adj.c, adj.dt, ptr(lam), stream_ptr())
-    mu = lam                                 # mu_K
+    reach = record.reach
+    # (while a graph is captured the host cannot ask: whole orders)
+    limited = bool(starts and adj.K and reach < T)
+    ask = limited and not torch.cuda.is_current_stream_capturing()
+    call("spr_collect_adjoint_finite", adj.R, P, D, B, T, ptr(gH),
+         ptr(adj.rpts), ptr(adj._geom["centers"]), ptr(adj.ridx),
+         ptr(adj.rfactor), ptr(adj.air), adj.c, adj.dt, ptr(lam),
+         adj.finite.ask() if ask else None, stream_ptr())
+    if ask:
+        adj.finite.asked()
     if not starts or not adj.K:
-        return mu
+        return lam                           # mu_K
     mus = (state(), state())                 # even orders, odd orders
     scratch = [state() for _ in range(min(adj.every, adj.K) - 1)]
-    if limited and not adj.finite.answer():
-        # an infinite or NaN gradient times the zeros of an unreached bin is
-        # NaN: whole orders
-        for k, x in checkpoints.items():     # (set on their reached bins)
-            x[..., min(T, reach + k * adj.plan.limits[0]):] = 0
-        reach = T
-    for s in reversed(starts):
-        n = min(s + adj.every, adj.K) - s
-        segment(s, [checkpoints[s]] + scratch[:n - 1], reach, lam, mu, *mus)
-        mu = mus[s % 2]
-    return mu
+
+    def orders(reach):
+        mu = lam
+        for s in reversed(starts):
+            n = min(s + adj.every, adj.K) - s
+            segment(s, [checkpoints[s]] + scratch[:n - 1], reach, lam, mu,
+                    *mus)
+            mu = mus[s % 2]
+        return mu
+    if ask or not limited:
+        mu = orders(reach)
+        if not ask or adj.finite.answer():
+            return mu
+    # an infinite or NaN lambda times the zeros of an unreached bin is NaN:
+    # whole orders, from checkpoints that were set on their reached bins only
+    for k, x in checkpoints.items():
+        x[..., min(T, reach + k * adj.plan.limits[0]):] = 0
+    sums.zero_()
+    return orders(T)
 
 
 class ExchangeAdjoint:
@@ -282,7 +288,7 @@ class ExchangeAdjoint:
                  ptr(self.tm), ptr(twa), ptr(twc), ptr(lam), ptr(mu),
                  ptr(mu_even), ptr(mu_odd), ptr(musum), ptr(ga),
                  stream_ptr())
-        mu = _backward(self, grad_hist, record, segment)
+        mu = _backward(self, grad_hist, record, segment, ga)
         gA = torch.zeros((self.NK, B), dtype=torch.float64, device=dev)
         gC = torch.zeros_like(gA)
         call("spr_ds_injection_grad", P, D, B, T, ptr(self.energy0),
@@ -469,7 +475,7 @@ class BRDFExchangeAdjoint:
                  ptr(self.tgrp), ptr(self.tlag), ptr(self.tscal), ptr(lam),
                  ptr(mu), ptr(mu_even), ptr(mu_odd), ptr(nu), ptr(gg),
                  stream_ptr())
-        mu = _backward(self, grad_hist, record, segment)
+        mu = _backward(self, grad_hist, record, segment, gg)
         gt = torch.zeros((self.NK, D, B), dtype=torch.float64, device=dev)
         call("spr_grouped_key_grad", G, D, B, ptr(p.grp_key), ptr(gg),
              ptr(gt), stream_ptr())

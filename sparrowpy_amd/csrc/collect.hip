@@ -155,7 +155,8 @@ __global__ __launch_bounds__(256) void collect_adjoint_kernel(
     const float *__restrict__ grad, const double *__restrict__ points,
     const double *__restrict__ centers, const int64_t *__restrict__ idx,
     const double *__restrict__ factor, const double *__restrict__ air,
-    double c, double dt, float *__restrict__ lam) {
+    double c, double dt, float *__restrict__ lam,
+    int32_t *__restrict__ finite) {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= P * B * T) return;
   const int64_t s = q % T, b = (q / T) % B, k = q / (B * T);
@@ -170,7 +171,12 @@ __global__ __launch_bounds__(256) void collect_adjoint_kernel(
     if (t >= T) t -= T;
     const double a = exp(-air[b] * dist);
     float *row = lam + ((k * D + idx[r * P + k]) * B + b) * T;
-    row[s] = (float)((double)row[s] + (g * a) * (double)grad[(r * B + b) * T + t]);
+    const float v =
+        (float)((double)row[s] + (g * a) * (double)grad[(r * B + b) * T + t]);
+    row[s] = v;
+    if (finite && !(fabsf(v) < __builtin_inff()))
+      __hip_atomic_store(finite, 0, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -228,13 +234,11 @@ extern "C" int spr_collect(int64_t NR, int64_t P, int64_t D, int64_t B,
   return SPR_OK;
 }
 
-extern "C" int spr_collect_adjoint(int64_t NR, int64_t P, int64_t D,
-                                   int64_t B, int64_t T, const float *grad,
-                                   const double *points,
-                                   const double *centers, const int64_t *idx,
-                                   const double *factor, const double *air,
-                                   double c, double dt, float *lam,
-                                   void *stream) {
+extern "C" int spr_collect_adjoint_finite(
+    int64_t NR, int64_t P, int64_t D, int64_t B, int64_t T, const float *grad,
+    const double *points, const double *centers, const int64_t *idx,
+    const double *factor, const double *air, double c, double dt, float *lam,
+    int32_t *finite, void *stream) {
   SPR_REQUIRE(NR > 0 && P > 0 && D > 0 && B > 0 && T > 0 && c > 0 && dt > 0,
               "spr_collect_adjoint: bad sizes");
   SPR_REQUIRE(grad && points && centers && idx && factor && air && lam,
@@ -245,7 +249,18 @@ extern "C" int spr_collect_adjoint(int64_t NR, int64_t P, int64_t D,
   hipLaunchKernelGGL(collect_adjoint_kernel,
                      dim3((unsigned)ceil_div(P * B * T, 256)), dim3(256), 0,
                      s, NR, P, D, B, T, grad, points, centers, idx, factor,
-                     air, c, dt, lam);
+                     air, c, dt, lam, finite);
   SPR_LAUNCH_CHECK();
   return SPR_OK;
+}
+
+extern "C" int spr_collect_adjoint(int64_t NR, int64_t P, int64_t D,
+                                   int64_t B, int64_t T, const float *grad,
+                                   const double *points,
+                                   const double *centers, const int64_t *idx,
+                                   const double *factor, const double *air,
+                                   double c, double dt, float *lam,
+                                   void *stream) {
+  return spr_collect_adjoint_finite(NR, P, D, B, T, grad, points, centers, idx,
+                                    factor, air, c, dt, lam, nullptr, stream);
 }

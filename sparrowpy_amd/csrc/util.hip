@@ -1,5 +1,4 @@
 // Error reporting, version, and small shared kernels (scan, fills).
-#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 
@@ -155,31 +154,7 @@ template int fill<int64_t>(int64_t *, int64_t, int64_t, hipStream_t);
 template int fill<int32_t>(int32_t *, int64_t, int32_t, hipStream_t);
 template int fill<uint8_t>(uint8_t *, int64_t, uint8_t, hipStream_t);
 
-namespace {
-__global__ __launch_bounds__(1024) void all_finite_kernel(
-    int64_t n, const float *__restrict__ x, int32_t *__restrict__ flag) {
-  bool finite = true;
-  const int64_t stride = (int64_t)gridDim.x * 1024;
-  for (int64_t k = (int64_t)blockIdx.x * 1024 + threadIdx.x; k < n;
-       k += stride)
-    finite &= fabsf(x[k]) < __builtin_inff();
-  if (!finite)
-    __hip_atomic_store(flag, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-}  // namespace
-
 }  // namespace spr
-
-extern "C" int spr_all_finite(int64_t n, const float *x, int32_t *flag,
-                              void *stream) {
-  SPR_REQUIRE(n >= 0 && x && flag, "spr_all_finite: bad arguments");
-  const int64_t blocks = std::min<int64_t>(spr::ceil_div(n, 4096), 1024);
-  if (!blocks) return SPR_OK;
-  hipLaunchKernelGGL(spr::all_finite_kernel, dim3((unsigned)blocks),
-                     dim3(1024), 0, spr::as_stream(stream), n, x, flag);
-  SPR_LAUNCH_CHECK();
-  return SPR_OK;
-}
 
 extern "C" const char *spr_last_error(void) { return spr::g_last_error; }
 
